@@ -1,7 +1,7 @@
 // Internal (non-ABI) launchers shared between translation units.
 #pragma once
 
-#define OMNI_PA_MERGE_CNT 512            // arrival counters a paged-attention workspace opens with (zero between launches)
+#define OMNI_PA_MERGE_CNT 512            // arrival counters a paged-attention workspace opens with (its owner's launches: zero between them)
 #include <stdint.h>
 
 #include "../../include/omni_talker.h"
@@ -58,7 +58,8 @@ int k_attn_decode_fused(const void* qkv, const void* qnorm_w, const void* knorm_
                         const int32_t* num_live = nullptr /* device: rows >= *num_live write no KV / slot */,
                         const int32_t* rope_delta = nullptr /* device [B]: rotary position = positions[b] + rope_delta[b] */,
                         int rope_rows = 0 /* rows of cos_sin: positions + rope_delta is clamped into the table (0: no clamp) */,
-                        const float* scale_dev = nullptr /* fp8 KV: device {k_scale, v_scale} read at run time instead of the arguments */);
+                        const float* scale_dev = nullptr /* fp8 KV: device {k_scale, v_scale} read at run time instead of the arguments */,
+                        bool ws_counted = false /* the workspace opens with OMNI_PA_MERGE_CNT counters that only these launches write */);
 int k_paged_attn_prefill(const void* q, const void* k_cache, const void* v_cache, const float* k_scales,
                          const float* v_scales, const int32_t* block_table, int bt_stride, const int32_t* req_of_tok,
                          const int32_t* positions, void* out, int T, int q_heads, int kv_heads, int head_dim, int block_size,

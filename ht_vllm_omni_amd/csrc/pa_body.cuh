@@ -26,7 +26,8 @@ struct PAArgs {
     void* k_cache; void* v_cache; float* k_scales; float* v_scales;
     const int32_t* block_table; int bt_stride; const int32_t* seq_lens; const int32_t* req_of_row; int seq_from_pos;
     uint16_t* out; float* partial;
-    unsigned* merge_cnt;           // KV splits merged by the LAST ARRIVER of a (row, virtual kv head): its arrival counters (NULL: debug library, a merge launch)
+    unsigned* merge_cnt;           // KV splits merged by the LAST ARRIVER of a (row, virtual kv head): its arrival counters (NULL: a merge launch)
+    bool ws_counted;               // host: the workspace's owner keeps those counters zero between launches
     int q_heads, kv_heads, bs; float k_scale, v_scale, sm_scale; int nsplit;
     int bs_shift;                  // log2(bs): the paged kernels take power-of-two blocks (vLLM's 8 ... 256) -- token -> (block, offset)
                                    // by shift and mask; a runtime division cost every (token group, batch) ~20 quarter-rate instructions

@@ -10,7 +10,7 @@
 // the sequence length is known: unallocated block-table entries point at the null block).  The
 // G = Hq/Hkv query heads share every K/V load.  Dequant in registers, fp32 scores, online softmax
 // per 8-lane group (no cross-wave traffic in the loop), one LDS combine at the end; optional KV
-// splits merged by the last of them to arrive.  Output = oracle attention_rows (fp32 softmax and PV, one
+// splits merged by the last of them to arrive, or by a launch.  Output = oracle attention_rows (fp32 softmax and PV, one
 // rounding to bf16); the fused prologue = oracle rms_norm / apply_rope / fp8_quant / int8_quant.
 #include "common.cuh"
 #include "kernels.h"
@@ -354,8 +354,7 @@ int k_attn_pair01(const void* qkv, int row1_off, const void* qnorm_w, const void
     return OMNI_OK;
 }
 
-#ifdef OMNI_DEBUG_HOOKS
-// the launch that the merge inside the attention is compared with: one 128-thread block per (row, q-head)
+// KV splits merged by a launch of their own, behind a caller's workspace: one 128-thread block per (row, q-head)
 __global__ __launch_bounds__(128) void paged_attn_merge_kernel(const float* __restrict__ partial,
                                                                uint16_t* __restrict__ out, int nsplit, float v_mul,
                                                                int q_heads, int out_frag, const float* __restrict__ v_mul_dev) {
@@ -368,7 +367,6 @@ __global__ __launch_bounds__(128) void paged_attn_merge_kernel(const float* __re
     const int row = (int)(rh / q_heads), qh = (int)(rh % q_heads);
     out[out_frag ? frag_off(row, qh * 128 + d, q_heads * 128) : rh * 128 + d] = f2bf(L > 0.f ? (A / L) * v_mul : 0.f);
 }
-#endif
 
 static int pick_nsplit(int rows, int kv_heads, int max_seq_len) {
     const int wgs = rows * kv_heads;
@@ -384,7 +382,8 @@ static int pick_nsplit(int rows, int kv_heads, int max_seq_len) {
     return ns < 1 ? 1 : ns;
 }
 
-// workspace = PA_MERGE_CNT arrival counters (zero when handed over; every launch leaves them zero) + the splits' partial records
+// workspace = PA_MERGE_CNT arrival counters + the splits' partial records.  The counters count only where the workspace's owner keeps them zero between
+// launches (PAArgs::ws_counted: a talker's own); of a caller's workspace they are 2 KB that nobody reads
 #define PA_MERGE_CNT OMNI_PA_MERGE_CNT      // kernels.h
 extern "C" int64_t omni_paged_attn_workspace_bytes(int B, int q_heads, int head_dim, int max_seq_len) {
     (void)head_dim;
@@ -392,12 +391,13 @@ extern "C" int64_t omni_paged_attn_workspace_bytes(int B, int q_heads, int head_
     return (int64_t)PA_MERGE_CNT * 4 + (int64_t)B * q_heads * 16 * PA_REC * sizeof(float);
 }
 
-// g_pa_merge_inkernel: the KV splits are merged by whichever of a (row, virtual head)'s workgroups arrives last, which saves a launch and its boundary.
-// Measured per decode step of 28 layers, against a merge launch, both with every record asked for at once (pa_merge_records): 1 row (16 splits) 2.767 -> 2.728
-// ms, 2 rows 2.755 -> 2.738, 16 rows 2.770 -> 2.742, 32 rows 2.808 -> 2.779.  0 (the launch): the debug library's other arm.
-OMNI_KNOB g_pa_int8_max_g = 2, g_pa_tail_chunks = 1, g_pa_merge_inkernel = 1;
+// g_pa_merge_inkernel: -1: the KV splits of a workspace with live counters are merged by whichever of a (row, virtual head)'s workgroups arrives last, which
+// saves a launch and its boundary; a caller's workspace, which may hold anything, takes the merge launch.  Measured per decode step of 28 layers, last
+// arriver against a merge launch, both with every record asked for at once (pa_merge_records): 1 row (16 splits) 2.767 -> 2.728 ms, 2 rows 2.755 -> 2.738,
+// 16 rows 2.770 -> 2.742, 32 rows 2.808 -> 2.779.  0 / 1: always the launch / the last arriver (debug library).
+OMNI_KNOB g_pa_int8_max_g = 2, g_pa_tail_chunks = 1, g_pa_merge_inkernel = -1;
 #ifdef OMNI_DEBUG_HOOKS
-extern "C" void omni_debug_pa_merge(int inkernel) { g_pa_merge_inkernel = inkernel; }      // 1: KV splits merged by their last arriver (A/B arm)
+extern "C" void omni_debug_pa_merge(int inkernel) { g_pa_merge_inkernel = inkernel; }
 extern "C" void omni_debug_int8_max_g(int g) { g_pa_int8_max_g = g; }
 extern "C" void omni_debug_pa_tail(int on) { g_pa_tail_chunks = on; }      // A/B: the tail round as contiguous chunks (PAArgs::tail_chunks)
 #endif
@@ -411,12 +411,13 @@ static int launch_pa(const PAArgs& a_in, int rows, hipStream_t st) {
     const int max_g = (KV == OMNI_KV_INT8) ? g_pa_int8_max_g : 4;
     while (G > max_g && G % 2 == 0) { G /= 2; a.kv_rep *= 2; }
     if (rows * a.kv_heads * a.kv_rep >= 512) a.nsplit = 1;      // the virtual heads already fill the chip: no KV split
-    // the workspace opens with the arrival counters of the in-kernel merge (a split launch has fewer than 512 (row, virtual head) pairs)
+    // (a split launch has fewer than 512 (row, virtual head) pairs)
     float* ws = a.partial;
     a.merge_cnt = nullptr;
     if (ws != nullptr) {
         a.partial = ws + PA_MERGE_CNT;
-        if (a.nsplit > 1 && g_pa_merge_inkernel && rows * a.kv_heads * a.kv_rep <= PA_MERGE_CNT) a.merge_cnt = reinterpret_cast<unsigned*>(ws);
+        const bool inside = g_pa_merge_inkernel < 0 ? a.ws_counted : g_pa_merge_inkernel != 0;
+        if (a.nsplit > 1 && inside && rows * a.kv_heads * a.kv_rep <= PA_MERGE_CNT) a.merge_cnt = reinterpret_cast<unsigned*>(ws);
     }
     dim3 grid(a.kv_heads * a.kv_rep, rows, a.nsplit), block(PA_THREADS);
     const size_t lds = (size_t)PA_LDS_FLOATS(G) * sizeof(float);
@@ -429,14 +430,12 @@ static int launch_pa(const PAArgs& a_in, int rows, hipStream_t st) {
     }
 #undef LAUNCH
     OMNI_CHECK_LAUNCH("omni_paged_attn_decode");
-#ifdef OMNI_DEBUG_HOOKS
     if (a.nsplit > 1 && a.merge_cnt == nullptr) {
         hipLaunchKernelGGL(paged_attn_merge_kernel, dim3(rows * a.q_heads), dim3(128), 0, st, (const float*)a.partial,
                            a.out, a.nsplit, KV == OMNI_KV_FP8 ? a.v_scale : 1.0f, a.q_heads, a.out_frag,
                            KV == OMNI_KV_FP8 ? a.scale_dev : nullptr);
         OMNI_CHECK_LAUNCH("omni_paged_attn_merge");
     }
-#endif
     return OMNI_OK;
 }
 
@@ -490,8 +489,9 @@ int k_attn_decode_fused(const void* qkv, const void* qnorm_w, const void* knorm_
                         const int32_t* block_table, int bt_stride, const int32_t* seq_lens, int64_t* slot_out, void* out,
                         void* workspace, int B, int q_heads, int kv_heads, int head_dim, int block_size, int kv_dtype,
                         float k_scale, float v_scale, float sm_scale, int max_seq_len, int out_frag, int dense_pos,
-                        void* stream, const int32_t* num_live, const int32_t* rope_delta, int rope_rows, const float* scale_dev) {
+                        void* stream, const int32_t* num_live, const int32_t* rope_delta, int rope_rows, const float* scale_dev, bool ws_counted) {
     PAArgs a{};
+    a.ws_counted = ws_counted;
     a.rope_delta = rope_delta;
     a.rope_rows = rope_delta ? rope_rows : 0;
     a.scale_dev = kv_dtype == OMNI_KV_FP8 ? scale_dev : nullptr;

@@ -378,7 +378,7 @@ def test_paged_attn_decode(ops, kv, hq, hkv, split):
 @pytest.mark.parametrize("kv", ["fp8", "bf16", "int8"])
 @pytest.mark.parametrize("hq,hkv", [(16, 8), (16, 2)])
 def test_kv_splits_merged_inside_the_attention_launch_equal_the_merge_launch(ops, kv, hq, hkv):
-    """Both arms of the debug library (the product merges inside the launch): at 1-32 rows the context of a (row, kv head) is split over several workgroups; the LAST of them to arrive merges the splits inside the attention
+    """Both arms of the debug library (a talker merges inside the launch, behind a caller's workspace a merge launch runs): at 1-32 rows the context of a (row, kv head) is split over several workgroups; the LAST of them to arrive merges the splits inside the attention
     launch (arrival counters at the head of the workspace, write-through records).  Same arithmetic in split order: bit-identical to the
     merge launch, whoever arrives last; the counters are zero again after every launch, so one workspace serves call after call."""
     import ctypes as C
@@ -418,13 +418,36 @@ def test_kv_splits_merged_inside_the_attention_launch_equal_the_merge_launch(ops
                 assert int(ws[:512].view(torch.int32).abs().sum()) == 0, "arrival counters left non-zero"
                 res[inkernel] = outs
         finally:
-            lib.omni_debug_pa_merge(1)
+            lib.omni_debug_pa_merge(-1)
     for a, b in zip(res[0], res[1]):
         assert torch.equal(a, b)
     for r, n in enumerate(seq_lens):         # ... and both are the oracle's attention
         kk, vv = pk.gather(bt[r].tolist(), n)
         ref = O.attention_rows(qs[2][r].cpu().view(1, hq, D), kk, vv, torch.tensor([n - 1]), D ** -0.5)
         assert_bf16_close(res[1][2][r].cpu().view(1, hq, D), ref, ulps=1, max_mismatch=0.05, what=f"attn row {r} len {n}")
+
+
+@pytest.mark.parametrize("kv", ["fp8", "bf16", "int8"])
+@pytest.mark.parametrize("B", [1, 5])
+@pytest.mark.parametrize("bits", [0x00000001, 0x7FFFFFFF, -1])
+def test_a_workspace_may_hold_anything(ops, kv, B, bits):
+    """Scratch straight from an allocator (counters of 1, of -1, NaN records): the rows are those of a zero-filled workspace, call after call."""
+    from ht_vllm_omni_amd import _lib as L
+    D, bs, hq, hkv, nb = 128, 16, 16, 8, 130
+    g = torch.Generator().manual_seed(B)
+    pk = _fill_cache(kv, nb, bs, hkv, D, g, 0.5, 2.0)
+    cache = (pk.data.view(torch.uint8) if kv == "fp8" else pk.data).cuda()
+    sc = pk.scales.cuda() if kv == "int8" else (None, None)
+    seq = torch.tensor([2000, 257, 1, 700, 1024][:B], dtype=torch.int32).cuda()
+    bt = torch.arange(1, 126, dtype=torch.int32).repeat(B, 1).cuda()
+    qs = [_rand(g, B, hq * D, scale=1.0).cuda() for _ in range(3)]          # (an output left unwritten holds another query's rows)
+    words = L.load().omni_paged_attn_workspace_bytes(B, hq, D, 2048) // 4
+    got = []
+    for fill in (0, bits):
+        ws = torch.full((words,), fill, dtype=torch.int32, device="cuda").view(torch.float32)
+        got.append([ops.paged_attn_decode(q, cache[0], cache[1], bt, seq, q_heads=hq, kv_heads=hkv, head_dim=D, block_size=bs, kv_dtype=L.KV_CODES[kv], k_scale=0.5,
+                                          v_scale=2.0, k_scales=sc[0], v_scales=sc[1], max_seq_len=2048, workspace=ws).clone() for q in qs])
+    assert all(torch.equal(a, b) and bool(a.isfinite().all()) for a, b in zip(*got))
 
 
 @pytest.mark.parametrize("kv", ["bf16", "fp8", "int8"])

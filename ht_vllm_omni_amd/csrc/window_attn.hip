@@ -230,8 +230,10 @@ __global__ __launch_bounds__(256, 3) void window_prefill_dma_kernel(const WinArg
         for (int s = 0; s < WS; ++s) Q[rg][s] = ld16(a.q + ((size_t)tok * a.heads + head) * dp + 32 * s + 8 * qk);
 #pragma unroll
         for (int d = 0; d < 2 * WS; ++d) O[rg][d] = (f32x4){0.f, 0.f, 0.f, 0.f};
-        m[rg] = a.sink ? a.sink[head] * LA_LOG2E : LA_SENT;
-        l[rg] = a.sink && qk == 0 ? 1.f : 0.f;
+        // a sink of -inf is none: the finite sentinel, against which a tile that holds no key of the row weighs nothing (of +inf: not a number, as its softmax)
+        const float sink = a.sink ? a.sink[head] * LA_LOG2E : -INFINITY;
+        m[rg] = sink < LA_SENT ? LA_SENT : (sink == INFINITY ? NAN : sink);
+        l[rg] = sink < LA_SENT || qk != 0 ? 0.f : 1.f;
     }
     // keys the wave's rows see, the keys every one of them sees (no masks in a tile inside), and the tile's: positions grow along the rows
     const bool any = wave * WR < nrows;

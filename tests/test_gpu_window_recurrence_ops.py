@@ -336,6 +336,27 @@ def test_the_sink_takes_its_share(elem):
     assert abs(float(s.run(0.2, None).float().norm()) / outs[0] - 1) < 1e-3
 
 
+@pytest.mark.parametrize("dim", [64, 96, 128])
+@pytest.mark.parametrize("window", [None, 7, 50])
+def test_a_sink_of_minus_infinity_is_none(dim, window):
+    """... also for rows that see no key of the first tiles their workgroup walks (a window), beside heads whose sinks are numbers."""
+    s = Seqs([33, 129, 300, 16, 90], [33, 128, 100, 16, 1], 6, 2, dim, dim, 0, seed=dim)
+    s.sink[::2] = -float("inf")
+    close(s.run(0.3, window), s.reference(0.3, window), SAFE[0])
+
+
+@pytest.mark.parametrize("dim", [64, 96, 128])
+@pytest.mark.parametrize("window", [None, 40])
+def test_keys_that_are_no_numbers_reach_the_rows_that_see_them(dim, window):
+    """NaN and infinite keys: rows whose window and past do not hold them are untouched; of the others, those with a score of -inf lose the key alone."""
+    s = Seqs([129, 300], [129, 100], 4, 2, dim, dim, 0, seed=dim, sink=False)
+    s.k[0][70, :, 3], s.k[1][230, :, 5], s.k[1][290, 0, 0] = float("nan"), float("inf"), -float("inf")
+    got, ref = s.run(0.3, window).double(), s.reference(0.3, window)
+    assert torch.equal(got.isnan(), ref.isnan()) and bool(ref.isnan().any())
+    ok = ~ref.isnan()
+    close(got.where(ok, torch.zeros(())), ref.where(ok, torch.zeros(())), SAFE[0])
+
+
 @pytest.mark.parametrize("window", [None, 700, 2049])
 def test_splits_and_single_walk_agree(window):
     s = Seqs([2500, 40], [1, 1], 16, 2, 128, 128, 0, seed=4)

@@ -117,17 +117,21 @@ __global__ __launch_bounds__(DR_THREADS) void stream_rows_kernel(const omni_stre
             const int row = a.row_of_tok[t];
             const bool first = t == 0 || a.row_of_tok[t - 1] != row;
             if (first) {
-                const bool zero = a.positions[t] == 0;
-                const float* st = a.state + (size_t)a.state_slot[row] * wp;
-                raw4<float> r[MAXC];
+                if (a.positions[t] == 0) {                 // zeros; the slot of a sequence that begins may not be set yet
 #pragma unroll
-                for (int c = 0; c < MAXC; ++c) r[c].load(st + at(c));
+                    for (int c = 0; c < MAXC; ++c) prev[c][0] = prev[c][1] = prev[c][2] = prev[c][3] = 0.f;
+                } else {
+                    const float* st = a.state + (size_t)a.state_slot[row] * wp;
+                    raw4<float> r[MAXC];
 #pragma unroll
-                for (int c = 0; c < MAXC; ++c) {
-                    r[c].get(prev[c]);
+                    for (int c = 0; c < MAXC; ++c) r[c].load(st + at(c));
 #pragma unroll
-                    for (int e = 0; e < 4; ++e)
-                        if (zero || !in_row(c)) prev[c][e] = 0.f;
+                    for (int c = 0; c < MAXC; ++c) {
+                        r[c].get(prev[c]);
+#pragma unroll
+                        for (int e = 0; e < 4; ++e)
+                            if (!in_row(c)) prev[c][e] = 0.f;
+                    }
                 }
             } else if (i == i0) {
                 if (a.ids) {

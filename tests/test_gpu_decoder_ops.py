@@ -109,6 +109,29 @@ def test_stream_rows_embedding_and_final_norm(elem):
 
 
 @pytest.mark.parametrize("elem", [0, 1])
+@pytest.mark.parametrize("source", ["rows", "ids"])
+@pytest.mark.parametrize("width,T", [(72, 3), (3000, 1030)])
+def test_a_sequence_that_begins_has_no_slot_yet(elem, source, width, T):
+    """At position 0 the shift takes zeros: the row's slot is not looked up (here it lies far outside the states), whatever the row's source and strip."""
+    g, wp, V = gen(T), r32(width), 9
+    new = torch.randn(T, width, generator=g)
+    mu = torch.rand(width, generator=g).to(ELEMS[elem])
+    ids = torch.randint(0, V, (T,), generator=g).to(torch.int32)
+    table = torch.randn(V, width, generator=g).to(ELEMS[elem])
+    src = dict(x_in=dev(padc(new, wp))) if source == "rows" else dict(ids=dev(ids), table=dev(padc(table, wp)), vocab=V)
+    if source == "ids":
+        new = table[ids.long()]
+    cut = T // 2 + 1                                                                  # two sequences begin in this batch
+    row = (torch.arange(T) >= cut).to(torch.int32)
+    pos = torch.cat([torch.arange(cut), torch.arange(T - cut)]).to(torch.int32)
+    h = torch.zeros(T, wp, dtype=ELEMS[elem], device="cuda")
+    run_struct("omni_stream_rows_run", L.StreamRows(), **src, mu=dev(padc(mu, wp)), state=torch.zeros(1, wp, device="cuda"), state_slot=torch.full((2,), 1 << 24, dtype=torch.int32, device="cuda"),
+               row_of_tok=dev(row), positions=dev(pos), h_out=h, rows=T, width=width, wp=wp, elem=elem)
+    ref = torch.cat([D.token_shift(new[:cut].double(), mu.double()), D.token_shift(new[cut:].double(), mu.double())])
+    close(h[:, :width], ref, RTOL[elem])
+
+
+@pytest.mark.parametrize("elem", [0, 1])
 @pytest.mark.parametrize("q_rank,kv_rank,heads,gated", [(8, 8, 1, True), (48, 56, 3, False), (1500, 500, 33, True), (160, 264, 20, False)])
 def test_latent_write(elem, q_rank, kv_rank, heads, gated):
     g, T, bs, width = gen(q_rank), 9, 16, 72

@@ -38,7 +38,7 @@ typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
 typedef __attribute__((address_space(3))) void lds_void_t;
 
 struct TileArgs {
-    const uint16_t* x; int64_t x_rows; int ldx;
+    const uint16_t* x; int64_t x_rows; int ldx, x_bytes;      // x_bytes: what the descriptor of x covers
     int seg_len, seg_rows, row_off;
     const uint16_t* W; const float* bias; const float* scale;
     const float* resid; int ldr;
@@ -312,7 +312,7 @@ __global__ __launch_bounds__(TG_THREADS) void gemm_tile_kernel(const TileArgs a_
     const int nsteps = a.K >> 5;                                              // 32-deep slices
 
     const __amdgpu_buffer_rsrc_t rw = __builtin_amdgcn_make_buffer_rsrc((void*)a.W, 0, (int)((size_t)a.N * a.K * 2), 0x00020000);
-    const __amdgpu_buffer_rsrc_t rx = __builtin_amdgcn_make_buffer_rsrc((void*)a.x, 0, (int)((a.x_rows * a.ldx - x_skip) * 2), 0x00020000);
+    const __amdgpu_buffer_rsrc_t rx = __builtin_amdgcn_make_buffer_rsrc((void*)a.x, 0, a.x_bytes - (int)(x_skip * 2), 0x00020000);
 
     // ---- staging.  Slice image: W tile f at f KB, x tile g at (NTILES + g) KB.  Wave w issues W tiles w + 8 i (i < NLW; a wave
     // without an i-th tile loads zeros into a spare KB so that every wave has the same count in flight) and x tiles w + 8 i.
@@ -494,7 +494,7 @@ __global__ __launch_bounds__(TG_THREADS) void gemm_tile_pp_kernel(const TileArgs
     }
     const int nkt = (nsteps + 1) >> 1;
     const __amdgpu_buffer_rsrc_t rw = __builtin_amdgcn_make_buffer_rsrc((void*)a.W, 0, (int)((size_t)a.N * a.K * 2), 0x00020000);
-    const __amdgpu_buffer_rsrc_t rx = __builtin_amdgcn_make_buffer_rsrc((void*)a.x, 0, (int)(a.x_rows * a.ldx * 2), 0x00020000);
+    const __amdgpu_buffer_rsrc_t rx = __builtin_amdgcn_make_buffer_rsrc((void*)a.x, 0, a.x_bytes, 0x00020000);
 
     // staging: piece e (0 / 1) of a half-tile = fragment f = wave + 8 e of its 16 = (slot t = f >> 1, k-step f & 1).  Slot t of an x half is
     // the t-th m-tile of [group 0's half | group 1's half]; slot t of a W half is n-tile 4 (t >> 1) + (t & 1) (+ 2 in the high half).
@@ -740,7 +740,7 @@ __global__ __launch_bounds__(WAVES * 64, 2) void gemm_mid_kernel(const TileArgs 
     // per-lane constant (out of the descriptor, i.e. zeros, for rows that are not there) plus the step's scalar offset; the pieces behind the last
     // step fetch the first one's bytes again, for the count: nothing reads them.
     const __amdgpu_buffer_rsrc_t rw = __builtin_amdgcn_make_buffer_rsrc((void*)a.W, 0, (int)((size_t)a.N * a.K * 2), 0x00020000);
-    const __amdgpu_buffer_rsrc_t rx = __builtin_amdgcn_make_buffer_rsrc((void*)a.x, 0, (int)((a.x_rows * a.ldx - x_skip) * 2), 0x00020000);
+    const __amdgpu_buffer_rsrc_t rx = __builtin_amdgcn_make_buffer_rsrc((void*)a.x, 0, a.x_bytes - (int)(x_skip * 2), 0x00020000);
     const int ks = wave & 1;
     unsigned wofs[G::PW], xofs[G::PX];
     int xrow[G::PX];
@@ -975,6 +975,8 @@ extern "C" int omni_gemm_tile(const omni_tile_gemm* g, void* stream) {
                                    (g->out_group_cols == 0 || (!g->out2 && !g->resid))),
                    "omni_gemm_tile: group columns leave the rows of x / out");
     a.gx_cols = groups > 1 ? g->x_group_cols : 0; a.gout_cols = groups > 1 ? g->out_group_cols : 0;
+    // up to the end of the last row's last column: rows of a wider array need not be followed by anything
+    a.x_bytes = (int)(((g->x_rows - 1) * g->ldx + (groups - 1) * a.gx_cols + seg_len) * 2);
     hipStream_t st = (hipStream_t)stream;
     const int N = g->N;
     OMNI_CHECK_ARG(g->k_splits >= 0 && g->k_splits <= 4 && (g->k_splits <= 1 || (tile_epi(a) == EPI_ACT && g->act == OMNI_TILE_ACT_NONE && !g->out && groups == 1 && g->k_splits <= g->K / 32 &&

@@ -67,6 +67,19 @@ def test_mid_size_tiles_at_their_edges(M, N, K, taps, dil):
         assert torch.equal(out[:M], ref) and bool((out[M:] == 7.0).all()), hint
 
 
+@pytest.mark.parametrize("M,K,splits", [(33, 32, 1), (70, 96, 3), (129, 160, 4), (65, 64, 1)])
+def test_rows_that_end_an_array(M, K, splits):
+    """x is the last columns of a wider array and a run of K steps is a single one: what a tile fetches ahead of its last step lies past the last row."""
+    ops, L, frag_shuffle, _ = _ops()
+    g = torch.Generator().manual_seed(M)
+    wide, w = torch.randn(M, K + 64, generator=g).to(BF16), (torch.randn(48, K, generator=g) * 0.05).to(BF16)
+    x = wide.cuda()[:, 64:]
+    ref, mag = wide[:, 64:].double() @ w.double().T, wide[:, 64:].double().abs() @ w.double().abs().T
+    for hint in (0, 2, 8, 9, 10, 11, 12, 13) + ((1,) if splits == 1 else ()):
+        y = ops.gemm_tile(x, frag_shuffle(w).cuda(), want="f", splits=splits, tile_hint=hint)
+        assert bool((((y.double().sum(0) if splits > 1 else y.double()).cpu() - ref).abs() <= mag * 2.0 ** -18).all()), hint
+
+
 @pytest.mark.parametrize("M,N,K", [(70, 32, 256), (490, 2048, 9216), (257, 1040, 800), (1030, 512, 2080)])
 def test_partial_sums_add_up(M, N, K):
     """splits: the partial sums of runs of K steps, on the dispatch rule's tile and on both kernels by hint; their fp32 sum against fp64 with the

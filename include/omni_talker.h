@@ -54,8 +54,10 @@ extern "C" {
                                  * finished act columns, so any number of tiles per workgroup divides the chip evenly */
 
 const char* omni_last_error(void);
-int omni_abi_version(void);   /* 7: omni_tile_gemm activations RELU2, SILU_SIGMOID, GELU_MUL (6: column groups, xIELU; 5: omni_ar_peers.tile_flags, omni_talker_set_chains
-                                 modes 2 / 3, a zero-filled attention workspace) */
+int omni_abi_version(void);   /* 8: omni_tile_gemm.k_splits / slab_stride, omni_gemm_tile_splits, omni_res_unit.row_tiles, omni_window_attn.key_base / k_row /
+                                 v_row / head_gate, omni_latent_gather; an attention workspace may hold anything (7: omni_tile_gemm activations RELU2, SILU_SIGMOID,
+                                 GELU_MUL; 6: column groups, xIELU; 5: omni_ar_peers.tile_flags, omni_talker_set_chains modes 2 / 3).  A library reads whole structs of
+                                 its own version: a caller compares this with the header it was built against */
 
 /* ------------------------------------------------------------------ per-op entry points */
 

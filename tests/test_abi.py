@@ -27,8 +27,25 @@ def test_header_symbols_exported_and_bound():
     for n in names:
         assert hasattr(lib, n), f"{n} declared in include/*.h but not exported"
         assert n in _lib.SIGNATURES, f"{n} has no ctypes signature"
-    assert lib.omni_abi_version() == 7
+    assert lib.omni_abi_version() == 8
     assert lib.omni_last_error() is not None
+
+
+def test_structs_of_this_abi_version(tmp_path):
+    """Callers allocate these structs and the library reads all of them: one that grows takes a new version number, then its size here."""
+    from ht_vllm_omni_amd import _lib
+    sizes = {"omni_tile_gemm": 272, "omni_res_unit": 104, "omni_window_attn": 192, "omni_latent_attn": 128, "omni_latent_write": 184, "omni_stream_rows": 184,
+             "omni_qkv_write": 168, "omni_gated_norm": 80, "omni_decay_rec": 168, "omni_row_table": 24, "omni_talker_desc": 344, "omni_step_io": 224,
+             "omni_layer_weights": 128, "omni_ar_peers": 216, "omni_row_sampling": 48}
+    src = tmp_path / "sz.c"
+    src.write_text("#include <stdio.h>\n" + "".join(f'#include "{ROOT}/include/{h}.h"\n' for h in ("omni_talker", "omni_codec", "omni_decoder"))
+                   + "int main(){%s return 0;}\n" % "".join(f'printf("%zu\\n",sizeof({n}));' for n in sizes))
+    exe = tmp_path / "sz"
+    subprocess.check_call(["gcc", str(src), "-o", str(exe)])
+    assert dict(zip(sizes, (int(x) for x in subprocess.check_output([str(exe)]).split()))) == sizes
+    assert _lib.load().omni_abi_version() == _lib.load_decoder().omni_abi_version() == 8
+    for c, t in (("omni_window_attn", _lib.WindowAttn), ("omni_res_unit", _lib.ResUnit), ("omni_tile_gemm", _lib.TileGemm)):
+        assert C.sizeof(t) == sizes[c]
 
 
 def test_struct_layout_matches_c(tmp_path):

@@ -103,6 +103,23 @@ def test_portions_over_expanded_keys_and_values(dims, monkeypatch):
     assert True in said and False in said
 
 
+@pytest.mark.parametrize("n", [1281, 3900])
+def test_a_prompt_does_not_depend_on_the_batches_before_it(n):
+    """Products that leave as partial sums over K leave as many before and after a larger batch has grown the scratch: the same bits."""
+    sizes = dict(heads=4, dim=64, vdim=64, kv_rank=64, q_rank=96, ff=9216)
+    d = dims_from_config(config([layer(**sizes)], width=2048, vocab=90), 8300)
+    eng = DecoderEngine(d, make_decoder_weights(d, seed=4, device="cuda"), num_blocks=600, max_batch=2)
+    eng.block_table[0, :514] = torch.arange(1, 515, dtype=torch.int32)
+    eng.state_slot[0] = 1
+
+    def run(T):
+        b = eng.make_batch(torch.tensor(tokens(T, d.vocab, T)), np.zeros(T, np.int32), np.arange(T), [T])
+        return eng.forward(b, sel=torch.arange(T - 64, T, dtype=torch.int32, device="cuda")).clone()
+    before = run(n)
+    run(8192)
+    assert torch.equal(run(n), before)
+
+
 # ---------------------------------------------------------------- decoding and portions
 @pytest.mark.parametrize("dtype", DTYPES)
 @pytest.mark.parametrize("name", ["mixed", "narrow", "behind", "k_mixed", "k_narrow", "k_state"])

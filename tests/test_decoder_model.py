@@ -1,16 +1,18 @@
 """Decoder-only language models, everything that needs no GPU: configuration and registry, checkpoint checks, open prompts in the scheduler,
 state slots, attention work items, and the oracle's mechanisms against loops over single numbers."""
 import math
+from types import SimpleNamespace
 
 import pytest
 import torch
 
+from ht_vllm_omni_amd import _lib as L
 from ht_vllm_omni_amd import models
 from ht_vllm_omni_amd.checkpoint import load_decoder_checkpoint
 from ht_vllm_omni_amd.config import TalkerDims
 from ht_vllm_omni_amd.decoder_config import dims_from_config, tensor_shapes
-from ht_vllm_omni_amd.decoder_mixers import (LATENT_WIDTHS, attention_tiles, cache_row_widths, cache_traffic, latent_width, pad_head_cols, pad_head_rows, pad_heads,
-                                             recurrence_chunks, recurrence_segments, state_bytes)
+from ht_vllm_omni_amd.decoder_mixers import (LATENT_WIDTHS, LatentMixer, attention_tiles, cache_row_widths, cache_traffic, cached_rows, first_rows, latent_width,
+                                             pad_head_cols, pad_head_rows, pad_heads, recurrence_chunks, recurrence_segments, state_bytes)
 from ht_vllm_omni_amd.payloads import OmniModelRunnerOutput, SamplingParams
 from ht_vllm_omni_amd.sched import SlotPool
 from ht_vllm_omni_amd.scheduler import MI355XARScheduler, Request
@@ -122,6 +124,38 @@ def test_state_slots_are_unique_and_come_back():
     p.release("b")
     p.release("b")
     assert p.acquire("d") == got[1]
+
+
+@pytest.mark.parametrize("segs", [[(1, 0, 0)], [(16, 16, 3), (5, 0, 0), (1, 1000, 2)], [(33, 95, 1), (128, 0, 7)]])
+def test_cached_rows_name_every_key_of_every_segment(segs):
+    """... once, in order, at the row where first_rows says the segment's keys begin."""
+    want, at, first = [], 0, {}
+    for n, p, r in segs:
+        first[r] = at
+        want += [(r, k, at + k) for k in range(p + n)]
+        at += p + n
+    got = []
+    for r, key, n, to in cached_rows(segs).tolist():
+        assert 0 < n <= L.GATHER_ROWS and key % L.GATHER_ROWS == 0
+        got += [(r, key + i, to + i) for i in range(n)]
+    assert got == want
+    starts = first_rows(segs)
+    assert len(starts) == max(first) + 1 and all(int(starts[r, 0]) == a for r, a in first.items())
+
+
+def test_items_of_a_batch_are_those_its_mixers_will_walk():
+    """The lists of expanded keys are asked for where a latent mixer expands the batch, and its tiles of latents where not: never both, and of none that is
+    too large, or too small, to be expanded."""
+    m = LatentMixer.__new__(LatentMixer)
+    m.spec, m.rp, m.dp, m.vp, m.ukv = SimpleNamespace(heads=16), 512, 128, 128, object()
+    m.tiles, m.head_tiles = ("tiles", 16, 128), ("tiles", 1, 128)
+    m.work = (m.tiles,)
+    batch = lambda segs, n_decode=0: SimpleNamespace(T=n_decode + sum(n for n, _ in segs), n_decode=n_decode, segs=segs)  # noqa: E731
+    assert m.work_for(batch([(2000, 0)])) == (m.head_tiles, ("cached_rows",), ("first_rows",))
+    assert m.work_for(batch([(251, 512)] * 2, 48)) == (m.head_tiles, ("cached_rows",), ("first_rows",))
+    assert m.work_for(batch([(32, 8000)] * 60)) == m.work_for(batch([(3, 900)], 2)) == m.work_for(batch([], 3)) == (m.tiles,)
+    m.ukv = None
+    assert m.work_for(batch([(2000, 0)])) == (m.tiles,)
 
 
 def test_attention_tiles_cover_every_row_once_and_never_straddle_sequences():

@@ -103,6 +103,18 @@ def test_portions_over_expanded_keys_and_values(dims, monkeypatch):
     assert True in said and False in said
 
 
+@pytest.mark.parametrize("name", ["wide", "k_mixed"])
+def test_segments_of_no_tokens(name):
+    """... in front, between and behind the others: the batch without them."""
+    d, w, _ = model(name, seed=6)
+    eng = DecoderEngine(d, w, num_blocks=40, max_batch=3, block_size=16)
+    eng.block_table[:3, :8] = torch.arange(1, 25, dtype=torch.int32).view(3, 8)
+    eng.state_slot[:] = torch.arange(1, 4)
+    ids, row, pos = torch.tensor(tokens(170, d.vocab)), np.repeat([0, 2], [100, 70]), np.concatenate([np.arange(100), np.arange(70)])
+    want = eng.forward(eng.make_batch(ids, row, pos, [100, 70])).clone()
+    assert torch.equal(eng.forward(eng.make_batch(ids, row, pos, [0, 100, 0, 70, 0])), want)
+
+
 @pytest.mark.parametrize("n", [1281, 3900])
 def test_a_prompt_does_not_depend_on_the_batches_before_it(n):
     """Products that leave as partial sums over K leave as many before and after a larger batch has grown the scratch: the same bits."""

@@ -115,6 +115,23 @@ def test_segments_of_no_tokens(name):
     assert torch.equal(eng.forward(eng.make_batch(ids, row, pos, [0, 100, 0, 70, 0])), want)
 
 
+def test_the_memory_probe_holds_the_scratch_of_every_step():
+    """Behind profile_run no step allocates for its expanded keys: portions of all rows behind as much as the model's length lets them have."""
+    sizes = dict(heads=16, dim=128, vdim=128, kv_rank=512, q_rank=64, ff=64)
+    d = dims_from_config(config([layer(**sizes)], width=128, vocab=90), 3000)
+    eng = DecoderEngine(d, make_decoder_weights(d, seed=7, device="cuda"), num_blocks=16, max_batch=4)
+    eng.profile_run(64, 4)
+    eng.resize_kv_cache(760)
+    eng.block_table[:] = torch.arange(4 * 188, dtype=torch.int32).view(4, 188) + 1
+    held = {k: (t.data_ptr(), t.numel()) for k, t in eng._grown.items()}
+    assert held["latent_kv"][1] >= 4 * 3000 * 16 * 256
+    row, pos = np.repeat(np.arange(4), 100), np.tile(np.arange(2900, 3000), 4)
+    b = eng.make_batch(torch.zeros(400, dtype=torch.int32), row, pos, [100] * 4)
+    assert eng.layer_w[0].mixer.expands(b)
+    eng.forward(b)
+    assert held == {k: (t.data_ptr(), t.numel()) for k, t in eng._grown.items()}
+
+
 @pytest.mark.parametrize("n", [1281, 3900])
 def test_a_prompt_does_not_depend_on_the_batches_before_it(n):
     """Products that leave as partial sums over K leave as many before and after a larger batch has grown the scratch: the same bits."""

@@ -859,7 +859,7 @@ static int launch_mid(TileArgs a, hipStream_t st, int groups) {
     return OMNI_OK;
 }
 
-// waves, waves along n, n-tiles x m-tiles per wave, ring: 32 x 32 | 32 x 64 | 64 x 64 | 128 x 64 (rows x columns; two workgroups fit a CU) |
+// waves, waves along n, n-tiles x m-tiles per wave, ring: 32 x 32 | 32 x 64 | 64 x 64 | 64 x 128 (rows x columns; two workgroups fit a CU) |
 // 128 x 128 | 256 x 128 | 128 x 256 (one)
 #define MID_LIST(X) X(0, 4, 2, 1, 1, 9) X(1, 4, 2, 2, 1, 6) X(2, 4, 2, 2, 2, 4) X(3, 8, 4, 2, 2, 3) X(4, 8, 4, 2, 4, 4) X(5, 8, 2, 4, 4, 3) X(6, 8, 4, 4, 4, 3)
 template <bool GU8, bool WINDOW>
@@ -880,19 +880,26 @@ static int launch_mid_of(int geom, const TileArgs& a, hipStream_t st, int groups
 // Numbers: ns, from sweeps of M 66 ... 6000 over the weight shapes of the 1024- and 2048-wide models and of the vocoder's convolutions at 12 ... 325
 // frames, weights cold.  With this rule against the two tiles there were (the 256 x 256 family, and 64 x 128 below 96 of those): 490 x 9216 x 2048
 // 45 -> 33 us, 490 x 2048 x 2048 18.3 -> 11.5, 1450 x 2048 x 9216 101 -> 67, 800 x 5120 x 2048 40 -> 31, 50 x 1024 x 3072 20.9 -> 8.8.
+// (The 64 x 128 tile's numbers are from a sweep of its own, M 50 ... 1800, over all tiles' times: 390 x 9216 x 2048 31.5 -> 24.5, 1100 x 1024 x 4608
+// 32.4 -> 23.0, 560 x 2048 x 2048 16.0 -> 12.4 against its size taken for 128 x 64; what the rule picks is 2.2 % behind the best tile on average, from 3.9.)
 enum { KIND_MID, KIND_PP, KIND_LARGE };
 struct TileChoice {
     int kind, geom, bm, bn;          // geom: MID_LIST index, or rows of the two-group / lockstep tile
     int round1, slice1, round2, slice2;      // alone on a CU; two per CU (0: one fits)
+    bool whole;                      // two per CU: a third waits for the round
 };
+#define MID_SIZE_CASE(I, A, B, C, D, E) if (I == i) return rows ? MidGeom<A, B, C, D, E>::BM : MidGeom<A, B, C, D, E>::BN;
+static constexpr int mid_size(int i, bool rows) { MID_LIST(MID_SIZE_CASE) return 0; }
+#undef MID_SIZE_CASE
+#define MID(I) KIND_MID, I, mid_size(I, true), mid_size(I, false)
 static const TileChoice TILE_CHOICES[] = {
-    {KIND_MID, 0, 32, 32, 1300, 140, 1900, 230},      {KIND_MID, 1, 32, 64, 1300, 175, 2200, 335},    {KIND_MID, 2, 64, 64, 1400, 270, 2400, 440},
-    {KIND_MID, 3, 128, 64, 1700, 440, 2600, 540},     {KIND_MID, 4, 128, 128, 2200, 500, 0, 0},       {KIND_MID, 5, 256, 128, 4000, 830, 0, 0},
-    {KIND_MID, 6, 128, 256, 4200, 900, 0, 0},         {KIND_PP, 192, 192, 256, 5000, 1130, 0, 0},     {KIND_PP, 224, 224, 256, 5500, 1200, 0, 0},
-    {KIND_PP, 256, 256, 256, 6000, 1280, 0, 0},       {KIND_LARGE, 192, 192, 256, 6000, 1150, 0, 0},  {KIND_LARGE, 224, 224, 256, 6500, 1250, 0, 0},
-    {KIND_LARGE, 256, 256, 256, 7500, 1350, 0, 0},    {KIND_LARGE, 0, 256, 192, 6000, 1180, 0, 0},    {KIND_LARGE, 0, 512, 128, 7500, 1650, 0, 0},
-    {KIND_LARGE, 0, 512, 96, 7000, 1500, 0, 0},
+    {MID(0), 1300, 140, 1900, 230, false}, {MID(1), 1300, 175, 2200, 335, false}, {MID(2), 1400, 270, 2400, 440, false}, {MID(3), 1600, 480, 3000, 600, true},
+    {MID(4), 2200, 500},                   {MID(5), 4000, 830},                   {MID(6), 4200, 900},
+    {KIND_PP, 192, 192, 256, 5000, 1130},    {KIND_PP, 224, 224, 256, 5500, 1200},    {KIND_PP, 256, 256, 256, 6000, 1280},
+    {KIND_LARGE, 192, 192, 256, 6000, 1150}, {KIND_LARGE, 224, 224, 256, 6500, 1250}, {KIND_LARGE, 256, 256, 256, 7500, 1350},
+    {KIND_LARGE, 0, 256, 192, 6000, 1180},   {KIND_LARGE, 0, 512, 128, 7500, 1650},   {KIND_LARGE, 0, 512, 96, 7000, 1500},
 };
+#undef MID
 static const TileChoice& pick_tile(int M, int N, int K, int groups, int splits, bool plain, bool gu8, long long* ns) {
     const TileChoice* best = nullptr;
     long long least = 0;
@@ -903,8 +910,8 @@ static const TileChoice& pick_tile(int M, int N, int K, int groups, int splits, 
         if (c.kind == KIND_LARGE && (c.bn != large_bn || (plain && c.bn == 256) || splits > 1)) continue;
         const long long tiles = (long long)((M + c.bm - 1) / c.bm) * ((N + c.bn - 1) / c.bn) * groups * splits;
         long long t;
-        // (a CU that gets a third small tile while the first two run does not wait for a round of two; the 128-row tile's measured like whole rounds)
-        if (c.slice2 && tiles > 256) t = (c.round2 + slices * c.slice2) * (c.bm < 128 ? (tiles + 255) / 256 : 2 * ((tiles + 511) / 512)) / 2;
+        // (a CU that gets a third small tile while the first two run does not wait for a round of two; the 64 x 128 tile measured like whole rounds)
+        if (c.slice2 && tiles > 256) t = (c.round2 + slices * c.slice2) * (c.whole ? 2 * ((tiles + 511) / 512) : (tiles + 255) / 256) / 2;
         else t = (c.round1 + slices * c.slice1) * ((tiles + 255) / 256);
         if (!best || t < least) { best = &c; least = t; }
     }

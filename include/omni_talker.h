@@ -175,7 +175,7 @@ typedef struct omni_tile_gemm {
     void* out; int ldo;
     void* out2; int ldo2; const float* snake_alpha; const float* snake_inv_beta;
     int M, N, K;
-    int tile_hint;   /* 0: automatic; 1: the large output tiles (256 x 256 ...); 2: the tile of 128 rows x 64 columns;
+    int tile_hint;   /* 0: automatic; 1: the large output tiles (256 x 256 ...); 2: the tile of 64 rows x 128 columns;
                         3 / 4: 256 columns x 224 / 192 rows (N % 256 == 0); 5 / 6 / 7: the two-group form of the 256-column tile at
                         256 / 224 / 192 rows (plain GEMMs only); 8 ... 13: 32 x 32, 32 x 64, 64 x 64, 128 x 128, 256 x 128, 128 x 256
                         rows x columns.  Same results whatever the tile */

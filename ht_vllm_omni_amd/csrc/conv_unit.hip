@@ -57,8 +57,8 @@ struct RuGeom {
     static_assert(TT_BYTES <= WIN_BYTES && LDS_BYTES <= 160 * 1024, "LDS budget");
 };
 
-// <C, m tiles per wave, ring depth>.  Up to two m tiles a wave's registers and a block's LDS leave room for two workgroups per CU, whose memory phases
-// (window load, stream read / write) overlap each other's MFMA phase.
+// <C, m tiles per wave, ring depth>.  With one m tile a wave a block takes 74 KB of LDS: two workgroups fit a CU, and their memory phases (window load, stream
+// read / write) overlap each other's MFMA phase.  Two tiles take 87 KB (C = 96) or 108 KB (C = 192), four 139 or 158 KB: one workgroup per CU.
 template <int C, int WM_, int NBUF_>
 __global__ __launch_bounds__(RU_THREADS, (RuGeom<C, WM_, NBUF_>::LDS_BYTES <= 80 * 1024 ? 4 : 2)) void res_unit_kernel(const ResUnitArgs a) {
     using G = RuGeom<C, WM_, NBUF_>;
@@ -283,15 +283,17 @@ static int launch_unit(const ResUnitArgs& a, hipStream_t st) {
 
 #define RU_MAX_TILES 4
 // m tiles per wave: the fewest rounds of the chip's 256 CUs, at what a round costs.  A block's weights, latencies and epilogue cost as much as 1.6 (C = 192)
-// or 1.3 (C = 96) of its m tiles, whatever their number.  Measured, us, 1 / 2 / 3 / 4 tiles: C = 192, 2560 rows 18 / 23 / 31 / 38, 32000 rows
-// (125 blocks of 256: half the chip) 38 / 33 / 39 / 44, 40960 rows 55 / 54 / 41 / 47, 64000 rows 69 / 61 / 73 / 54; C = 96, 7680 rows 12 / 16 / 22 / 27,
-// 96000 rows 36 / 40 / 34 / 35, 288000 rows 84 / 93 / 88 / 101.
+// or 1.3 (C = 96) of its m tiles, whatever their number; a round of blocks of one tile, two to a CU, 28 (C = 96) or 42 (C = 192) in the same units of a tenth
+// tile, where one to a CU is 23 or 26.  Measured, us, 1 / 2 / 3 / 4 tiles: C = 192, 2560 rows 18 / 23 / 31 / 38, 32000 rows (125 blocks of 256: half the chip)
+// 38 / 33 / 39 / 44, 40960 rows 57 / 53 / 41 / 46, 64000 rows 70 / 59 / 73 / 54; C = 96, 7680 rows 12 / 16 / 22 / 27, 96000 rows 35 / 40 / 34 / 35,
+// 134400 rows 49 / 57 / 55 / 65, 288000 rows 84 / 93 / 89 / 102.  Over 4 ... 325 frames the choice is 1.5 % (C = 96) and 0.1 % (C = 192) behind the best.
 static int ru_row_tiles(int C, int T) {
-    const int rows = C == 96 ? 128 : 64, fixed = C == 96 ? 13 : 16;
+    const int rows = C == 96 ? 128 : 64, fixed = C == 96 ? 13 : 16, pair = C == 96 ? 28 : 42;
     int best = 1;
     int64_t cost = INT64_MAX;
     for (int wm = 1; wm <= RU_MAX_TILES; ++wm) {
-        const int64_t blocks = ((int64_t)T + rows * wm - 1) / (rows * wm), c = (blocks + 255) / 256 * (fixed + 10 * wm);
+        const int64_t blocks = ((int64_t)T + rows * wm - 1) / (rows * wm);
+        const int64_t c = wm == 1 && blocks > 256 ? (blocks + 511) / 512 * pair : (blocks + 255) / 256 * (fixed + 10 * wm);
         if (c < cost) { cost = c; best = wm; }
     }
     return best;

@@ -314,7 +314,9 @@ __global__ __launch_bounds__(256, 3) void window_prefill_dma_kernel(const WinArg
 #pragma unroll
             for (int j = 1; j < 8; ++j) mx = fmaxf(mx, p[j]);
             mx = xor32_max(xor16_max(mx)) * a.qs;
-            // the maximum follows once a row has outgrown it by 2^LAZY: weights up to that size lose nothing in fp32, nor in three terms
+            // the maximum follows once a row has outgrown it by 2^LAZY (the conditional rescaling of FlashAttention-4): weights up to that size lose nothing
+            // in fp32, nor in three terms.  The 16 rows of a group move together, so a row's last bits depend on the rows it shares a group with,
+            // that is on where its portion was cut
             if (__any(mx > m[rg] + LAZY)) {
                 const float mn = fmaxf(m[rg], mx), alpha = exp2_w(m[rg] - mn);      // (never below the finite sentinel: 1, harmless, where l = 0, O = 0)
                 m[rg] = mn;

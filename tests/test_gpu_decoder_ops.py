@@ -7,6 +7,7 @@ import torch
 from ht_vllm_omni_amd import _lib as L
 from ht_vllm_omni_amd import ops
 from ht_vllm_omni_amd.decoder_engine import attention_tiles, r32
+from ht_vllm_omni_amd.decoder_mixers import cached_rows
 from ht_vllm_omni_amd.engine import frag_shuffle, frag_unshuffle
 from oracle import decoder_oracle as D
 
@@ -51,6 +52,28 @@ def padc(t, n):
 
 def unfrag(h, rows, width):
     return frag_unshuffle(h.view(-1, width))[:rows]
+
+
+# ---------------------------------------------------------------- cached rows side by side
+@pytest.mark.parametrize("rp", [32, 40, 256, 512])
+@pytest.mark.parametrize("bs", [1, 8, 16, 64])
+@pytest.mark.parametrize("segs", [[(1, 0, 0)], [(16, 0, 2), (3, 30, 0)], [(33, 95, 1), (1, 15, 3), (17, 512, 0)]])
+def test_latent_gather(rp, bs, segs):
+    """Every key of every segment, in order, out of scrambled blocks; nothing behind the last."""
+    g = gen(rp + bs)
+    keys = [n + p for n, p, _ in segs]
+    need = [-(-k // bs) for k in keys]
+    ids = (torch.randperm(sum(need) + 3, generator=g) + 1).tolist()
+    cache = torch.randn(sum(need) + 4, bs, rp, generator=g).bfloat16()
+    bt = torch.zeros(max(r for _, _, r in segs) + 1, max(need), dtype=torch.int32)
+    want = []
+    for (_, _, r), k, n in zip(segs, keys, need):
+        bt[r, :n] = torch.tensor([ids.pop() for _ in range(n)])
+        want.append(cache[bt[r, :n].long()].reshape(-1, rp)[:k])
+    items = cached_rows(segs)
+    out = torch.full((sum(keys) + 5, rp), 7.0, dtype=torch.bfloat16, device="cuda")
+    call("omni_latent_gather", dev(cache), dev(bt), bt.shape[1], bs, dev(torch.tensor(items, dtype=torch.int32)), len(items), out, rp)
+    assert torch.equal(out[:sum(keys)].cpu(), torch.cat(want)) and bool((out[sum(keys):] == 7.0).all())
 
 
 # ---------------------------------------------------------------- residual stream, shift, norms

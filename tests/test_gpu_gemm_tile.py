@@ -30,7 +30,7 @@ def _close(got, ref, mag, what):
                                    (1111, 96, 672), (255, 288, 96), (70, 48, 32), (900, 272, 160), (6400, 2048, 2048),
                                    (700, 256, 64), (1300, 768, 96), (515, 256, 32), (2000, 1024, 6144)])
 def test_plain_gemm_every_tile_configuration(M, N, K):
-    """tile_hint 1 = the large tiles (256 / 192 / 128 / 96 columns by N; the lockstep kernel), 2 = the 128 x 64 small-M tile, 0 = the
+    """tile_hint 1 = the large tiles (256 / 192 / 128 / 96 columns by N; the lockstep kernel), 2 = the 64 x 128 tile of few rows, 0 = the
     dispatch rule (plain GEMMs with N % 256 == 0: the two-group kernel)."""
     ops, L, frag_shuffle, _ = _ops()
     g = torch.Generator().manual_seed(M * 7 + N)

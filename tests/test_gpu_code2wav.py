@@ -229,6 +229,34 @@ def test_window_attention_kernel(hd, nh, nkv, T, window, ldo):
     assert float((d - ref.abs() * 2.0 ** -8).max()) <= 4 * 2.0 ** -13
 
 
+@pytest.mark.parametrize("Q,bins,C,T", [(1, 1, 4, 1), (7, 5, 260, 3), (16, 300, 512, 50), (64, 40, 516, 9), (65, 40, 1028, 5), (130, 3, 12, 33)])
+def test_code_lookup(Q, bins, C, T):
+    """Ids of 64 quantizers at a time, eight rows in flight, columns past a block's width and ids outside the table (clamped): fp32 sums in quantizer order."""
+    from ht_vllm_omni_amd import _lib as L
+    g = torch.Generator().manual_seed(Q + C)
+    codes, table = torch.randint(-2, bins + 2, (Q, T + 3), generator=g).cuda(), torch.randn(Q, bins, C, generator=g).cuda()
+    out = torch.full((T + 1, C), 7.0, dtype=torch.bfloat16, device="cuda")
+    L.check(L.load().omni_codec_rvq_embed(codes.data_ptr(), T + 3, table.data_ptr(), out.data_ptr(), T, Q, bins, C, L.current_stream()), "omni_codec_rvq_embed")
+    ref = torch.zeros(T, C, device="cuda")
+    for q in range(Q):
+        ref = ref + table[q][codes[q, :T].clamp(0, bins - 1)]
+    assert torch.equal(out[:T], ref.to(torch.bfloat16)) and bool((out[T:] == 7.0).all())
+
+
+@pytest.mark.parametrize("H", [4, 252, 512, 516, 1024, 1028, 1600])
+def test_codec_norm(H):
+    """Rows that end inside a piece, and the widths at which the kernel changes.  Bound: one rounding to bf16 (8 significant bits: half a unit in the
+    last place is at most 2^-8 of the value) beside fp32 sums."""
+    from ht_vllm_omni_amd import _lib as L
+    g, T = torch.Generator().manual_seed(H), 7
+    x, w = torch.randn(T, H + 4, generator=g).cuda() * 3, torch.randn(H, generator=g).cuda()
+    out = torch.full((T + 1, H), 7.0, dtype=torch.bfloat16, device="cuda")
+    L.check(L.load().omni_codec_rmsnorm(x.data_ptr(), H + 4, w.data_ptr(), 1e-5, out.data_ptr(), T, H, L.current_stream()), "omni_codec_rmsnorm")
+    v = x[:, :H].double()
+    ref = w.double() * v / torch.sqrt(v.pow(2).mean(-1, keepdim=True) + 1e-5)
+    assert bool(((out[:T].double() - ref).abs() <= ref.abs() * (2.0 ** -8 + 2.0 ** -16)).all()) and bool((out[T:] == 7.0).all())
+
+
 @pytest.mark.parametrize("C,T,taps", [(8, 1, 7), (96, 255, 7), (96, 257, 7), (72, 600, 3), (96, 300, 1), (112, 513, 12), (256, 300, 7), (520, 260, 7)])
 def test_last_conv(C, T, taps):
     """Blocks of 256 samples and their edges, samples before the first whole window, rows in LDS and rows too wide for it.  Bound: 2^-24 of the sum of

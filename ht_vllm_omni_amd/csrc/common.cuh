@@ -154,15 +154,38 @@ __device__ __forceinline__ void wave_argmax(float& v, int& idx) {
 __device__ __forceinline__ float wave_sum(float v) { return xor32_sum(xor16_sum(row16_sum(v))); }
 __device__ __forceinline__ float wave_max(float v) { return xor32_max(xor16_max(row16_max(v))); }
 
-// ---- xIELU: a quadratic branch above zero, an exponential one below, both with slope 1/2 at zero; ap, an are the two positive coefficients
+// ---- xIELU: a quadratic branch above zero, an exponential one below, both with slope 1/2 at zero; ap, an are the two positive coefficients.
+// Down to -1 it is z^2 times a polynomial (minimax for (e^z - 1 - z) / z^2, 5e-10 off), where the difference of expm1 and z would cancel, and the
+// hardware's exponential below; an enters the coefficients, which a loop of calls computes once.  An epilogue is a phase of its own behind the matrix
+// pipe: behind expm1f, 6001 x 9216 x 2048 took 31 us longer than the plain product, 502 rows 6, 64 rows 1.3; so 18, 4 and 0.8.
 __device__ __forceinline__ float xielu(float z, float ap, float an) {
-    return fmaf(0.5f, z, z > 0.f ? ap * z * z : an * (expm1f(fminf(z, 0.f)) - z));
+    float p = fmaf(an * 1.6879887851e-5f, z, an * 1.8817880123e-4f);
+    p = fmaf(p, z, an * 1.3820756500e-3f);
+    p = fmaf(p, z, an * 8.3309630941e-3f);
+    p = fmaf(p, z, an * 4.1666269431e-2f);
+    p = fmaf(p, z, an * 1.6666664144e-1f);
+    p = fmaf(p, z, an * 0.5f);
+    const float near = fmaf((z > 0.f ? ap : p) * z, z, 0.5f * z);
+    const float far = fmaf(an, __builtin_amdgcn_exp2f(z * 1.4426950408889634f), fmaf(z, 0.5f - an, -an));
+    return z < -1.0f ? far : near;
 }
 
 // ---- the other activations of the language models' products
 __device__ __forceinline__ float relu2(float z) { z = fmaxf(z, 0.f); return z * z; }
 __device__ __forceinline__ float gelu_tanh(float z) { return 0.5f * z * (1.0f + tanhf(0.79788456080286536f * fmaf(0.044715f * z * z, z, z))); }
 __device__ __forceinline__ float sigmoidf_(float z) { return 1.0f / (1.0f + expf(-z)); }
+// the same in two thirds of the instructions, for the epilogues behind the matrix pipe: the hardware's exponential of z log2(e) with what that product's
+// rounding lost put back, and its reciprocal with a Newton step, 2^24 up so that no reciprocal is denormal.  Within 1.7e-7; SiLU of a bf16 is the one
+// expf and a division give, bit for bit (65536 of 65536 inputs); the clamps turn what infinities leave in the corrections into numbers: results are those of above.
+// 6267 x 12288 x 2048 with SiLU(gate) * up 269 -> 263 us (the
+// plain product: 262), 6001 x 8192 x 2048 with SiLU and the logistic 188 -> 178 (155).
+__device__ __forceinline__ float sigmoid_w(float z) {
+    const float t = z * -1.4426950408889634f;
+    const float r = __builtin_amdgcn_fmed3f(fmaf(z, -1.9259629911e-8f, fmaf(z, -1.4426950408889634f, -t)), -1e-4f, 1e-4f);
+    const float d = fmaf(__builtin_amdgcn_exp2f(t), fmaf(r, 0.6931471806f, 1.0f), 1.0f) * 0x1p-24f;
+    const float y = __builtin_amdgcn_rcpf(d);
+    return fmaf(__builtin_amdgcn_fmed3f(fmaf(-d, y, 1.0f), -1e-4f, 1e-4f), y, y) * 0x1p-24f;
+}
 
 // ---- OCP e4m3fn <-> f32 (saturating, round-nearest-even: clamp then hardware cvt)
 #define OMNI_FP8_MAX 448.0f

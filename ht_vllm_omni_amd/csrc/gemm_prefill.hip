@@ -123,7 +123,7 @@ __device__ __forceinline__ void tile_epilogue(const TileArgs& a, f32x4 (&acc)[WN
         if (EPI == EPI_ACT && a.act == OMNI_TILE_ACT_XIELU) write_as(pass, [&](float z, int, float, float) { return xielu(z, a.act_p, a.act_n); });
         else if (EPI == EPI_ACT && a.act == OMNI_TILE_ACT_RELU2) write_as(pass, [&](float z, int, float, float) { return relu2(z); });
         else if (EPI == EPI_ACT && a.act == OMNI_TILE_ACT_SILU_SIGMOID)
-            write_as(pass, [&](float z, int j, float, float) { return (nw0 + j * 16 + 4 * q < a.act_cols ? z : 1.0f) * sigmoidf_(z); });
+            write_as(pass, [&](float z, int j, float, float) { return (nw0 + j * 16 + 4 * q < a.act_cols ? z : 1.0f) * sigmoid_w(z); });
         else if (mul) write_as(pass, [&](float z, int, float, float) { return gelu_tanh(z); });
         else if (gelu) write_as(pass, [&](float z, int, float b, float s) { return tg_gelu(z + b) * s; });
         else if (EPI == EPI_FULL) write_as(pass, [&](float z, int, float b, float s) { return (z + b) * s; });
@@ -164,7 +164,7 @@ __device__ __forceinline__ void tile_epilogue(const TileArgs& a, f32x4 (&acc)[WN
                 for (int e = 0; e < 4; ++e) {
                     const float g0 = bfround(gp[2 * e]), g1 = bfround(gp[2 * e + 1]);
                     const float u0 = bfround(gp[8 + 2 * e]), u1 = bfround(gp[8 + 2 * e + 1]);
-                    const float s0 = bfround(g0 / (1.0f + expf(-g0))), s1 = bfround(g1 / (1.0f + expf(-g1)));   // torch: F.silu(bf16) is bf16
+                    const float s0 = bfround(g0 * sigmoid_w(g0)), s1 = bfround(g1 * sigmoid_w(g1));   // torch: F.silu(bf16) is bf16
                     o[e] = pack_bf2(s0 * u0, s1 * u1);
                 }
                 *reinterpret_cast<u32x4*>(a.out + (size_t)m * a.ldo + (n >> 1)) = o;

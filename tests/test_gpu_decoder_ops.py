@@ -287,6 +287,32 @@ def test_xielu_epilogues(M):
     assert float(err.max()) <= 8e-3, float(err.max())
 
 
+def test_activations_of_the_tile_epilogues_to_32_bits():
+    """XIELU and SiLU / sigmoid of given fp32 values (a product with unit rows of W), from 1e-30 to 1e30 in either sign, in fp32: six roundings and two
+    1-ulp instructions are under 5e-7 of the larger of the result and its largest term; not-a-number stays one, and large values do not become one."""
+    v = torch.cat([torch.logspace(-30, 30, 2400, dtype=torch.double), torch.logspace(-2, 2.2, 4000, dtype=torch.double)]).bfloat16()
+    v = torch.cat([v, -v, torch.zeros(64, dtype=torch.bfloat16)])
+    v = v[:v.numel() // 96 * 96].reshape(-1, 96)
+    x, w = torch.zeros(v.shape[0], 96, dtype=torch.bfloat16), torch.eye(96, dtype=torch.bfloat16)
+    x.copy_(v)
+    z, lib = v.double(), L.load_decoder()
+    got = ops.gemm_tile(dev(x), frag_shuffle(dev(w)), act=L.TILE_ACT_XIELU, act_params=(0.7, 0.8), want="f", lib=lib).double().cpu()
+    n = z.clamp_max(0)
+    small = n * n * (0.5 + n / 6 + n * n / 24)                                        # expm1(n) - n cancels in doubles too
+    e = torch.where(n > -1e-3, small, torch.expm1(n) - n)
+    ref = 0.5 * z + torch.where(z > 0, 0.7 * z * z, 0.8 * e)
+    fits = ref.abs() < 3e38
+    assert bool(((got - ref).abs() <= 5e-7 * torch.maximum(ref.abs(), z.abs()) + 1e-37)[fits].all())
+    for cols in (96, 0):
+        got = ops.gemm_tile(dev(x), frag_shuffle(dev(w)), act=L.TILE_ACT_SILU_SIGMOID, act_cols=cols, want="f", lib=lib).double().cpu()
+        ref = torch.sigmoid(z) * (z if cols else 1.0)
+        keep = z > -87                                                                # below: the logistic leaves fp32's normal range, for either
+        assert bool(((got - ref).abs() <= 5e-7 * ref.abs() + 1e-37)[keep].all()) and bool((got[~keep].abs() <= 1e-35).all())
+    x[0, 0] = float("nan")
+    for kw in (dict(act=L.TILE_ACT_XIELU, act_params=(0.7, 0.8)), dict(act=L.TILE_ACT_SILU_SIGMOID, act_cols=96), dict(act=L.TILE_ACT_SILU_SIGMOID)):
+        assert bool(ops.gemm_tile(dev(x), frag_shuffle(dev(w)), want="f", lib=lib, **kw)[0].isnan().all())
+
+
 # ---------------------------------------------------------------- attention
 class Seqs:
     """Sequences of given lengths in a scrambled paged cache; the last `new[r]` tokens of each are the batch."""

@@ -860,8 +860,9 @@ static int launch_mid(TileArgs a, hipStream_t st, int groups) {
 }
 
 // waves, waves along n, n-tiles x m-tiles per wave, ring: 32 x 32 | 32 x 64 | 64 x 64 | 64 x 128 (rows x columns; two workgroups fit a CU) |
-// 128 x 128 | 256 x 128 | 128 x 256 (one)
-#define MID_LIST(X) X(0, 4, 2, 1, 1, 9) X(1, 4, 2, 2, 1, 6) X(2, 4, 2, 2, 2, 4) X(3, 8, 4, 2, 2, 3) X(4, 8, 4, 2, 4, 4) X(5, 8, 2, 4, 4, 3) X(6, 8, 4, 4, 4, 3)
+// 128 x 128 | 256 x 128 | 128 x 256 (one) | 96 x 64 (two) | 192 x 128 | 96 x 128 (one)
+#define MID_LIST(X) X(0, 4, 2, 1, 1, 9) X(1, 4, 2, 2, 1, 6) X(2, 4, 2, 2, 2, 4) X(3, 8, 4, 2, 2, 3) X(4, 8, 4, 2, 4, 4) X(5, 8, 2, 4, 4, 3) X(6, 8, 4, 4, 4, 3) \
+                    X(7, 4, 2, 2, 3, 4) X(8, 8, 2, 4, 3, 4) X(9, 4, 2, 4, 3, 4)
 template <bool GU8, bool WINDOW>
 static int launch_mid_of(int geom, const TileArgs& a, hipStream_t st, int groups) {
     switch (geom) {
@@ -877,27 +878,29 @@ static int launch_mid_of(int geom, const TileArgs& a, hipStream_t st, int groups
 // costs is what a CU takes in -- 60 - 90 GB/s of operands in every geometry (a slice of the 32 x 64 tile is 12 KB in 0.17 us, of the 256 x 256 tile
 // 64 KB in 1.1 - 1.3 us) -- so small grids want small tiles on all 256 CUs and large ones tall tiles.  Two workgroups on a CU share that rate
 // but hide each other's barriers: 0.44 us for a slice of each of two 64 x 64 tiles, 0.27 alone.
-// Numbers: ns, from sweeps of M 66 ... 6000 over the weight shapes of the 1024- and 2048-wide models and of the vocoder's convolutions at 12 ... 325
-// frames, weights cold.  With this rule against the two tiles there were (the 256 x 256 family, and 64 x 128 below 96 of those): 490 x 9216 x 2048
-// 45 -> 33 us, 490 x 2048 x 2048 18.3 -> 11.5, 1450 x 2048 x 9216 101 -> 67, 800 x 5120 x 2048 40 -> 31, 50 x 1024 x 3072 20.9 -> 8.8.
-// (The 64 x 128 tile's numbers are from a sweep of its own, M 50 ... 1800, over all tiles' times: 390 x 9216 x 2048 31.5 -> 24.5, 1100 x 1024 x 4608
-// 32.4 -> 23.0, 560 x 2048 x 2048 16.0 -> 12.4 against its size taken for 128 x 64; what the rule picks is 2.2 % behind the best tile on average, from 3.9.)
+// Numbers: ns above what every launch costs, least squares over M 13 ... 6300 x the weight shapes of the language models, talkers and the vocoder, 600
+// products by every tile and count of partial sums, every weight out of HBM; what the rule picks is 0.9 % behind the best tile on average, 0.5 % over the
+// vocoder's windows.  (Weights that are in the last-level cache want fewer, larger tiles: 50 x 1024 x 3072 by 32 x 64 9.5, by 32 x 32 10.5; out of HBM the
+// other way round.  A step's weights do not stay there.)
+// The heights between the powers of two are there for the rounds: a product of 500 rows by 9216 columns is 288 tiles of 128 x 128 on 256 CUs (two rounds,
+// 34.8 us), 144 of 256 x 128 (33.0) and 216 of 192 x 128 (25.8); 200 x 4608 x 1024 7.5 -> 6.9 by 96 x 64, 800 x 5120 x 2048 34.6 -> 25.0, 1000 x 2560 x 1024
+// 10.6 -> 9.6 by 96 x 128.  On average over those products the three are worth 1.8 %.
 enum { KIND_MID, KIND_PP, KIND_LARGE };
 struct TileChoice {
     int kind, geom, bm, bn;          // geom: MID_LIST index, or rows of the two-group / lockstep tile
     int round1, slice1, round2, slice2;      // alone on a CU; two per CU (0: one fits)
-    bool whole;                      // two per CU: a third waits for the round
 };
 #define MID_SIZE_CASE(I, A, B, C, D, E) if (I == i) return rows ? MidGeom<A, B, C, D, E>::BM : MidGeom<A, B, C, D, E>::BN;
 static constexpr int mid_size(int i, bool rows) { MID_LIST(MID_SIZE_CASE) return 0; }
 #undef MID_SIZE_CASE
 #define MID(I) KIND_MID, I, mid_size(I, true), mid_size(I, false)
 static const TileChoice TILE_CHOICES[] = {
-    {MID(0), 1300, 140, 1900, 230, false}, {MID(1), 1300, 175, 2200, 335, false}, {MID(2), 1400, 270, 2400, 440, false}, {MID(3), 1600, 480, 3000, 600, true},
-    {MID(4), 2200, 500},                   {MID(5), 4000, 830},                   {MID(6), 4200, 900},
-    {KIND_PP, 192, 192, 256, 5000, 1130},    {KIND_PP, 224, 224, 256, 5500, 1200},    {KIND_PP, 256, 256, 256, 6000, 1280},
-    {KIND_LARGE, 192, 192, 256, 6000, 1150}, {KIND_LARGE, 224, 224, 256, 6500, 1250}, {KIND_LARGE, 256, 256, 256, 7500, 1350},
-    {KIND_LARGE, 0, 256, 192, 6000, 1180},   {KIND_LARGE, 0, 512, 128, 7500, 1650},   {KIND_LARGE, 0, 512, 96, 7000, 1500},
+    {MID(0), 2390, 140, 2750, 231}, {MID(1), 2490, 202, 2660, 306}, {MID(2), 2660, 280, 3110, 427}, {MID(3), 3100, 466, 4990, 650},
+    {MID(4), 4400, 475},            {MID(5), 5230, 871},            {MID(6), 5800, 912},
+    {MID(7), 3010, 306, 4090, 542}, {MID(8), 5380, 570},            {MID(9), 4150, 425},
+    {KIND_PP, 192, 192, 256, 8570, 996},     {KIND_PP, 224, 224, 256, 9350, 1044},    {KIND_PP, 256, 256, 256, 10300, 1088},
+    {KIND_LARGE, 192, 192, 256, 9600, 1015}, {KIND_LARGE, 224, 224, 256, 10300, 1090}, {KIND_LARGE, 256, 256, 256, 11800, 1150},
+    {KIND_LARGE, 0, 256, 192, 9600, 1040},   {KIND_LARGE, 0, 512, 128, 11800, 1450},  {KIND_LARGE, 0, 512, 96, 11300, 1320},
 };
 #undef MID
 static const TileChoice& pick_tile(int M, int N, int K, int groups, int splits, bool plain, bool gu8, long long* ns) {
@@ -910,8 +913,8 @@ static const TileChoice& pick_tile(int M, int N, int K, int groups, int splits, 
         if (c.kind == KIND_LARGE && (c.bn != large_bn || (plain && c.bn == 256) || splits > 1)) continue;
         const long long tiles = (long long)((M + c.bm - 1) / c.bm) * ((N + c.bn - 1) / c.bn) * groups * splits;
         long long t;
-        // (a CU that gets a third small tile while the first two run does not wait for a round of two; the 64 x 128 tile measured like whole rounds)
-        if (c.slice2 && tiles > 256) t = (c.round2 + slices * c.slice2) * (c.whole ? 2 * ((tiles + 511) / 512) : (tiles + 255) / 256) / 2;
+        // (a CU that gets a third small tile while the first two run does not wait for a round of two)
+        if (c.slice2 && tiles > 256) t = (c.round2 + slices * c.slice2) * ((tiles + 255) / 256) / 2;
         else t = (c.round1 + slices * c.slice1) * ((tiles + 255) / 256);
         if (!best || t < least) { best = &c; least = t; }
     }
@@ -949,7 +952,7 @@ extern "C" int omni_gemm_tile(const omni_tile_gemm* g, void* stream) {
     OMNI_CHECK_ARG(g->act != OMNI_TILE_ACT_SILU_SIGMOID || (g->act_cols >= 0 && g->act_cols % 4 == 0), "omni_gemm_tile: act_cols=%d (%% 4)", g->act_cols);
     OMNI_CHECK_ARG(g->act != OMNI_TILE_ACT_GELU_MUL || (g->mul_table && g->mul_ids && g->mul_rows > 0 && g->mul_ld >= g->N && g->mul_ld % 8 == 0 && g->out && !g->out2 && !g->resid &&
                                                         g->groups <= 1), "omni_gemm_tile: the row table takes ids, mul_ld >= N (%% 8), a bf16 output and one group");
-    OMNI_CHECK_ARG(g->tile_hint >= 0 && g->tile_hint <= 13, "omni_gemm_tile: tile_hint=%d", g->tile_hint);
+    OMNI_CHECK_ARG(g->tile_hint >= 0 && g->tile_hint <= 16, "omni_gemm_tile: tile_hint=%d", g->tile_hint);
     OMNI_CHECK_ARG(g->tile_hint < 3 || g->tile_hint > 7 || g->N % 256 == 0, "omni_gemm_tile: tile_hint=%d needs N %% 256 == 0", g->tile_hint);
     OMNI_CHECK_ARG(!gu8 || (g->out && !g->resid && !g->out2 && !g->out_f32), "omni_gemm_tile: SiLU-mul takes out only");
     OMNI_CHECK_ARG(!g->out2 || (g->snake_alpha && g->snake_inv_beta), "omni_gemm_tile: out2 needs the snake parameters");
@@ -990,7 +993,7 @@ extern "C" int omni_gemm_tile(const omni_tile_gemm* g, void* stream) {
     OMNI_CHECK_ARG(g->k_splits >= 0 && g->k_splits <= 4 && (g->k_splits <= 1 || (tile_epi(a) == EPI_ACT && g->act == OMNI_TILE_ACT_NONE && !g->out && groups == 1 && g->k_splits <= g->K / 32 &&
                    g->slab_stride >= (int64_t)(g->M - 1) * g->ldf + N && g->slab_stride % 4 == 0)), "omni_gemm_tile: k_splits=%d (<= K / 32; one group, fp32 output alone)", g->k_splits);
     a.splits = g->k_splits > 1 ? g->k_splits : 1; a.slab_stride = g->slab_stride;
-    // tile_hint: 1 the large lockstep tiles, 2 and 8 ... 13 the mid-size ones, 3 / 4 lockstep and 5 / 6 / 7 two-group at 224 / 192 and 256 / 224 / 192 rows
+    // tile_hint: 1 the large lockstep tiles, 2 and 8 ... 16 the mid-size ones, 3 / 4 lockstep and 5 / 6 / 7 two-group at 224 / 192 and 256 / 224 / 192 rows
     const bool plain = groups == 1 && !g->group_rows && seg_len == g->K && g->row_off == 0;
     OMNI_CHECK_ARG(g->tile_hint < 5 || g->tile_hint > 7 || plain, "omni_gemm_tile: tile_hint=%d (two-group tile) takes a plain GEMM", g->tile_hint);
     OMNI_CHECK_ARG(a.splits == 1 || g->tile_hint == 0 || g->tile_hint == 2 || g->tile_hint >= 5, "omni_gemm_tile: tile_hint=%d takes no k_splits", g->tile_hint);

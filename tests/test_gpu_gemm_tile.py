@@ -67,6 +67,23 @@ def test_mid_size_tiles_at_their_edges(M, N, K, taps, dil):
         assert torch.equal(out[:M], ref) and bool((out[M:] == 7.0).all()), hint
 
 
+@pytest.mark.parametrize("M,N,K,taps,dil", [(1, 16, 32, 1, 1), (95, 48, 64, 1, 1), (97, 144, 96, 1, 1), (193, 80, 32 * 7, 7, 9), (385, 272, 1056, 1, 1), (577, 1040, 288, 1, 1)])
+def test_tiles_of_96_and_192_rows_at_their_edges(M, N, K, taps, dil):
+    """tile_hints 14 ... 16, as above; with partial sums, and SiLU * up of interleaved gates where it is no window."""
+    ops, L, frag_shuffle, gu8_shuffle = _ops()
+    g = torch.Generator().manual_seed(M * 13 + K)
+    x, w = torch.randn(M, K // taps, generator=g).to(BF16).cuda(), (torch.randn(N, K, generator=g) * 0.05).to(BF16)
+    b, wf, wg = torch.randn(N, generator=g).cuda(), frag_shuffle(w).cuda(), gu8_shuffle(w).cuda()
+    for hint in (14, 15, 16):
+        out = torch.full((M + 3, N), 7.0, dtype=BF16, device="cuda")
+        ops.gemm_tile(x, wf, bias=b, taps=taps, dilation=dil, tile_hint=hint, out=out[:M])
+        assert torch.equal(out[:M], ops.gemm_tile(x, wf, bias=b, taps=taps, dilation=dil, tile_hint=1)) and bool((out[M:] == 7.0).all()), hint
+        if taps == 1:
+            assert torch.equal(*(ops.gemm_tile(x, wg, act=L.TILE_ACT_SILU_MUL_GU8, tile_hint=h) for h in (hint, 1))), hint
+        if taps == 1 and K >= 96:
+            assert torch.equal(*(ops.gemm_tile(x, wf, want="f", splits=3, tile_hint=h) for h in (hint, 2))), hint
+
+
 @pytest.mark.parametrize("M,K,splits", [(33, 32, 1), (70, 96, 3), (129, 160, 4), (65, 64, 1)])
 def test_rows_that_end_an_array(M, K, splits):
     """x is the last columns of a wider array and a run of K steps is a single one: what a tile fetches ahead of its last step lies past the last row."""

@@ -195,6 +195,22 @@ __global__ __launch_bounds__(64) void window_merge_kernel(const WinArgs a, int m
 // chain over the keys is then what a tile takes, and one group's is shorter.  Us, two groups / one, heads x keys' heads of 128: 16 x 4, 52 tiles of portions
 // behind 512 tokens 30.4 / 19.9, 252 tiles (a prompt of 2000 in windows of 512) 30.5 / 27.7; 16 x 16, 256 tiles of 97 rows 11.2 / 9.9, 64 tiles behind 1000
 // tokens 66 / 44.
+// Order.  An XCD deals its workgroups out in turn over its 32 CUs, three to a CU, and the tiles of a causal prompt are as long as the keys they see: by length
+// the first CU gets the longest of each turn (one prompt of 6001 tokens, 47 tiles of 16 heads: 94 units of keys against 70 on average).  wa_deal orders the
+// first turns so that what a CU gets adds up to the same (72): that prompt 394 -> 342 us a layer, one of 3000 152 -> 143, one of
+// 2500 in windows of 1024 61 -> 57, with a step's address arithmetic and maxima cut down (4 prompts of up to 2048 in such windows, balanced before: 91.8 -> 90.9).
+// (The dealing is how an idle XCD was seen to go about it; another one costs time, never a result.)
+__device__ __forceinline__ int wa_deal(int slot, int n) {                     // workgroup of an XCD -> rank by length among its n
+    constexpr int C = 32;
+    const int turn = slot / C, j = slot - turn * C, i = j >> 1;
+    if (n <= C || turn >= 3) return slot;
+    if (n <= 2 * C) return turn == 0 ? C - 1 - j : slot;                      // the shortest of the first turn get the longest of the second
+    const int last = min(n - 2 * C, C);                                       // three turns: sums of three orders, 46 or 47 of 93 where all are full
+    if (turn == 0) return j;
+    if (turn == 1) return C + (j & 1 ? C - 1 - i : C / 2 - 1 - i);
+    return 2 * C + (j & 1 ? last / 2 - 1 - i : last - 1 - i);
+}
+
 template <int WS, int RG>
 __global__ __launch_bounds__(256, 3) void window_prefill_dma_kernel(const WinArgs a, int n_tiles) {
     constexpr int WR = 16 * RG, PARTS = 2 / RG, HALF = WS * 1024, IMAGE = 4 * HALF, NB = 3, dp = 32 * WS;
@@ -205,8 +221,8 @@ __global__ __launch_bounds__(256, 3) void window_prefill_dma_kernel(const WinArg
     int tile, g;
     {
         const int id = blockIdx.x, xcd = id & 7, slot = id >> 3, G = a.kv_heads;
-        if (G % 8 == 0) { g = slot / n_tiles * 8 + xcd; tile = slot % n_tiles; }
-        else if (8 % G == 0) { g = xcd % G; tile = slot * (8 / G) + xcd / G; }
+        if (G % 8 == 0) { const int r = wa_deal(slot, n_tiles * (G / 8)); tile = r / (G / 8); g = (r - tile * (G / 8)) * 8 + xcd; }
+        else if (8 % G == 0) { g = xcd % G; tile = wa_deal(slot, (int)gridDim.x >> 3) * (8 / G) + xcd / G; }
         else { g = id / n_tiles; tile = id - g * n_tiles; }
     }
     if (tile >= n_tiles || g >= a.kv_heads) return;
@@ -260,13 +276,23 @@ __global__ __launch_bounds__(256, 3) void window_prefill_dma_kernel(const WinArg
         if (!a.key_base) ids = bt[b];
         asm volatile("" : "+v"(ids));                  // waited for here, not where the lookups are
     };
-    auto block_of = [&](int k0) {
-        if (((k0 + LA_KEYS - 1) >> a.bs_shift) - cached > 63) load_ids(k0);
-        return __shfl(ids, (min(k0 + lkey, nkeys - 1) >> a.bs_shift) - cached, 64);
-    };
+    const int lkey0 = 16 * (wave & 1);
     auto stage = [&](int k0, int buf) {                                       // keys past the end: a valid row, masked below
-        const int blk = block_of(min(k0, nkeys - 1));
-        const uint16_t* p = src + (size_t)blk * lblock + (size_t)(min(k0 + lkey, nkeys - 1) & a.bs_mask) * lrow;
+        k0 = min(k0, nkeys - 1);
+        const int off = min(k0 + lkey, nkeys - 1) & a.bs_mask;
+        const uint16_t* p = src;
+        if (a.bs_shift >= 4) {                                                // (uniform) the wave's 16 keys lie in one block
+            int blk = min(k0 + lkey0, nkeys - 1) >> a.bs_shift;
+            if (!a.key_base) {
+                if (((k0 + LA_KEYS - 1) >> a.bs_shift) - cached > 63) load_ids(k0);
+                blk = __builtin_amdgcn_readlane(ids, blk - cached);
+            }
+            p += (int64_t)blk * lblock;
+        } else {
+            if (((k0 + LA_KEYS - 1) >> a.bs_shift) - cached > 63) load_ids(k0);
+            p += (int64_t)__shfl(ids, (min(k0 + lkey, nkeys - 1) >> a.bs_shift) - cached, 64) * lblock;
+        }
+        p += (uint64_t)(unsigned)off * (unsigned)lrow;
         unsigned char* d = dst0 + buf * IMAGE;
 #pragma unroll
         for (int s = 0; s < WS; ++s)
@@ -313,12 +339,11 @@ __global__ __launch_bounds__(256, 3) void window_prefill_dma_kernel(const WinArg
             mx = p[0];
 #pragma unroll
             for (int j = 1; j < 8; ++j) mx = fmaxf(mx, p[j]);
-            mx = xor32_max(xor16_max(mx)) * a.qs;
             // the maximum follows once a row has outgrown it by 2^LAZY (the conditional rescaling of FlashAttention-4): weights up to that size lose nothing
             // in fp32, nor in three terms.  The 16 rows of a group move together, so a row's last bits depend on the rows it shares a group with,
             // that is on where its portion was cut
-            if (__any(mx > m[rg] + LAZY)) {
-                const float mn = fmaxf(m[rg], mx), alpha = exp2_w(m[rg] - mn);      // (never below the finite sentinel: 1, harmless, where l = 0, O = 0)
+            if (__any(mx * a.qs > m[rg] + LAZY)) {                 // (any lane's own keys: the row's maximum is put together only then)
+                const float mn = fmaxf(m[rg], xor32_max(xor16_max(mx)) * a.qs), alpha = exp2_w(m[rg] - mn);      // (never below the finite sentinel: 1, harmless, where l = 0, O = 0)
                 m[rg] = mn;
                 l[rg] *= alpha;
 #pragma unroll

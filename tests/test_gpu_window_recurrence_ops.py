@@ -284,6 +284,15 @@ def test_prompt_tiles_that_fill_the_chip(heads, kv, dim, bs, window, scale):
     close(s.run(scale, window), s.reference(scale, window), SAFE[0])
 
 
+@pytest.mark.parametrize("tiles", [33, 47, 64, 65, 79, 96, 97, 131])
+@pytest.mark.parametrize("heads,kv", [(8, 8), (4, 4), (16, 16)])
+def test_every_tile_is_dealt_once(heads, kv, tiles):
+    """An XCD's workgroups in one, two, three and more turns over its CUs, whole turns and one more or less (a tile per short sequence)."""
+    lens = [2 + r % 4 for r in range(tiles)]
+    s = Seqs([n + r % 3 for r, n in enumerate(lens)], lens, heads, kv, 64, 64, 0, seed=tiles)
+    close(s.run(0.3, None), s.reference(0.3, None), SAFE[0])
+
+
 @pytest.mark.parametrize("heads,kv,dim,vdim", [(8, 8, 128, 128), (3, 3, 64, 64), (6, 2, 40, 24), (4, 4, 96, 128), (2, 2, 200, 256)])
 @pytest.mark.parametrize("window", [None, 50])
 def test_keys_in_one_array_and_a_gate_per_head(heads, kv, dim, vdim, window):

@@ -195,6 +195,12 @@ __global__ __launch_bounds__(64) void window_merge_kernel(const WinArgs a, int m
 // chain over the keys is then what a tile takes, and one group's is shorter.  Us, two groups / one, heads x keys' heads of 128: 16 x 4, 52 tiles of portions
 // behind 512 tokens 30.4 / 19.9, 252 tiles (a prompt of 2000 in windows of 512) 30.5 / 27.7; 16 x 16, 256 tiles of 97 rows 11.2 / 9.9, 64 tiles behind 1000
 // tokens 66 / 44.
+// KT: teams of four waves that take the workgroup's 32-key steps in turn, each with a ring and running sums of its own; the first adds up.  Three, one
+// workgroup to a CU, where the half tiles are no more than the CUs: a step is a chain of LDS reads, 8 + 24 MFMAs and the softmax between (0.85 us for one wave
+// a SIMD, 1.6 for three in turn), and nothing else is there to fill its gaps.  Up to four steps are one team's: the others leave at once.  Us, one
+// team / three, heads x keys' heads of 128: 16 x 16, portions of 251 and 130 tokens behind 512 26.3 / 18.8 (two: 19.9), 64 behind 1500 43.9 / 28.3 (31.7), a
+// prompt of 1000 33.8 / 23.0 (24.6), of 300 12.8 / 11.0, of 66 6.3 / 6.5; 16 x 4, a prompt of 1000 31.3 / 22.3, 8 of 100 7.4 / 7.8.  Above 256 half tiles two
+// workgroups of one team share a CU instead: 256 tiles of up to 128 tokens 9.4, by three teams in turns 15.8.
 // Order.  An XCD deals its workgroups out in turn over its 32 CUs, three to a CU, and the tiles of a causal prompt are as long as the keys they see: by length
 // the first CU gets the longest of each turn (one prompt of 6001 tokens, 47 tiles of 16 heads: 94 units of keys against 70 on average).  wa_deal orders the
 // first turns so that what a CU gets adds up to the same (72): that prompt 394 -> 342 us a layer, one of 3000 152 -> 143, one of
@@ -211,12 +217,12 @@ __device__ __forceinline__ int wa_deal(int slot, int n) {                     //
     return 2 * C + (j & 1 ? last / 2 - 1 - i : last - 1 - i);
 }
 
-template <int WS, int RG>
-__global__ __launch_bounds__(256, 3) void window_prefill_dma_kernel(const WinArgs a, int n_tiles) {
+template <int WS, int RG, int KT>
+__global__ __launch_bounds__(256 * KT, KT == 1 ? 3 : KT) void window_prefill_dma_kernel(const WinArgs a, int n_tiles) {
     constexpr int WR = 16 * RG, PARTS = 2 / RG, HALF = WS * 1024, IMAGE = 4 * HALF, NB = 3, dp = 32 * WS;
     constexpr float LAZY = 8.0f;
     extern __shared__ __attribute__((aligned(1024))) unsigned char lds[];     // [ring][keys 0-15 | keys 16-31 | values 0-15 | values 16-31][32-wide pieces]
-    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane((threadIdx.x >> 6) & 3), team = KT == 1 ? 0 : __builtin_amdgcn_readfirstlane(threadIdx.x >> 8);
     const int c = lane & 15, qk = lane >> 4;
     int tile, g;
     {
@@ -247,7 +253,7 @@ __global__ __launch_bounds__(256, 3) void window_prefill_dma_kernel(const WinArg
 #pragma unroll
         for (int d = 0; d < 2 * WS; ++d) O[rg][d] = (f32x4){0.f, 0.f, 0.f, 0.f};
         // a sink of -inf is none: the finite sentinel, against which a tile that holds no key of the row weighs nothing (of +inf: not a number, as its softmax)
-        const float sink = a.sink ? a.sink[head] * LA_LOG2E : -INFINITY;
+        const float sink = a.sink && team == 0 ? a.sink[head] * LA_LOG2E : -INFINITY;
         m[rg] = sink < LA_SENT ? LA_SENT : (sink == INFINITY ? NAN : sink);
         l[rg] = sink < LA_SENT || qk != 0 ? 0.f : 1.f;
     }
@@ -259,13 +265,16 @@ __global__ __launch_bounds__(256, 3) void window_prefill_dma_kernel(const WinArg
     const int fhi = wave * WR + WR <= nrows ? wfirst + 1 : 0, flo = wa_first(whi - 1, a.window);
     const int nkeys = a.positions[(row0 + nrows - 1) / a.rep] + 1;
     const int kbeg = wa_first(a.positions[tok0], a.window) & ~(LA_KEYS - 1);
+    const int teams = KT == 1 || nkeys - kbeg <= 4 * LA_KEYS ? 1 : KT, stride = LA_KEYS * teams;      // (uniform) four steps are walked sooner than merged
+    if (team >= teams) return;
     // loader: wave -> keys 16 (wave & 1) ... of the keys (waves 0, 1) or the values (2, 3); lane -> key lane / 4, 16-byte quarter lane % 4 of every piece
     const bool vals = wave >= 2;
     const int lkey = 16 * (wave & 1) + (lane >> 2);
     const int lrow = vals ? a.v_row : a.k_row;
     const int64_t lblock = vals ? a.v_block : a.k_block;
     const uint16_t* src = (vals ? a.vc + first * a.v_row + (size_t)g * a.v_head : a.kc + first * a.k_row + (size_t)g * a.k_head) + 8 * (lane & 3);
-    unsigned char* const dst0 = lds + wave * HALF;
+    unsigned char* const ring = lds + team * (NB * IMAGE);
+    unsigned char* const dst0 = ring + wave * HALF;
     // block ids: 64 of the sequence's table in the lanes of a register, looked up by a lane exchange (a load per tile would be waited for together with
     // the tiles in flight); read again when a tile leaves them
     int cached = 0, ids = 0;
@@ -299,14 +308,15 @@ __global__ __launch_bounds__(256, 3) void window_prefill_dma_kernel(const WinArg
             __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)(p + 32 * s), (__attribute__((address_space(3))) void*)(d + s * 1024), 16, 0, 0);
     };
     load_ids(kbeg);
-    stage(kbeg, 0);
-    stage(kbeg + LA_KEYS, 1);
+    stage(kbeg + LA_KEYS * team, 0);
+    stage(kbeg + LA_KEYS * team + stride, 1);
     int buf = 0;
-    for (int k0 = kbeg; k0 < nkeys; k0 += LA_KEYS) {
+    for (int base = kbeg; base < nkeys; base += stride) {              // (as many turns for every team; one past the end stages a valid row and skips)
+        const int k0 = base + LA_KEYS * team;
         asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"n"(WS) : "memory");      // this tile is there; the one before is read by no wave any more
-        stage(k0 + 2 * LA_KEYS, buf >= 1 ? buf - 1 : NB - 1);                  // into the place that tile left
-        const unsigned char* kimg = lds + buf * IMAGE + (c * 4 + qk) * 16;
-        const unsigned char* vimg = lds + buf * IMAGE + 2 * HALF + (4 * qk + (c >> 2)) * 64 + (c & 3) * 8;
+        stage(k0 + 2 * stride, buf >= 1 ? buf - 1 : NB - 1);                  // into the place that tile left
+        const unsigned char* kimg = ring + buf * IMAGE + (c * 4 + qk) * 16;
+        const unsigned char* vimg = ring + buf * IMAGE + 2 * HALF + (4 * qk + (c >> 2)) * 64 + (c & 3) * 8;
         buf = buf + 1 == NB ? 0 : buf + 1;
         if (k0 >= whi || k0 + LA_KEYS <= wlo) continue; // (wave-uniform; loads and barriers above stay common)
         f32x4 S[RG][2];
@@ -375,16 +385,43 @@ __global__ __launch_bounds__(256, 3) void window_prefill_dma_kernel(const WinArg
                          : "v"(vaddr), "n"(d0 * 512), "n"(d0 * 512 + 32), "n"(d0 * 512 + 1024), "n"(d0 * 512 + 1056), "n"(d0 * 512 + HALF), "n"(d0 * 512 + 32 + HALF),
                            "n"(d0 * 512 + 1024 + HALF), "n"(d0 * 512 + 1056 + HALF));
 #pragma unroll
-            for (int d = 0; d < 4; ++d) {
-                const u32x4 VT = {x[d][0], x[d][1], y[d][0], y[d][1]};
+            for (int k = 2; k >= 0; --k)
 #pragma unroll
-                for (int k = 2; k >= 0; --k)
+                for (int d = 0; d < 4; ++d)
 #pragma unroll
-                    for (int rg = 0; rg < RG; ++rg) O[rg][d0 + d] = mfma16(VT, w3[rg][k], O[rg][d0 + d]);
-            }
+                    for (int rg = 0; rg < RG; ++rg) O[rg][d0 + d] = mfma16((u32x4){x[d][0], x[d][1], y[d][0], y[d][1]}, w3[rg][k], O[rg][d0 + d]);
         }
     }
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // the tiles behind the last one land before the LDS is another workgroup's
+    if constexpr (KT > 1) if (teams > 1) {             // the other teams' rows into the first one's: [team][wave][row group][d tile | m, l][lane]
+        constexpr int REC = RG * (2 * WS + 1) * 64;
+        static_assert((KT - 1) * 4 * REC * 16 <= KT * NB * IMAGE, "the records lie in the rings");
+        f32x4* const recs = reinterpret_cast<f32x4*>(lds) + (size_t)wave * REC + lane;
+        __syncthreads();
+        if (team) {
+            f32x4* const rec = recs + (size_t)(team - 1) * (4 * REC);
+#pragma unroll
+            for (int rg = 0; rg < RG; ++rg) {
+#pragma unroll
+                for (int d = 0; d < 2 * WS; ++d) rec[(rg * (2 * WS + 1) + d) * 64] = O[rg][d];
+                rec[(rg * (2 * WS + 1) + 2 * WS) * 64] = (f32x4){m[rg], l[rg], 0.f, 0.f};
+            }
+        }
+        __syncthreads();
+        if (team) return;
+#pragma unroll
+        for (int o = 0; o < KT - 1; ++o)
+#pragma unroll
+            for (int rg = 0; rg < RG; ++rg) {
+                const f32x4* const rec = recs + (size_t)o * (4 * REC) + rg * (2 * WS + 1) * 64;
+                const f32x4 ml = rec[2 * WS * 64];
+                const float mn = fmaxf(m[rg], ml[0]), mine = exp2_w(m[rg] - mn), theirs = exp2_w(ml[0] - mn);      // (a team without a key of the row: the sentinel, l = 0, O = 0)
+                m[rg] = mn;
+                l[rg] = l[rg] * mine + ml[1] * theirs;
+#pragma unroll
+                for (int d = 0; d < 2 * WS; ++d) O[rg][d] = O[rg][d] * mine + rec[d * 64] * theirs;
+            }
+    }
 #pragma unroll
     for (int rg = 0; rg < RG; ++rg) {
         const float L = xor32_sum(xor16_sum(l[rg]));
@@ -639,15 +676,17 @@ static int wa_run(const omni_window_attn& p, WinArgs a, hipStream_t st) {
     if (p.n_tiles > 0) {
         if constexpr (EX && WS <= 4) if (a.qs > 0.f) {
             constexpr int LDS = 3 * 4 * WS * 1024;
-            static const int rc = wa_lds(window_prefill_dma_kernel<WS, 2>, LDS), rc1 = wa_lds(window_prefill_dma_kernel<WS, 1>, LDS);
+            static const int rc = wa_lds(window_prefill_dma_kernel<WS, 2, 1>, LDS), rc1 = wa_lds(window_prefill_dma_kernel<WS, 1, 1>, LDS), rc3 = wa_lds(window_prefill_dma_kernel<WS, 1, 3>, 3 * LDS);
             if (rc != OMNI_OK) return rc;
             if (rc1 != OMNI_OK) return rc1;
+            if (rc3 != OMNI_OK) return rc3;
             const int G = p.kv_heads, per = 8 % G == 0 ? 8 / G : 1;           // workgroups in whole groups of 8 where an XCD takes part of one head's tiles
             const bool halves = (int64_t)p.n_tiles * G <= 256;
             const int n = halves ? 2 * p.n_tiles : p.n_tiles;
             const int64_t wgs = 8 % G == 0 ? (int64_t)(n + per - 1) / per * 8 : (int64_t)n * G;
-            if (halves) hipLaunchKernelGGL((window_prefill_dma_kernel<WS, 1>), dim3((unsigned)wgs), dim3(256), LDS, st, a, n);
-            else hipLaunchKernelGGL((window_prefill_dma_kernel<WS, 2>), dim3((unsigned)wgs), dim3(256), LDS, st, a, n);
+            if (halves && (int64_t)n * G <= 256) hipLaunchKernelGGL((window_prefill_dma_kernel<WS, 1, 3>), dim3((unsigned)wgs), dim3(768), 3 * LDS, st, a, n);
+            else if (halves) hipLaunchKernelGGL((window_prefill_dma_kernel<WS, 1, 1>), dim3((unsigned)wgs), dim3(256), LDS, st, a, n);
+            else hipLaunchKernelGGL((window_prefill_dma_kernel<WS, 2, 1>), dim3((unsigned)wgs), dim3(256), LDS, st, a, n);
             OMNI_CHECK_LAUNCH("omni_window_attn(prefill)");
             return OMNI_OK;
         }

@@ -284,6 +284,21 @@ def test_prompt_tiles_that_fill_the_chip(heads, kv, dim, bs, window, scale):
     close(s.run(scale, window), s.reference(scale, window), SAFE[0])
 
 
+@pytest.mark.parametrize("heads,kv,dim,sinks", [(8, 8, 128, True), (6, 2, 64, True), (2, 2, 128, False)])
+@pytest.mark.parametrize("keys,window", [(127, None), (128, None), (129, None), (160, None), (161, None), (225, None), (290, 100), (900, 129), (1111, 400), (333, 161)])
+def test_steps_shared_out_over_teams(heads, kv, dim, sinks, keys, window):
+    """Few half tiles: up to four steps of 32 keys by one team of waves, more by three in turn, counts that do and do not divide by three, rows whose window
+    holds no key of a team's steps, a first step in the middle of the keys."""
+    s = Seqs([keys, keys + 40, 33], [70, 2, 17], heads, kv, dim, dim, 0, seed=keys + dim, sink=sinks)
+    close(s.run(0.3, window), s.reference(0.3, window), SAFE[0])
+
+
+def test_half_tiles_two_to_a_compute_unit():
+    """More half tiles than compute units, and not as many whole ones: one team walks."""
+    s = Seqs([200, 140, 161] * 7, [70, 64, 130] * 7, 8, 8, 128, 128, 0, seed=9)
+    close(s.run(0.3, None), s.reference(0.3, None), SAFE[0])
+
+
 @pytest.mark.parametrize("tiles", [33, 47, 64, 65, 79, 96, 97, 131])
 @pytest.mark.parametrize("heads,kv", [(8, 8), (4, 4), (16, 16)])
 def test_every_tile_is_dealt_once(heads, kv, tiles):

@@ -1,26 +1,6 @@
 // Row-wise kernels of the decoder-only language models (include/omni_decoder.h): everything between two matrix products of a layer.
 // The residual stream is fp32; norms, gates and the token-shift state are fp32; only matrix operands are rounded (once) to bf16.
-#include "row_io.cuh"
-
-#define DR_THREADS 256
-#define DR_WAVES (DR_THREADS / 64)
-
-// sum over the workgroup, result in every thread; `buf` alternates between calls so that one barrier per sum is enough
-struct BlockSum {
-    float* lds;      // [2][DR_WAVES]
-    int flip;
-    __device__ __forceinline__ float operator()(float v) {
-        v = wave_sum(v);
-        float* b = lds + flip * DR_WAVES;
-        flip ^= 1;
-        if ((threadIdx.x & 63) == 0) b[threadIdx.x >> 6] = v;
-        __syncthreads();
-        float t = 0.f;
-#pragma unroll
-        for (int w = 0; w < DR_WAVES; ++w) t += b[w];
-        return t;
-    }
-};
+#include "stream_row.cuh"
 
 // A workgroup walks `strip` consecutive tokens so that the token shift finds the previous token's NEW stream row in registers; only the
 // strip's first token rebuilds its predecessor (or reads it from the sequence's state, or takes zeros).
@@ -31,88 +11,17 @@ struct BlockSum {
 template <typename E, int MAXC, bool SHIFT, bool SPLIT>
 __global__ __launch_bounds__(DR_THREADS) void stream_rows_kernel(const omni_stream_rows a, int strip) {
     __shared__ float red[2 * DR_WAVES];
-    BlockSum bsum{red, 0};
-    const int wp = a.wp;
-    const E* table = reinterpret_cast<const E*>(a.table);
-    const E* yw = reinterpret_cast<const E*>(a.y_w);
-    const E* fw = reinterpret_cast<const E*>(a.final_w);
+    StreamRow<E, MAXC, SPLIT> sr{a, (int)threadIdx.x, BlockSum{red, 0}};
+    using Pieces = typename StreamRow<E, MAXC, SPLIT>::Pieces;
     E* h_out = reinterpret_cast<E*>(a.h_out);
-    auto at = [&](int c) { return min((c * DR_THREADS + (int)threadIdx.x) * 4, wp - 4); };
-    auto in_row = [&](int c) { return (c * DR_THREADS + (int)threadIdx.x) * 4 < wp; };
-    struct Pieces {
-        raw4<float> x[MAXC];
-        slab_pieces<MAXC, SPLIT> y;
-    };
-    auto fetch = [&](int t, Pieces& r) {                   // (without y: x again, not used)
-        const float* x = a.x_in + (size_t)t * wp;
-#pragma unroll
-        for (int c = 0; c < MAXC; ++c) r.x[c].load(x + at(c));
-        r.y.load(a.y ? a.y + (size_t)t * wp : x, a.y_slabs, a.y_stride, at);
-    };
-    raw4<E> ywr[MAXC], mur[MAXC];
-    auto embed = [&](int t, float (&v)[MAXC][4]) {         // the stream row of token t: its table row
-        const int id = a.ids[t];
-        const bool ok = id >= 0 && id < a.vocab;
-        raw4<E> r[MAXC];
-#pragma unroll
-        for (int c = 0; c < MAXC; ++c) r[c].load(table + (size_t)(ok ? id : 0) * wp + at(c));
-#pragma unroll
-        for (int c = 0; c < MAXC; ++c) {
-            r[c].get(v[c]);
-#pragma unroll
-            for (int e = 0; e < 4; ++e) {
-                if (!ok || !in_row(c)) v[c][e] = 0.f;
-                if (a.table_scale != 0.f) v[c][e] *= a.table_scale;
-            }
-        }
-    };
-    auto join = [&](const Pieces& r, float (&v)[MAXC][4]) { // ... or its row behind the sublayer that just ran
-        float y[MAXC][4], ss = 0.f;
-#pragma unroll
-        for (int c = 0; c < MAXC; ++c) {
-            r.x[c].get(v[c]);
-            r.y.sum(c, a.y_slabs, y[c]);
-            if (!in_row(c)) {
-#pragma unroll
-                for (int e = 0; e < 4; ++e) v[c][e] = y[c][e] = 0.f;
-            }
-        }
-        if (!a.y) return;
-        if (a.post) {                                      // the norm takes the sum, not the sublayer's output
-#pragma unroll
-            for (int c = 0; c < MAXC; ++c)
-#pragma unroll
-                for (int e = 0; e < 4; ++e) { y[c][e] = fmaf(a.alpha, v[c][e], y[c][e]); v[c][e] = 0.f; }
-        }
-#pragma unroll
-        for (int c = 0; c < MAXC; ++c) ss += sq4_sum(y[c][0], y[c][1], y[c][2], y[c][3]);
-        ss = bsum(ss);
-        const float g = (yw ? 1.0f : a.gain) / sqrtf(ss / (float)a.width + a.eps);
-#pragma unroll
-        for (int c = 0; c < MAXC; ++c) {
-            if (yw) {
-                float w[4];
-                ywr[c].get(w);
-#pragma unroll
-                for (int e = 0; e < 4; ++e) y[c][e] *= in_row(c) ? w[e] : 0.f;
-            }
-#pragma unroll
-            for (int e = 0; e < 4; ++e) v[c][e] = fmaf(y[c][e], g, v[c][e]);
-        }
-    };
+    const int wp = a.wp;
     const int i0 = blockIdx.x * strip, i1 = min(i0 + strip, a.rows);
     float cur[MAXC][4], prev[MAXC][4];
     for (int i = i0; i < i1; ++i) {
         const int t = a.sel ? a.sel[i] : i;
         Pieces now;
-        if (!a.ids) fetch(t, now);
-        if (i == i0) {
-#pragma unroll
-            for (int c = 0; c < MAXC; ++c) {
-                if (yw) ywr[c].load(yw + at(c));
-                if (SHIFT) mur[c].load(reinterpret_cast<const E*>(a.mu) + at(c));
-            }
-        }
+        if (!a.ids) sr.fetch(t, now);
+        if (i == i0) sr.weights(SHIFT);
         if (SHIFT) {
             const int row = a.row_of_tok[t];
             const bool first = t == 0 || a.row_of_tok[t - 1] != row;
@@ -121,25 +30,15 @@ __global__ __launch_bounds__(DR_THREADS) void stream_rows_kernel(const omni_stre
 #pragma unroll
                     for (int c = 0; c < MAXC; ++c) prev[c][0] = prev[c][1] = prev[c][2] = prev[c][3] = 0.f;
                 } else {
-                    const float* st = a.state + (size_t)a.state_slot[row] * wp;
-                    raw4<float> r[MAXC];
-#pragma unroll
-                    for (int c = 0; c < MAXC; ++c) r[c].load(st + at(c));
-#pragma unroll
-                    for (int c = 0; c < MAXC; ++c) {
-                        r[c].get(prev[c]);
-#pragma unroll
-                        for (int e = 0; e < 4; ++e)
-                            if (!in_row(c)) prev[c][e] = 0.f;
-                    }
+                    sr.shifted_in(row, prev);
                 }
             } else if (i == i0) {
                 if (a.ids) {
-                    embed(t - 1, prev);
+                    sr.embed(t - 1, prev);
                 } else {
                     Pieces before;
-                    fetch(t - 1, before);
-                    join(before, prev);
+                    sr.fetch(t - 1, before);
+                    sr.join(before, prev);
                 }
             } else {
 #pragma unroll
@@ -148,15 +47,9 @@ __global__ __launch_bounds__(DR_THREADS) void stream_rows_kernel(const omni_stre
                     for (int e = 0; e < 4; ++e) prev[c][e] = cur[c][e];
             }
         }
-        if (a.ids) embed(t, cur);
-        else join(now, cur);
-        float rf = 0.f;
-        if (!SHIFT && a.use_final) {
-            float ss = 0.f;
-#pragma unroll
-            for (int c = 0; c < MAXC; ++c) ss += sq4_sum(cur[c][0], cur[c][1], cur[c][2], cur[c][3]);
-            rf = (fw ? 1.0f : a.final_gain) / sqrtf(bsum(ss) / (float)a.width + a.eps);
-        }
+        if (a.ids) sr.embed(t, cur);
+        else sr.join(now, cur);
+        const float rf = !SHIFT && a.use_final ? sr.final_factor(cur) : 0.f;
 #pragma unroll
         for (int c = 0; c < MAXC; ++c) {
             const int k = (c * DR_THREADS + threadIdx.x) * 4;
@@ -164,21 +57,7 @@ __global__ __launch_bounds__(DR_THREADS) void stream_rows_kernel(const omni_stre
             if (a.x_out) st4<float>(a.x_out + (size_t)t * wp + k, cur[c]);
             if (!h_out) continue;
             float h[4];
-            if (SHIFT) {
-                float m[4];
-                mur[c].get(m);
-#pragma unroll
-                for (int e = 0; e < 4; ++e) h[e] = fmaf(prev[c][e] - cur[c][e], m[e], cur[c][e]);
-            } else {
-#pragma unroll
-                for (int e = 0; e < 4; ++e) h[e] = a.use_final ? cur[c][e] * rf : cur[c][e];
-                if (a.use_final && fw) {
-                    float w[4];
-                    ld4<E>(fw + k, w);
-#pragma unroll
-                    for (int e = 0; e < 4; ++e) h[e] *= w[e];
-                }
-            }
+            sr.operand(SHIFT, c, cur[c], prev[c], rf, h);
             st4<E>(h_out + (a.frag ? frag_off(i, k, wp) : (size_t)i * wp + k), h);
         }
     }
@@ -205,8 +84,8 @@ static int stream_rows_pick(const omni_stream_rows& a, int strip, hipStream_t st
     return OMNI_OK;
 }
 
-extern "C" int omni_stream_rows_run(const omni_stream_rows* p, void* stream) {
-    OMNI_CHECK_ARG(p && (p->ids ? p->table != nullptr : p->x_in != nullptr) && (p->x_out || p->h_out), "omni_stream_rows: null pointer");
+int omni_stream_rows_check(const omni_stream_rows* p) {
+    OMNI_CHECK_ARG(p && (p->ids ? p->table != nullptr : p->x_in != nullptr), "omni_stream_rows: null pointer");
     const omni_stream_rows& a = *p;
     OMNI_CHECK_ARG(a.width > 0 && a.wp >= a.width && a.wp % 32 == 0 && a.wp <= DR_THREADS * 4 * 8, "omni_stream_rows: width=%d wp=%d (multiple of 32, <= 8192)", a.width, a.wp);
     OMNI_CHECK_ARG(a.y_slabs <= OMNI_STREAM_MAX_SPLITS, "omni_stream_rows: y_slabs=%d", a.y_slabs);
@@ -217,6 +96,14 @@ extern "C" int omni_stream_rows_run(const omni_stream_rows* p, void* stream) {
     OMNI_CHECK_ARG(!a.post || (a.y && !a.ids), "omni_stream_rows: the norm behind the sum needs y");
     // (a strip's first token and the shift read rows of x_in that another workgroup may already have rewritten: never in place)
     OMNI_CHECK_ARG(a.x_out == nullptr || a.x_out != a.x_in, "omni_stream_rows: x_out must not be x_in");
+    return OMNI_OK;
+}
+
+extern "C" int omni_stream_rows_run(const omni_stream_rows* p, void* stream) {
+    const int rc = omni_stream_rows_check(p);
+    if (rc != OMNI_OK) return rc;
+    const omni_stream_rows& a = *p;
+    OMNI_CHECK_ARG(a.x_out || a.h_out, "omni_stream_rows: null pointer");
     if (a.rows <= 0) return OMNI_OK;
     const int strip = a.mu && a.rows > 1024 ? 4 : 1;
     return a.elem ? stream_rows_pick<float>(a, strip, (hipStream_t)stream) : stream_rows_pick<uint16_t>(a, strip, (hipStream_t)stream);
@@ -298,8 +185,8 @@ __global__ __launch_bounds__(DR_THREADS) void latent_write_kernel(const omni_lat
     }
 }
 
-extern "C" int omni_latent_write_run(const omni_latent_write* p, void* stream) {
-    OMNI_CHECK_ARG(p && p->proj && p->qw && p->kw && p->cq && p->cache && p->block_table && p->row_of_tok && p->positions, "omni_latent_write: null pointer");
+int omni_latent_write_check(const omni_latent_write* p) {
+    OMNI_CHECK_ARG(p && p->proj && p->qw && p->kw && p->cache && p->block_table && p->row_of_tok && p->positions, "omni_latent_write: null pointer");
     const omni_latent_write& a = *p;
     OMNI_CHECK_ARG(a.q_rank > 0 && a.kv_rank > 0 && a.qp >= a.q_rank && a.rp >= a.kv_rank && a.qp % 32 == 0 && a.rp % 32 == 0 && a.ld % 4 == 0 &&
                    a.ld >= a.qp + a.rp + (a.gate ? a.heads : 0), "omni_latent_write: q %d / %d, kv %d / %d, ld %d", a.q_rank, a.qp, a.kv_rank, a.rp, a.ld);
@@ -308,6 +195,14 @@ extern "C" int omni_latent_write_run(const omni_latent_write* p, void* stream) {
     OMNI_CHECK_ARG(a.elem == 1 || a.elem == 0, "omni_latent_write: elem=%d", a.elem);
     OMNI_CHECK_ARG(!a.frag || a.elem == 0, "omni_latent_write: fragment-major output is bf16");
     OMNI_CHECK_ARG(a.slabs <= OMNI_STREAM_MAX_SPLITS, "omni_latent_write: slabs=%d", a.slabs);
+    return OMNI_OK;
+}
+
+extern "C" int omni_latent_write_run(const omni_latent_write* p, void* stream) {
+    const int rc = omni_latent_write_check(p);
+    if (rc != OMNI_OK) return rc;
+    const omni_latent_write& a = *p;
+    OMNI_CHECK_ARG(a.cq, "omni_latent_write: null pointer");
     OMNI_CHECK_ARG(a.ld <= 15 * 1024, "omni_latent_write: ld=%d (<= 15360: a token's projections are staged in LDS)", a.ld);
     if (a.T <= 0) return OMNI_OK;
     const size_t lds = (size_t)a.ld * sizeof(float);

@@ -261,6 +261,56 @@ __global__ __launch_bounds__(128) void latent_merge_kernel(const float* __restri
     *reinterpret_cast<uint2*>(out + rh * rp + k) = make_uint2(pack_bf2(v[0], v[1]), pack_bf2(v[2], v[3]));
 }
 
+// The merge inside the per-head product that follows, for one row or two: every workgroup merges its head's rows for itself (128 threads each) into LDS while
+// its weights are on their way, then multiplies as head_gemm_kernel does with its waves splitting K.  A merge of its own is 3.5 us of launch and trips to
+// memory: 16 heads, latents of 256, 352 keys, a step of 8 layers 301 -> 292 us.
+__global__ __launch_bounds__(256) void latent_values_kernel(const float* __restrict__ partial, const float* __restrict__ gate, const uint16_t* __restrict__ merged,
+                                                            const int32_t* __restrict__ positions, const uint16_t* __restrict__ w, uint16_t* __restrict__ out, int T, int heads,
+                                                            int max_split, int per, int rp, int n, int frag) {
+    constexpr int P = 4, WAVES = 4;
+    extern __shared__ __attribute__((aligned(16))) uint16_t xs[];      // [T][rp]
+    __shared__ f32x4 part[WAVES][64];
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), c = lane & 15, q = lane >> 4;
+    const int h = blockIdx.y, nt = blockIdx.x, nsteps = rp >> 5, mine = nsteps > wave ? (nsteps - wave + WAVES - 1) / WAVES : 0;
+    const uint16_t* wp = w + ((size_t)h * (n >> 4) + nt) * nsteps * 512 + lane * 8;
+    u32x4 W[P];
+    auto load = [&](int d, int s) { W[d] = ld16(wp + (size_t)min(wave + s * WAVES, nsteps - 1) * 512); };      // (past the last step: that one again, not used)
+    const int t = min(wave >> 1, T - 1), k = (threadIdx.x & 127) * 4;
+    const size_t rh = (size_t)t * heads + h;
+    const int nsplit = la_row_splits((positions[t] + 16) / 16, max_split, per);
+    const float* base = partial + rh * max_split * (rp + 4);
+    const float2 ml = lane < nsplit && nsplit > 1 ? *reinterpret_cast<const float2*>(base + (size_t)lane * (rp + 4)) : make_float2(LA_SENT, 0.f);
+    const uint2 whole = k < rp ? *reinterpret_cast<const uint2*>(merged + rh * rp + k) : make_uint2(0, 0);      // (one split: the decode kernel wrote the row)
+#pragma unroll
+    for (int d = 0; d < P; ++d) load(d, d);
+    const float M = wave_max(ml.x), e = lane < nsplit ? exp2f(ml.x - M) : 0.f, L = wave_sum(ml.y * e);
+    f32x4 m = (f32x4){0.f, 0.f, 0.f, 0.f};
+    if (k < rp && nsplit > 1)
+#pragma unroll 4
+        for (int s = 0; s < nsplit; ++s)
+            m += *reinterpret_cast<const f32x4*>(base + (size_t)s * (rp + 4) + 4 + k) * __int_as_float(__builtin_amdgcn_readlane(__float_as_int(e), s));
+    m *= (L > 0.f ? 1.0f / L : 0.f) * (gate ? gate[rh] : 1.0f);
+    if (k < rp && wave >> 1 == t) *reinterpret_cast<uint2*>(xs + (size_t)t * rp + k) = nsplit > 1 ? make_uint2(pack_bf2(m[0], m[1]), pack_bf2(m[2], m[3])) : whole;
+    __syncthreads();
+    const uint16_t* xp = xs + (size_t)min(c, T - 1) * rp + wave * 32 + 8 * q;
+    f32x4 acc = (f32x4){0.f, 0.f, 0.f, 0.f};
+    for (int s = 0; s < mine; s += P)
+#pragma unroll
+        for (int d = 0; d < P; ++d) {
+            if (s + d >= mine) break;
+            acc = mfma16(W[d], *reinterpret_cast<const u32x4*>(xp + (size_t)(s + d) * (WAVES * 32)), acc);
+            if (s + d + P < mine) load(d, s + d + P);
+        }
+    part[wave][lane] = acc;
+    __syncthreads();
+    if (wave > 0 || c >= T) return;
+    f32x4 v = part[0][lane];
+#pragma unroll
+    for (int u = 1; u < WAVES; ++u) v += part[u][lane];
+    const int col = h * n + nt * 16 + 4 * q;
+    *reinterpret_cast<uint2*>(out + (frag ? frag_off(c, col, heads * n) : (size_t)c * heads * n + col)) = make_uint2(pack_bf2(v[0], v[1]), pack_bf2(v[2], v[3]));
+}
+
 template <int RS, int PW>
 __global__ __launch_bounds__(64 * PW, 2) void latent_prefill_kernel(const LatentArgs a) {
     using G = LatentGeom<RS>;
@@ -455,8 +505,9 @@ static int la_lds(K kernel, int bytes) {
     return OMNI_OK;
 }
 
+struct LatentValues { const uint16_t* w; uint16_t* out; int n, frag; };      // the per-head product behind decode tokens; w NULL: none
 template <int RS>
-static int la_run(const omni_latent_attn& p, LatentArgs a, hipStream_t st) {
+static int la_run(const omni_latent_attn& p, LatentArgs a, const LatentValues& then, hipStream_t st) {
     using G = LatentGeom<RS>;
     if (p.n_decode > 0) {
         constexpr int LDS = LA_DEC_WAVES * 16 * G::PITCH + LA_DEC_WAVES / 2 * 3 * 1024;
@@ -469,7 +520,11 @@ static int la_run(const omni_latent_attn& p, LatentArgs a, hipStream_t st) {
         a.per = p.n_decode * ((p.heads + 15) / 16) <= 8 ? 4 : 8;
         hipLaunchKernelGGL(latent_decode_kernel<RS>, dim3((p.heads + 15) / 16, p.n_decode, a.nsplit), dim3(64 * LA_DEC_WAVES), LDS, st, a);
         OMNI_CHECK_LAUNCH("omni_latent_attn(decode)");
-        if (a.nsplit > 1) {
+        if (then.w) {
+            hipLaunchKernelGGL(latent_values_kernel, dim3(then.n / 16, p.heads), dim3(256), p.n_decode * p.rp * 2, st, (const float*)a.partial, a.gate, (const uint16_t*)a.out, a.positions,
+                               then.w, then.out, p.n_decode, p.heads, a.nsplit, a.per, p.rp, then.n, then.frag);
+            OMNI_CHECK_LAUNCH("omni_latent_attn(values)");
+        } else if (a.nsplit > 1) {
             hipLaunchKernelGGL(latent_merge_kernel, dim3(p.n_decode * p.heads), dim3(p.rp > 256 ? 128 : 64), 0, st, (const float*)a.partial, a.gate, a.out, a.positions, p.heads, a.nsplit, a.per, p.rp);
             OMNI_CHECK_LAUNCH("omni_latent_attn(merge)");
         }
@@ -484,7 +539,7 @@ static int la_run(const omni_latent_attn& p, LatentArgs a, hipStream_t st) {
     return OMNI_OK;
 }
 
-extern "C" int omni_latent_attn_run(const omni_latent_attn* pp, void* stream) {
+static int la_any(const omni_latent_attn* pp, const LatentValues& then, hipStream_t st) {
     OMNI_CHECK_ARG(pp && pp->q && pp->cache && pp->out && pp->block_table && pp->row_of_tok && pp->positions, "omni_latent_attn: null pointer");
     const omni_latent_attn& p = *pp;
     OMNI_CHECK_ARG(p.heads > 0 && p.rp > 0 && p.rp % 32 == 0 && p.rp <= LA_PLAIN_MAX, "omni_latent_attn: heads=%d latent width %d (multiple of 32, <= %d)", p.heads, p.rp, LA_PLAIN_MAX);
@@ -494,7 +549,6 @@ extern "C" int omni_latent_attn_run(const omni_latent_attn* pp, void* stream) {
     OMNI_CHECK_ARG(p.n_tiles == 0 || p.tile_rows == la_tile_rows(p.rp), "omni_latent_attn: tile_rows=%d (omni_latent_attn_tile_rows(%d) = %d)", p.tile_rows, p.rp, la_tile_rows(p.rp));
     OMNI_CHECK_ARG(!p.workspace || p.workspace_bytes >= omni_latent_attn_workspace_bytes(p.n_decode, p.heads, p.rp), "omni_latent_attn: workspace of %lld bytes", (long long)p.workspace_bytes);
     if (p.T <= 0) return OMNI_OK;
-    hipStream_t st = (hipStream_t)stream;
     if (p.elem == 1 || !omni_latent_attn_mfma(p.rp)) {
         const dim3 grid((unsigned)((int64_t)p.T * p.heads)), block(64);
         if (p.elem == 1)
@@ -512,9 +566,19 @@ extern "C" int omni_latent_attn_run(const omni_latent_attn* pp, void* stream) {
     a.row_of_tok = p.row_of_tok; a.positions = p.positions; a.tiles = p.tiles;
     a.heads = p.heads; a.qs = p.scale * LA_LOG2E; a.partial = p.workspace; a.nsplit = 1; a.per = 8;
     switch (p.rp / 32) {
-#define X(RS_) case RS_: return la_run<RS_>(p, a, st);
+#define X(RS_) case RS_: return la_run<RS_>(p, a, then, st);
         LA_WIDTHS(X)
 #undef X
         default: return OMNI_EINVAL;
     }
+}
+
+extern "C" int omni_latent_attn_run(const omni_latent_attn* p, void* stream) { return la_any(p, LatentValues{}, (hipStream_t)stream); }
+
+extern "C" int omni_latent_attn_values(const omni_latent_attn* p, const void* w, void* out, int n, int frag, void* stream) {
+    OMNI_CHECK_ARG(p && w && out, "omni_latent_attn_values: null pointer");
+    OMNI_CHECK_ARG(p->T >= 1 && p->T == p->n_decode && p->T <= OMNI_STREAM_LATENT_ROWS && p->n_tiles == 0 && p->elem == 0 && p->rp <= 512 && omni_latent_attn_mfma(p->rp),
+                   "omni_latent_attn_values: T=%d n_decode=%d rp=%d (decode tokens, <= %d, bf16)", p->T, p->n_decode, p->rp, OMNI_STREAM_LATENT_ROWS);
+    OMNI_CHECK_ARG(n > 0 && n % 16 == 0 && (!frag || p->heads * n % 32 == 0), "omni_latent_attn_values: n=%d (%% 16) frag=%d", n, frag);
+    return la_any(p, LatentValues{(const uint16_t*)w, (uint16_t*)out, n, frag}, (hipStream_t)stream);
 }

@@ -107,6 +107,15 @@ int omni_gemm_f32_rows(const float* x, int ldx, const float* w, float* out, int 
 int omni_gemm_stream(const void* x, const void* w, void* out, int M, int N, int K, int kind, int one, float act_p, float act_n, int out_frag, void* stream);
 int omni_gemm_stream_rows(const void* x, const void* w, void* out, int M, int N, int K, const omni_row_table* rt, int out_frag, void* stream);
 int omni_gemm_stream_splits(int M, int N, int K);
+/* omni_gemm_stream of a few rows that it makes itself, in one launch, bit for bit:
+ *   _joined:  the rows omni_stream_rows_run would leave in h_out (not written here; x_out is), K = wp: up to OMNI_STREAM_JOINED_ROWS of wp <= 1024, 2 of wp <=
+ *             2048.  kind 0, 2 or 3; rt != NULL: the row table's activation; with mu: kind 0
+ *   _latents: the rows omni_latent_write_run would leave in cq (not written here; cache, gate and state are), K = qp: up to OMNI_STREAM_LATENT_ROWS of ld <=
+ *             3072.  bf16 out, row-major                                                                                                             */
+#define OMNI_STREAM_JOINED_ROWS 4
+#define OMNI_STREAM_LATENT_ROWS 2
+int omni_gemm_stream_joined(const omni_stream_rows* r, const void* w, void* out, int N, int kind, int one, float act_p, float act_n, const omni_row_table* rt, int out_frag, void* stream);
+int omni_gemm_stream_latents(const omni_latent_write* r, const void* w, void* out, int N, void* stream);
 
 /* Causal attention over a paged cache of latents shared by all heads (keys and values are the same rp-wide rows):
  *   out[t, h] = gate[t, h] * sum_j softmax_j(scale * q[t, h] . c_j) c_j,   j <= positions[t],   q / out elem [T, heads, rp].
@@ -121,6 +130,9 @@ typedef struct omni_latent_attn {
     int T, n_decode, heads, rp; float scale; int max_keys; float* workspace; int64_t workspace_bytes; int elem;
 } omni_latent_attn;
 int omni_latent_attn_run(const omni_latent_attn* a, void* stream);
+/* Decode tokens alone (T = n_decode <= OMNI_STREAM_LATENT_ROWS, bf16, a width of omni_latent_attn_mfma, rp <= 512) and the per-head product behind it:
+ * out[t, h] = (what omni_latent_attn_run leaves in a->out) . w[h]^T as omni_head_gemm, in one launch less; a->out is scratch                        */
+int omni_latent_attn_values(const omni_latent_attn* a, const void* w, void* out, int n, int frag, void* stream);
 int64_t omni_latent_attn_workspace_bytes(int n_decode, int heads, int rp);
 int omni_latent_attn_tile_rows(int rp);
 /* 1 when the matrix-core kernels take this padded latent width (else the plain kernel runs it) */

@@ -184,6 +184,7 @@ SIGNATURES = {
     # include/omni_codec.h
     "omni_codec_rvq_embed": (i32, [vp, i32, vp, vp, i32, i32, i32, i32, vp]),
     "omni_codec_rmsnorm": (i32, [vp, i32, vp, f32, vp, i32, i32, vp]),
+    "omni_codec_add_rmsnorm": (i32, [vp, i32, vp, i32, i64, vp, vp, f32, vp, i32, i32, vp]),
     "omni_codec_rope": (i32, [vp, i32, i32, i32, i32, i32, f32, vp]),
     "omni_codec_window_attn": (i32, [vp, i32, vp, i32, i32, i32, i32, i32, i32, f32, vp]),
     "omni_codec_dwconv_ln": (i32, [vp, i32, vp, vp, vp, vp, f32, vp, i32, i32, i32, vp]),

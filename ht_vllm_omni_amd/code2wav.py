@@ -33,6 +33,9 @@ from .engine import frag_shuffle, gu8_shuffle
 
 logger = logging.getLogger(__name__)
 BF16 = torch.bfloat16
+# Up to so many frames the transformer's products that join the stream may leave partial sums (their tiles are fewer than the compute units: 50 rows x 1024 columns
+# are 64).  Measured, us, the decode of 12 frames 890 / 870, 30 989 / 966, 50 1087 / 1062, 75 1703 / 1684, 325 4407 / 4376; of 160 and 230 the same
+SPLIT_FRAMES = 512
 
 
 @dataclass
@@ -272,17 +275,39 @@ class Code2WavDecoder:
         h = self.in_proj(x, want="f")
         a = torch.empty(T, H, dtype=BF16, device=dev)
         attn = torch.empty(T, nh * hd, dtype=BF16, device=dev)
+        # few frames: the products that join the stream leave partial sums over K, which the next norm adds up
+        behind = None
+        few = T <= SPLIT_FRAMES and H <= 1024
+        parts = torch.empty(L.STREAM_MAX_SPLITS, T, H, dtype=torch.float32, device=dev) if few else None
+
+        def joins(g, x):
+            nonlocal behind
+            n = lib.omni_gemm_tile_splits(T, H, x.shape[1]) if few else 1
+            if n == 1:
+                g(x, resid=h, out_f32=h, want="f")
+            else:
+                ops.gemm_tile(x, g.w, out_f32=parts[:n], want="f", splits=n)
+                behind = n, g.scale
+
+        def norm(w):
+            nonlocal behind
+            if behind is None:
+                self._check(lib.omni_codec_rmsnorm(h.data_ptr(), H, w.data_ptr(), c.rms_norm_eps, a.data_ptr(), T, H, st), "omni_codec_rmsnorm")
+            else:
+                n, scale = behind
+                self._check(lib.omni_codec_add_rmsnorm(h.data_ptr(), H, parts.data_ptr(), n, T * H, scale.data_ptr(), w.data_ptr(), c.rms_norm_eps, a.data_ptr(), T, H, st),
+                            "omni_codec_add_rmsnorm")
+                behind = None
         for lw in self.layers:
-            self._check(lib.omni_codec_rmsnorm(h.data_ptr(), H, lw["ln1"].data_ptr(), c.rms_norm_eps, a.data_ptr(), T, H, st), "omni_codec_rmsnorm")
+            norm(lw["ln1"])
             qkv = lw["qkv"](a)
             self._check(lib.omni_codec_rope(qkv.data_ptr(), qkv.stride(0), T, nh, nkv, hd, float(c.rope_theta), st), "omni_codec_rope")
             self._check(lib.omni_codec_window_attn(qkv.data_ptr(), qkv.stride(0), attn.data_ptr(), attn.stride(0), T, nh, nkv, hd,
                                                    c.sliding_window, hd ** -0.5, st), "omni_codec_window_attn")
-            lw["o"](attn, resid=h, out_f32=h, want="f")
-            self._check(lib.omni_codec_rmsnorm(h.data_ptr(), H, lw["ln2"].data_ptr(), c.rms_norm_eps, a.data_ptr(), T, H, st), "omni_codec_rmsnorm")
-            act = lw["gu"](a, act=L.TILE_ACT_SILU_MUL_GU8)
-            lw["down"](act, resid=h, out_f32=h, want="f")
-        self._check(lib.omni_codec_rmsnorm(h.data_ptr(), H, self.final_norm.data_ptr(), c.rms_norm_eps, a.data_ptr(), T, H, st), "omni_codec_rmsnorm")
+            joins(lw["o"], attn)
+            norm(lw["ln2"])
+            joins(lw["down"], lw["gu"](a, act=L.TILE_ACT_SILU_MUL_GU8))
+        norm(self.final_norm)
         x = self.out_proj(a)
         tap("pre_transformer", x)
         # ---- upsample stages

@@ -60,9 +60,11 @@ extern "C" int omni_codec_rvq_embed(const int64_t* codes, int ld_codes, const fl
 // ---------------------------------------------------------------- RMSNorm of the fp32 stream: one wave per row
 // The row and the weights are asked for at once and stay in registers (PIECES of 256 columns; the row was walked twice, a wait per piece).  Measured in the
 // decode of 50 frames, 17 of these launches over 50 rows of 1024: 1158 -> 1143 us.  Wider rows take the kernel that walks them.
-template <int PIECES>
-__global__ __launch_bounds__(256) void codec_rmsnorm_kernel(const float* __restrict__ x, int ldx, const float* __restrict__ w, float eps,
-                                                            uint16_t* __restrict__ out, int T, int H) {
+// ADD: what the sublayer in front left joins the row first: partial sums of a product whose few tiles would each walk all of K alone (omni_gemm_tile k_splits).
+struct CodecAdd { float* x; const float* y; const float* scale; int slabs; long long stride; };
+template <int PIECES, bool ADD>
+__global__ __launch_bounds__(256) void codec_rmsnorm_kernel(const float* x, int ldx, const float* __restrict__ w, float eps,
+                                                            uint16_t* __restrict__ out, int T, int H, const CodecAdd add) {
     const int lane = threadIdx.x & 63;
     const int t = blockIdx.x * 4 + (threadIdx.x >> 6);
     if (t >= T) return;
@@ -72,6 +74,26 @@ __global__ __launch_bounds__(256) void codec_rmsnorm_kernel(const float* __restr
     for (int i = 0; i < PIECES; ++i) v[i] = *reinterpret_cast<const f32x4*>(xr + min(lane * 4 + 256 * i, H - 4));
 #pragma unroll
     for (int i = 0; i < PIECES; ++i) g[i] = *reinterpret_cast<const f32x4*>(w + min(lane * 4 + 256 * i, H - 4));
+    if constexpr (ADD) {
+        constexpr int S = 4;                               // all partial sums leave at once (past the last: that one again, not added)
+        f32x4 y[PIECES][S], sc[PIECES];
+#pragma unroll
+        for (int i = 0; i < PIECES; ++i)
+#pragma unroll
+            for (int s = 0; s < S; ++s) y[i][s] = *reinterpret_cast<const f32x4*>(add.y + min(s, add.slabs - 1) * add.stride + (size_t)t * H + min(lane * 4 + 256 * i, H - 4));
+#pragma unroll
+        for (int i = 0; i < PIECES; ++i) sc[i] = *reinterpret_cast<const f32x4*>(add.scale + min(lane * 4 + 256 * i, H - 4));
+#pragma unroll
+        for (int i = 0; i < PIECES; ++i) {
+#pragma unroll
+            for (int s = 1; s < S; ++s)
+#pragma unroll
+                for (int e = 0; e < 4; ++e) y[i][0][e] += s < add.slabs ? y[i][s][e] : 0.f;
+#pragma unroll
+            for (int e = 0; e < 4; ++e) v[i][e] = fmaf(y[i][0][e], sc[i][e], v[i][e]);
+            if (lane * 4 + 256 * i < H) *reinterpret_cast<f32x4*>(add.x + (size_t)t * ldx + lane * 4 + 256 * i) = v[i];
+        }
+    }
     float ss = 0.f;
 #pragma unroll
     for (int i = 0; i < PIECES; ++i)
@@ -113,10 +135,21 @@ __global__ __launch_bounds__(256) void codec_rmsnorm_wide_kernel(const float* __
 extern "C" int omni_codec_rmsnorm(const float* x, int ldx, const float* w, float eps, void* out, int T, int H, void* stream) {
     OMNI_CHECK_ARG(x && w && out && T > 0 && H > 0 && H % 4 == 0 && ldx >= H && ldx % 4 == 0, "omni_codec_rmsnorm: T=%d H=%d ldx=%d", T, H, ldx);
     const dim3 grid((T + 3) / 4), block(256);
-    if (H <= 512) hipLaunchKernelGGL(codec_rmsnorm_kernel<2>, grid, block, 0, (hipStream_t)stream, x, ldx, w, eps, (uint16_t*)out, T, H);
-    else if (H <= 1024) hipLaunchKernelGGL(codec_rmsnorm_kernel<4>, grid, block, 0, (hipStream_t)stream, x, ldx, w, eps, (uint16_t*)out, T, H);
+    if (H <= 512) hipLaunchKernelGGL((codec_rmsnorm_kernel<2, false>), grid, block, 0, (hipStream_t)stream, x, ldx, w, eps, (uint16_t*)out, T, H, CodecAdd{});
+    else if (H <= 1024) hipLaunchKernelGGL((codec_rmsnorm_kernel<4, false>), grid, block, 0, (hipStream_t)stream, x, ldx, w, eps, (uint16_t*)out, T, H, CodecAdd{});
     else hipLaunchKernelGGL(codec_rmsnorm_wide_kernel, grid, block, 0, (hipStream_t)stream, x, ldx, w, eps, (uint16_t*)out, T, H);
     OMNI_CHECK_LAUNCH("omni_codec_rmsnorm");
+    return OMNI_OK;
+}
+
+extern "C" int omni_codec_add_rmsnorm(float* x, int ldx, const float* y, int slabs, int64_t slab_stride, const float* scale, const float* w, float eps, void* out, int T, int H, void* stream) {
+    OMNI_CHECK_ARG(x && y && scale && w && out && T > 0 && H > 0 && H % 4 == 0 && H <= 1024 && ldx >= H && ldx % 4 == 0 && slabs >= 1 && slabs <= 4 &&
+                   (slabs == 1 || slab_stride >= (int64_t)T * H) && slab_stride % 4 == 0, "omni_codec_add_rmsnorm: T=%d H=%d (<= 1024) ldx=%d slabs=%d (<= 4)", T, H, ldx, slabs);
+    const dim3 grid((T + 3) / 4), block(256);
+    const CodecAdd add{x, y, scale, slabs, slab_stride};
+    if (H <= 512) hipLaunchKernelGGL((codec_rmsnorm_kernel<2, true>), grid, block, 0, (hipStream_t)stream, x, ldx, w, eps, (uint16_t*)out, T, H, add);
+    else hipLaunchKernelGGL((codec_rmsnorm_kernel<4, true>), grid, block, 0, (hipStream_t)stream, x, ldx, w, eps, (uint16_t*)out, T, H, add);
+    OMNI_CHECK_LAUNCH("omni_codec_add_rmsnorm");
     return OMNI_OK;
 }
 

@@ -26,6 +26,9 @@ int omni_codec_rvq_embed(const int64_t* codes, int ld_codes, const float* table,
 
 /* Qwen3TTSTokenizerV2DecoderRMSNorm (…:397-414) on the fp32 residual stream: out bf16 [T, H] = w * (x * rsqrt(mean(x^2) + eps)). */
 int omni_codec_rmsnorm(const float* x, int ldx, const float* w, float eps, void* out, int T, int H, void* stream);
+/* ... behind x += scale * (the sum of `slabs` <= 4 arrays y [T, H], slab_stride elements apart), scale fp32 [H]; H <= 1024 */
+int omni_codec_add_rmsnorm(float* x, int ldx, const float* y, int slabs, int64_t slab_stride, const float* scale, const float* w, float eps, void* out, int T, int H,
+                           void* stream);
 
 /* apply_rotary_pos_emb (…:90-121) with the default rope init (…:51-66), positions 0..T-1, in place on the q and k heads of fused
  * qkv rows: bf16 [T, ld], row = [q_heads | kv_heads (k) | kv_heads (v)] x head_dim. */

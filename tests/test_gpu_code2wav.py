@@ -257,6 +257,28 @@ def test_codec_norm(H):
     assert bool(((out[:T].double() - ref).abs() <= ref.abs() * (2.0 ** -8 + 2.0 ** -16)).all()) and bool((out[T:] == 7.0).all())
 
 
+@pytest.mark.parametrize("H", [4, 260, 512, 516, 1024])
+@pytest.mark.parametrize("T,slabs", [(1, 1), (7, 2), (50, 4), (9, 3)])
+def test_norm_behind_partial_sums(H, T, slabs):
+    """The stream takes the scaled sum, whatever stands behind the last slab, and the norm takes the stream.  Bounds: of the stream half a unit in the last place (2^-24)
+    of the magnitudes for each of slabs + 1 operations; of the output one rounding to bf16 beside fp32 sums, from the stream as it came out."""
+    from ht_vllm_omni_amd import _lib as L
+    g = torch.Generator().manual_seed(H + T)
+    x, w, sc = torch.randn(T, H + 4, generator=g) * 3, torch.randn(H, generator=g), torch.randn(H, generator=g) * 0.3
+    y = torch.full((slabs + 1, T, H), float("nan"))
+    y[:slabs] = torch.randn(slabs, T, H, generator=g)
+    xd, yd, wd, sd = (t.cuda() for t in (x, y, w, sc))
+    out = torch.full((T + 1, H), 7.0, dtype=torch.bfloat16, device="cuda")
+    L.check(L.load().omni_codec_add_rmsnorm(xd.data_ptr(), H + 4, yd.data_ptr(), slabs, T * H, sd.data_ptr(), wd.data_ptr(), 1e-5, out.data_ptr(), T, H, L.current_stream()), "add")
+    got = xd.cpu()
+    ref = x[:, :H].double() + sc.double() * y[:slabs].double().sum(0)
+    mag = x[:, :H].double().abs() + sc.double().abs() * y[:slabs].double().abs().sum(0)
+    assert bool(((got[:, :H].double() - ref).abs() <= mag * (slabs + 1) * 2.0 ** -24).all()) and torch.equal(got[:, H:], x[:, H:])
+    v = got[:, :H].double()
+    ref = w.double() * v / torch.sqrt(v.pow(2).mean(-1, keepdim=True) + 1e-5)
+    assert bool(((out[:T].cpu().double() - ref).abs() <= ref.abs() * (2.0 ** -8 + 2.0 ** -16)).all()) and bool((out[T:] == 7.0).all())
+
+
 @pytest.mark.parametrize("C,T,taps", [(8, 1, 7), (96, 255, 7), (96, 257, 7), (72, 600, 3), (96, 300, 1), (112, 513, 12), (256, 300, 7), (520, 260, 7)])
 def test_last_conv(C, T, taps):
     """Blocks of 256 samples and their edges, samples before the first whole window, rows in LDS and rows too wide for it.  Bound: 2^-24 of the sum of

@@ -39,9 +39,9 @@ __device__ __forceinline__ u32x4 la_transposed_at(const unsigned char* img, int 
     return (u32x4){x[0], x[1], y[0], y[1]};
 }
 
-// workgroups of a decode launch -> KV splits: two workgroups per CU, at least one 16-key tile per wave and split
-static inline int la_split_count(int wgs, int max_keys) {
-    int ns = 512 / (wgs > 0 ? wgs : 1);
+// workgroups of a decode launch -> KV splits: as many as make `fill` workgroups, at least one 16-key tile per wave and split
+static inline int la_split_count(int wgs, int max_keys, int fill) {
+    int ns = fill / (wgs > 0 ? wgs : 1);
     const int cap = (max_keys + 63) / 64;
     if (ns > cap) ns = cap;
     if (ns > LA_MAX_SPLIT) ns = LA_MAX_SPLIT;

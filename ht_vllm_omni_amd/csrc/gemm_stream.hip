@@ -300,18 +300,22 @@ __global__ __launch_bounds__(GS_THREADS) void gemm_behind_kernel(const StreamArg
     gs_store<1, NT, KIND>(a, part, 0);
 }
 
-// Columns per workgroup and K splits.  A workgroup's registers and LDS leave room for one per CU at 64 rows, so a grid runs in rounds of 256; a
-// workgroup's time goes with the operand tiles it reads (NT of W and MT of x per k-step) plus its epilogue, a split also costs its consumer.
-// Measured at 64 rows: 9216 x 2048 by 3 (192 workgroups) 12.1 us, by 2 (288: two rounds) 15.0; 2048 x 9216 by 2 in 4 splits (256) 11.4, in 6 13.3.
+// Columns per workgroup and K splits.  At more than 32 rows a workgroup's registers and LDS leave room for one per CU, so a grid runs in rounds of 256; below,
+// several share a CU and a further round costs three quarters of the first.  A workgroup's time goes with the operand tiles it reads per k-step (NT of W; of x,
+// which is in L2, three quarters of MT) plus its epilogue, NT * MT sums of eight waves through LDS; a split also costs its reader.
+// Measured over 1 ... 64 rows x the weight shapes of the language models, 1600 products out of HBM, the reader of partial sums at 30 ns and 8 TB/s a slab: what
+// the rule picks is 0.5 % behind the best on average (rounds in full, MT in full and a fifth of the epilogue: 2.1 %).  Us, before / now, 8 rows, rows x K:
+// 8192 x 2048 8.9 / 7.8 (4 column tiles in 2 splits / 2 in one), 5120 x 2048 6.4 / 5.8, 5120 x 1024 4.5 / 4.4, 1024 x 2048 3.4 / 3.0; 64 rows 8192 x 2048 10.9 / 10.1.
+// As before: 9216 x 2048 by 3 (192 workgroups; by 2, 288 of them, 2 us more), 2048 x 9216 by 2 in 4 splits.
 static void gs_policy(int M, int N, int nsteps, bool slabs, int* nt, int* splits) {
     const int tiles = N / 16, mt = M > 32 ? 4 : (M > 16 ? 2 : 1);
     long best = -1;
     for (int n = 1; n <= 4; ++n) {
         if (tiles % n) continue;
         for (int s = 1; s <= (slabs ? OMNI_STREAM_MAX_SPLITS : 1); ++s) {
-            if (s > 1 && nsteps / s < 2 * GS_WAVES) break;
-            const long rounds = ((long)tiles / n * s + 255) / 256;
-            const long cost = rounds * ((n + mt) * ((nsteps + s - 1) / s) + 4 * n * mt) + 12 * s;
+            if (s > 1 && nsteps / s < GS_WAVES) break;
+            const long rounds = ((long)tiles / n * s + 255) / 256, quarters = mt == 4 ? 4 * rounds : 1 + 3 * rounds;
+            const long cost = quarters * ((4 * n + 3 * mt) * ((nsteps + s - 1) / s) + (mt == 4 ? 44 : 80) * n * mt) + (mt == 4 ? 0 : 128) * s;
             if (best < 0 || cost < best) { best = cost; *nt = n; *splits = s; }
         }
     }

@@ -1,6 +1,6 @@
 // Linear recurrence with one decay per head (include/omni_decoder.h omni_decay_rec): S <- decay S + k v^T, out = S^T q, fp32 state per sequence.
 //
-//   rec_run_kernel          token by token: a workgroup keeps 64 or 128 columns of one head's S in registers while it walks its tokens.  A decoded token
+//   rec_run_kernel          token by token: a workgroup keeps 32, 64 or 128 columns of one head's S in registers while it walks its tokens.  A decoded token
 //                           is a run of one: S is read and written once -- that traffic is the op's bound
 //   chunks of 128 tokens, for prompts (matrix cores; a decay's powers enter as fp32 factors, fp32 operands as three bf16 terms whose sum is the value):
 //   rec_chunk_state_kernel  what a chunk adds to S:  sum_j decay^(n-1-j) k_j v_j^T, every chunk on its own
@@ -17,6 +17,30 @@ __device__ __forceinline__ float rc_silu(float z) { return z * sigmoidf_(z); }
 
 // ---- token by token.  Threads: CQ column quads x 256 / CQ row groups; row group g owns rows g, g + 256 / CQ, ...
 // RAW: projections fp32 (partial sums), SiLU here; else bf16 behind it
+template <bool RAW>
+struct RcValues {                    // four values of a token's projections, as loaded: on their way while the state is asked for and the token before is summed
+    slab_pieces<1, true> raw;
+    __device__ __forceinline__ void load(const omni_decay_rec& a, int t, int c) {
+        raw.load(reinterpret_cast<const float*>(a.proj) + (size_t)t * a.ld + c, a.slabs, a.slab_stride, [](int) { return 0; });
+    }
+    static __device__ __forceinline__ void now(const omni_decay_rec& a, int t, int c, float (&v)[4]) {
+        ld4_slabs(reinterpret_cast<const float*>(a.proj) + (size_t)t * a.ld + c, a.slabs, a.slab_stride, v);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) v[e] = rc_silu(v[e]);
+    }
+    __device__ __forceinline__ void get(int slabs, float (&v)[4]) const {
+        raw.sum(0, slabs, v);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) v[e] = rc_silu(v[e]);
+    }
+};
+template <>
+struct RcValues<false> {
+    raw4<uint16_t> raw;
+    __device__ __forceinline__ void load(const omni_decay_rec& a, int t, int c) { raw.load(reinterpret_cast<const uint16_t*>(a.proj) + (size_t)t * a.ld + c); }
+    __device__ __forceinline__ void get(int, float (&v)[4]) const { raw.get(v); }
+    static __device__ __forceinline__ void now(const omni_decay_rec& a, int t, int c, float (&v)[4]) { ld4<uint16_t>(reinterpret_cast<const uint16_t*>(a.proj) + (size_t)t * a.ld + c, v); }
+};
 template <int CQ, int MAXR, bool RAW>
 __global__ __launch_bounds__(256) void rec_run_kernel(const omni_decay_rec a, const int32_t* items) {
     constexpr int RG = 256 / CQ;
@@ -27,7 +51,16 @@ __global__ __launch_bounds__(256) void rec_run_kernel(const omni_decay_rec a, co
     const int row = a.row_of_tok[t0];
     if (a.num_live && row >= *a.num_live) return;
     const int cq = tid % CQ, g = tid / CQ, col = (blockIdx.x * CQ + cq) * 4;
-    const bool mine = col < a.vp;
+    const bool mine = col < a.vp, qk = tid * 4 < 2 * a.dp;      // (2 dp <= 1024: a thread's four of q or k)
+    RcValues<RAW> zqk, zv;
+    const int cqk = !qk ? 0 : tid * 4 < a.dp ? h * a.dp + tid * 4 : a.heads * a.dp + h * a.dp + tid * 4 - a.dp, cv = 2 * a.heads * a.dp + h * a.vp + (mine ? col : 0);
+    // ahead of the state and a token early where few workgroups wait for trips to memory; where many share a CU, their number -- registers -- hides those
+    // (64 sequences: 23.2 us a layer, 26 with the values held)
+    constexpr bool AHEAD = CQ == 8;
+    if constexpr (AHEAD) {
+        zqk.load(a, t0, cqk);
+        zv.load(a, t0, cv);
+    }
     float* sq = qk_lds;
     float* sk = qk_lds + a.dp;
     float* st = a.state + ((size_t)a.state_slot[row] * a.heads + h) * a.dp * a.vp + col;
@@ -40,24 +73,19 @@ __global__ __launch_bounds__(256) void rec_run_kernel(const omni_decay_rec a, co
         if (mine && !zero && d < a.dp) S[i] = *reinterpret_cast<const f32x4*>(st + (size_t)d * a.vp);
     }
     const float decay = a.decay[h];
-    auto value = [&](int t, int c, float (&v)[4]) {
-        if constexpr (RAW) {
-            ld4_slabs(reinterpret_cast<const float*>(a.proj) + (size_t)t * a.ld + c, a.slabs, a.slab_stride, v);
-#pragma unroll
-            for (int e = 0; e < 4; ++e) v[e] = rc_silu(v[e]);
-        } else {
-            ld4<uint16_t>(reinterpret_cast<const uint16_t*>(a.proj) + (size_t)t * a.ld + c, v);
-        }
-    };
-    const int kcol = a.heads * a.dp, vcol = 2 * a.heads * a.dp;
     for (int t = t0; t < t0 + n; ++t) {
-        for (int c = tid * 4; c < 2 * a.dp; c += 1024) {
-            float z[4];
-            value(t, c < a.dp ? h * a.dp + c : kcol + h * a.dp + c - a.dp, z);
-            st4<float>(qk_lds + c, z);
+        float z[4], v[4];
+        if constexpr (AHEAD) {
+            zqk.get(a.slabs, z);
+            zv.get(a.slabs, v);
         }
-        float v[4] = {0.f, 0.f, 0.f, 0.f};
-        if (mine) value(t, vcol + h * a.vp + col, v);
+        if (!AHEAD && qk) RcValues<RAW>::now(a, t, cqk, z);
+        if (qk) st4<float>(qk_lds + tid * 4, z);
+        if constexpr (!AHEAD) RcValues<RAW>::now(a, t, cv, v);
+        if (AHEAD && t + 1 < t0 + n) {
+            zqk.load(a, t + 1, cqk);
+            zv.load(a, t + 1, cv);
+        }
         __syncthreads();                              // q and k of this token
         f32x4 o = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
@@ -72,7 +100,10 @@ __global__ __launch_bounds__(256) void rec_run_kernel(const omni_decay_rec a, co
             }
         }
 #pragma unroll
-        for (int e = 0; e < 4; ++e) o[e] = xor32_sum(CQ == 16 ? xor16_sum(o[e]) : o[e]);
+        for (int e = 0; e < 4; ++e) {
+            if (CQ == 8) o[e] += dpp_f<OMNI_DPP_ROR8>(o[e]);
+            o[e] = xor32_sum(CQ <= 16 ? xor16_sum(o[e]) : o[e]);
+        }
         if ((tid & 63) < CQ) red[tid >> 6][cq] = o;
         __syncthreads();                              // the waves' sums (and: nobody reads this token's q, k any more)
         if (tid < CQ && mine) {
@@ -329,7 +360,11 @@ static void rec_runs_launch(const omni_decay_rec& a, const int32_t* items, int n
 template <bool RAW>
 static int rec_runs(const omni_decay_rec& a, const int32_t* items, int n, hipStream_t st) {
     if (n <= 0) return OMNI_OK;
-    if (a.vp > 64 && a.dp <= 256) rec_runs_launch<32, RAW>(a, items, n, st);
+    // Columns per workgroup: 32 where 128 would leave CUs idle -- a state is then asked for by four times as many waves -- else 128, whose q and k are summed and
+    // activated once.  Us, 16 heads of 128 x 128, one token of 1 | 2 | 4 | 8 | 12 | 16 | 24 | 48 sequences, by 128 columns 7.5 | 7.7 | 8.1 | 9.0 | 9.9 | 11.0 | 14.8 | 22.0, by 32
+    // 4.4 | 4.7 | 5.1 | 6.4 | 7.6 | 9.2 | 14.7 | 23.6.
+    if ((int64_t)a.heads * n * ((a.vp + 127) / 128) <= 256) rec_runs_launch<8, RAW>(a, items, n, st);
+    else if (a.vp > 64 && a.dp <= 256) rec_runs_launch<32, RAW>(a, items, n, st);
     else rec_runs_launch<16, RAW>(a, items, n, st);
     OMNI_CHECK_LAUNCH("omni_decay_rec(runs)");
     return OMNI_OK;

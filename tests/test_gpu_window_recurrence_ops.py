@@ -477,6 +477,13 @@ def test_rows_past_the_live_count_keep_their_state():
     run_recurrence([1, 1, 1, 1], [4, 0, 9, 2], 2, 40, 24, [0.9, 0.7], "sums", dead=(2, 3))
 
 
+@pytest.mark.parametrize("form", ["sums", "rows"])
+@pytest.mark.parametrize("heads,dim,vdim,n", [(16, 32, 40, 16), (16, 32, 40, 17), (16, 264, 72, 17), (16, 40, 136, 8), (16, 40, 136, 9), (20, 130, 8, 12), (20, 130, 8, 13)])
+def test_runs_by_32_64_and_128_columns(heads, dim, vdim, n, form):
+    """As many workgroups of 128 columns as compute units and more, one token and two of every sequence, sequences that begin."""
+    run_recurrence([1] * (n - 1) + [2], [r % 3 for r in range(n)], heads, dim, vdim, [0.9 - 0.02 * h for h in range(heads)], form, seed=n + dim)
+
+
 def test_argument_errors_come_back_as_errors():
     lib = L.load_decoder()
     for fn, s in (("omni_qkv_write_run", L.QkvWrite()), ("omni_gated_norm_run", L.GatedNorm()), ("omni_window_attn_run", L.WindowAttn()), ("omni_decay_rec_run", L.DecayRec())):

@@ -56,7 +56,7 @@ __device__ __forceinline__ void ld4_slabs(const float* p, int slabs, int64_t str
 }
 
 // N such pieces of an array, piece c at element at(c): all their loads leave before the first piece is added up, with no branch between them (a branch per
-// piece, taken or not, is a wait per piece).  SPLIT: more than one slab
+// piece, taken or not, is a wait per piece).  SPLIT: there may be more than one slab (0, 1: one)
 template <int N, bool SPLIT>
 struct slab_pieces {
     raw4<float> z[N][SPLIT ? OMNI_STREAM_MAX_SPLITS : 1];
@@ -65,7 +65,7 @@ struct slab_pieces {
 #pragma unroll
         for (int c = 0; c < N; ++c)
 #pragma unroll
-            for (int s = 0; s < (SPLIT ? OMNI_STREAM_MAX_SPLITS : 1); ++s) z[c][s].load(p + at(c) + (SPLIT ? min(s, slabs - 1) * stride : 0));
+            for (int s = 0; s < (SPLIT ? OMNI_STREAM_MAX_SPLITS : 1); ++s) z[c][s].load(p + at(c) + (SPLIT ? min(s, max(slabs, 1) - 1) * stride : 0));
     }
     __device__ __forceinline__ void sum(int c, int slabs, float (&v)[4]) const {
         z[c][0].get(v);

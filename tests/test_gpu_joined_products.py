@@ -81,7 +81,7 @@ def test_rows_of_the_stream(form, rows, width, N):
         src.update(post=1, alpha=1.6, y_w=r(1, dt=BF))
         kind, frag = 3, 1
     elif form == "plain":
-        kind = 2
+        kind, src["y"], src["y_slabs"] = 2, r(1, T), 0      # no count of slabs is one
     elif form == "final":
         src.update(use_final=1, final_w=r(1, dt=BF), sel=dev(torch.randperm(T, generator=g).to(torch.int32)))
         one = 1
@@ -115,12 +115,12 @@ def test_latents(T, q_rank, kv_rank, heads, N, form):
     g = gen(T + q_rank + N)
     r32 = lambda n: (n + 31) // 32 * 32  # noqa: E731
     qp, rp = r32(q_rank), r32(kv_rank)
-    ld, W, bs, slabs = qp + rp + r32(heads), 96, 4, 1 + (q_rank + T) % 4
+    ld, W, bs, slabs = qp + rp + r32(heads), 96, 4, 1 if form == "one sequence" else 1 + (q_rank + T) % 4
     parts = torch.zeros(slabs, T, ld)
     parts[..., :q_rank], parts[..., qp:qp + kv_rank] = torch.randn(slabs, T, q_rank, generator=g), torch.randn(slabs, T, kv_rank, generator=g)
     parts[..., qp + rp:qp + rp + heads] = torch.randn(slabs, T, heads, generator=g)
     w = dev(torch.randn(N * qp, generator=g) * 0.1, BF)
-    fixed = dict(proj=dev(parts), slabs=slabs, slab_stride=T * ld, ld=ld, q_rank=q_rank, qp=qp, kv_rank=kv_rank, rp=rp, heads=max(heads, 1), qw=dev(padc(torch.randn(q_rank, generator=g), qp), BF),
+    fixed = dict(proj=dev(parts), slabs=0 if form == "one sequence" else slabs, slab_stride=T * ld, ld=ld, q_rank=q_rank, qp=qp, kv_rank=kv_rank, rp=rp, heads=max(heads, 1), qw=dev(padc(torch.randn(q_rank, generator=g), qp), BF),
                  kw=dev(padc(torch.randn(kv_rank, generator=g), rp), BF), eps=1e-6, block_table=dev(torch.tensor([[2, 0, 1], [4, 3, 5]], dtype=torch.int32)), bt_stride=3, block_size=bs,
                  row_of_tok=dev(torch.tensor([0, 0 if form == "one sequence" else 1], dtype=torch.int32)[:T]), positions=dev(torch.tensor([6, 7], dtype=torch.int32)[:T]),
                  x=dev(torch.randn(T, W, generator=g)), wp=W, state_slot=dev(torch.tensor([1, 2], dtype=torch.int32)), T=T, elem=0)

@@ -58,7 +58,7 @@ __device__ __forceinline__ void gs_store(const StreamArgs& a, const f32x4* part,
     }}
 
 // P: k-steps in flight per wave: 2 on a grid that fills the chip (4 measured the same or slower at 1 .. 64 rows).
-// grid.z: groups of MT row tiles (more than one on narrow products only)
+// grid.z: groups of MT row tiles (more than one where the columns alone leave CUs idle)
 template <int MT, int NT, int KIND, int P>
 __global__ __launch_bounds__(GS_THREADS) void gemm_stream_kernel(const StreamArgs a) {
     extern __shared__ __attribute__((aligned(16))) f32x4 part[];      // [wave][NT * MT][lane]
@@ -343,8 +343,12 @@ static int gs_run(StreamArgs a, int kind, bool one, hipStream_t st) {
     int nt, splits;
     gs_policy(a.M, a.N, a.nsteps, kind == GS_F32 && !one, &nt, &splits);
     a.split_steps = (a.nsteps + splits - 1) / splits;
-    const int mt = a.M > 32 ? 4 : (a.M > 16 ? 2 : 1);
-    // a narrow product (a side input's gate): its few workgroups would each pull all of x through one CU, so the rows are dealt out as well
+    int mt = a.M > 32 ? 4 : (a.M > 16 ? 2 : 1);
+    // Where the columns leave half of the CUs idle the rows are dealt out as well: a workgroup's time goes with the x it pulls through its CU, and W is read by the
+    // second group out of a cache.  The same sums.  Us, rows x columns x K, all rows / dealt out: 64 x 2048 x 1536 6.4 / 4.9, 64 x 2048 x 768 4.5 / 3.9, 32 x 2048 x 1536
+    // 4.9 / 4.2, 64 x 1024 x 256 3.0 / 2.7; beyond one round of 256 workgroups the other way round: 64 x 4608 x 1024 6.3 / 7.0, 32 x 9216 x 2048 11.0 / 15.0.
+    while (mt > 1 && a.N / 16 / nt * splits * (((a.M + 15) / 16 + mt / 2 - 1) / (mt / 2)) <= 256) mt /= 2;
+    // a narrow product (a side input's gate), more steps in flight
     if (a.N / 16 * splits <= 32) {
         if (kind == GS_F32) return gs_launch<1, 1, GS_F32, 4>(a, splits, st);
         return kind == GS_BF16 ? gs_launch<1, 1, GS_BF16, 4>(a, splits, st) : gs_launch<1, 1, GS_ACT, 4>(a, splits, st);

@@ -269,6 +269,25 @@ def test_gemm_stream(M, N, K):
         close(unfrag(b, M, N), ref, 8e-3)
 
 
+@pytest.mark.parametrize("M", [17, 31, 33, 48, 49, 64])
+@pytest.mark.parametrize("N", [32, 1024, 2048, 2064, 4096])
+def test_rows_dealt_out_over_workgroups(M, N):
+    """Columns that leave compute units idle take the rows in groups of 64, 32 and 16: every row has the bits it has in a product of its own 16."""
+    K = 96
+    g = gen(M + N)
+    x, w = (torch.randn(M, K, generator=g)).bfloat16(), dev((torch.randn(N * K, generator=g) * 0.1).bfloat16())
+    xp = torch.zeros((M + 15) // 16 * 16, K, dtype=torch.bfloat16)
+    xp[:M] = x
+    out = torch.full((M + 1, N), 7.0, dtype=torch.bfloat16, device="cuda")
+    call("omni_gemm_stream", frag_shuffle(dev(xp)), w, out, M, N, K, L.STREAM_BF16, 0, 0.0, 0.0, 0)
+    for m in range(0, M, 16):
+        n = min(16, M - m)
+        part = torch.empty(n, N, dtype=torch.bfloat16, device="cuda")
+        call("omni_gemm_stream", frag_shuffle(dev(xp[m:m + 16])), w, part, n, N, K, L.STREAM_BF16, 0, 0.0, 0.0, 0)
+        assert torch.equal(out[m:m + n], part)
+    assert bool((out[M] == 7.0).all())
+
+
 @pytest.mark.parametrize("M", [1, 17, 64, 65, 300])
 def test_xielu_epilogues(M):
     """The activation inside both GEMMs, over values far into either branch and around zero."""

@@ -75,9 +75,13 @@ extern "C" int omni_head_gemm(const void* x, const void* w, void* out, int T, in
     OMNI_CHECK_ARG(heads > 0 && heads <= 65535 && n > 0 && n % 16 == 0 && k > 0 && k % 32 == 0, "omni_head_gemm: heads=%d n=%d (%% 16) k=%d (%% 32)", heads, n, k);
     OMNI_CHECK_ARG(!frag || heads * n % 32 == 0, "omni_head_gemm: fragment-major output needs heads * n %% 32 == 0");
     if (T <= 0) return OMNI_OK;
-    const int mt = T > 32 ? 4 : (T > 16 ? 2 : 1);
     const bool ks = k >= 256;
-    const dim3 grid(ks ? n / 16 : (n / 16 + HG_WAVES - 1) / HG_WAVES, (T + 16 * mt - 1) / (16 * mt), heads), block(64 * HG_WAVES);
+    const int cols = ks ? n / 16 : (n / 16 + HG_WAVES - 1) / HG_WAVES;
+    int mt = T > 32 ? 4 : (T > 16 ? 2 : 1);
+    // rows are dealt out where columns and heads leave half of the CUs idle: a wave's chain is its loads of x.  The same sums.  Us, 16 heads, columns x K, 64 rows
+    // in one workgroup / dealt out: 512 x 128 4.4 / 3.4, 128 x 512 4.3 / 3.3, 256 x 128 4.2 / 2.7, 128 x 256 3.4 / 2.9; 32 rows 3.3 / 2.7, 3.2 / 2.9, 3.2 / 2.8, 2.9 / 2.6
+    while (mt > 1 && (int64_t)cols * heads * ((T + 8 * mt - 1) / (8 * mt)) <= 256) mt /= 2;
+    const dim3 grid(cols, (T + 16 * mt - 1) / (16 * mt), heads), block(64 * HG_WAVES);
     OMNI_CHECK_ARG(grid.y <= 65535, "omni_head_gemm: T=%d", T);
 #define HG(MT_, KS_) hipLaunchKernelGGL((head_gemm_kernel<MT_, KS_>), grid, block, 0, (hipStream_t)stream, (const uint16_t*)x, (const uint16_t*)w, (uint16_t*)out, T, heads, n, k, frag)
     if (ks) { if (mt == 4) HG(4, true); else if (mt == 2) HG(2, true); else HG(1, true); }

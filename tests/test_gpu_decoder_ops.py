@@ -269,6 +269,22 @@ def test_gemm_stream(M, N, K):
         close(unfrag(b, M, N), ref, 8e-3)
 
 
+@pytest.mark.parametrize("T", [17, 32, 33, 48, 64, 70])
+@pytest.mark.parametrize("heads,n,k", [(1, 64, 64), (16, 512, 128), (16, 128, 512), (16, 128, 256), (40, 256, 128)])
+def test_head_products_dealt_out_by_rows(T, heads, n, k):
+    """Rows in groups of 64, 32 and 16, as many as make a workgroup per compute unit: every row has the bits it has in a product of its own 16."""
+    g = gen(T + n)
+    x, w = dev(torch.randn(T, heads * k, generator=g).bfloat16()), dev((torch.randn(heads * n * k, generator=g) * 0.1).bfloat16())
+    out = torch.full((T + 1, heads * n), 7.0, dtype=torch.bfloat16, device="cuda")
+    call("omni_head_gemm", x, w, out, T, heads, n, k, 0)
+    for t in range(0, T, 16):
+        m = min(16, T - t)
+        part = torch.empty(m, heads * n, dtype=torch.bfloat16, device="cuda")
+        call("omni_head_gemm", x[t:t + m].contiguous(), w, part, m, heads, n, k, 0)
+        assert torch.equal(out[t:t + m], part)
+    assert bool((out[T] == 7.0).all())
+
+
 @pytest.mark.parametrize("M", [17, 31, 33, 48, 49, 64])
 @pytest.mark.parametrize("N", [32, 1024, 2048, 2064, 4096])
 def test_rows_dealt_out_over_workgroups(M, N):

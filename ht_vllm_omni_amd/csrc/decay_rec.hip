@@ -346,6 +346,7 @@ __global__ __launch_bounds__(512, 2) void rec_chunk_out_kernel(const omni_decay_
 }
 
 // ---- host side
+static constexpr int RC_RUN_DP = 512;      // most rows of S of the kernels that walk runs: their registers hold 32 of a thread's
 template <int CQ, bool RAW>
 static void rec_runs_launch(const omni_decay_rec& a, const int32_t* items, int n, hipStream_t st) {
     constexpr int RG = 256 / CQ;
@@ -353,8 +354,8 @@ static void rec_runs_launch(const omni_decay_rec& a, const int32_t* items, int n
     const size_t lds = 2 * (size_t)a.dp * sizeof(float);
     if (a.dp <= 4 * RG) hipLaunchKernelGGL((rec_run_kernel<CQ, 4, RAW>), grid, block, lds, st, a, items);
     else if (a.dp <= 8 * RG) hipLaunchKernelGGL((rec_run_kernel<CQ, 8, RAW>), grid, block, lds, st, a, items);
-    else if (a.dp <= 16 * RG) hipLaunchKernelGGL((rec_run_kernel<CQ, 16, RAW>), grid, block, lds, st, a, items);
-    else hipLaunchKernelGGL((rec_run_kernel<CQ, 32, RAW>), grid, block, lds, st, a, items);
+    else if (16 * RG >= RC_RUN_DP || a.dp <= 16 * RG) hipLaunchKernelGGL((rec_run_kernel<CQ, 16, RAW>), grid, block, lds, st, a, items);
+    else if constexpr (16 * RG < RC_RUN_DP) hipLaunchKernelGGL((rec_run_kernel<CQ, 32, RAW>), grid, block, lds, st, a, items);      // (else: nothing comes here)
 }
 
 template <bool RAW>
@@ -383,8 +384,8 @@ static int rec_out(const omni_decay_rec& a, hipStream_t st) {
 extern "C" int omni_decay_rec_run(const omni_decay_rec* p, void* stream) {
     OMNI_CHECK_ARG(p && p->proj && p->decay && p->log2_decay && p->state && p->state_slot && p->row_of_tok && p->positions && p->out, "omni_decay_rec: null pointer");
     const omni_decay_rec& a = *p;
-    OMNI_CHECK_ARG(a.heads > 0 && a.heads <= 65535 && a.dp > 0 && a.dp % 32 == 0 && a.dp <= 512 && a.vp > 0 && a.vp % 32 == 0 && a.ld >= a.heads * (2 * a.dp + a.vp) && a.ld % 8 == 0,
-                   "omni_decay_rec: heads=%d dp=%d (multiple of 32, <= 512) vp=%d ld=%d", a.heads, a.dp, a.vp, a.ld);
+    OMNI_CHECK_ARG(a.heads > 0 && a.heads <= 65535 && a.dp > 0 && a.dp % 32 == 0 && a.dp <= RC_RUN_DP && a.vp > 0 && a.vp % 32 == 0 && a.ld >= a.heads * (2 * a.dp + a.vp) && a.ld % 8 == 0,
+                   "omni_decay_rec: heads=%d dp=%d (multiple of 32, <= %d) vp=%d ld=%d", a.heads, a.dp, RC_RUN_DP, a.vp, a.ld);
     OMNI_CHECK_ARG(a.slabs >= 0 && a.slabs <= OMNI_STREAM_MAX_SPLITS, "omni_decay_rec: slabs=%d", a.slabs);
     OMNI_CHECK_ARG(a.n_decode >= 0 && a.n_decode <= 65535 && a.n_runs >= 0 && a.n_runs <= 65535 && (a.n_runs == 0 || a.runs), "omni_decay_rec: n_decode=%d n_runs=%d", a.n_decode, a.n_runs);
     OMNI_CHECK_ARG(a.n_chunks >= 0 && (a.n_chunks == 0) == (a.n_segs == 0) && a.n_segs <= 65535, "omni_decay_rec: n_chunks=%d n_segs=%d", a.n_chunks, a.n_segs);

@@ -63,3 +63,11 @@ def test_no_kernel_holds_a_packed_fp32_op(tmp_path, defines):
         scratch = {n: scratch_bytes(lines) for n, lines in zip(names, asms) if n in B.DECODER_SOURCES}
         assert sum(map(len, scratch.values())) > 50
         assert not any(map(any, scratch.values())), {n: v for n, v in scratch.items() if any(v)}
+
+
+@pytest.mark.skipif(not os.path.exists(B.LIB_DECODER), reason="libomni_decoder.so is not built")
+def test_no_kernel_of_runs_that_nothing_reaches():
+    """32 row groups of 16 rows are all 512 rows of S that omni_decay_rec takes: no form by 32 columns holds 32 rows a thread.  16 groups need it."""
+    code = open(B.LIB_DECODER, "rb").read()
+    assert b"rec_run_kernelILi8ELi16E" in code and b"rec_run_kernelILi16ELi32E" in code
+    assert b"rec_run_kernelILi8ELi32E" not in code

@@ -174,17 +174,28 @@ __device__ __forceinline__ float xielu(float z, float ap, float an) {
 __device__ __forceinline__ float relu2(float z) { z = fmaxf(z, 0.f); return z * z; }
 __device__ __forceinline__ float gelu_tanh(float z) { return 0.5f * z * (1.0f + tanhf(0.79788456080286536f * fmaf(0.044715f * z * z, z, z))); }
 __device__ __forceinline__ float sigmoidf_(float z) { return 1.0f / (1.0f + expf(-z)); }
-// the same in two thirds of the instructions, for the epilogues behind the matrix pipe: the hardware's exponential of z log2(e) with what that product's
-// rounding lost put back, and its reciprocal with a Newton step, 2^24 up so that no reciprocal is denormal.  Within 1.7e-7; SiLU of a bf16 is the one
-// expf and a division give, bit for bit (65536 of 65536 inputs); the clamps turn what infinities leave in the corrections into numbers: results are those of above.
-// 6267 x 12288 x 2048 with SiLU(gate) * up 269 -> 263 us (the
-// plain product: 262), 6001 x 8192 x 2048 with SiLU and the logistic 188 -> 178 (155).
-__device__ __forceinline__ float sigmoid_w(float z) {
+// The same without a division, for the epilogues behind the matrix pipe, and closer: the hardware's exponential of z log2(e); what rounding that product and the
+// sum lost enters the reciprocal's Newton step, 2^24 down so that no reciprocal is denormal.  Largest error over every fp32 of a range, this / expf and a division, units
+// of 1e-7: z of -30 ... -8 1.10 / 1.63, -8 ... -1 1.10 / 1.34, -1 ... 0 1.01 / 1.31, 0 ... 1 0.80 / 1.13, 1 ... 8 0.57 / 1.02 (rms nowhere larger).  The clamps turn what
+// infinities leave in the corrections into numbers: results are those of above.  6001 x 8192 x 2048 with SiLU and the logistic 189 -> 184 us (the plain product: 153).
+struct LogisticTerms { float E, r; };         // exp(-z), but for a factor of 1 + r ln 2
+__device__ __forceinline__ LogisticTerms logistic_terms(float z) {
     const float t = z * -1.4426950408889634f;
-    const float r = __builtin_amdgcn_fmed3f(fmaf(z, -1.9259629911e-8f, fmaf(z, -1.4426950408889634f, -t)), -1e-4f, 1e-4f);
-    const float d = fmaf(__builtin_amdgcn_exp2f(t), fmaf(r, 0.6931471806f, 1.0f), 1.0f) * 0x1p-24f;
+    return {__builtin_amdgcn_exp2f(t), __builtin_amdgcn_fmed3f(fmaf(z, -1.9259629911e-8f, fmaf(z, -1.4426950408889634f, -t)), -1e-4f, 1e-4f)};
+}
+__device__ __forceinline__ float sigmoid_w(float z) {
+    const LogisticTerms e = logistic_terms(z);
+    const float s = e.E + 1.0f, d = s * 0x1p-24f, lost = fmaf(e.E, e.r * 0.6931471806f, (fmaxf(e.E, 1.0f) - s) + fminf(e.E, 1.0f)) * 0x1p-24f;
     const float y = __builtin_amdgcn_rcpf(d);
-    return fmaf(__builtin_amdgcn_fmed3f(fmaf(-d, y, 1.0f), -1e-4f, 1e-4f), y, y) * 0x1p-24f;
+    return fmaf(__builtin_amdgcn_fmed3f(fmaf(-lost, y, fmaf(-d, y, 1.0f)), -1e-4f, 1e-4f), y, y) * 0x1p-24f;
+}
+// SiLU of a bf16, to be rounded to bf16: the sum's rounding is not followed up (2.2e-7 at most), and every bf16 rounds as it does behind expf and a division.
+// 6267 x 12288 x 2048 with SiLU(gate) * up 268 -> 260 us (by sigmoid_w 264; the plain product: 247)
+__device__ __forceinline__ float silu_b(float z) {
+    const LogisticTerms e = logistic_terms(z);
+    const float d = fmaf(e.E, fmaf(e.r, 0.6931471806f, 1.0f), 1.0f) * 0x1p-24f;
+    const float y = __builtin_amdgcn_rcpf(d);
+    return z * (fmaf(__builtin_amdgcn_fmed3f(fmaf(-d, y, 1.0f), -1e-4f, 1e-4f), y, y) * 0x1p-24f);
 }
 
 // ---- OCP e4m3fn <-> f32 (saturating, round-nearest-even: clamp then hardware cvt)

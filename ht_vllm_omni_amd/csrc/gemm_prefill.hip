@@ -164,7 +164,7 @@ __device__ __forceinline__ void tile_epilogue(const TileArgs& a, f32x4 (&acc)[WN
                 for (int e = 0; e < 4; ++e) {
                     const float g0 = bfround(gp[2 * e]), g1 = bfround(gp[2 * e + 1]);
                     const float u0 = bfround(gp[8 + 2 * e]), u1 = bfround(gp[8 + 2 * e + 1]);
-                    const float s0 = bfround(g0 * sigmoid_w(g0)), s1 = bfround(g1 * sigmoid_w(g1));   // torch: F.silu(bf16) is bf16
+                    const float s0 = bfround(silu_b(g0)), s1 = bfround(silu_b(g1));   // torch: F.silu(bf16) is bf16
                     o[e] = pack_bf2(s0 * u0, s1 * u1);
                 }
                 *reinterpret_cast<u32x4*>(a.out + (size_t)m * a.ldo + (n >> 1)) = o;

@@ -8,7 +8,7 @@ from ht_vllm_omni_amd import _lib as L
 from ht_vllm_omni_amd import ops
 from ht_vllm_omni_amd.decoder_engine import attention_tiles, r32
 from ht_vllm_omni_amd.decoder_mixers import cached_rows
-from ht_vllm_omni_amd.engine import frag_shuffle, frag_unshuffle
+from ht_vllm_omni_amd.engine import frag_shuffle, frag_unshuffle, gu8_shuffle
 from oracle import decoder_oracle as D
 
 pytestmark = pytest.mark.gpu
@@ -323,7 +323,7 @@ def test_xielu_epilogues(M):
 
 
 def test_activations_of_the_tile_epilogues_to_32_bits():
-    """XIELU and SiLU / sigmoid of given fp32 values (a product with unit rows of W), from 1e-30 to 1e30 in either sign, in fp32: six roundings and two
+    """XIELU and SiLU / sigmoid of given bf16 values (a product with unit rows of W), from 1e-30 to 1e30 in either sign, in fp32: six roundings and two
     1-ulp instructions are under 5e-7 of the larger of the result and its largest term; not-a-number stays one, and large values do not become one."""
     v = torch.cat([torch.logspace(-30, 30, 2400, dtype=torch.double), torch.logspace(-2, 2.2, 4000, dtype=torch.double)]).bfloat16()
     v = torch.cat([v, -v, torch.zeros(64, dtype=torch.bfloat16)])
@@ -346,6 +346,40 @@ def test_activations_of_the_tile_epilogues_to_32_bits():
     x[0, 0] = float("nan")
     for kw in (dict(act=L.TILE_ACT_XIELU, act_params=(0.7, 0.8)), dict(act=L.TILE_ACT_SILU_SIGMOID, act_cols=96), dict(act=L.TILE_ACT_SILU_SIGMOID)):
         assert bool(ops.gemm_tile(dev(x), frag_shuffle(dev(w)), want="f", lib=lib, **kw)[0].isnan().all())
+
+
+@pytest.mark.parametrize("lo,hi", [(-86.0, -30.0), (-30.0, -8.0), (-8.0, -1.0), (-1.0, 0.0), (0.0, 1.0), (1.0, 8.0), (8.0, 30.0)])
+def test_logistic_of_full_fp32_accumulators(lo, hi):
+    """Accumulators with all 24 bits: the three bf16 terms of a value, added up by the product without rounding.  Bound: the hardware's exponential is within a unit
+    in the last place (2^-23), which the sum 1 + e takes in proportion e / (1 + e); the result is rounded once (2^-24); SiLU's product once more."""
+    g = gen(int(lo * 8 + 800))
+    z = (torch.rand(16384, 32, generator=g, dtype=torch.double) * (hi - lo) + lo).float()
+    hi16 = z.bfloat16()
+    mid = (z - hi16.float()).bfloat16()
+    x = torch.cat([hi16, mid, (z - hi16.float() - mid.float()).bfloat16()], 1)
+    w, lib, zd = dev(frag_shuffle(torch.eye(32).repeat(1, 3).bfloat16())), L.load_decoder(), z.double()
+    assert torch.equal(ops.gemm_tile(dev(x), w, want="f", lib=lib).cpu(), z)
+    e = torch.exp(-zd)
+    for cols in (0, 32):
+        got = ops.gemm_tile(dev(x), w, act=L.TILE_ACT_SILU_SIGMOID, act_cols=cols, want="f", lib=lib).double().cpu()
+        bound = 2.0 ** -23 * e / (1 + e) + 2.0 ** -24 * (1 + cols // 32)
+        err = (got / ((zd if cols else 1.0) / (1 + e)) - 1).abs()
+        assert bool((err <= bound * 1.001).all()), (cols, float((err / bound).max()))
+
+
+def test_silu_of_every_bf16():
+    """The interleaved epilogue's SiLU rounds as 64 bits do, save where the value is within 2^-21 of the middle between two bf16."""
+    z = torch.arange(-32768, 32768, dtype=torch.int32).to(torch.int16).view(torch.bfloat16)
+    z = z[(z.float() > -87) & (z.float() < 1e30) & (z.float().abs() > 1e-30)]
+    z = z[:z.numel() // 32 * 32].reshape(-1, 32)
+    x = torch.cat([z, torch.ones(z.shape[0], 32, dtype=torch.bfloat16)], 1)
+    w = torch.zeros(64, 64)
+    w[:32, :32], w[32:, 32] = torch.eye(32), 1.0
+    got = ops.gemm_tile(dev(x), dev(gu8_shuffle(w.bfloat16())), act=L.TILE_ACT_SILU_MUL_GU8, lib=L.load_decoder()).cpu()
+    ref = z.double() / (1 + torch.exp(-z.double()))
+    near = [(ref * (1 + s * 2.0 ** -21)).float().bfloat16() for s in (-1, 0, 1)]
+    assert bool(((got == near[0]) | (got == near[1]) | (got == near[2])).all())
+    assert int((got != near[1]).sum()) <= int((near[0] != near[2]).sum())
 
 
 # ---------------------------------------------------------------- attention

@@ -126,8 +126,8 @@ __global__ __launch_bounds__(GS_THREADS) void gemm_stream_kernel(const StreamArg
 // a layer) is gone.  One workgroup (`writer`) leaves what others read later.  Us, a decode step of 8 layers, launches of their own / rows made by the
 // product: Zefedra, 1024 wide, 1 row 330 / 280 (its latents and the merge of attention's splits among them: rows of the stream alone 301), 2 rows 334 / 286,
 // 2048 wide 457 / 400 and 464 / 413; Koronex 323 / 277, 330 / 284, 440 / 407, 444 / 416.
-// How many rows: a third and a fourth are summed behind the first two, which costs what it saves where a row is wide (3 rows of 2048: Zefedra 463 / 479, of 1024
-// 342 / 336, Koronex 332 / 312; 4 rows 343 / 321), and for latents always (4 rows 347 / 363).
+// How many rows it takes: a third and a fourth are summed behind the first two, which costs what it saves where a row is wide (3 rows of 2048: Zefedra 463 / 479), and for
+// latents always (4 rows 347 / 363).  Which products are given theirs: omni_gemm_stream_joins.
 constexpr int gs_joined_rows(int maxc) { return maxc == 1 ? OMNI_STREAM_JOINED_ROWS : 2; }
 template <int MAXC, bool SHIFT>
 struct RowsPro {                                          // a row of the residual stream (decoder_rows.hip stream_rows_kernel)
@@ -396,6 +396,21 @@ static int gs_behind(StreamArgs a, bool one, const typename PRO::Args& pa, hipSt
     GS(1) GS(2) GS(3) GS(4)
 #undef GS
     return OMNI_EINVAL;
+}
+
+// Every workgroup makes the rows: what the launch in front costs is saved once, what the rows cost is paid by every round of workgroups -- and hidden behind the weights
+// of the round before where a row is as wide as those are long.  Us, rows made by the product against launches of their own, behind four partial sums, a row or two: up to
+// 256 workgroups -1.2 ... -2.5 at every width; 512 -0.3 ... -0.7 (widths to 640), -1 ... -2.5 (wider); 768 of one column tile -0.0 ... -0.6, of two and more +1.4 ... +2.6
+// (256 to 512 wide); 2374 +12 ... +22 (to 384), +5.4 (512), +3.9 (640), +0.4 (768), -0.5 (896), -1.2 ... -3.1 (1024 to 2048).  With the token shift, whose state is one more
+// trip: 192 -0.6 ... -1.2, 512 and 576 -0.9 ... +3.2.  Three and four rows: 256 workgroups 0 ... -1.2, 288 and more +0.3 ... +1.9; with the shift +0.2 ... +6.6.
+extern "C" int omni_gemm_stream_joins(int rows, int wp, int N, int shift, int sums) {
+    if (rows < 1 || wp < 32 || wp % 32 || wp > 2 * DR_THREADS * 4 || rows > gs_joined_rows(wp > DR_THREADS * 4 ? 2 : 1) || N < 16 || N % 16 || (shift && rows > 2)) return 0;
+    int nt, splits;
+    gs_policy(rows, N, wp / 32, sums != 0, &nt, &splits);
+    if (N / 16 * splits <= 32) nt = 1;
+    const int wgs = N / 16 / nt * splits;
+    if (shift || rows > 2) return wgs <= 256;
+    return wp > 768 || wgs <= (nt == 1 ? 768 : 512);
 }
 
 extern "C" int omni_gemm_stream_joined(const omni_stream_rows* r, const void* w, void* out, int N, int kind, int one, float act_p, float act_n, const omni_row_table* rt, int out_frag, void* stream) {

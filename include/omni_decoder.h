@@ -110,11 +110,13 @@ int omni_gemm_stream_splits(int M, int N, int K);
 /* omni_gemm_stream of a few rows that it makes itself, in one launch, bit for bit:
  *   _joined:  the rows omni_stream_rows_run would leave in h_out (not written here; x_out is), K = wp: up to OMNI_STREAM_JOINED_ROWS of wp <= 1024, 2 of wp <=
  *             2048.  kind 0, 2 or 3; rt != NULL: the row table's activation; with mu: kind 0
+ *   _joins:   1 where _joined takes `rows` rows of wp by N columns and is faster than two launches (shift: with mu; sums: kind 0 and not `one`)
  *   _latents: the rows omni_latent_write_run would leave in cq (not written here; cache, gate and state are), K = qp: up to OMNI_STREAM_LATENT_ROWS of ld <=
  *             3072.  bf16 out, row-major                                                                                                             */
 #define OMNI_STREAM_JOINED_ROWS 4
 #define OMNI_STREAM_LATENT_ROWS 2
 int omni_gemm_stream_joined(const omni_stream_rows* r, const void* w, void* out, int N, int kind, int one, float act_p, float act_n, const omni_row_table* rt, int out_frag, void* stream);
+int omni_gemm_stream_joins(int rows, int wp, int N, int shift, int sums);
 int omni_gemm_stream_latents(const omni_latent_write* r, const void* w, void* out, int N, void* stream);
 
 /* Causal attention over a paged cache of latents shared by all heads (keys and values are the same rp-wide rows):

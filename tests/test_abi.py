@@ -181,3 +181,14 @@ def test_tile_flag_block_matches_the_kernels_indexing():
     assert tp_comm.CTL_BYTES == tp_comm.TILE_OFF + tp_comm.TILE_BYTES and tp_comm.TILE_OFF >= tp_comm.ERROR_OFF + 4
     assert tiles >= 256, "the o_proj / down_proj tile grid of the 64-row stage set: up to 128 column tiles x 2 row tiles"
 
+
+@pytest.mark.parametrize("args,joins", [
+    ((1, 1024, 3072, 0, 0), 1), ((4, 1024, 3072, 0, 0), 1), ((2, 2048, 9216, 0, 0), 1), ((2, 1024, 1056, 1, 1), 1), ((1, 32, 16, 0, 0), 1), ((2, 1024, 16384, 0, 0), 1),
+    ((1, 1024, 151936, 0, 0), 1), ((2, 512, 12288, 0, 0), 1), ((2, 640, 24576, 0, 0), 1), ((1, 1024, 5120, 0, 1), 1),
+    ((4, 1024, 16384, 0, 0), 0), ((1, 768, 151936, 0, 0), 0), ((2, 512, 24576, 0, 0), 0), ((3, 512, 4608, 0, 0), 0), ((3, 1024, 1056, 1, 1), 0), ((1, 2048, 16384, 1, 1), 0), ((1, 1024, 4608, 1, 1), 0),
+    ((5, 1024, 64, 0, 0), 0), ((3, 2048, 64, 0, 0), 0), ((1, 2080, 64, 0, 0), 0), ((0, 1024, 64, 0, 0), 0), ((1, 0, 64, 0, 0), 0), ((1, 1000, 64, 0, 0), 0), ((1, 1024, 0, 0, 0), 0), ((1, 1024, 24, 0, 0), 0)])
+def test_which_products_make_their_rows(args, joins):
+    """(rows, width, columns, token shift, partial sums): one round of workgroups, two or three for a row or two without the shift, any number where that row is wide;
+    what the entry does not take, never."""
+    from ht_vllm_omni_amd import _lib
+    assert _lib.load_decoder().omni_gemm_stream_joins(*args) == joins

@@ -9,6 +9,7 @@ import numpy as np
 import pytest
 import torch
 
+from ht_vllm_omni_amd import _lib as L
 from ht_vllm_omni_amd.decoder_config import dims_from_config
 from ht_vllm_omni_amd.decoder_engine import DecoderEngine
 from ht_vllm_omni_amd.decoder_mixers import LatentMixer
@@ -17,7 +18,7 @@ from ht_vllm_omni_amd.replay import Replayer
 from ht_vllm_omni_amd.scheduler import Request
 from ht_vllm_omni_amd.serving import serve
 from ht_vllm_omni_amd.weights import make_decoder_weights
-from tests.decoder_util import CONFIGS, TOL, assert_logits, config, layer, model, oracle, oracle_logits, tokens
+from tests.decoder_util import CONFIGS, G, TOL, assert_logits, config, layer, model, oracle, oracle_logits, tokens
 
 pytestmark = pytest.mark.gpu
 ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
@@ -150,6 +151,27 @@ def test_a_prompt_does_not_depend_on_the_batches_before_it(n):
 
 
 # ---------------------------------------------------------------- decoding and portions
+@pytest.mark.parametrize("n", [1, 2, 4])
+def test_a_large_head_takes_rows_that_are_made_once(n):
+    """A few rows are made by the products with few columns and by a launch of their own for the head of a large vocabulary."""
+    cfg = config([layer(), layer(G)], vocab=50000)
+    d = dims_from_config(cfg, 512)
+    w = make_decoder_weights(d, seed=4)
+    eng = DecoderEngine(d, w, dtype="bfloat16", num_blocks=8, max_batch=2, block_size=8)
+    made, mm = {}, eng._mm
+
+    def spy(x, m, *a, **kw):
+        made.setdefault(id(m), set()).add(isinstance(x, L.StreamRows))
+        return mm(x, m, *a, **kw)
+    eng._mm = spy
+    toks = tokens(n, d.vocab)
+    eng.block_table[0, :1] = 3
+    logits = eng.forward(eng.make_batch(torch.tensor(toks), np.zeros(n), np.arange(n), [n]))
+    lw = eng.layer_w[0]
+    assert [made[id(m)] for m in (eng.head, lw.up, lw.mixer.down)] == [{False}, {True}, {n <= 2}]
+    assert_logits(logits[:, :d.vocab], oracle_logits(w, cfg, toks), "bfloat16")
+
+
 @pytest.mark.parametrize("dtype", DTYPES)
 @pytest.mark.parametrize("name", ["mixed", "narrow", "behind", "k_mixed", "k_narrow", "k_state"])
 def test_token_by_token_equals_the_whole_prompt(name, dtype):

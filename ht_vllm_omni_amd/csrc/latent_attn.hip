@@ -581,5 +581,11 @@ extern "C" int omni_latent_attn_values(const omni_latent_attn* p, const void* w,
     OMNI_CHECK_ARG(p->T >= 1 && p->T == p->n_decode && p->T <= OMNI_STREAM_LATENT_ROWS && p->n_tiles == 0 && p->elem == 0 && p->rp <= 512 && omni_latent_attn_mfma(p->rp),
                    "omni_latent_attn_values: T=%d n_decode=%d rp=%d (decode tokens, <= %d, bf16)", p->T, p->n_decode, p->rp, OMNI_STREAM_LATENT_ROWS);
     OMNI_CHECK_ARG(n > 0 && n % 16 == 0 && (!frag || p->heads * n % 32 == 0), "omni_latent_attn_values: n=%d (%% 16) frag=%d", n, frag);
+    // A head's rows are merged n / 16 times over: past one round of workgroups the merge of its own is no slower.  Us, two rows of 2048 keys, heads x 128 by latents of 512 (256),
+    // two launches / one: 16 heads 19.8 / 18.7 (16.1 / 14.9), 32 20.7 / 20.6 (16.8 / 16.0), 64 23.0 / 24.2 (17.9 / 18.2), 128 28.4 / 34.8 (21.4 / 22.2).
+    if ((int64_t)p->heads * (n / 16) > 256) {
+        const int rc = omni_latent_attn_run(p, stream);
+        return rc != OMNI_OK ? rc : omni_head_gemm(p->out, w, out, p->T, p->heads, n, p->rp, frag, stream);
+    }
     return la_any(p, LatentValues{(const uint16_t*)w, (uint16_t*)out, n, frag}, (hipStream_t)stream);
 }

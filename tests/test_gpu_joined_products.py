@@ -144,11 +144,8 @@ def test_latents(T, q_rank, kv_rank, heads, N, form):
     assert outs[0][0].abs().max() > 0
 
 
-@pytest.mark.parametrize("lens", [[1], [64], [65], [352], [17, 900], [2100, 60]])
-@pytest.mark.parametrize("heads,rp,n,gated", [(1, 32, 32, True), (16, 256, 128, False), (16, 512, 128, True), (20, 96, 48, True)])
-@pytest.mark.parametrize("split,frag", [(True, 1), (False, 0)])
-def test_values_of_merged_splits(lens, heads, rp, n, gated, split, frag):
-    """Rows of one split beside rows of several, and no workspace for any."""
+def values_both_ways(lens, heads, rp, n, gated, split, frag):
+    """The per-head product behind the attention of decode tokens, by two entries and by one."""
     g, T, bs = gen(sum(lens) + rp), len(lens), 16
     need = [(k + bs - 1) // bs for k in lens]
     bt = torch.zeros(T, max(need), dtype=torch.int32)
@@ -175,9 +172,26 @@ def test_values_of_merged_splits(lens, heads, rp, n, gated, split, frag):
             call("omni_latent_attn_run", C.byref(a))
             call("omni_head_gemm", a.keep["out"], w, out, T, heads, n, rp, frag)
         outs.append(out)
+    return outs
+
+
+@pytest.mark.parametrize("lens", [[1], [64], [65], [352], [17, 900], [2100, 60]])
+@pytest.mark.parametrize("heads,rp,n,gated", [(1, 32, 32, True), (16, 256, 128, False), (16, 512, 128, True), (20, 96, 48, True)])
+@pytest.mark.parametrize("split,frag", [(True, 1), (False, 0)])
+def test_values_of_merged_splits(lens, heads, rp, n, gated, split, frag):
+    """Rows of one split beside rows of several, and no workspace for any."""
+    outs = values_both_ways(lens, heads, rp, n, gated, split, frag)
     assert torch.isfinite(outs[0].float()).all()
     close = torch.equal(*outs) if rp >= 256 else torch.allclose(outs[0].float(), outs[1].float(), rtol=2 ** -7, atol=1e-3)      # (narrower: head_gemm's waves do not split K, so one rounding to bf16 may fall the other way)
     assert close
+
+
+@pytest.mark.parametrize("lens", [[40], [352], [2100, 60]])
+@pytest.mark.parametrize("heads,rp,n", [(33, 64, 128), (80, 96, 64), (260, 32, 16)])
+def test_values_of_more_heads_than_merge_for_themselves(lens, heads, rp, n):
+    """More workgroups than compute units: the splits are merged once, the same bits at every width."""
+    outs = values_both_ways(lens, heads, rp, n, True, True, 0)
+    assert torch.isfinite(outs[0].float()).all() and torch.equal(*outs)
 
 
 def test_what_is_refused():

@@ -99,7 +99,7 @@ class WindowAttn(C.Structure):
     """omni_window_attn."""
     _fields_ = [("q", vp), ("kc", vp), ("vc", vp), ("gate", vp), ("sink", vp), ("out", vp), ("frag", i32), ("block_table", vp), ("bt_stride", i32), ("block_size", i32),
                 ("row_of_tok", vp), ("positions", vp), ("tiles", vp), ("n_tiles", i32), ("tile_rows", i32), ("T", i32), ("n_decode", i32), ("heads", i32), ("kv_heads", i32),
-                ("dp", i32), ("vp", i32), ("scale", f32), ("window", i32), ("max_keys", i32), ("workspace", vp), ("workspace_bytes", i64), ("elem", i32),
+                ("dp", i32), ("vp", i32), ("scale", f32), ("window", i32), ("max_keys", i32), ("workspace", vp), ("workspace_bytes", i64), ("elem", i32), ("prompt_keys", i32),
                 ("key_base", vp), ("k_row", i32), ("v_row", i32), ("head_gate", vp)]
 
 

@@ -197,10 +197,11 @@ __global__ __launch_bounds__(64) void window_merge_kernel(const WinArgs a, int m
 // tokens 66 / 44.
 // KT: teams of four waves that take the workgroup's 32-key steps in turn, each with a ring and running sums of its own; the first adds up.  Three, one
 // workgroup to a CU, where the half tiles are no more than the CUs: a step is a chain of LDS reads, 8 + 24 MFMAs and the softmax between (0.85 us for one wave
-// a SIMD, 1.6 for three in turn), and nothing else is there to fill its gaps.  Up to four steps are one team's: the others leave at once.  Us, one
-// team / three, heads x keys' heads of 128: 16 x 16, portions of 251 and 130 tokens behind 512 26.3 / 18.8 (two: 19.9), 64 behind 1500 43.9 / 28.3 (31.7), a
-// prompt of 1000 33.8 / 23.0 (24.6), of 300 12.8 / 11.0, of 66 6.3 / 6.5; 16 x 4, a prompt of 1000 31.3 / 22.3, 8 of 100 7.4 / 7.8.  Above 256 half tiles two
-// workgroups of one team share a CU instead: 256 tiles of up to 128 tokens 9.4, by three teams in turns 15.8.
+// a SIMD, 1.6 for three in turn), and nothing else is there to fill its gaps.  Us, one team / three, heads x keys' heads of 128: 16 x 16, portions of 251 and 130
+// tokens behind 512 26.3 / 18.8 (two: 19.9), 64 behind 1500 43.9 / 28.3 (31.7), a prompt of 1000 33.8 / 23.0 (24.6), of 300 12.8 / 11.0; 16 x 4, a prompt of 1000 31.3 /
+// 22.3.  Up to WA_TEAM_KEYS keys the merge and the larger workgroups' start cost more: 16 x 4, 4 prompts of 96 7.7 / 8.3, of 128 8.5 / 9.2, of 160 9.7 / 10.2, of 176
+// to 224 the same, of 256 12.7 / 12.2; where a batch's longest portion sees no more, one team is launched, and in other batches the first walks such a tile alone:
+// the same sums either way.  Above 256 half tiles two workgroups of one team share a CU instead: 256 tiles of up to 128 tokens 9.4, by three teams in turns 15.8.
 // Order.  An XCD deals its workgroups out in turn over its 32 CUs, three to a CU, and the tiles of a causal prompt are as long as the keys they see: by length
 // the first CU gets the longest of each turn (one prompt of 6001 tokens, 47 tiles of 16 heads: 94 units of keys against 70 on average).  wa_deal orders the
 // first turns so that what a CU gets adds up to the same (72): that prompt 394 -> 342 us a layer, one of 3000 152 -> 143, one of
@@ -217,6 +218,7 @@ __device__ __forceinline__ int wa_deal(int slot, int n) {                     //
     return 2 * C + (j & 1 ? last / 2 - 1 - i : last - 1 - i);
 }
 
+#define WA_TEAM_KEYS 160
 template <int WS, int RG, int KT>
 __global__ __launch_bounds__(256 * KT, KT == 1 ? 3 : KT) void window_prefill_dma_kernel(const WinArgs a, int n_tiles) {
     constexpr int WR = 16 * RG, PARTS = 2 / RG, HALF = WS * 1024, IMAGE = 4 * HALF, NB = 3, dp = 32 * WS;
@@ -265,7 +267,7 @@ __global__ __launch_bounds__(256 * KT, KT == 1 ? 3 : KT) void window_prefill_dma
     const int fhi = wave * WR + WR <= nrows ? wfirst + 1 : 0, flo = wa_first(whi - 1, a.window);
     const int nkeys = a.positions[(row0 + nrows - 1) / a.rep] + 1;
     const int kbeg = wa_first(a.positions[tok0], a.window) & ~(LA_KEYS - 1);
-    const int teams = KT == 1 || nkeys - kbeg <= 4 * LA_KEYS ? 1 : KT, stride = LA_KEYS * teams;      // (uniform) four steps are walked sooner than merged
+    const int teams = KT == 1 || nkeys - kbeg <= WA_TEAM_KEYS ? 1 : KT, stride = LA_KEYS * teams;     // (uniform)
     if (team >= teams) return;
     // loader: wave -> keys 16 (wave & 1) ... of the keys (waves 0, 1) or the values (2, 3); lane -> key lane / 4, 16-byte quarter lane % 4 of every piece
     const bool vals = wave >= 2;
@@ -688,7 +690,8 @@ static int wa_run(const omni_window_attn& p, WinArgs a, hipStream_t st) {
             const bool halves = (int64_t)p.n_tiles * G <= 256;
             const int n = halves ? 2 * p.n_tiles : p.n_tiles;
             const int64_t wgs = 8 % G == 0 ? (int64_t)(n + per - 1) / per * 8 : (int64_t)n * G;
-            if (halves && (int64_t)n * G <= 256) hipLaunchKernelGGL((window_prefill_dma_kernel<WS, 1, 3>), dim3((unsigned)wgs), dim3(768), 3 * LDS, st, a, n);
+            const bool one_team = p.prompt_keys > 0 && p.prompt_keys <= WA_TEAM_KEYS;
+            if (halves && (int64_t)n * G <= 256 && !one_team) hipLaunchKernelGGL((window_prefill_dma_kernel<WS, 1, 3>), dim3((unsigned)wgs), dim3(768), 3 * LDS, st, a, n);
             else if (halves) hipLaunchKernelGGL((window_prefill_dma_kernel<WS, 1, 1>), dim3((unsigned)wgs), dim3(256), LDS, st, a, n);
             else hipLaunchKernelGGL((window_prefill_dma_kernel<WS, 2, 1>), dim3((unsigned)wgs), dim3(256), LDS, st, a, n);
             OMNI_CHECK_LAUNCH("omni_window_attn(prefill)");

@@ -152,12 +152,13 @@ int omni_latent_gather(const void* cache, const int32_t* block_table, int bt_str
  * it the denominator is the sum alone).
  * Tokens [0, n_decode) are single-token sequences (workspace for the splits); the others are covered by `tiles` (int32 [n_tiles][2], device:
  * first flat row t * (heads / kv_heads) + r and row count <= tile_rows; one sequence each; every key / value head walks the same tiles).
- * max_keys bounds positions[t] + 1 of the decode tokens (split choice only).                                                          */
+ * max_keys bounds positions[t] + 1 of the decode tokens (split choice only), prompt_keys of the others (0: not known; choice of kernel only: it lies
+ * where the struct had padding, and whatever a caller built before it left there costs time, never a result).                         */
 typedef struct omni_window_attn {
     const void* q; const void* kc; const void* vc; const void* gate; const float* sink; void* out; int frag;
     const int32_t* block_table; int bt_stride, block_size; const int32_t* row_of_tok; const int32_t* positions;
     const int32_t* tiles; int n_tiles, tile_rows;
-    int T, n_decode, heads, kv_heads, dp, vp; float scale; int window, max_keys; float* workspace; int64_t workspace_bytes; int elem;
+    int T, n_decode, heads, kv_heads, dp, vp; float scale; int window, max_keys; float* workspace; int64_t workspace_bytes; int elem, prompt_keys;
     /* prompt tiles alone (n_decode = 0): key_base int32 [batch rows]: keys and values are rows of plain arrays instead of pages -- key j of a sequence is row
      * key_base[row] + j, kc elem [rows, k_row] with head g at column g * dp, vc likewise; head_gate fp32 [T, heads] in the gate's place */
     const int32_t* key_base; int k_row, v_row; const float* head_gate;

@@ -342,3 +342,8 @@ def test_oracle_koronex_layer_parts():
         assert torch.allclose(got, r / math.sqrt(float((r * r).mean()) + 0.1) * s["norm"])
     m = dict(up=rnd(3, 4), down=rnd(4, 3))
     assert torch.allclose(D.relu2_mlp(x, m)[0], m["down"] @ torch.tensor([max(float(r @ x[0]), 0.0) ** 2 for r in m["up"]], dtype=torch.float64))
+
+
+def test_keys_that_the_longest_portion_sees():
+    from ht_vllm_omni_amd.decoder_engine import Batch
+    assert Batch(5, 1, segs=[(3, 10), (1, 2)]).prompt_keys == 13 and Batch(70, 0, segs=[(70, 0)]).prompt_keys == 70 and Batch(4, 4, max_keys=900).prompt_keys == 0

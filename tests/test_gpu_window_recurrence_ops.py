@@ -205,7 +205,7 @@ class Seqs:
         out = torch.cat(out).reshape(-1, self.heads * self.vdim)
         return out if self.gate is None else out * self.gate.double()
 
-    def run(self, scale, window, split=True, frag=0, rows_of=None):
+    def run(self, scale, window, split=True, frag=0, rows_of=None, prompt_keys=0):
         """rows_of: keys and values as rows of one array each, spaced `rows_of` sequences apart, instead of pages; a gate per head."""
         order = sorted(range(len(self.lens)), key=lambda r: self.new[r] > 1)
         ones = sum(1 for n in self.new if n == 1)
@@ -240,7 +240,7 @@ class Seqs:
         run_struct("omni_window_attn_run", L.WindowAttn(), **more, q=q, kc=kc, vc=vc, gate=gate, sink=None if self.sink is None else dev(self.sink), out=out, frag=frag,
                    block_table=dev(self.bt), bt_stride=self.bt.shape[1], block_size=self.bs, row_of_tok=dev(row), positions=dev(pos), tiles=tiles, n_tiles=0 if tiles is None else len(tiles), tile_rows=rows,
                    T=T, n_decode=ones, heads=H, kv_heads=self.kv, dp=dp, vp=vp, scale=scale, window=window or 0, max_keys=max([self.lens[r] for r in order[:ones]] or [0]),
-                   workspace=torch.full((nb // 4,), float("nan"), device="cuda") if split else None, workspace_bytes=nb if split else 0, elem=self.elem)
+                   workspace=torch.full((nb // 4,), float("nan"), device="cuda") if split else None, workspace_bytes=nb if split else 0, elem=self.elem, prompt_keys=prompt_keys)
         got = (unfrag(out, T, H * vp) if frag else out[:T]).cpu().reshape(T, H, vp)
         assert not got[:, :, self.vdim:].any() or self.gate is None
         res = torch.empty(T, H * self.vdim, dtype=got.dtype)
@@ -287,10 +287,20 @@ def test_prompt_tiles_that_fill_the_chip(heads, kv, dim, bs, window, scale):
 @pytest.mark.parametrize("heads,kv,dim,sinks", [(8, 8, 128, True), (6, 2, 64, True), (2, 2, 128, False)])
 @pytest.mark.parametrize("keys,window", [(127, None), (128, None), (129, None), (160, None), (161, None), (225, None), (290, 100), (900, 129), (1111, 400), (333, 161)])
 def test_steps_shared_out_over_teams(heads, kv, dim, sinks, keys, window):
-    """Few half tiles: up to four steps of 32 keys by one team of waves, more by three in turn, counts that do and do not divide by three, rows whose window
+    """Few half tiles: up to five steps of 32 keys by one team of waves, more by three in turn, counts that do and do not divide by three, rows whose window
     holds no key of a team's steps, a first step in the middle of the keys."""
     s = Seqs([keys, keys + 40, 33], [70, 2, 17], heads, kv, dim, dim, 0, seed=keys + dim, sink=sinks)
     close(s.run(0.3, window), s.reference(0.3, window), SAFE[0])
+
+
+@pytest.mark.parametrize("heads,kv,dim", [(8, 8, 128), (8, 2, 64)])
+@pytest.mark.parametrize("keys", [33, 96, 128, 129, 159, 160])
+def test_short_portions_by_one_team(keys, heads, kv, dim):
+    """A batch whose longest portion is short, told so: the sums of a launch that does not know."""
+    s = Seqs([keys, min(keys, 40), 33], [min(keys, 70), 2, 17], heads, kv, dim, dim, 0, seed=keys + dim)
+    got = s.run(0.3, None, prompt_keys=keys)
+    close(got, s.reference(0.3, None), SAFE[0])
+    assert torch.equal(got, s.run(0.3, None))
 
 
 def test_half_tiles_two_to_a_compute_unit():

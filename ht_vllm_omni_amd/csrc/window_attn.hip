@@ -204,8 +204,11 @@ __global__ __launch_bounds__(64) void window_merge_kernel(const WinArgs a, int m
 // the same sums either way.  Above 256 half tiles two workgroups of one team share a CU instead: 256 tiles of up to 128 tokens 9.4, by three teams in turns 15.8.
 // Order.  An XCD deals its workgroups out in turn over its 32 CUs, three to a CU, and the tiles of a causal prompt are as long as the keys they see: by length
 // the first CU gets the longest of each turn (one prompt of 6001 tokens, 47 tiles of 16 heads: 94 units of keys against 70 on average).  wa_deal orders the
-// first turns so that what a CU gets adds up to the same (72): that prompt 394 -> 342 us a layer, one of 3000 152 -> 143, one of
-// 2500 in windows of 1024 61 -> 57, with a step's address arithmetic and maxima cut down (4 prompts of up to 2048 in such windows, balanced before: 91.8 -> 90.9).
+// first turns so that what a CU gets adds up to the same (72).  Us a layer, that prompt, head after head 359, every head's tiles by length 312, dealt 304; one of 3000
+// 147 / 139 / 136, of 2500 122 / 117 / 115; 16 x 4, by length / dealt, one of 6001 310 / 301, 24 of 128 15.6 / 14.0.
+// The row's maximum is put together only where it moves: 312 -> 303 of that prompt, 16 x 4, 4 of up to 2048 99 -> 97.
+// (Tried in the loop: blocks looked up by the scalar unit, 16 keys at a time -- 8 x 8 of 64, one of 3000, 66 -> 73 us, 16 x 4 of 128, one of 2048, 57 -> 60; the second product
+// term by term over four column tiles: 0 to 3 % slower.)
 // (The dealing is how an idle XCD was seen to go about it; another one costs time, never a result.)
 __device__ __forceinline__ int wa_deal(int slot, int n) {                     // workgroup of an XCD -> rank by length among its n
     constexpr int C = 32;
@@ -287,23 +290,13 @@ __global__ __launch_bounds__(256 * KT, KT == 1 ? 3 : KT) void window_prefill_dma
         if (!a.key_base) ids = bt[b];
         asm volatile("" : "+v"(ids));                  // waited for here, not where the lookups are
     };
-    const int lkey0 = 16 * (wave & 1);
+    auto block_of = [&](int k0) {
+        if (((k0 + LA_KEYS - 1) >> a.bs_shift) - cached > 63) load_ids(k0);
+        return __shfl(ids, (min(k0 + lkey, nkeys - 1) >> a.bs_shift) - cached, 64);
+    };
     auto stage = [&](int k0, int buf) {                                       // keys past the end: a valid row, masked below
-        k0 = min(k0, nkeys - 1);
-        const int off = min(k0 + lkey, nkeys - 1) & a.bs_mask;
-        const uint16_t* p = src;
-        if (a.bs_shift >= 4) {                                                // (uniform) the wave's 16 keys lie in one block
-            int blk = min(k0 + lkey0, nkeys - 1) >> a.bs_shift;
-            if (!a.key_base) {
-                if (((k0 + LA_KEYS - 1) >> a.bs_shift) - cached > 63) load_ids(k0);
-                blk = __builtin_amdgcn_readlane(ids, blk - cached);
-            }
-            p += (int64_t)blk * lblock;
-        } else {
-            if (((k0 + LA_KEYS - 1) >> a.bs_shift) - cached > 63) load_ids(k0);
-            p += (int64_t)__shfl(ids, (min(k0 + lkey, nkeys - 1) >> a.bs_shift) - cached, 64) * lblock;
-        }
-        p += (uint64_t)(unsigned)off * (unsigned)lrow;
+        const int blk = block_of(min(k0, nkeys - 1));
+        const uint16_t* p = src + (size_t)blk * lblock + (size_t)(min(k0 + lkey, nkeys - 1) & a.bs_mask) * lrow;
         unsigned char* d = dst0 + buf * IMAGE;
 #pragma unroll
         for (int s = 0; s < WS; ++s)
@@ -387,11 +380,13 @@ __global__ __launch_bounds__(256 * KT, KT == 1 ? 3 : KT) void window_prefill_dma
                          : "v"(vaddr), "n"(d0 * 512), "n"(d0 * 512 + 32), "n"(d0 * 512 + 1024), "n"(d0 * 512 + 1056), "n"(d0 * 512 + HALF), "n"(d0 * 512 + 32 + HALF),
                            "n"(d0 * 512 + 1024 + HALF), "n"(d0 * 512 + 1056 + HALF));
 #pragma unroll
-            for (int k = 2; k >= 0; --k)
+            for (int d = 0; d < 4; ++d) {
+                const u32x4 VT = {x[d][0], x[d][1], y[d][0], y[d][1]};
 #pragma unroll
-                for (int d = 0; d < 4; ++d)
+                for (int k = 2; k >= 0; --k)
 #pragma unroll
-                    for (int rg = 0; rg < RG; ++rg) O[rg][d0 + d] = mfma16((u32x4){x[d][0], x[d][1], y[d][0], y[d][1]}, w3[rg][k], O[rg][d0 + d]);
+                    for (int rg = 0; rg < RG; ++rg) O[rg][d0 + d] = mfma16(VT, w3[rg][k], O[rg][d0 + d]);
+            }
         }
     }
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // the tiles behind the last one land before the LDS is another workgroup's

@@ -363,8 +363,11 @@ static int rec_runs(const omni_decay_rec& a, const int32_t* items, int n, hipStr
     if (n <= 0) return OMNI_OK;
     // Columns per workgroup: 32 where 128 would leave CUs idle -- a state is then asked for by four times as many waves -- else 128, whose q and k are summed and
     // activated once.  Us, 16 heads of 128 x 128, one token of 1 | 2 | 4 | 8 | 12 | 16 | 24 | 48 sequences, by 128 columns 7.5 | 7.7 | 8.1 | 9.0 | 9.9 | 11.0 | 14.8 | 22.0, by 32
-    // 4.4 | 4.7 | 5.1 | 6.4 | 7.6 | 9.2 | 14.7 | 23.6.
-    if ((int64_t)a.heads * n * ((a.vp + 127) / 128) <= 256) rec_runs_launch<8, RAW>(a, items, n, st);
+    // 4.4 | 4.7 | 5.1 | 6.4 | 7.6 | 9.2 | 14.7 | 23.6.  Longer columns fill a CU's registers sooner, and what does not fit at once is a round more: 4 heads, by 128 / by 32, 256 x 128
+    // of 32 sequences 15.6 / 12.8, of 36 16.6 / 19.0, of 64 23.1 / 23.8; 160 x 128 of 32 10.8 / 8.6, of 36 11.2 / 12.6, of 64 15.6 / 18.8; 8 of 256 x 64 of 24 10.0 / 9.4, of 32 11.4 / 13.0;
+    // above 256 rows, by 64 / by 32, 512 x 128 of 48 25.6 / 24.6, of 56 29.1 / 32.9; 288 x 128 17.4 / 14.2, 19.2 / 20.5; 8 of 512 x 64 of 32 22.4 / 18.3.
+    const int64_t wide = (int64_t)a.heads * n * ((a.vp + 127) / 128), narrow = (int64_t)a.heads * n * ((a.vp + 31) / 32);
+    if (wide <= (a.dp > 128 && a.dp <= 256 ? 192 : 256) && (a.dp <= 128 || narrow <= (a.dp <= 256 ? 512 : 768))) rec_runs_launch<8, RAW>(a, items, n, st);
     else if (a.vp > 64 && a.dp <= 256) rec_runs_launch<32, RAW>(a, items, n, st);
     else rec_runs_launch<16, RAW>(a, items, n, st);
     OMNI_CHECK_LAUNCH("omni_decay_rec(runs)");

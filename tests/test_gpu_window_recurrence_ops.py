@@ -494,6 +494,13 @@ def test_runs_by_32_64_and_128_columns(heads, dim, vdim, n, form):
     run_recurrence([1] * (n - 1) + [2], [r % 3 for r in range(n)], heads, dim, vdim, [0.9 - 0.02 * h for h in range(heads)], form, seed=n + dim)
 
 
+@pytest.mark.parametrize("form", ["sums", "rows"])
+@pytest.mark.parametrize("heads,dim,vdim,n", [(16, 136, 128, 8), (16, 136, 128, 9), (16, 256, 64, 12), (16, 256, 64, 13), (16, 264, 128, 12), (16, 264, 128, 13), (16, 512, 64, 16), (16, 512, 64, 17)])
+def test_runs_of_long_columns(heads, dim, vdim, n, form):
+    """Columns of more than 128 and of more than 256 rows, up to the last sequence that goes by 32 of them and the next."""
+    run_recurrence([1] * (n - 1) + [2], [r % 3 for r in range(n)], heads, dim, vdim, [0.9 - 0.02 * h for h in range(heads)], form, seed=n + dim)
+
+
 def test_argument_errors_come_back_as_errors():
     lib = L.load_decoder()
     for fn, s in (("omni_qkv_write_run", L.QkvWrite()), ("omni_gated_norm_run", L.GatedNorm()), ("omni_window_attn_run", L.WindowAttn()), ("omni_decay_rec_run", L.DecayRec())):

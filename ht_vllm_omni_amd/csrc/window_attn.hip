@@ -665,8 +665,11 @@ static int wa_run(const omni_window_attn& p, WinArgs a, hipStream_t st) {
         // One workgroup per CU.  A second to each halves no walk that two CUs' worth of keys in flight do not already fill, and its records cost their writing and a
         // merge.  Us with the merge, by two / one, 16 heads over 4 of 128, window 1024, contexts of up to 352 | 700 | 2048: 8 rows 10.0 / 10.0 | 11.2 / 11.1 |
         // 14.7 / 12.3, 16 rows 10.7 / 10.5 | 13.5 / 12.3 | 16.4 / 15.2, 32 rows 13.0 / 11.9 | 17.0 / 16.3 | 22.6 / 22.7, 64 rows -- which then leave no records -- 16.5 / 13.4 |
-        // 25.2 / 22.0 | 37.5 / 35.2.  (By one per two CUs: 32 rows of up to 2048 29.8.  Eight waves a workgroup: 64 rows 14.1 | 23.8 | 37.4.)
-        a.nsplit = p.workspace ? la_split_count(wgs * p.n_decode, p.window > 0 && p.window < p.max_keys ? p.window + 15 : p.max_keys, 256) : 1;
+        // 25.2 / 22.0 | 37.5 / 35.2.  (By one per two CUs: 32 rows of up to 2048 29.8.  Eight waves a workgroup: 64 rows 14.1 | 23.8 | 37.4.)  What it costs: one row of
+        // 8192 keys beside 31 of 100, no window, 47.9 / 49.9.
+        // Heads of up to 64 are half the bytes a key, and one workgroup's walk no longer fills a CU: two per CU, as ever (8 heads over 2 of 64, two / one: 64 rows of up to
+        // 2048 20.3 / 22.4, in windows of 1024 14.5 / 15.4, one of 8192 beside 63 of 100 44.0 / 60.2; 32 rows 14.6 / 15.0, 12.5 / 11.5, 26.6 / 33.9).
+        a.nsplit = p.workspace ? la_split_count(wgs * p.n_decode, p.window > 0 && p.window < p.max_keys ? p.window + 15 : p.max_keys, WS <= 2 ? 512 : 256) : 1;
         hipLaunchKernelGGL((window_decode_kernel<WS, EX>), dim3(wgs, p.n_decode, a.nsplit), dim3(64 * LA_DEC_WAVES), lds, st, a);
         OMNI_CHECK_LAUNCH("omni_window_attn(decode)");
         if (a.nsplit > 1) {

@@ -303,9 +303,10 @@ __global__ __launch_bounds__(GS_THREADS) void gemm_behind_kernel(const StreamArg
 // Columns per workgroup and K splits.  At more than 32 rows a workgroup's registers and LDS leave room for one per CU, so a grid runs in rounds of 256; below,
 // several share a CU and a further round costs three quarters of the first.  A workgroup's time goes with the operand tiles it reads per k-step (NT of W; of x,
 // which is in L2, three quarters of MT) plus its epilogue, NT * MT sums of eight waves through LDS; a split also costs its reader.
-// Measured over 1 ... 64 rows x the weight shapes of the language models, 1600 products out of HBM, the reader of partial sums at 30 ns and 8 TB/s a slab: what
-// the rule picks is 0.5 % behind the best on average (rounds in full, MT in full and a fifth of the epilogue: 2.1 %).  Us, before / now, 8 rows, rows x K:
-// 8192 x 2048 8.9 / 7.8 (4 column tiles in 2 splits / 2 in one), 5120 x 2048 6.4 / 5.8, 5120 x 1024 4.5 / 4.4, 1024 x 2048 3.4 / 3.0; 64 rows 8192 x 2048 10.9 / 10.1.
+// The numbers are a fit with all rows in a workgroup, over 1 ... 64 rows x the weight shapes of the language models; gs_run then deals rows out.  As launched, over 297 products
+// out of HBM and every choice of columns, splits and rows, the reader of partial sums at 30 ns and 8 TB/s a slab, it is 1.0 % behind the best on average (the rule before,
+// rounds, MT and splits in full and a fifth of the epilogue: 4.1 %); table: profiles/gemm_stream_sweep.txt.  Us, before / now, 8 rows, columns x K: 8192 x 2048 8.8 / 7.7 (4 column
+// tiles in 2 splits / 2 in one), 5120 x 2048 6.5 / 5.8, 5120 x 1024 4.6 / 4.4, 1024 x 2048 3.5 / 3.0.  Slower: 2064 columns, 129 tiles, at 17 - 32 rows, 4.4 / 4.7.
 // As before: 9216 x 2048 by 3 (192 workgroups; by 2, 288 of them, 2 us more), 2048 x 9216 by 2 in 4 splits.
 static void gs_policy(int M, int N, int nsteps, bool slabs, int* nt, int* splits) {
     const int tiles = N / 16, mt = M > 32 ? 4 : (M > 16 ? 2 : 1);

@@ -1,5 +1,6 @@
 """Decoder-only language models end to end on the GPU, against the plain whole-sequence oracle: prompts, decoding, portions, mixed batches, reused
 pages and slots, generation through scheduler and runner, the command line."""
+import ctypes as C
 import json
 import os
 import subprocess
@@ -170,6 +171,16 @@ def test_a_large_head_takes_rows_that_are_made_once(n):
     lw = eng.layer_w[0]
     assert [made[id(m)] for m in (eng.head, lw.up, lw.mixer.down)] == [{False}, {True}, {n <= 2}]
     assert_logits(logits[:, :d.vocab], oracle_logits(w, cfg, toks), "bfloat16")
+
+
+@pytest.mark.parametrize("name", ["mixed", "k_mixed"])
+def test_a_forward_leaves_no_pointers_behind(name):
+    """What a product makes its few rows of names the batch's arrays: nothing keeps it once the forward is over."""
+    d, w, _ = model(name, seed=5)
+    eng = DecoderEngine(d, w, dtype="bfloat16", num_blocks=8, max_batch=2, block_size=8)
+    eng.block_table[0, :1], eng.state_slot[0] = 3, 1
+    eng.forward(eng.make_batch(torch.tensor(tokens(2, d.vocab)), np.zeros(2), np.arange(2), [2]))
+    assert not [k for o in (eng, eng._any, *eng.layer_w.values()) for k, v in vars(o).items() if isinstance(v, C.Structure)]
 
 
 @pytest.mark.parametrize("dtype", DTYPES)

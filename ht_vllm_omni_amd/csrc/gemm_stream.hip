@@ -304,9 +304,9 @@ __global__ __launch_bounds__(GS_THREADS) void gemm_behind_kernel(const StreamArg
 // several share a CU and a further round costs three quarters of the first.  A workgroup's time goes with the operand tiles it reads per k-step (NT of W; of x,
 // which is in L2, three quarters of MT) plus its epilogue, NT * MT sums of eight waves through LDS; a split also costs its reader.
 // The numbers are a fit with all rows in a workgroup, over 1 ... 64 rows x the weight shapes of the language models; gs_run then deals rows out.  As launched, over 297 products
-// out of HBM and every choice of columns, splits and rows, the reader of partial sums at 30 ns and 8 TB/s a slab, it is 1.0 % behind the best on average (the rule before,
-// rounds, MT and splits in full and a fifth of the epilogue: 4.1 %); table: profiles/gemm_stream_sweep.txt.  Us, before / now, 8 rows, columns x K: 8192 x 2048 8.8 / 7.7 (4 column
-// tiles in 2 splits / 2 in one), 5120 x 2048 6.5 / 5.8, 5120 x 1024 4.6 / 4.4, 1024 x 2048 3.5 / 3.0.  Slower: 2064 columns, 129 tiles, at 17 - 32 rows, 4.4 / 4.7.
+// out of HBM and every choice of columns, splits and rows, the reader of partial sums at 30 ns and 8 TB/s a slab, it is 1.3 % behind the best on average (the rule before,
+// rounds, MT and splits in full and a fifth of the epilogue: 4.2 %); table: profiles/gemm_stream_sweep.txt.  Us, before / now, 8 rows, columns x K: 8192 x 2048 8.6 / 7.4 (4 column
+// tiles in 2 splits / 2 in one), 5120 x 2048 6.1 / 5.6, 1024 x 2048 3.2 / 2.8.  Slower: 2064 columns, 129 tiles, at 17 - 32 rows, 4.2 / 4.5.
 // As before: 9216 x 2048 by 3 (192 workgroups; by 2, 288 of them, 2 us more), 2048 x 9216 by 2 in 4 splits.
 static void gs_policy(int M, int N, int nsteps, bool slabs, int* nt, int* splits) {
     const int tiles = N / 16, mt = M > 32 ? 4 : (M > 16 ? 2 : 1);
@@ -346,8 +346,8 @@ static int gs_run(StreamArgs a, int kind, bool one, hipStream_t st) {
     a.split_steps = (a.nsteps + splits - 1) / splits;
     int mt = a.M > 32 ? 4 : (a.M > 16 ? 2 : 1);
     // Where the columns leave half of the CUs idle the rows are dealt out as well: a workgroup's time goes with the x it pulls through its CU, and W is read by the
-    // second group out of a cache.  The same sums.  Us, rows x columns x K, all rows / dealt out: 64 x 2048 x 1536 6.4 / 4.9, 64 x 2048 x 768 4.5 / 3.9, 32 x 2048 x 1536
-    // 4.9 / 4.2, 64 x 1024 x 256 3.0 / 2.7; beyond one round of 256 workgroups the other way round: 64 x 4608 x 1024 6.3 / 7.0, 32 x 9216 x 2048 11.0 / 15.0.
+    // second group out of a cache.  The same sums.  Us, rows x columns x K, all rows / dealt out: 64 x 2048 x 1536 6.1 / 4.6, 64 x 2048 x 768 4.1 / 3.6, 32 x 2048 x 1536
+    // 4.7 / 4.0, 64 x 1024 x 256 2.7 / 2.4; beyond one round of 256 workgroups the other way round: 64 x 4608 x 1024 6.3 / 7.0, 32 x 9216 x 2048 11.0 / 15.0.
     while (mt > 1 && a.N / 16 / nt * splits * (((a.M + 15) / 16 + mt / 2 - 1) / (mt / 2)) <= 256) mt /= 2;
     // a narrow product (a side input's gate), more steps in flight
     if (a.N / 16 * splits <= 32) {

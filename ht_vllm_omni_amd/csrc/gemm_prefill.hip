@@ -879,8 +879,8 @@ static int launch_mid_of(int geom, const TileArgs& a, hipStream_t st, int groups
 // 64 KB in 1.1 - 1.3 us) -- so small grids want small tiles on all 256 CUs and large ones tall tiles.  Two workgroups on a CU share that rate
 // but hide each other's barriers: 0.44 us for a slice of each of two 64 x 64 tiles, 0.27 alone.
 // Numbers: ns above what every launch costs, least squares over M 13 ... 6300 x the weight shapes of the language models, talkers and the vocoder by every tile and count
-// of partial sums; those of the small tiles, of 192 x 128 and of omni_gemm_tile_splits then moved, within a few per cent, to where the fp32 products' counts are the better ones
-// and no other product of 1100 changes its tile.  What the rule picks is 0.9 % behind the best on average; 28 of them take more than 3 % longer than under the rule of
+// of partial sums; those of the small tiles, of 192 x 128, 256 x 128 and of omni_gemm_tile_splits then moved, within a few per cent, to where the fp32 products' counts are the better ones
+// and no other product of 1100 changes its tile (one: 16 heads of 2000 x 512 x 128, 18.0 -> 13.8 us).  What the rule picks is 0.9 % behind the best on average; 27 of them take more than 3 % longer than under the rule of
 // fewer tiles before it.  Table: profiles/gemm_tile_sweep.txt.  Every weight comes out of HBM there, 700 MB of them in turn, as in a step: weights that are in the
 // last-level cache want fewer, larger tiles (50 x 1024 x 3072 by 32 x 32 9.8, by 32 x 64 11.7; the other way round from 150 MB in turn), and numbers searched on those cost the
 // vocoder 2 %.
@@ -898,7 +898,7 @@ static constexpr int mid_size(int i, bool rows) { MID_LIST(MID_SIZE_CASE) return
 #define MID(I) KIND_MID, I, mid_size(I, true), mid_size(I, false)
 static const TileChoice TILE_CHOICES[] = {
     {MID(0), 2484, 140, 2750, 249}, {MID(1), 2402, 196, 2909, 306}, {MID(2), 2660, 280, 3110, 432}, {MID(3), 3100, 466, 4990, 650},
-    {MID(4), 4400, 447},            {MID(5), 5230, 871},            {MID(6), 5800, 912},
+    {MID(4), 4400, 447},            {MID(5), 5450, 871},            {MID(6), 5800, 912},
     {MID(7), 3010, 306, 4090, 542}, {MID(8), 5178, 572},            {MID(9), 4150, 425},
     {KIND_PP, 192, 192, 256, 8570, 996},     {KIND_PP, 224, 224, 256, 9350, 1044},    {KIND_PP, 256, 256, 256, 10300, 1088},
     {KIND_LARGE, 192, 192, 256, 9600, 1015}, {KIND_LARGE, 224, 224, 256, 10300, 1090}, {KIND_LARGE, 256, 256, 256, 11800, 1150},

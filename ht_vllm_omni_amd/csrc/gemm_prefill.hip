@@ -879,14 +879,14 @@ static int launch_mid_of(int geom, const TileArgs& a, hipStream_t st, int groups
 // 64 KB in 1.1 - 1.3 us) -- so small grids want small tiles on all 256 CUs and large ones tall tiles.  Two workgroups on a CU share that rate
 // but hide each other's barriers: 0.44 us for a slice of each of two 64 x 64 tiles, 0.27 alone.
 // Numbers: ns above what every launch costs, least squares over M 13 ... 6300 x the weight shapes of the language models, talkers and the vocoder by every tile and count
-// of partial sums; those of the small tiles, of 192 x 128, 256 x 128 and of omni_gemm_tile_splits then moved, within a few per cent, to where the fp32 products' counts are the better ones
-// and no other product of 1100 changes its tile (one: 16 heads of 2000 x 512 x 128, 18.0 -> 13.8 us).  What the rule picks is 0.9 % behind the best on average; 27 of them take more than 3 % longer than under the rule of
-// fewer tiles before it.  Table: profiles/gemm_tile_sweep.txt.  Every weight comes out of HBM there, 700 MB of them in turn, as in a step: weights that are in the
-// last-level cache want fewer, larger tiles (50 x 1024 x 3072 by 32 x 32 9.8, by 32 x 64 11.7; the other way round from 150 MB in turn), and numbers searched on those cost the
-// vocoder 2 %.
+// of partial sums; some were then moved by a few per cent, with those of omni_gemm_tile_splits, to where the fp32 products' counts are the better ones and no other product of
+// 1400 takes a slower tile.  What the rule picks is 0.7 % behind the best on average, 1.1 % over 376 rows and sizes it was not found on (before: 0.9 %, 1.2 % of the fp32
+// products); 41 of 1300 take more than 3 % longer than under the rule of fewer tiles before it, all together 4 % less.  Table: profiles/gemm_tile_sweep.txt.  Every weight
+// comes out of HBM there, 700 MB of them in turn, as in a step: weights that are in the last-level cache want fewer, larger tiles (50 x 1024 x 3072 by 32 x 32 9.8, by 32 x 64
+// 11.7; the other way round from 150 MB in turn), and numbers searched on those cost the vocoder 2 %.
 // The heights between the powers of two are there for the rounds: a product of 500 rows by 9216 columns is 288 tiles of 128 x 128 on 256 CUs (two rounds,
-// 36 us), 144 of 256 x 128 (33.1) and 216 of 192 x 128 (24.0); 251 x 5120 x 2048 18.7 -> 13.1 by 96 x 64, 800 x 5120 x 2048 31.6 -> 21.6, 502 x 5120 x 2048
-// 20.6 -> 16.4 by 96 x 128.  On average over those products the three are worth 3.3 %.  (Not taken where it would pay: 200 x 4608 x 1024, 96 x 64 8.0, taken 32 x 64 9.3.)
+// 36 us), 144 of 256 x 128 (33.2) and 216 of 192 x 128 (24.7); 200 x 4608 x 1024 9.1 -> 8.0 by 96 x 64, 251 x 5120 x 2048 18.7 -> 13.1, 800 x 5120 x 2048 32 -> 22 by
+// 192 x 128, 502 x 5120 x 2048 20.6 -> 16.5 by 96 x 128.  On average over those products the three are worth 3.3 %.
 enum { KIND_MID, KIND_PP, KIND_LARGE };
 struct TileChoice {
     int kind, geom, bm, bn;          // geom: MID_LIST index, or rows of the two-group / lockstep tile
@@ -897,9 +897,9 @@ static constexpr int mid_size(int i, bool rows) { MID_LIST(MID_SIZE_CASE) return
 #undef MID_SIZE_CASE
 #define MID(I) KIND_MID, I, mid_size(I, true), mid_size(I, false)
 static const TileChoice TILE_CHOICES[] = {
-    {MID(0), 2484, 140, 2750, 249}, {MID(1), 2402, 196, 2909, 306}, {MID(2), 2660, 280, 3110, 432}, {MID(3), 3100, 466, 4990, 650},
+    {MID(0), 2484, 140, 2750, 249}, {MID(1), 2402, 196, 2909, 316}, {MID(2), 2563, 280, 3110, 432}, {MID(3), 3100, 466, 4990, 650},
     {MID(4), 4400, 447},            {MID(5), 5450, 871},            {MID(6), 5800, 912},
-    {MID(7), 3010, 306, 4090, 542}, {MID(8), 5178, 572},            {MID(9), 4150, 425},
+    {MID(7), 3010, 306, 4090, 542}, {MID(8), 5178, 572},            {MID(9), 3999, 425},
     {KIND_PP, 192, 192, 256, 8570, 996},     {KIND_PP, 224, 224, 256, 9350, 1044},    {KIND_PP, 256, 256, 256, 10300, 1088},
     {KIND_LARGE, 192, 192, 256, 9600, 1015}, {KIND_LARGE, 224, 224, 256, 10300, 1090}, {KIND_LARGE, 256, 256, 256, 11800, 1150},
     {KIND_LARGE, 0, 256, 192, 9600, 1040},   {KIND_LARGE, 0, 512, 128, 11800, 1450},  {KIND_LARGE, 0, 512, 96, 11300, 1320},
@@ -913,6 +913,8 @@ static const TileChoice& pick_tile(int M, int N, int K, int groups, int splits, 
     for (const TileChoice& c : TILE_CHOICES) {
         if (c.kind == KIND_PP && !plain) continue;                            // the two-group tile takes a plain product, the lockstep ones the others
         if (c.kind == KIND_LARGE && (c.bn != large_bn || (plain && c.bn == 256) || splits > 1)) continue;
+        // 96 x 128 is four waves: where it makes as many row blocks as 128 x 128 (rows 257 ... 288; below, its blocks are the fuller ones) eight are faster, 284 x 7936 x 2048 19.5 / 18.0 us
+        if (c.kind == KIND_MID && c.geom == 9 && M > 256 && (M + 95) / 96 == (M + 127) / 128) continue;
         const long long tiles = (long long)((M + c.bm - 1) / c.bm) * ((N + c.bn - 1) / c.bn) * groups * splits;
         long long t;
         // (a CU that gets a third small tile while the first two run does not wait for a round of two)
@@ -925,9 +927,9 @@ static const TileChoice& pick_tile(int M, int N, int K, int groups, int splits, 
 }
 
 // Partial sums for the reader of an fp32 product to add up: as many as make the product and their extra traffic (written here, read there) cheapest; at
-// most 4, what the readers take (OMNI_STREAM_MAX_SPLITS).  The traffic at 3.3 TB/s and 23 ns, found with the tiles' numbers: over 258 fp32 products of up to 1100 rows
-// product and reader (a slab read at 8 TB/s and 30 ns) are 0.6 % behind the best tile and count on average.  At 3.8 TB/s and 100 ns, from before the tiles' numbers moved,
-// 1.2 %: 66 x 2080 x 2048 in four took 7.6 us, in two 6.5, 800 x 2048 x 7936 in three 39 to 43, in two 35.
+// most 4, what the readers take (OMNI_STREAM_MAX_SPLITS).  The traffic at 3.5 TB/s and 124 ns, found with the tiles' numbers: over 316 fp32 products of up to 1100 rows
+// product and reader (a slab read at 8 TB/s and 30 ns) are 0.8 % behind the best tile and count on average.  At 3.8 TB/s and 100 ns, from before the tiles' numbers moved,
+// 1.3 %: 66 x 2080 x 2048 in four took 7.6 us, in two 6.4, 800 x 2048 x 7936 in three 40 to 43, in two 34.
 extern "C" int omni_gemm_tile_splits(int M, int N, int K) {
     int best = 1;
     long long least = -1;
@@ -935,7 +937,7 @@ extern "C" int omni_gemm_tile_splits(int M, int N, int K) {
         if (s > 1 && (K / 32 < 8 * s || N % 16)) break;
         long long t;
         pick_tile(M, N, K, 1, s, true, false, &t);
-        t += (long long)(s - 1) * M * N * 8 / 3301 + (s > 1 ? 23 : 0);
+        t += (long long)(s - 1) * M * N * 8 / 3500 + (s > 1 ? 124 : 0);
         if (least < 0 || t < least) { least = t; best = s; }
     }
     return best;

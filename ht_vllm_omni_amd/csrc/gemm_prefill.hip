@@ -880,8 +880,8 @@ static int launch_mid_of(int geom, const TileArgs& a, hipStream_t st, int groups
 // but hide each other's barriers: 0.44 us for a slice of each of two 64 x 64 tiles, 0.27 alone.
 // Numbers: ns above what every launch costs, least squares over M 13 ... 6300 x the weight shapes of the language models, talkers and the vocoder by every tile and count
 // of partial sums; some were then moved by a few per cent, with those of omni_gemm_tile_splits, to where the fp32 products' counts are the better ones and no other product of
-// 1400 takes a slower tile.  What the rule picks is 0.7 % behind the best on average, 1.1 % over 376 rows and sizes it was not found on (before: 0.9 %, 1.2 % of the fp32
-// products); 41 of 1300 take more than 3 % longer than under the rule of fewer tiles before it, all together 4 % less.  Table: profiles/gemm_tile_sweep.txt.  Every weight
+// 1400 takes a slower tile.  What the rule picks is 0.8 % behind the best on average, 1.0 % over 398 rows and sizes it was not found on (before: 0.9 %, of the fp32 products
+// 1.2 %); 38 of 1323 take more than 3 % longer than under the rule of fewer tiles before it, all together 4 % less.  Table: profiles/gemm_tile_sweep.txt.  Every weight
 // comes out of HBM there, 700 MB of them in turn, as in a step: weights that are in the last-level cache want fewer, larger tiles (50 x 1024 x 3072 by 32 x 32 9.8, by 32 x 64
 // 11.7; the other way round from 150 MB in turn), and numbers searched on those cost the vocoder 2 %.
 // The heights between the powers of two are there for the rounds: a product of 500 rows by 9216 columns is 288 tiles of 128 x 128 on 256 CUs (two rounds,
@@ -920,6 +920,8 @@ static const TileChoice& pick_tile(int M, int N, int K, int groups, int splits, 
         // (a CU that gets a third small tile while the first two run does not wait for a round of two)
         if (c.slice2 && tiles > 256) t = (c.round2 + slices * c.slice2) * ((tiles + 255) / 256) / 2;
         else t = (c.round1 + slices * c.slice1) * ((tiles + 255) / 256);
+        // 192 x 128 in runs of K costs 80 ns a slice more than whole: 700 x 2048 x 9216 in four runs 43 us, by 96 x 128 in two 35
+        if (c.kind == KIND_MID && c.geom == 8 && splits > 1) t += 80 * slices * ((tiles + 255) / 256);
         if (!best || t < least) { best = &c; least = t; }
     }
     if (ns) *ns = least;
@@ -927,9 +929,9 @@ static const TileChoice& pick_tile(int M, int N, int K, int groups, int splits, 
 }
 
 // Partial sums for the reader of an fp32 product to add up: as many as make the product and their extra traffic (written here, read there) cheapest; at
-// most 4, what the readers take (OMNI_STREAM_MAX_SPLITS).  The traffic at 3.5 TB/s and 124 ns, found with the tiles' numbers: over 316 fp32 products of up to 1100 rows
-// product and reader (a slab read at 8 TB/s and 30 ns) are 0.8 % behind the best tile and count on average.  At 3.8 TB/s and 100 ns, from before the tiles' numbers moved,
-// 1.3 %: 66 x 2080 x 2048 in four took 7.6 us, in two 6.4, 800 x 2048 x 7936 in three 40 to 43, in two 34.
+// most 4, what the readers take (OMNI_STREAM_MAX_SPLITS).  The traffic at 3.5 TB/s and 124 ns, found with the tiles' numbers: over 325 fp32 products of up to 1100 rows
+// product and reader (a slab read at 8 TB/s and 30 ns) are 0.6 % behind the best tile and count on average.  At 3.8 TB/s and 100 ns, from before the tiles' numbers moved,
+// 1.2 %: 66 x 2080 x 2048 in four took 7.6 us, in two 6.4, 800 x 2048 x 7936 in three 40 to 43, in two 34.
 extern "C" int omni_gemm_tile_splits(int M, int N, int K) {
     int best = 1;
     long long least = -1;

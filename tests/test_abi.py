@@ -195,7 +195,7 @@ def test_which_products_make_their_rows(args, joins):
 
 
 @pytest.mark.parametrize("M,N,K,best", [(66, 2080, 2048, {2}), (75, 2048, 2048, {2, 4}), (200, 1056, 1024, {2}), (800, 2048, 7936, {2}), (50, 1024, 3072, {4}), (13, 2048, 9216, {4}),
-                                        (390, 1024, 4608, {3}), (640, 2048, 9216, {3})])
+                                        (390, 1024, 4608, {3}), (640, 2048, 9216, {3}), (700, 2048, 7936, {2}), (760, 2048, 9216, {2})])
 def test_counts_of_partial_sums_that_measured_best(M, N, K, best):
     """Counts that with their reader are within 3 % of the fastest over all tiles (profiles/gemm_tile_sweep.txt)."""
     from ht_vllm_omni_amd import _lib

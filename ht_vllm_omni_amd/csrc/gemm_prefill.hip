@@ -68,11 +68,12 @@ __device__ __forceinline__ float tg_gelu(float v) { return 0.5f * v * (1.0f + er
 
 // Epilogues, each a body of its own: one that held every activation outgrew the compiler's unrolling of its passes at 256 rows, and accumulators
 // indexed by a run-time pass live in scratch memory (+ 25 us per launch).
-//   EPI_PLAIN  bf16 out        EPI_ACT  XIELU, RELU2, SILU_SIGMOID, GELU_MUL or none -> bf16 and / or fp32 out
+//   EPI_PLAIN  bf16 out        EPI_F32  fp32 out        EPI_ACT  XIELU, RELU2, SILU_SIGMOID, GELU_MUL or none -> bf16 and / or fp32 out
 //   EPI_FULL   bias, scale, GELU or none, residual, any outputs
-enum { EPI_PLAIN = 0, EPI_ACT = 1, EPI_FULL = 2 };
+enum { EPI_PLAIN = 0, EPI_ACT = 1, EPI_FULL = 2, EPI_F32 = 3 };
 __host__ __device__ __forceinline__ int tile_epi(const TileArgs& a) {
     if (a.bias || a.scale || a.act == OMNI_TILE_ACT_GELU || a.resid || a.out2) return EPI_FULL;
+    if (a.out_f32 && !a.out && a.act == OMNI_TILE_ACT_NONE) return EPI_F32;
     return a.out_f32 || a.act >= OMNI_TILE_ACT_XIELU ? EPI_ACT : EPI_PLAIN;
 }
 
@@ -88,9 +89,13 @@ __device__ __forceinline__ void tile_epilogue(const TileArgs& a, f32x4 (&acc)[WN
     // of an fp32 output (whole 128-byte lines); + fp32 residual (the pass's residual loads are issued before its image is written:
     // the epilogue of a residual GEMM is an HBM phase, not a chain of load -> add -> store round trips), then up to three stores of
     // the SAME fp32 value: fp32 (the residual stream), bf16 (the next GEMM's operand), bf16(snake(y)) (the next conv's operand).
+    // fp32 alone (EPI_F32, the products that a row kernel reads): 4 columns per lane, so that a wave's store is whole rows of 256 contiguous bytes; two stores of 16 of every
+    // 32 bytes, as behind the other outputs, write at 3 - 4 TB/s.  Us, before / now: 1547 x 1024 x 2048 in two partial sums 13.8 / 12.5, 1000 x 2048 x 2048 in two 16.3 / 14.9,
+    // 6001 x 2048 x 2048 48.8 / 46.2, 70 x 2048 x 2048 in four 6.4 / 6.2; straight from the registers, 64 bytes a row, 13.6, 15.4 and 46.6.  With a residual or a second output
+    // it is the other way round (twice the instructions: 6001 x 2048 x 2048 58.2 / 59.1, with GELU 56.7 / 58.8).
     // (Two images per wave, pass p + 1's written before pass p's is read back, measured SLOWER: 5.9 k -> 8.5 k cycles per epilogue.)
     constexpr int IPITCH = WN * 64 + 16;                  // bytes per image row
-    constexpr int PER_ROW = GU8 ? WN : WN * 2;            // lane items per image row: a [8 gate | 8 up] tile, or 8 columns
+    constexpr int PER_ROW = GU8 ? WN : EPI == EPI_F32 ? WN * 4 : WN * 2;      // lane items per image row: a [8 gate | 8 up] tile, 4 columns, or 8
     constexpr int RIT = (16 * PER_ROW + 63) / 64;         // row-side iterations per pass
     uint8_t* img = lds + wave * (16 * IPITCH);
     auto bias_scale = [&](int j, f32x4& b, f32x4& s) {
@@ -169,6 +174,14 @@ __device__ __forceinline__ void tile_epilogue(const TileArgs& a, f32x4 (&acc)[WN
                 }
                 *reinterpret_cast<u32x4*>(a.out + (size_t)m * a.ldo + (n >> 1)) = o;
             }
+        } else if (EPI == EPI_F32) {
+#pragma unroll
+            for (int it = 0; it < RIT; ++it) {
+                const int idx = lane + 64 * it;
+                const int row = idx / PER_ROW, ch = idx - row * PER_ROW;
+                const int m = mp0 + row, n = nw0 + ch * 4;
+                if (m < a.M && n < a.N) *reinterpret_cast<f32x4*>(a.out_f32 + (size_t)m * a.ldf + n) = *reinterpret_cast<const f32x4*>(img + row * IPITCH + ch * 16);
+            }
         } else {
 #pragma unroll
             for (int it = 0; it < RIT; ++it) {
@@ -235,6 +248,7 @@ template <int WN, int WM, bool GU8>
 __device__ __forceinline__ void tile_epilogue_of(const TileArgs& a, f32x4 (&acc)[WN][WM], uint8_t* lds, int wave, int lane, int mw0, int nw0) {
     const int epi = tile_epi(a);
     if (epi == EPI_PLAIN) tile_epilogue<WN, WM, GU8, EPI_PLAIN>(a, acc, lds, wave, lane, mw0, nw0);
+    else if (!GU8 && epi == EPI_F32) tile_epilogue<WN, WM, GU8, EPI_F32>(a, acc, lds, wave, lane, mw0, nw0);
     else if (!GU8 && epi == EPI_ACT) tile_epilogue<WN, WM, GU8, EPI_ACT>(a, acc, lds, wave, lane, mw0, nw0);
     else tile_epilogue<WN, WM, GU8, EPI_FULL>(a, acc, lds, wave, lane, mw0, nw0);
 }
@@ -997,7 +1011,7 @@ extern "C" int omni_gemm_tile(const omni_tile_gemm* g, void* stream) {
     a.x_bytes = (int)(((g->x_rows - 1) * g->ldx + (groups - 1) * a.gx_cols + seg_len) * 2);
     hipStream_t st = (hipStream_t)stream;
     const int N = g->N;
-    OMNI_CHECK_ARG(g->k_splits >= 0 && g->k_splits <= 4 && (g->k_splits <= 1 || (tile_epi(a) == EPI_ACT && g->act == OMNI_TILE_ACT_NONE && !g->out && groups == 1 && g->k_splits <= g->K / 32 &&
+    OMNI_CHECK_ARG(g->k_splits >= 0 && g->k_splits <= 4 && (g->k_splits <= 1 || (tile_epi(a) == EPI_F32 && groups == 1 && g->k_splits <= g->K / 32 &&
                    g->slab_stride >= (int64_t)(g->M - 1) * g->ldf + N && g->slab_stride % 4 == 0)), "omni_gemm_tile: k_splits=%d (<= K / 32; one group, fp32 output alone)", g->k_splits);
     a.splits = g->k_splits > 1 ? g->k_splits : 1; a.slab_stride = g->slab_stride;
     // tile_hint: 1 the large lockstep tiles, 2 and 8 ... 16 the mid-size ones, 3 / 4 lockstep and 5 / 6 / 7 two-group at 224 / 192 and 256 / 224 / 192 rows

@@ -84,6 +84,20 @@ def test_tiles_of_96_and_192_rows_at_their_edges(M, N, K, taps, dil):
             assert torch.equal(*(ops.gemm_tile(x, wf, want="f", splits=3, tile_hint=h) for h in (hint, 2))), hint
 
 
+@pytest.mark.parametrize("M,N,K", [(1, 16, 32), (33, 48, 64), (95, 144, 96), (257, 272, 160), (300, 768, 288)])
+def test_fp32_output_alone_at_every_tiles_edges(M, N, K):
+    """A product that leaves fp32 alone stores 4 columns a lane: the bits of the form that leaves both outputs, at M and N inside, on and one past a tile, and nothing of the
+    rows' rest or of the rows behind them."""
+    ops, L, frag_shuffle, _ = _ops()
+    g = torch.Generator().manual_seed(M * 17 + K)
+    x, w = torch.randn(M, K, generator=g).to(BF16).cuda(), frag_shuffle((torch.randn(N, K, generator=g) * 0.05).to(BF16)).cuda()
+    ref, _ = ops.gemm_tile(x, w, want="fb")
+    for hint in (0, 1, 2) + tuple(range(8, 17)) + ((3, 4, 5, 6, 7) if N % 256 == 0 else ()):
+        out = torch.full((M + 3, N + 12), 7.0, device="cuda")
+        ops.gemm_tile(x, w, want="f", out_f32=out[:M, :N], tile_hint=hint)
+        assert torch.equal(out[:M, :N], ref) and bool((out[M:] == 7.0).all()) and bool((out[:, N:] == 7.0).all()), hint
+
+
 @pytest.mark.parametrize("M,K,splits", [(33, 32, 1), (70, 96, 3), (129, 160, 4), (65, 64, 1)])
 def test_rows_that_end_an_array(M, K, splits):
     """x is the last columns of a wider array and a run of K steps is a single one: what a tile fetches ahead of its last step lies past the last row."""

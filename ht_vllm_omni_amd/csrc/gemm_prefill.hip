@@ -860,7 +860,13 @@ static int launch_mid(TileArgs a, hipStream_t st, int groups) {
         const int per_xcd = (a.mblocks * a.nblocks + 7) / 8;
         int band = 1;
         while (band * band < per_xcd) ++band;
-        a.band = band > a.mblocks ? a.mblocks : band;
+        // Row blocks of up to 5 stay together: a panel of W, which comes out of HBM, is fetched by one XCD then, and the rows of so few blocks fit its L2; more in
+        // bands of equal height, not 6 and 1.  The same products in a whole forward, us (in launches of one product in turn x stays in the L2s and the
+        // difference is another): one prompt of 130 tokens 459 / 447, 2 of 251 1101 / 1076, 48 decoded tokens beside two portions 1477 / 1454; the mean of forty
+        // forwards 0.5 % less (up to 8 blocks together 0.6, with products of 16 rows in two runs of K slower).  W fetched past the caches where only one XCD reads
+        // it is up to 20 % faster in such launches, and up to 7 % slower in forwards of a model whose weights the last-level cache holds.
+        const int bands = (a.mblocks + band - 1) / band;
+        a.band = a.mblocks <= 5 ? a.mblocks : (a.mblocks + bands - 1) / bands;
     }
     static bool attr_set = false;
     if (!attr_set) {

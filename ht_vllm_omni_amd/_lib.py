@@ -239,6 +239,7 @@ DECODER_SIGNATURES = {
     **{n: SIGNATURES[n] for n in ("omni_last_error", "omni_abi_version", "omni_gemm_tile", "omni_gemm_tile_splits", "omni_sample", "omni_sample_rows")},
     "omni_stream_rows_run": (i32, [C.POINTER(StreamRows), vp]),
     "omni_latent_write_run": (i32, [C.POINTER(LatentWrite), vp]),
+    "omni_latent_write_rows": (i32, [C.POINTER(LatentWrite), vp, vp, i32, vp]),
     "omni_latent_attn_run": (i32, [C.POINTER(LatentAttn), vp]),
     "omni_latent_attn_workspace_bytes": (i64, [i32, i32, i32]),
     "omni_latent_attn_mfma": (i32, [i32]),

@@ -54,6 +54,8 @@ typedef struct omni_latent_write {
     int T, elem;
 } omni_latent_write;
 int omni_latent_write_run(const omni_latent_write* a, void* stream);
+/* ... and the new latents of tokens from .. T - 1 (bf16) to a second array besides: token t of batch row b to row row_base[b] + positions[t] of rows [.., rp] */
+int omni_latent_write_rows(const omni_latent_write* a, void* rows, const int32_t* row_base, int from, void* stream);
 
 /* Behind the joint projection proj fp32 [T, ld] (the sum of `slabs` such arrays) of a grouped attention layer, every head padded with zeros:
  *   [q heads * dp | k kv_heads * dp | v kv_heads * vp | gate logits heads * vp]        (kc == NULL: no k and v, another layer's are read;

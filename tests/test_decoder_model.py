@@ -11,7 +11,7 @@ from ht_vllm_omni_amd import models
 from ht_vllm_omni_amd.checkpoint import load_decoder_checkpoint
 from ht_vllm_omni_amd.config import TalkerDims
 from ht_vllm_omni_amd.decoder_config import dims_from_config, tensor_shapes
-from ht_vllm_omni_amd.decoder_mixers import (LATENT_WIDTHS, LatentMixer, attention_tiles, cache_row_widths, cache_traffic, cached_rows, first_rows, latent_width,
+from ht_vllm_omni_amd.decoder_mixers import (LATENT_WIDTHS, LatentMixer, attention_tiles, cache_row_widths, cache_traffic, cached_rows, earlier_rows, first_rows, latent_width,
                                              pad_head_cols, pad_head_rows, pad_heads, recurrence_chunks, recurrence_segments, state_bytes)
 from ht_vllm_omni_amd.payloads import OmniModelRunnerOutput, SamplingParams
 from ht_vllm_omni_amd.sched import SlotPool
@@ -139,6 +139,8 @@ def test_cached_rows_name_every_key_of_every_segment(segs):
         assert 0 < n <= L.GATHER_ROWS and key % L.GATHER_ROWS == 0
         got += [(r, key + i, to + i) for i in range(n)]
     assert got == want
+    earlier = [(r, key + i, to + i) for r, key, n, to in earlier_rows(segs).tolist() for i in range(n)]
+    assert earlier == [(r, k, a) for (r, k, a) in want if k < dict((s, p) for _, p, s in segs)[r]]
     starts = first_rows(segs)
     assert len(starts) == max(first) + 1 and all(int(starts[r, 0]) == a for r, a in first.items())
 

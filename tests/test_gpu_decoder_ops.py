@@ -196,6 +196,41 @@ def test_latent_write(elem, q_rank, kv_rank, heads, gated):
     assert torch.equal(state.cpu(), ws), "state: each live sequence's last token, nothing else"
 
 
+@pytest.mark.parametrize("q_rank,kv_rank,slabs", [(8, 8, 1), (160, 264, 3), (1500, 500, 2)])
+def test_latent_write_rows(q_rank, kv_rank, slabs):
+    """The second place of new latents: the cache's own bits at row_base + position for tokens from `start` on, nothing anywhere else; the rest of the launch as without."""
+    g, T, bs, start = gen(kv_rank), 9, 16, 2
+    qp, rp = r32(q_rank), r32(kv_rank)
+    ld = qp + rp
+    parts = torch.zeros(slabs, T, ld)
+    parts[..., :q_rank], parts[..., qp:qp + kv_rank] = torch.randn(slabs, T, q_rank, generator=g), torch.randn(slabs, T, kv_rank, generator=g)
+    row = torch.tensor([0, 2, 1, 1, 1, 3, 3, 3, 3], dtype=torch.int32)
+    pos = torch.tensor([31, 5, 15, 16, 17, 0, 1, 2, 3], dtype=torch.int32)
+    bt = torch.tensor([[5, 2], [3, 8], [7, 1], [9, 10]], dtype=torch.int32)
+    base = torch.tensor([1 << 20, 4, 1 << 20, 0], dtype=torch.int32)                # rows 0 and 2 are decoded tokens: never looked up
+    got = []
+    for second in (False, True):
+        cq, cache = torch.zeros(16, qp, dtype=torch.bfloat16, device="cuda"), torch.full((11, bs, rp), 5.0, dtype=torch.bfloat16, device="cuda")
+        a = L.LatentWrite(slabs=slabs, slab_stride=T * ld, ld=ld, q_rank=q_rank, qp=qp, kv_rank=kv_rank, rp=rp, heads=1, eps=1e-5, bt_stride=2, block_size=bs, T=T)
+        held = dict(proj=dev(parts), qw=dev(padc(torch.ones(q_rank), qp).to(torch.bfloat16)), kw=dev(padc(torch.ones(kv_rank), rp).to(torch.bfloat16)), cq=cq, cache=cache, block_table=dev(bt), row_of_tok=dev(row),
+                    positions=dev(pos))
+        for k, v in held.items():
+            setattr(a, k, v.data_ptr())
+        side, b = torch.full((24, rp), 7.0, dtype=torch.bfloat16, device="cuda"), dev(base)
+        if second:
+            call("omni_latent_write_rows", C.byref(a), side, b, start)
+        else:
+            call("omni_latent_write_run", C.byref(a))
+        got.append((cq, cache))
+    assert all(torch.equal(x, y) for x, y in zip(*got))
+    want = torch.full((24, rp), 7.0, dtype=torch.bfloat16)
+    for t in range(start, T):
+        want[int(base[row[t]]) + int(pos[t])] = got[0][1][int(bt[row[t], pos[t] // bs]), int(pos[t]) % bs].cpu()
+    assert torch.equal(side.cpu(), want)
+    lib = L.load_decoder()
+    assert lib.omni_latent_write_rows(C.byref(a), side.data_ptr(), b.data_ptr(), T + 1, None) == -1 and lib.omni_latent_write_rows(C.byref(a), None, b.data_ptr(), 0, None) == -1
+
+
 # ---------------------------------------------------------------- products
 @pytest.mark.parametrize("T", [1, 7, 16, 33, 64, 200])
 @pytest.mark.parametrize("heads,n,k", [(1, 32, 32), (3, 64, 32), (5, 48, 96), (16, 512, 128), (16, 128, 512), (2, 16, 288)])

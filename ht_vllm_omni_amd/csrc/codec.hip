@@ -13,6 +13,7 @@
 // it calls); oracle: oracle/code2wav_oracle.py.
 #include "common.cuh"
 #include "kernels.h"
+#include <initializer_list>
 
 typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
 
@@ -61,12 +62,15 @@ extern "C" int omni_codec_rvq_embed(const int64_t* codes, int ld_codes, const fl
 // The row and the weights are asked for at once and stay in registers (PIECES of 256 columns; the row was walked twice, a wait per piece).  Measured in the
 // decode of 50 frames, 17 of these launches over 50 rows of 1024: 1158 -> 1143 us.  Wider rows take the kernel that walks them.
 // ADD: what the sublayer in front left joins the row first: partial sums of a product whose few tiles would each walk all of K alone (omni_gemm_tile k_splits).
+// A few rows are dealt out a wave to a workgroup: with partial sums a row is 28 KB, and four of them on one CU wait for its intake
+// (the 17 norms of 50 frames, all together 15 us less).
+static int norm_rows(int T) { return T <= 1024 ? 1 : 4; }
 struct CodecAdd { float* x; const float* y; const float* scale; int slabs; long long stride; };
 template <int PIECES, bool ADD>
 __global__ __launch_bounds__(256) void codec_rmsnorm_kernel(const float* x, int ldx, const float* __restrict__ w, float eps,
                                                             uint16_t* __restrict__ out, int T, int H, const CodecAdd add) {
     const int lane = threadIdx.x & 63;
-    const int t = blockIdx.x * 4 + (threadIdx.x >> 6);
+    const int t = blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6);
     if (t >= T) return;
     const float* xr = x + (size_t)t * ldx;
     f32x4 v[PIECES], g[PIECES];
@@ -134,7 +138,8 @@ __global__ __launch_bounds__(256) void codec_rmsnorm_wide_kernel(const float* __
 
 extern "C" int omni_codec_rmsnorm(const float* x, int ldx, const float* w, float eps, void* out, int T, int H, void* stream) {
     OMNI_CHECK_ARG(x && w && out && T > 0 && H > 0 && H % 4 == 0 && ldx >= H && ldx % 4 == 0, "omni_codec_rmsnorm: T=%d H=%d ldx=%d", T, H, ldx);
-    const dim3 grid((T + 3) / 4), block(256);
+    const int per = H <= 1024 ? norm_rows(T) : 4;
+    const dim3 grid((T + per - 1) / per), block(64 * per);
     if (H <= 512) hipLaunchKernelGGL((codec_rmsnorm_kernel<2, false>), grid, block, 0, (hipStream_t)stream, x, ldx, w, eps, (uint16_t*)out, T, H, CodecAdd{});
     else if (H <= 1024) hipLaunchKernelGGL((codec_rmsnorm_kernel<4, false>), grid, block, 0, (hipStream_t)stream, x, ldx, w, eps, (uint16_t*)out, T, H, CodecAdd{});
     else hipLaunchKernelGGL(codec_rmsnorm_wide_kernel, grid, block, 0, (hipStream_t)stream, x, ldx, w, eps, (uint16_t*)out, T, H);
@@ -145,7 +150,8 @@ extern "C" int omni_codec_rmsnorm(const float* x, int ldx, const float* w, float
 extern "C" int omni_codec_add_rmsnorm(float* x, int ldx, const float* y, int slabs, int64_t slab_stride, const float* scale, const float* w, float eps, void* out, int T, int H, void* stream) {
     OMNI_CHECK_ARG(x && y && scale && w && out && T > 0 && H > 0 && H % 4 == 0 && H <= 1024 && ldx >= H && ldx % 4 == 0 && slabs >= 1 && slabs <= 4 &&
                    (slabs == 1 || slab_stride >= (int64_t)T * H) && slab_stride % 4 == 0, "omni_codec_add_rmsnorm: T=%d H=%d (<= 1024) ldx=%d slabs=%d (<= 4)", T, H, ldx, slabs);
-    const dim3 grid((T + 3) / 4), block(256);
+    const int per = norm_rows(T);
+    const dim3 grid((T + per - 1) / per), block(64 * per);
     const CodecAdd add{x, y, scale, slabs, slab_stride};
     if (H <= 512) hipLaunchKernelGGL((codec_rmsnorm_kernel<2, true>), grid, block, 0, (hipStream_t)stream, x, ldx, w, eps, (uint16_t*)out, T, H, add);
     else hipLaunchKernelGGL((codec_rmsnorm_kernel<4, true>), grid, block, 0, (hipStream_t)stream, x, ldx, w, eps, (uint16_t*)out, T, H, add);
@@ -332,10 +338,59 @@ __global__ __launch_bounds__(256) void codec_dwconv_ln_kernel(const float* __res
     }
 }
 
+// Seven taps, channels in pieces of 16 bytes: everything a thread needs -- its four channels of seven rows, 28 weights, bias, gain and offset -- is asked for at once
+// (a channel and a tap after the other, a wait each: 11.8 us for 100 frames of 1024, so 4.7).  The same sums per channel.
+__global__ __launch_bounds__(256) void codec_dwconv7_ln_kernel(const float* __restrict__ x, int ldx, const float* __restrict__ w, const float* __restrict__ b,
+                                                               const float* __restrict__ ln_w, const float* __restrict__ ln_b, float eps, uint16_t* __restrict__ out, int T, int C) {
+    constexpr int TAPS = 7;
+    __shared__ float red[2][4];
+    const int t = blockIdx.x, tid = threadIdx.x, lane = tid & 63, wv = tid >> 6, c = min(tid * 4, C - 4);
+    const bool mine = tid * 4 < C;
+    f32x4 xv[TAPS], wq[TAPS];
+#pragma unroll
+    for (int j = 0; j < TAPS; ++j) xv[j] = *reinterpret_cast<const f32x4*>(x + (size_t)max(t - (TAPS - 1) + j, 0) * ldx + c);
+#pragma unroll
+    for (int j = 0; j < TAPS; ++j) wq[j] = *reinterpret_cast<const f32x4*>(w + (size_t)c * TAPS + 4 * j);      // float k of the 28: channel c + k / 7, tap k % 7
+    f32x4 y = *reinterpret_cast<const f32x4*>(b + c);
+    const f32x4 gw = *reinterpret_cast<const f32x4*>(ln_w + c), gb = *reinterpret_cast<const f32x4*>(ln_b + c);
+#pragma unroll
+    for (int j = 0; j < TAPS; ++j)
+        if (t - (TAPS - 1) + j >= 0)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) y[e] += wq[(e * TAPS + j) >> 2][(e * TAPS + j) & 3] * xv[j][e];
+    float sum = mine ? (y[0] + y[1]) + (y[2] + y[3]) : 0.f;
+    sum = wave_sum(sum);
+    if (lane == 0) red[0][wv] = sum;
+    __syncthreads();
+    const float mean = (red[0][0] + red[0][1] + red[0][2] + red[0][3]) / (float)C;
+    float var = 0.f;
+    if (mine)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) var += (y[e] - mean) * (y[e] - mean);
+    var = wave_sum(var);
+    if (lane == 0) red[1][wv] = var;
+    __syncthreads();
+    const float rstd = rsqrtf((red[1][0] + red[1][1] + red[1][2] + red[1][3]) / (float)C + eps);
+    if (!mine) return;
+    float o[4];
+#pragma unroll
+    for (int e = 0; e < 4; ++e) o[e] = (y[e] - mean) * rstd * gw[e] + gb[e];
+    *reinterpret_cast<uint2*>(out + (size_t)t * C + c) = make_uint2(pack_bf2(o[0], o[1]), pack_bf2(o[2], o[3]));
+}
+
+static bool aligned16(std::initializer_list<const void*> ps) {
+    for (const void* p : ps)
+        if ((uintptr_t)p & 15) return false;
+    return true;
+}
+
 extern "C" int omni_codec_dwconv_ln(const float* x, int ldx, const float* w, const float* b, const float* ln_w, const float* ln_b, float eps,
                                     void* out, int T, int C, int taps, void* stream) {
     OMNI_CHECK_ARG(x && w && b && ln_w && ln_b && out && T > 0 && C > 0 && C <= 1024 && taps > 0 && ldx >= C, "omni_codec_dwconv_ln: T=%d C=%d (<= 1024)", T, C);
-    hipLaunchKernelGGL(codec_dwconv_ln_kernel, dim3(T), dim3(256), 0, (hipStream_t)stream, x, ldx, w, b, ln_w, ln_b, eps, (uint16_t*)out, T, C, taps);
+    if (taps == 7 && C % 4 == 0 && ldx % 4 == 0 && aligned16({x, w, b, ln_w, ln_b}) && (uintptr_t)out % 8 == 0)
+        hipLaunchKernelGGL(codec_dwconv7_ln_kernel, dim3(T), dim3(256), 0, (hipStream_t)stream, x, ldx, w, b, ln_w, ln_b, eps, (uint16_t*)out, T, C);
+    else
+        hipLaunchKernelGGL(codec_dwconv_ln_kernel, dim3(T), dim3(256), 0, (hipStream_t)stream, x, ldx, w, b, ln_w, ln_b, eps, (uint16_t*)out, T, C, taps);
     OMNI_CHECK_LAUNCH("omni_codec_dwconv_ln");
     return OMNI_OK;
 }
@@ -384,6 +439,72 @@ __global__ __launch_bounds__(OC_ROWS) void codec_out_conv_kernel(const uint16_t*
     wav[t] = fminf(fmaxf(acc, -1.0f), 1.0f);
 }
 
+// Up to eight taps, rows of whole 32-channel steps: every row times every tap on the matrix cores, the fp32 weights as three bf16 terms whose sum they are (16 columns: the
+// taps' first terms | their second; 16 more for the third), then a sample adds up `taps` numbers out of LDS.  A lane's operand is 16 bytes of a row: rows are read once, in place,
+// and nothing waits for weights 32 at a time (21.1 us of the decode of 50 frames, 7.2 so).  Closer than a chain of 672 fp32 additions.  A sample
+// that is no finite number is added up as in the kernel above: a term of an infinite weight or row is no number here.
+#define OM_ROWS 256
+template <int KS>
+__global__ __launch_bounds__(256) void codec_out_mfma_kernel(const uint16_t* __restrict__ x, const float* __restrict__ w, float bias, float* __restrict__ wav, int T, int taps) {
+    constexpr int C = 32 * KS, TILES = OM_ROWS / 64;
+    __shared__ float part[OM_ROWS][9];
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, c = lane & 15, q = lane >> 4;
+    const int outs = OM_ROWS - (taps - 1), t0 = blockIdx.x * outs, r0 = t0 - (taps - 1);
+    u32x4 X[TILES][KS];
+#pragma unroll
+    for (int i = 0; i < TILES; ++i) {
+        const int r = r0 + (wave * TILES + i) * 16 + c;
+#pragma unroll
+        for (int k = 0; k < KS; ++k) {
+            X[i][k] = *reinterpret_cast<const u32x4*>(x + (size_t)min(max(r, 0), T - 1) * C + 32 * k + 8 * q);
+            if (r < 0) X[i][k] = u32x4{0, 0, 0, 0};
+        }
+    }
+    u32x4 W0[KS], W1[KS];
+    const int tap = c & 7;
+#pragma unroll
+    for (int k = 0; k < KS; ++k) {
+        const float* wp = w + (size_t)min(tap, taps - 1) * C + 32 * k + 8 * q;
+        const f32x4 a = *reinterpret_cast<const f32x4*>(wp), b = *reinterpret_cast<const f32x4*>(wp + 4);
+        const float v[8] = {a[0], a[1], a[2], a[3], b[0], b[1], b[2], b[3]};
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            const float w0 = tap < taps ? v[2 * e] : 0.f, w1 = tap < taps ? v[2 * e + 1] : 0.f;
+            const uint32_t hi = pack_bf2(w0, w1);
+            const float m0 = w0 - bf_lo(hi), m1 = w1 - bf_hi(hi);
+            const uint32_t mid = pack_bf2(m0, m1);
+            W0[k][e] = c < 8 ? hi : mid;
+            W1[k][e] = c < 8 ? pack_bf2(m0 - bf_lo(mid), m1 - bf_hi(mid)) : 0u;
+        }
+    }
+    auto mul = [](u32x4 a, u32x4 b, f32x4 d) { return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, a), __builtin_bit_cast(bf16x8, b), d, 0, 0, 0); };
+#pragma unroll
+    for (int i = 0; i < TILES; ++i) {
+        f32x4 d0 = {0.f, 0.f, 0.f, 0.f}, d1 = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int k = 0; k < KS; ++k) {
+            d0 = mul(X[i][k], W0[k], d0);
+            d1 = mul(X[i][k], W1[k], d1);
+        }
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            const float mid = __shfl_xor(d0[e], 8);
+            if (c < 8) part[(wave * TILES + i) * 16 + 4 * q + e][c] = (d1[e] + mid) + d0[e];
+        }
+    }
+    __syncthreads();
+    const int t = t0 + threadIdx.x;
+    if ((int)threadIdx.x >= outs || t >= T) return;
+    float acc = bias;
+    for (int j = 0; j < taps; ++j) acc += part[threadIdx.x + j][j];
+    if (!(fabsf(acc) < INFINITY)) {
+        acc = bias;
+        for (int j = 0; j < taps; ++j)
+            if (t - (taps - 1) + j >= 0) acc = oc_row(x + (size_t)(t - (taps - 1) + j) * C, w + j * C, C, acc);
+    }
+    wav[t] = fminf(fmaxf(acc, -1.0f), 1.0f);
+}
+
 // rows too wide for LDS: straight from memory, the weights in LDS
 __global__ __launch_bounds__(256) void codec_out_conv_wide_kernel(const uint16_t* __restrict__ x, const float* __restrict__ w, float bias,
                                                                   float* __restrict__ wav, int T, int C, int taps) {
@@ -401,7 +522,14 @@ __global__ __launch_bounds__(256) void codec_out_conv_wide_kernel(const uint16_t
 extern "C" int omni_codec_out_conv(const void* x, const float* w, float bias, float* wav, int T, int C, int taps, void* stream) {
     OMNI_CHECK_ARG(x && w && wav && T > 0 && C > 0 && C % 8 == 0 && taps > 0 && taps * C * 4 <= 64 * 1024, "omni_codec_out_conv: T=%d C=%d taps=%d", T, C, taps);
     const int64_t rows = (int64_t)(OC_ROWS + taps - 1) * oc_pitch(C);
-    if (rows <= 64 * 1024)
+    if (taps <= 8 && C % 32 == 0 && C <= 256 && aligned16({x, w})) {
+        const dim3 grid((T + OM_ROWS - taps) / (OM_ROWS - taps + 1)), block(256);
+        switch (C / 32) {
+#define OM(K) case K: hipLaunchKernelGGL(codec_out_mfma_kernel<K>, grid, block, 0, (hipStream_t)stream, (const uint16_t*)x, w, bias, wav, T, taps); break;
+            OM(1) OM(2) OM(3) OM(4) OM(5) OM(6) OM(7) OM(8)
+#undef OM
+        }
+    } else if (rows <= 64 * 1024)
         hipLaunchKernelGGL(codec_out_conv_kernel, dim3((T + OC_ROWS - 1) / OC_ROWS), dim3(OC_ROWS), (size_t)rows, (hipStream_t)stream,
                            (const uint16_t*)x, w, bias, wav, T, C, taps);
     else

@@ -6,6 +6,7 @@
     wrapper around the real decoder and the stage's request parsing / context trimming.
 Tolerances: the product computes with bf16 GEMM operands and fp32 accumulation / residual streams; the reference computes fp32.
 Measured on the fixture: |wav - ref| mean 1.9e-3, max 8e-3 at a signal of mean |wav| 0.15 (1.2 %); asserted at 2.5x that."""
+import math
 import os
 
 import numpy as np
@@ -294,6 +295,76 @@ def test_last_conv(C, T, taps):
     mag = 0.0625 + sum((xp[j:j + T] * w[j].double()).abs().sum(-1) for j in range(taps))
     assert bool((wav[T:] == 7.0).all())
     assert bool(((wav[:T].cpu().double() - ref.clamp(-1, 1)).abs() <= mag * (taps * C * 2.0 ** -24)).all())
+
+
+@pytest.mark.parametrize("C,T,taps", [(32, 1, 8), (32, 249, 8), (64, 251, 7), (96, 250, 7), (128, 1000, 2), (160, 255, 1), (192, 256, 3), (224, 17, 7), (256, 499, 8)])
+def test_last_conv_on_the_matrix_cores(C, T, taps):
+    """Every width that the kernel of matrix products takes, blocks of 256 - (taps - 1) samples and their edges; the bound of test_last_conv.  A row or a weight that is
+    no finite number reaches its own samples alone, as what the plain sum makes of it (an infinity times a weight is an infinity, not what its terms add up to)."""
+    from ht_vllm_omni_amd import _lib as L
+    g = torch.Generator().manual_seed(C + T)
+    x, w = torch.randn(T, C, generator=g).to(torch.bfloat16), torch.randn(taps, C, generator=g) * (0.3 / (taps * C) ** 0.5)
+
+    def run(x, w):
+        wav, xd, wd = torch.full((T + 4,), 7.0, device="cuda"), x.cuda(), w.cuda()
+        L.check(L.load().omni_codec_out_conv(xd.data_ptr(), wd.data_ptr(), 0.0625, wav.data_ptr(), T, C, taps, L.current_stream()), "omni_codec_out_conv")
+        assert bool((wav[T:] == 7.0).all())
+        return wav[:T].cpu()
+
+    def sums(x, w, absolute=False):
+        out = torch.full((T,), 0.0625, dtype=torch.float64)
+        for j in range(taps):                              # (rows in front of the first are none, not zeros)
+            lo = taps - 1 - j
+            y = x[:max(T - lo, 0)].double() * w[j].double()
+            out[lo:] += (y.abs() if absolute else y).sum(-1)
+        return out
+    plain = run(x, w)
+    assert bool(((plain.double() - sums(x, w).clamp(-1, 1)).abs() <= sums(x, w, True) * (taps * C * 2.0 ** -24)).all())
+    for row, bad in ((0, math.inf), (T // 2, -math.inf), (T - 1, math.nan)):
+        xb = x.clone()
+        xb[row, C - 1] = bad
+        ref, got = sums(xb, w), run(xb, w)
+        touched = ~torch.isfinite(ref)
+        assert torch.equal(got[~touched], plain[~touched])
+        want = torch.where(torch.isnan(ref), -torch.ones_like(ref), ref.clamp(-1, 1)).float()      # a NaN: max(NaN, -1)
+        assert torch.equal(got[touched], want[touched])
+    wb = w.clone()
+    wb[0, 0] = math.inf
+    ref, got = sums(x, wb), run(x, wb)
+    keep = torch.isfinite(ref)
+    assert torch.equal(got[~keep], torch.where(torch.isnan(ref), -torch.ones_like(ref), ref.clamp(-1, 1)).float()[~keep])
+
+
+@pytest.mark.parametrize("C,T,ldx,taps", [(4, 1, 4, 7), (252, 9, 256, 7), (1024, 3, 1024, 7), (1020, 40, 1028, 7), (256, 20, 257, 7), (130, 20, 130, 7), (64, 30, 64, 5)])
+def test_depthwise_conv_and_layer_norm(C, T, ldx, taps):
+    """Seven taps in pieces of four channels, and the general kernel where channels or pitch are no such pieces or the taps are others; frames before the first whole window.  Bound:
+    one rounding to bf16, and fp32 sums whose errors a small variance enlarges: 2^-20 of the largest gain."""
+    from ht_vllm_omni_amd import _lib as L
+    g = torch.Generator().manual_seed(C + T)
+    x, w, b = torch.randn(T, ldx, generator=g), torch.randn(C, taps, generator=g) * 0.4, torch.randn(C, generator=g) * 0.1
+    lw, lb = 1 + 0.1 * torch.randn(C, generator=g), 0.1 * torch.randn(C, generator=g)
+    out = torch.full((T + 1, C), 7.0, dtype=torch.bfloat16, device="cuda")
+    d = [t.cuda() for t in (x, w, b, lw, lb)]
+    L.check(L.load().omni_codec_dwconv_ln(d[0].data_ptr(), ldx, *(t.data_ptr() for t in d[1:]), 1e-6, out.data_ptr(), T, C, taps, L.current_stream()), "omni_codec_dwconv_ln")
+    xp = torch.cat([torch.zeros(taps - 1, C), x[:, :C]]).double()
+    y = b.double() + sum(xp[j:j + T] * w[:, j].double() for j in range(taps))
+    ref = torch.nn.functional.layer_norm(y, (C,), lw.double(), lb.double(), 1e-6)
+    assert bool(((out[:T].cpu().double() - ref).abs() <= ref.abs() * 2.0 ** -8 + 2.0 ** -18).all()) and bool((out[T:] == 7.0).all())
+
+
+@pytest.mark.parametrize("T", [1024, 1025, 1030])
+def test_norm_of_many_rows(T):
+    """A wave to a workgroup up to 1024 rows, four behind: the same bits."""
+    from ht_vllm_omni_amd import _lib as L
+    g, H = torch.Generator().manual_seed(T), 260
+    x, w = torch.randn(T, H, generator=g).cuda(), torch.randn(H, generator=g).cuda()
+    outs = []
+    for lo, n in ((0, T), (T - 24, 24)):
+        out = torch.full((n + 1, H), 7.0, dtype=torch.bfloat16, device="cuda")
+        L.check(L.load().omni_codec_rmsnorm(x[lo:].data_ptr(), H, w.data_ptr(), 1e-5, out.data_ptr(), n, H, L.current_stream()), "omni_codec_rmsnorm")
+        assert bool((out[n:] == 7.0).all())
+        outs.append(out[:n])
+    assert torch.equal(outs[0][T - 24:], outs[1])
 
 
 def test_window_attention_longer_than_the_window():

@@ -297,26 +297,51 @@ extern "C" int omni_codec_window_attn(const void* qkv, int ld, void* out, int ld
 
 // ---------------------------------------------------------------- ConvNeXt front: depthwise causal conv + LayerNorm over channels
 // y[t, c] = b[c] + sum_j w[c][j] x[t - (taps - 1) + j][c] (rows < 0 are zero);  out = bf16(LN(y) * g + beta).  One workgroup per frame.
+// Seven taps: the channels of seven rows, their weights, gains and offsets are asked for at once (a channel and a tap after the other, a wait each: 11.8 us
+// for 100 frames of 1024, so 3.9); the same sums.  TAPS 0: any number.
+template <int TAPS>
 __global__ __launch_bounds__(256) void codec_dwconv_ln_kernel(const float* __restrict__ x, int ldx, const float* __restrict__ w,
                                                               const float* __restrict__ b, const float* __restrict__ ln_w,
                                                               const float* __restrict__ ln_b, float eps, uint16_t* __restrict__ out,
                                                               int T, int C, int taps) {
     __shared__ float red[2][4];
     const int t = blockIdx.x, tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
-    float y[4];                                           // C <= 1024: channel tid + 256 i
+    float y[4], g[4], o[4];                               // C <= 1024: channel tid + 256 i
     float sum = 0.f;
+    if constexpr (TAPS > 0) {
+        float xv[4][TAPS], wq[4][TAPS];
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-        const int c = tid + 256 * i;
-        y[i] = 0.f;
-        if (c < C) {
-            float a = b[c];
-            for (int j = 0; j < taps; ++j) {
-                const int r = t - (taps - 1) + j;
-                if (r >= 0) a += w[c * taps + j] * x[(size_t)r * ldx + c];
+        for (int i = 0; i < 4; ++i) {
+            const int c = min(tid + 256 * i, C - 1);
+#pragma unroll
+            for (int j = 0; j < TAPS; ++j) {
+                xv[i][j] = x[(size_t)max(t - (TAPS - 1) + j, 0) * ldx + c];
+                wq[i][j] = w[c * TAPS + j];
             }
-            y[i] = a;
-            sum += a;
+            y[i] = b[c]; g[i] = ln_w[c]; o[i] = ln_b[c];
+        }
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+#pragma unroll
+            for (int j = 0; j < TAPS; ++j)
+                if (t - (TAPS - 1) + j >= 0) y[i] += wq[i][j] * xv[i][j];
+            if (tid + 256 * i >= C) y[i] = 0.f;
+            else sum += y[i];
+        }
+    } else {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const int c = tid + 256 * i;
+            y[i] = g[i] = o[i] = 0.f;
+            if (c < C) {
+                float a = b[c];
+                for (int j = 0; j < taps; ++j) {
+                    const int r = t - (taps - 1) + j;
+                    if (r >= 0) a += w[c * taps + j] * x[(size_t)r * ldx + c];
+                }
+                y[i] = a; g[i] = ln_w[c]; o[i] = ln_b[c];
+                sum += a;
+            }
         }
     }
     sum = wave_sum(sum);
@@ -334,48 +359,8 @@ __global__ __launch_bounds__(256) void codec_dwconv_ln_kernel(const float* __res
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
         const int c = tid + 256 * i;
-        if (c < C) out[(size_t)t * C + c] = f2bf((y[i] - mean) * rstd * ln_w[c] + ln_b[c]);
+        if (c < C) out[(size_t)t * C + c] = f2bf((y[i] - mean) * rstd * g[i] + o[i]);
     }
-}
-
-// Seven taps, channels in pieces of 16 bytes: everything a thread needs -- its four channels of seven rows, 28 weights, bias, gain and offset -- is asked for at once
-// (a channel and a tap after the other, a wait each: 11.8 us for 100 frames of 1024, so 4.7).  The same sums per channel.
-__global__ __launch_bounds__(256) void codec_dwconv7_ln_kernel(const float* __restrict__ x, int ldx, const float* __restrict__ w, const float* __restrict__ b,
-                                                               const float* __restrict__ ln_w, const float* __restrict__ ln_b, float eps, uint16_t* __restrict__ out, int T, int C) {
-    constexpr int TAPS = 7;
-    __shared__ float red[2][4];
-    const int t = blockIdx.x, tid = threadIdx.x, lane = tid & 63, wv = tid >> 6, c = min(tid * 4, C - 4);
-    const bool mine = tid * 4 < C;
-    f32x4 xv[TAPS], wq[TAPS];
-#pragma unroll
-    for (int j = 0; j < TAPS; ++j) xv[j] = *reinterpret_cast<const f32x4*>(x + (size_t)max(t - (TAPS - 1) + j, 0) * ldx + c);
-#pragma unroll
-    for (int j = 0; j < TAPS; ++j) wq[j] = *reinterpret_cast<const f32x4*>(w + (size_t)c * TAPS + 4 * j);      // float k of the 28: channel c + k / 7, tap k % 7
-    f32x4 y = *reinterpret_cast<const f32x4*>(b + c);
-    const f32x4 gw = *reinterpret_cast<const f32x4*>(ln_w + c), gb = *reinterpret_cast<const f32x4*>(ln_b + c);
-#pragma unroll
-    for (int j = 0; j < TAPS; ++j)
-        if (t - (TAPS - 1) + j >= 0)
-#pragma unroll
-            for (int e = 0; e < 4; ++e) y[e] += wq[(e * TAPS + j) >> 2][(e * TAPS + j) & 3] * xv[j][e];
-    float sum = mine ? (y[0] + y[1]) + (y[2] + y[3]) : 0.f;
-    sum = wave_sum(sum);
-    if (lane == 0) red[0][wv] = sum;
-    __syncthreads();
-    const float mean = (red[0][0] + red[0][1] + red[0][2] + red[0][3]) / (float)C;
-    float var = 0.f;
-    if (mine)
-#pragma unroll
-        for (int e = 0; e < 4; ++e) var += (y[e] - mean) * (y[e] - mean);
-    var = wave_sum(var);
-    if (lane == 0) red[1][wv] = var;
-    __syncthreads();
-    const float rstd = rsqrtf((red[1][0] + red[1][1] + red[1][2] + red[1][3]) / (float)C + eps);
-    if (!mine) return;
-    float o[4];
-#pragma unroll
-    for (int e = 0; e < 4; ++e) o[e] = (y[e] - mean) * rstd * gw[e] + gb[e];
-    *reinterpret_cast<uint2*>(out + (size_t)t * C + c) = make_uint2(pack_bf2(o[0], o[1]), pack_bf2(o[2], o[3]));
 }
 
 static bool aligned16(std::initializer_list<const void*> ps) {
@@ -387,10 +372,8 @@ static bool aligned16(std::initializer_list<const void*> ps) {
 extern "C" int omni_codec_dwconv_ln(const float* x, int ldx, const float* w, const float* b, const float* ln_w, const float* ln_b, float eps,
                                     void* out, int T, int C, int taps, void* stream) {
     OMNI_CHECK_ARG(x && w && b && ln_w && ln_b && out && T > 0 && C > 0 && C <= 1024 && taps > 0 && ldx >= C, "omni_codec_dwconv_ln: T=%d C=%d (<= 1024)", T, C);
-    if (taps == 7 && C % 4 == 0 && ldx % 4 == 0 && aligned16({x, w, b, ln_w, ln_b}) && (uintptr_t)out % 8 == 0)
-        hipLaunchKernelGGL(codec_dwconv7_ln_kernel, dim3(T), dim3(256), 0, (hipStream_t)stream, x, ldx, w, b, ln_w, ln_b, eps, (uint16_t*)out, T, C);
-    else
-        hipLaunchKernelGGL(codec_dwconv_ln_kernel, dim3(T), dim3(256), 0, (hipStream_t)stream, x, ldx, w, b, ln_w, ln_b, eps, (uint16_t*)out, T, C, taps);
+    if (taps == 7) hipLaunchKernelGGL(codec_dwconv_ln_kernel<7>, dim3(T), dim3(256), 0, (hipStream_t)stream, x, ldx, w, b, ln_w, ln_b, eps, (uint16_t*)out, T, C, taps);
+    else hipLaunchKernelGGL(codec_dwconv_ln_kernel<0>, dim3(T), dim3(256), 0, (hipStream_t)stream, x, ldx, w, b, ln_w, ln_b, eps, (uint16_t*)out, T, C, taps);
     OMNI_CHECK_LAUNCH("omni_codec_dwconv_ln");
     return OMNI_OK;
 }

@@ -337,7 +337,7 @@ def test_last_conv_on_the_matrix_cores(C, T, taps):
 
 @pytest.mark.parametrize("C,T,ldx,taps", [(4, 1, 4, 7), (252, 9, 256, 7), (1024, 3, 1024, 7), (1020, 40, 1028, 7), (256, 20, 257, 7), (130, 20, 130, 7), (64, 30, 64, 5)])
 def test_depthwise_conv_and_layer_norm(C, T, ldx, taps):
-    """Seven taps in pieces of four channels, and the general kernel where channels or pitch are no such pieces or the taps are others; frames before the first whole window.  Bound:
+    """Seven taps, and the general kernel of other counts; channels that end inside a round of threads, frames before the first whole window.  Bound:
     one rounding to bf16, and fp32 sums whose errors a small variance enlarges: 2^-20 of the largest gain."""
     from ht_vllm_omni_amd import _lib as L
     g = torch.Generator().manual_seed(C + T)

@@ -554,7 +554,9 @@ class MI355XCode2Wav:
             frames = n // q
             codes = r.reshape(q, frames)
             if self.validate_codes:
-                lo, hi = int(codes.min()), int(codes.max())
+                ends = torch.empty(2, dtype=codes.dtype, device=codes.device)      # (both in one launch, and one wait for them)
+                torch.aminmax(codes, out=(ends[0], ends[1]))
+                lo, hi = ends.tolist()
                 if lo < 0 or hi >= self.decoder.cfg.codebook_size:
                     raise ValueError(f"Code2Wav request {i}: codec ids in [{lo}, {hi}] outside [0, {self.decoder.cfg.codebook_size})")
             wav = self.decoder.chunked_decode(codes.unsqueeze(0)).reshape(-1)

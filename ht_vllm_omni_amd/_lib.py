@@ -254,6 +254,7 @@ DECODER_SIGNATURES = {
     "omni_gemm_stream_joins": (i32, [i32, i32, i32, i32, i32]),
     "omni_gemm_stream_latents": (i32, [C.POINTER(LatentWrite), vp, vp, i32, vp]),
     "omni_latent_attn_values": (i32, [C.POINTER(LatentAttn), vp, vp, i32, i32, vp]),
+    "omni_latent_attn_products": (i32, [C.POINTER(LatentAttn), vp, vp, i32, i32, vp]),
     "omni_gemm_f32_rows": (i32, [vp, i32, vp, vp, i32, i32, i32, i32, C.POINTER(RowTable), vp]),
     "omni_qkv_write_run": (i32, [C.POINTER(QkvWrite), vp]),
     "omni_gated_norm_run": (i32, [C.POINTER(GatedNorm), vp]),

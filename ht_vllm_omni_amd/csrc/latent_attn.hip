@@ -311,6 +311,92 @@ __global__ __launch_bounds__(256) void latent_values_kernel(const float* __restr
     *reinterpret_cast<uint2*>(out + (frag ? frag_off(c, col, heads * n) : (size_t)c * heads * n + col)) = make_uint2(pack_bf2(v[0], v[1]), pack_bf2(v[2], v[3]));
 }
 
+// The same for more rows: a workgroup merges `rows` rows of one head (128 threads each, eight records in flight) and multiplies them by all of the head's
+// columns, its waves taking K's steps in turn as head_gemm's do: the same sums.  A merge of its own and the product behind it are two launches and a round trip of the rows: with
+// the attention in front, us a layer, two launches / one, 16 heads of 128 by latents of 512 (256): 64 rows of up to 2048 keys 41.4 / 38.8 (27.1 / 24.4), 64 of up to 352 21.2 / 19.0
+// (15.1 / 13.9), 16 of up to 2048 24.2 / 21.9 (18.2 / 16.5), 3 of up to 352 14.3 / 12.8 (11.8 / 10.3), 20 of 40 keys, nothing to merge, 12.0 / 11.8 (9.3 / 9.1); 64 heads, 64 rows 99 / 92.5.
+// By four waves, two rows at a time and all columns to each, 39.3 of the first and 12.4 of the last but one.  What bounds it now: the records, 2 KB a split and row out of the last-level cache, and the head's weights, which stay in one XCD's L2 (heads are the grid's x).
+template <int NT>                                     // column tiles of a wave; two groups of four waves
+__global__ __launch_bounds__(512) void latent_rows_values_kernel(const float* __restrict__ partial, const float* __restrict__ gate, const uint16_t* __restrict__ merged,
+                                                                 const int32_t* __restrict__ positions, const uint16_t* __restrict__ w, uint16_t* __restrict__ out, int T, int heads,
+                                                                 int max_split, int per, int rp, int n, int frag, int rows) {
+    constexpr int P = 4, WAVES = 4, S = 8;
+    extern __shared__ __attribute__((aligned(16))) uint16_t xs[];      // [rows][rp + 8]
+    __shared__ f32x4 part[2 * WAVES][NT][64];
+    const int lane = threadIdx.x & 63, id = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), wave = id & 3, group = id >> 2, c = lane & 15, q = lane >> 4;
+    const int h = blockIdx.x, t0 = blockIdx.y * rows, n0 = (blockIdx.z * 2 + group) * NT, ntiles = n >> 4, nsteps = rp >> 5, mine = nsteps > wave ? (nsteps - wave + WAVES - 1) / WAVES : 0;
+    u32x4 W[P][NT];
+    auto load = [&](int d, int s) {                       // (past the last step or tile: that one again, not used)
+#pragma unroll
+        for (int j = 0; j < NT; ++j) W[d][j] = ld16(w + (((size_t)h * ntiles + min(n0 + j, ntiles - 1)) * nsteps + min(wave + s * WAVES, nsteps - 1)) * 512 + lane * 8);
+    };
+#pragma unroll
+    for (int d = 0; d < P; ++d) load(d, d);
+    const int k = (threadIdx.x & 127) * 4, kc = min(k, rp - 4);
+    for (int r0 = 0; r0 < rows; r0 += 8) {                // rows r0 + (id >> 1) and that + 4
+        float2 ml[2];
+        uint2 whole[2];
+        int ns[2];
+        const float* base[2];
+        f32x4 v[2][S];
+#pragma unroll
+        for (int u = 0; u < 2; ++u) {
+            const int t = min(t0 + min(r0 + 4 * u + (id >> 1), rows - 1), T - 1);
+            const size_t rh = (size_t)t * heads + h;
+            ns[u] = __builtin_amdgcn_readfirstlane(la_row_splits((positions[t] + 16) / 16, max_split, per));
+            base[u] = partial + rh * max_split * (rp + 4);
+            whole[u] = *reinterpret_cast<const uint2*>(merged + rh * rp + kc);      // (one split: the decode kernel wrote the row)
+            ml[u] = lane < ns[u] && ns[u] > 1 ? *reinterpret_cast<const float2*>(base[u] + (size_t)lane * (rp + 4)) : make_float2(LA_SENT, 0.f);
+            if (ns[u] > 1)
+#pragma unroll
+                for (int s = 0; s < S; ++s) v[u][s] = *reinterpret_cast<const f32x4*>(base[u] + (size_t)min(s, ns[u] - 1) * (rp + 4) + 4 + kc);
+        }
+#pragma unroll
+        for (int u = 0; u < 2; ++u) {
+            const int r = r0 + 4 * u + (id >> 1), t = min(t0 + r, T - 1);
+            if (r >= rows) continue;
+            uint2 o = whole[u];
+            if (ns[u] > 1) {
+                const float M = wave_max(ml[u].x), e = lane < ns[u] ? exp2f(ml[u].x - M) : 0.f, L = wave_sum(ml[u].y * e);
+                f32x4 m = (f32x4){0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+                for (int s = 0; s < S; ++s)
+                    if (s < ns[u]) m += v[u][s] * __int_as_float(__builtin_amdgcn_readlane(__float_as_int(e), s));
+                for (int s = S; s < ns[u]; ++s) m += *reinterpret_cast<const f32x4*>(base[u] + (size_t)s * (rp + 4) + 4 + kc) * __int_as_float(__builtin_amdgcn_readlane(__float_as_int(e), s));
+                m *= (L > 0.f ? 1.0f / L : 0.f) * (gate ? gate[(size_t)t * heads + h] : 1.0f);
+                o = make_uint2(pack_bf2(m[0], m[1]), pack_bf2(m[2], m[3]));
+            }
+            if (k < rp) *reinterpret_cast<uint2*>(xs + (size_t)r * (rp + 8) + k) = o;
+        }
+    }
+    __syncthreads();
+    const uint16_t* xp = xs + (size_t)min(c, rows - 1) * (rp + 8) + wave * 32 + 8 * q;
+    f32x4 acc[NT];
+#pragma unroll
+    for (int j = 0; j < NT; ++j) acc[j] = (f32x4){0.f, 0.f, 0.f, 0.f};
+    for (int s = 0; s < mine; s += P)
+#pragma unroll
+        for (int d = 0; d < P; ++d) {
+            if (s + d >= mine) break;
+            const u32x4 X = *reinterpret_cast<const u32x4*>(xp + (size_t)(s + d) * (WAVES * 32));
+#pragma unroll
+            for (int j = 0; j < NT; ++j) acc[j] = mfma16(W[d][j], X, acc[j]);
+            if (s + d + P < mine) load(d, s + d + P);
+        }
+#pragma unroll
+    for (int j = 0; j < NT; ++j) part[id][j][lane] = acc[j];
+    __syncthreads();
+    const int t = t0 + c;
+    if (c >= rows || t >= T) return;
+    for (int j = wave; j < min(NT, ntiles - n0); j += WAVES) {
+        f32x4 v = part[group * WAVES][j][lane];
+#pragma unroll
+        for (int u = 1; u < WAVES; ++u) v += part[group * WAVES + u][j][lane];
+        const int col = h * n + (n0 + j) * 16 + 4 * q;
+        *reinterpret_cast<uint2*>(out + (frag ? frag_off(t, col, heads * n) : (size_t)t * heads * n + col)) = make_uint2(pack_bf2(v[0], v[1]), pack_bf2(v[2], v[3]));
+    }
+}
+
 template <int RS, int PW>
 __global__ __launch_bounds__(64 * PW, 2) void latent_prefill_kernel(const LatentArgs a) {
     using G = LatentGeom<RS>;
@@ -506,7 +592,9 @@ static int la_lds(K kernel, int bytes) {
     return OMNI_OK;
 }
 
-struct LatentValues { const uint16_t* w; uint16_t* out; int n, frag; };      // the per-head product behind decode tokens; w NULL: none
+// the per-head product behind decode tokens; w NULL: none.  rows: of a workgroup of latent_rows_values_kernel; 0: latent_values_kernel
+struct LatentValues { const uint16_t* w; uint16_t* out; int n, frag, rows; };
+#define LA_VALUE_TILES 8
 template <int RS>
 static int la_run(const omni_latent_attn& p, LatentArgs a, const LatentValues& then, hipStream_t st) {
     using G = LatentGeom<RS>;
@@ -521,7 +609,12 @@ static int la_run(const omni_latent_attn& p, LatentArgs a, const LatentValues& t
         a.per = p.n_decode * ((p.heads + 15) / 16) <= 8 ? 4 : 8;
         hipLaunchKernelGGL(latent_decode_kernel<RS>, dim3((p.heads + 15) / 16, p.n_decode, a.nsplit), dim3(64 * LA_DEC_WAVES), LDS, st, a);
         OMNI_CHECK_LAUNCH("omni_latent_attn(decode)");
-        if (then.w) {
+        if (then.w && then.rows) {
+            hipLaunchKernelGGL(latent_rows_values_kernel<LA_VALUE_TILES / 2>, dim3(p.heads, (p.n_decode + then.rows - 1) / then.rows, (then.n / 16 + LA_VALUE_TILES - 1) / LA_VALUE_TILES), dim3(512),
+                               then.rows * (p.rp + 8) * 2, st, (const float*)a.partial, a.gate, (const uint16_t*)a.out, a.positions, then.w, then.out, p.n_decode, p.heads, a.nsplit, a.per, p.rp,
+                               then.n, then.frag, then.rows);
+            OMNI_CHECK_LAUNCH("omni_latent_attn(values)");
+        } else if (then.w) {
             hipLaunchKernelGGL(latent_values_kernel, dim3(then.n / 16, p.heads), dim3(256), p.n_decode * p.rp * 2, st, (const float*)a.partial, a.gate, (const uint16_t*)a.out, a.positions,
                                then.w, then.out, p.n_decode, p.heads, a.nsplit, a.per, p.rp, then.n, then.frag);
             OMNI_CHECK_LAUNCH("omni_latent_attn(values)");
@@ -576,6 +669,27 @@ static int la_any(const omni_latent_attn* pp, const LatentValues& then, hipStrea
 
 extern "C" int omni_latent_attn_run(const omni_latent_attn* p, void* stream) { return la_any(p, LatentValues{}, (hipStream_t)stream); }
 
+// rows of a workgroup that merges and multiplies: as few as make one round of workgroups; 0: not even 16 do
+static int la_value_rows(int T, int heads, int n) {
+    const int64_t cols = (int64_t)heads * ((n / 16 + LA_VALUE_TILES - 1) / LA_VALUE_TILES);
+    for (int r = 1; r <= 16; r *= 2)
+        if (cols * ((T + r - 1) / r) <= 256) return r;
+    return 0;
+}
+
+extern "C" int omni_latent_attn_products(const omni_latent_attn* p, const void* w, void* out, int n, int frag, void* stream) {
+    OMNI_CHECK_ARG(p && w && out, "omni_latent_attn_products: null pointer");
+    OMNI_CHECK_ARG(p->T >= 1 && p->T == p->n_decode && p->n_tiles == 0 && p->elem == 0 && p->rp <= 512 && omni_latent_attn_mfma(p->rp), "omni_latent_attn_products: T=%d n_decode=%d rp=%d (decode tokens, bf16)",
+                   p->T, p->n_decode, p->rp);
+    OMNI_CHECK_ARG(p->heads > 0 && n > 0 && n % 16 == 0 && (!frag || p->heads * n % 32 == 0), "omni_latent_attn_products: n=%d (%% 16) frag=%d", n, frag);
+    const int rows = la_value_rows(p->T, p->heads, n);
+    if (!rows || !p->workspace || la_splits(p->T, p->heads, p->max_keys) == 1) {
+        const int rc = omni_latent_attn_run(p, stream);
+        return rc != OMNI_OK ? rc : omni_head_gemm(p->out, w, out, p->T, p->heads, n, p->rp, frag, stream);
+    }
+    return la_any(p, LatentValues{(const uint16_t*)w, (uint16_t*)out, n, frag, rows}, (hipStream_t)stream);
+}
+
 extern "C" int omni_latent_attn_values(const omni_latent_attn* p, const void* w, void* out, int n, int frag, void* stream) {
     OMNI_CHECK_ARG(p && w && out, "omni_latent_attn_values: null pointer");
     OMNI_CHECK_ARG(p->T >= 1 && p->T == p->n_decode && p->T <= OMNI_STREAM_LATENT_ROWS && p->n_tiles == 0 && p->elem == 0 && p->rp <= 512 && omni_latent_attn_mfma(p->rp),
@@ -587,5 +701,5 @@ extern "C" int omni_latent_attn_values(const omni_latent_attn* p, const void* w,
         const int rc = omni_latent_attn_run(p, stream);
         return rc != OMNI_OK ? rc : omni_head_gemm(p->out, w, out, p->T, p->heads, n, p->rp, frag, stream);
     }
-    return la_any(p, LatentValues{(const uint16_t*)w, (uint16_t*)out, n, frag}, (hipStream_t)stream);
+    return la_any(p, LatentValues{(const uint16_t*)w, (uint16_t*)out, n, frag, 0}, (hipStream_t)stream);
 }

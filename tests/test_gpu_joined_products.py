@@ -144,7 +144,7 @@ def test_latents(T, q_rank, kv_rank, heads, N, form):
     assert outs[0][0].abs().max() > 0
 
 
-def values_both_ways(lens, heads, rp, n, gated, split, frag):
+def values_both_ways(lens, heads, rp, n, gated, split, frag, fn="omni_latent_attn_values"):
     """The per-head product behind the attention of decode tokens, by two entries and by one."""
     g, T, bs = gen(sum(lens) + rp), len(lens), 16
     need = [(k + bs - 1) // bs for k in lens]
@@ -165,9 +165,9 @@ def values_both_ways(lens, heads, rp, n, gated, split, frag):
         if split:
             a.keep["ws"] = ws = torch.full((nb // 4,), float("nan"), device="cuda")
             a.workspace, a.workspace_bytes = ws.data_ptr(), nb
-        out = torch.full((16 if frag else T, heads * n), 7.0, device="cuda", dtype=BF)
+        out = torch.full(((T + 15) // 16 * 16 if frag else T, heads * n), 7.0, device="cuda", dtype=BF)
         if joined:
-            call("omni_latent_attn_values", C.byref(a), w, out, n, frag)
+            call(fn, C.byref(a), w, out, n, frag)
         else:
             call("omni_latent_attn_run", C.byref(a))
             call("omni_head_gemm", a.keep["out"], w, out, T, heads, n, rp, frag)
@@ -194,6 +194,17 @@ def test_values_of_more_heads_than_merge_for_themselves(lens, heads, rp, n):
     assert torch.isfinite(outs[0].float()).all() and torch.equal(*outs)
 
 
+@pytest.mark.parametrize("T", [1, 3, 4, 5, 16, 17, 33, 64])
+@pytest.mark.parametrize("heads,rp,n", [(16, 512, 128), (16, 256, 128), (20, 96, 48), (3, 448, 144), (8, 32, 16), (256, 64, 16), (300, 64, 16)])
+def test_products_of_merged_rows(T, heads, rp, n):
+    """Rows of one split beside rows of up to 16, workgroups whose last rows are past the batch, columns that fill no second group of tiles, more heads than one round
+    takes; K's steps in head_gemm's order where its waves split K too, else within the order of the sums (a rounding to bf16 beside it)."""
+    lens = [(1, 64, 65, 352, 900, 2100, 17)[(5 * t) % 7] + t for t in range(T)]
+    outs = values_both_ways(lens, heads, rp, n, True, True, int(heads * n % 32 == 0 and T % 2), "omni_latent_attn_products")
+    assert torch.isfinite(outs[0].float()).all()
+    assert torch.equal(*outs) if rp >= 256 else torch.allclose(outs[0].float(), outs[1].float(), rtol=2 ** -7, atol=1e-3)
+
+
 def test_what_is_refused():
     lib = L.load_decoder()
     t = torch.zeros(1 << 16, device="cuda")
@@ -205,4 +216,5 @@ def test_what_is_refused():
     assert lib.omni_gemm_stream_joined(C.byref(a), p, p, 40, 2, 1, 0.0, 0.0, None, 0, None) == -1
     assert lib.omni_gemm_stream_joined(C.byref(a), p, p, 32, 1, 1, 0.0, 0.0, None, 0, None) == -1
     assert lib.omni_gemm_stream_latents(C.byref(L.LatentWrite()), p, p, 32, None) == -1
+    assert lib.omni_latent_attn_products(C.byref(L.LatentAttn(T=3, n_decode=2, rp=512)), p, p, 16, 0, None) == lib.omni_latent_attn_products(C.byref(L.LatentAttn(T=3, n_decode=3, rp=544)), p, p, 16, 0, None) == -1
     assert lib.omni_latent_attn_values(C.byref(L.LatentAttn(T=3, n_decode=3)), p, p, 16, 0, None) == -1

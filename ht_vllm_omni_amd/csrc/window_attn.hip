@@ -174,13 +174,20 @@ __global__ __launch_bounds__(64) void window_merge_kernel(const WinArgs a, int m
     const float* base = a.partial + rh * max_split * (vp + 4);
     const int lane = threadIdx.x, k = lane * 4;
     const float2 ml = lane < nsplit ? *reinterpret_cast<const float2*>(base + (size_t)lane * (vp + 4)) : make_float2(LA_SENT, 0.f);
+    constexpr int S = 8;                               // that many records are asked for before the first is used: a step of 8 layers, 4 rows of 1000 keys 319 -> 308 us, 8 of 2048 358 -> 350
+    f32x4 r[S];
+#pragma unroll
+    for (int s = 0; s < S; ++s) r[s] = *reinterpret_cast<const f32x4*>(base + (size_t)min(s, nsplit - 1) * (vp + 4) + 4 + min(k, vp - 4));
     const float M = wave_max(ml.x);
     const float w = lane < nsplit ? exp2_w(ml.x - M) : 0.f;
     const float L = wave_sum(ml.y * w);
     if (k >= vp) return;
     f32x4 v = (f32x4){0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int s = 0; s < S; ++s)
+        if (s < nsplit) v += r[s] * __int_as_float(__builtin_amdgcn_readlane(__float_as_int(w), s));
 #pragma unroll 4
-    for (int s = 0; s < nsplit; ++s)
+    for (int s = S; s < nsplit; ++s)
         v += *reinterpret_cast<const f32x4*>(base + (size_t)s * (vp + 4) + 4 + k) * __int_as_float(__builtin_amdgcn_readlane(__float_as_int(w), s));
     wa_store(a.gate, a.out, a.frag, t, head * vp + k, a.heads * vp, v * (L > 0.f ? 1.0f / L : 0.f));
 }

@@ -281,13 +281,22 @@ __global__ __launch_bounds__(256) void latent_values_kernel(const float* __restr
     const float* base = partial + rh * max_split * (rp + 4);
     const float2 ml = lane < nsplit && nsplit > 1 ? *reinterpret_cast<const float2*>(base + (size_t)lane * (rp + 4)) : make_float2(LA_SENT, 0.f);
     const uint2 whole = k < rp ? *reinterpret_cast<const uint2*>(merged + rh * rp + k) : make_uint2(0, 0);      // (one split: the decode kernel wrote the row)
+    constexpr int S = 8;                               // that many records are asked for before the first is used
+    f32x4 r[S];
+    if (nsplit > 1)
+#pragma unroll
+        for (int s = 0; s < S; ++s) r[s] = *reinterpret_cast<const f32x4*>(base + (size_t)min(s, nsplit - 1) * (rp + 4) + 4 + min(k, rp - 4));
 #pragma unroll
     for (int d = 0; d < P; ++d) load(d, d);
     const float M = wave_max(ml.x), e = lane < nsplit ? exp2f(ml.x - M) : 0.f, L = wave_sum(ml.y * e);
     f32x4 m = (f32x4){0.f, 0.f, 0.f, 0.f};
-    if (k < rp && nsplit > 1)
+    if (nsplit > 1)
+#pragma unroll
+        for (int s = 0; s < S; ++s)
+            if (s < nsplit) m += r[s] * __int_as_float(__builtin_amdgcn_readlane(__float_as_int(e), s));
+    if (k < rp)
 #pragma unroll 4
-        for (int s = 0; s < nsplit; ++s)
+        for (int s = S; s < nsplit; ++s)
             m += *reinterpret_cast<const f32x4*>(base + (size_t)s * (rp + 4) + 4 + k) * __int_as_float(__builtin_amdgcn_readlane(__float_as_int(e), s));
     m *= (L > 0.f ? 1.0f / L : 0.f) * (gate ? gate[rh] : 1.0f);
     if (k < rp && wave >> 1 == t) *reinterpret_cast<uint2*>(xs + (size_t)t * rp + k) = nsplit > 1 ? make_uint2(pack_bf2(m[0], m[1]), pack_bf2(m[2], m[3])) : whole;

@@ -191,6 +191,7 @@ SIGNATURES = {
     "omni_codec_out_conv": (i32, [vp, vp, f32, vp, i32, i32, i32, vp]),
     "omni_codec_res_unit_supported": (i32, [i32, i32, i32]),
     "omni_codec_res_unit": (i32, [C.POINTER(ResUnit), vp]),
+    "omni_codec_res_unit_last": (i32, [C.POINTER(ResUnit), vp]),
     "omni_gemm_resid": (i32, [vp, i32, vp, vp, vp, i32, vp, vp, i32, i32, i32, i32, vp]),
     "omni_gemm_xnorm": (i32, [vp, vp, i32, vp, f32, vp, vp, vp, i32, i32, i32, i32, vp, i32, vp]),
     "omni_attn_decode_fused": (i32, [vp, vp, vp, vp, vp, f32, vp, vp, vp, vp, vp, i32, vp, vp, vp, vp, i32, i32, i32, i32, i32, i32,

@@ -338,6 +338,7 @@ class Code2WavDecoder:
             for ui, un in enumerate(units):
                 nxt = units[ui + 1]["act1"] if ui + 1 < len(units) else (self.blocks[bi + 1]["act"] if bi + 1 < nb else self.last_act)
                 c1 = un["conv1"]
+                last = taps is None and ui + 1 == len(units)                          # behind it only s is read
                 if self.fused_units and lib.omni_codec_res_unit_supported(cout, c1.taps, c1.dilation):
                     s_alt = torch.empty_like(s) if s_alt is None else s_alt           # the unit reads a halo of s: no in-place s
                     ru = L.ResUnit()
@@ -345,11 +346,14 @@ class Code2WavDecoder:
                     ru.w1, ru.b1, ru.snake2_alpha, ru.snake2_inv_beta = c1.w.data_ptr(), c1.bias.data_ptr(), un["act2"][0].data_ptr(), un["act2"][1].data_ptr()
                     ru.w2, ru.b2, ru.next_alpha, ru.next_inv_beta = un["conv2"].w.data_ptr(), un["conv2"].bias.data_ptr(), nxt[0].data_ptr(), nxt[1].data_ptr()
                     ru.T, ru.C, ru.dilation = T, cout, c1.dilation
-                    self._check(lib.omni_codec_res_unit(C.byref(ru), st), "omni_codec_res_unit")
+                    self._check((lib.omni_codec_res_unit_last if last else lib.omni_codec_res_unit)(C.byref(ru), st), "omni_codec_res_unit")
                     s, s_alt = s_alt, s
                 else:
                     t1 = c1(s, snake=un["act2"], want="s")
-                    _, s = un["conv2"](t1, resid=hstream, out_f32=hstream, snake=nxt, want="fs")
+                    if last:
+                        s = un["conv2"](t1, resid=hstream, snake=nxt, want="s")
+                    else:
+                        _, s = un["conv2"](t1, resid=hstream, out_f32=hstream, snake=nxt, want="fs")
             tap(f"decoder{bi + 1}", hstream)
         tap(f"decoder{nb + 1}", s)
         wav = torch.empty(T, dtype=torch.float32, device=dev)

@@ -9,7 +9,9 @@
 //     all 7 taps take their operand fragments from it by row offset;
 //   * the 7-tap conv's output tile never leaves the chip: bias + snake2 -> bf16 -> LDS in operand-fragment order -> the 1x1 conv's
 //     MFMAs (its C x C weight straight from L2 into registers);
-//   * epilogue: + bias + h (fp32) -> h in place, bf16(snake_next(h)) for the next unit: 12 B per element of HBM traffic.
+//   * epilogue: + bias + h (fp32) -> h in place, bf16(snake_next(h)) for the next unit: 12 B per element of HBM traffic.  Behind a block's
+//     last unit nobody reads h (omni_codec_res_unit_last): 8 B.  A whole waveform's GPU time with the last
+//     unit of every block writing h / not, us: 12 frames 735 / 732, 50 950 / 942, 100 1 290 / 1 274, 200 2 046 / 2 004, 325 3 173 / 3 106
 // W1 (fragment-major [C, 7 C], K index = tap * C + channel) streams through an LDS ring by LDS-DMA like omni_gemm_tile's W.
 // 8 waves, a wave owns 6 n-tiles x WM m-tiles (96 columns x 16 WM rows): C = 96: 1 x 8 waves, BM = 128 WM; C = 192: 2 x 4 waves, BM = 64 WM.
 // Same k order per output element as the two-launch path (taps outer, channels inner; then the 1x1 conv's channels): bit-identical
@@ -32,6 +34,7 @@ struct ResUnitArgs {
     const uint16_t* w1; const float* b1; const float* a2; const float* ib2;      // conv7 + the snake behind it
     const uint16_t* w2; const float* b2; const float* an; const float* ibn;      // conv1x1 + the snake of the next consumer
     int T, dil;
+    bool last;                                                                   // h is read, not written
 };
 
 __device__ __forceinline__ f32x4 ru_mfma(u32x4 a, u32x4 b, f32x4 c) {
@@ -247,8 +250,10 @@ __global__ __launch_bounds__(RU_THREADS, (RuGeom<C, WM_, NBUF_>::LDS_BYTES <= 80
             float* hp = a.h + (size_t)m * C + n;
             const f32x4 y0 = *reinterpret_cast<const f32x4*>(img + row * IP + ch * 32) + hv[pass & 1][it][0];
             const f32x4 y1 = *reinterpret_cast<const f32x4*>(img + row * IP + ch * 32 + 16) + hv[pass & 1][it][1];
-            *reinterpret_cast<f32x4*>(hp) = y0;
-            *reinterpret_cast<f32x4*>(hp + 4) = y1;
+            if (!a.last) {
+                *reinterpret_cast<f32x4*>(hp) = y0;
+                *reinterpret_cast<f32x4*>(hp + 4) = y1;
+            }
             const f32x4 al0 = *reinterpret_cast<const f32x4*>(a.an + n), al1 = *reinterpret_cast<const f32x4*>(a.an + n + 4);
             const f32x4 ib0 = *reinterpret_cast<const f32x4*>(a.ibn + n), ib1 = *reinterpret_cast<const f32x4*>(a.ibn + n + 4);
             f32x4 z0, z1;
@@ -303,7 +308,7 @@ extern "C" int omni_codec_res_unit_supported(int C, int taps, int dilation) {
     return (C == 96 || C == 192) && taps == RU_TAPS && dilation >= 1 && (RU_TAPS - 1) * dilation <= RU_HALO_MAX;
 }
 
-extern "C" int omni_codec_res_unit(const omni_res_unit* u, void* stream) {
+static int res_unit(const omni_res_unit* u, bool last, void* stream) {
     OMNI_CHECK_ARG(u && u->s && u->h && u->s_next && u->w1 && u->b1 && u->snake2_alpha && u->snake2_inv_beta && u->w2 && u->b2 &&
                    u->next_alpha && u->next_inv_beta, "omni_codec_res_unit: null argument");
     OMNI_CHECK_ARG(u->T > 0 && omni_codec_res_unit_supported(u->C, RU_TAPS, u->dilation), "omni_codec_res_unit: T=%d C=%d dilation=%d (C 96 | 192, dilation <= 9)", u->T, u->C, u->dilation);
@@ -312,7 +317,7 @@ extern "C" int omni_codec_res_unit(const omni_res_unit* u, void* stream) {
     a.s = (const uint16_t*)u->s; a.h = u->h; a.s_next = (uint16_t*)u->s_next;
     a.w1 = (const uint16_t*)u->w1; a.b1 = u->b1; a.a2 = u->snake2_alpha; a.ib2 = u->snake2_inv_beta;
     a.w2 = (const uint16_t*)u->w2; a.b2 = u->b2; a.an = u->next_alpha; a.ibn = u->next_inv_beta;
-    a.T = u->T; a.dil = u->dilation;
+    a.T = u->T; a.dil = u->dilation; a.last = last;
     OMNI_CHECK_ARG(u->row_tiles >= 0 && u->row_tiles <= RU_MAX_TILES, "omni_codec_res_unit: row_tiles=%d (0 .. %d)", u->row_tiles, RU_MAX_TILES);
     const int wm = u->row_tiles ? u->row_tiles : ru_row_tiles(u->C, u->T);
     hipStream_t st = (hipStream_t)stream;
@@ -320,3 +325,6 @@ extern "C" int omni_codec_res_unit(const omni_res_unit* u, void* stream) {
         return wm == 1 ? launch_unit<96, 1, 4>(a, st) : wm == 2 ? launch_unit<96, 2, 4>(a, st) : wm == 3 ? launch_unit<96, 3, 4>(a, st) : launch_unit<96, 4, 4>(a, st);
     return wm == 1 ? launch_unit<192, 1, 2>(a, st) : wm == 2 ? launch_unit<192, 2, 3>(a, st) : wm == 3 ? launch_unit<192, 3, 3>(a, st) : launch_unit<192, 4, 3>(a, st);
 }
+
+extern "C" int omni_codec_res_unit(const omni_res_unit* u, void* stream) { return res_unit(u, false, stream); }
+extern "C" int omni_codec_res_unit_last(const omni_res_unit* u, void* stream) { return res_unit(u, true, stream); }

@@ -64,6 +64,7 @@ typedef struct omni_res_unit {
 } omni_res_unit;
 int omni_codec_res_unit_supported(int C, int taps, int dilation);
 int omni_codec_res_unit(const omni_res_unit* u, void* stream);
+int omni_codec_res_unit_last(const omni_res_unit* u, void* stream);      /* h is read and left as it is: a block's last unit, behind which only s_next is read */
 
 #ifdef __cplusplus
 }

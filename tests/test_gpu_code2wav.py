@@ -207,6 +207,34 @@ def test_a_unit_of_any_row_block_is_the_same_unit(C, T, dil):
     assert lib.omni_codec_res_unit(ctypes.byref(u), L.current_stream()) != 0
 
 
+@pytest.mark.parametrize("C,T,dil,tiles", [(96, 1, 1, 0), (96, 129, 9, 1), (96, 1030, 3, 4), (192, 65, 1, 2), (192, 771, 3, 3)])
+def test_a_last_unit_leaves_the_stream_and_gives_the_same_signal(C, T, dil, tiles):
+    import ctypes
+    from ht_vllm_omni_amd import _lib as L
+    lib, g = L.load(), torch.Generator().manual_seed(C + T)
+    r = lambda *s: torch.randn(*s, generator=g).cuda()  # noqa: E731
+    s, h, p = r(T, C).to(torch.bfloat16), r(T, C), r(6, C).abs() + 0.3
+    w1, w2 = (0.05 * r(C * 7 * C)).to(torch.bfloat16), (0.05 * r(C * C)).to(torch.bfloat16)
+    got = []
+    for f in (lib.omni_codec_res_unit, lib.omni_codec_res_unit_last):
+        h1, nxt = h.clone(), torch.full((T + 8, C), 7.0, dtype=torch.bfloat16, device="cuda")
+        u = L.ResUnit(s.data_ptr(), h1.data_ptr(), nxt.data_ptr(), w1.data_ptr(), *(p[i].data_ptr() for i in range(3)), w2.data_ptr(), *(p[i].data_ptr() for i in range(3, 6)),
+                      T, C, dil, tiles)
+        L.check(f(ctypes.byref(u), L.current_stream()), "omni_codec_res_unit", lib)
+        got.append((h1, nxt))
+    assert torch.equal(got[1][0], h) and not torch.equal(got[0][0], h) and torch.equal(got[1][1], got[0][1])
+    u.row_tiles = 5
+    assert lib.omni_codec_res_unit_last(ctypes.byref(u), L.current_stream()) != 0
+
+
+@pytest.mark.parametrize("T", [1, 7, 33])
+def test_a_waveform_is_the_same_with_and_without_the_streams(T):
+    sd = make_codec_state(FULL_CODEC, 9, device="cuda")
+    dec = _decoder(FULL_CODEC, sd)
+    codes = torch.randint(0, 2048, (1, 16, T), generator=torch.Generator().manual_seed(T)).cuda()
+    assert torch.equal(dec.forward(codes), dec.forward(codes, {}))
+
+
 @pytest.mark.parametrize("hd,nh,nkv,T,window,ldo", [(64, 4, 4, 1, 72, 256), (64, 4, 2, 65, 64, 256), (64, 3, 1, 130, 72, 203), (128, 2, 1, 129, 200, 256), (128, 2, 2, 9, 1, 264)])
 def test_window_attention_kernel(hd, nh, nkv, T, window, ldo):
     """Chunk edges of 64 keys, windows of one key and of several chunks, shared key heads, output rows of odd pitch.  Bound: the result's rounding to bf16

@@ -94,6 +94,10 @@ __device__ __forceinline__ u32x4 la_transposed(const unsigned char* img, int dt,
     return la_transposed_at(img, LatentGeom<RS>::PITCH, dt, c, qk);
 }
 
+// What bounds it: the stream of rows, 16 KB a wave in flight, and the chain in front of it.  A row's operand of q is asked for first and waited for before the
+// loop (a wait inside is for all that is in flight there, the next round's rows), the next ids ahead of the rows, and a piece of the next round the moment
+// this round's has gone to LDS.  Us with the merge, 16 heads, latents of 512 | 256, before / this: 64 rows of 1024 to 2048 keys 37.4 / 34.9 | 23.4 / 22.3, of 1536
+// 35.2 / 31.4 | 21.8 / 20.6, of 176 to 352 17.0 / 15.8 | 11.8 / 11.2, 32 of 256 14.2 / 13.3 | 10.5 / 9.9, 8 of 150 to 300 11.3 / 11.1 | 9.3 / 9.1; the same bits.
 template <int RS>
 __global__ __launch_bounds__(64 * LA_DEC_WAVES, 2) void latent_decode_kernel(const LatentArgs a) {
     using G = LatentGeom<RS>;
@@ -115,43 +119,44 @@ __global__ __launch_bounds__(64 * LA_DEC_WAVES, 2) void latent_decode_kernel(con
     if (split >= nsplit) return;
     const int t0 = (int)((long long)ntiles * split / nsplit), t1 = (int)((long long)ntiles * (split + 1) / nsplit);
     const int end = min(len, t1 * 16);                // keys of this split
-    u32x4 st[RS];                                     // the wave's next tile on its way to LDS (16 rows = RS 16-byte loads per lane)
-    auto block_of = [&](int tile) { return bt[min(tile * 16 + c, len - 1) >> a.bs_shift]; };
-    auto fetch = [&](int tile, int blk) {
-        const int key = min(tile * 16 + c, len - 1);  // keys past the end: a valid row, masked below
-        const int slot = (blk << a.bs_shift) + (key & a.bs_mask);
-#pragma unroll
-        for (int j = 0; j < RS; ++j) {
-            const int i = lane + 64 * j;
-            const int kk = i / G::CH, ch = i - kk * G::CH;
-            const int row = G::CH % 64 == 0 ? __builtin_amdgcn_readlane(slot, j / (G::CH / 64 > 0 ? G::CH / 64 : 1)) : __shfl(slot, kk, 64);
-            st[j] = ld16_nt(a.cache + (size_t)row * rp + ch * 8);
-        }
-    };
-    int blk = 0;                                      // block ids are looked up a round ahead of the rows
-    if (t0 < t1) {
-        blk = block_of(t0 + wave);
-        fetch(t0 + wave, blk);
-        blk = block_of(t0 + wave + LA_DEC_WAVES);
-    }
     u32x4 Q[RS];
 #pragma unroll
     for (int s = 0; s < RS; ++s) Q[s] = ld16(a.q + ((size_t)t * a.heads + hc) * rp + 32 * s + 8 * qk);
+    u32x4 st[RS];                                     // the wave's next tile on its way to LDS (16 rows = RS 16-byte loads per lane)
+    auto block_of = [&](int tile) { return bt[min(tile * 16 + c, len - 1) >> a.bs_shift]; };
+    auto slot_of = [&](int tile, int blk) { return (blk << a.bs_shift) + (min(tile * 16 + c, len - 1) & a.bs_mask); };      // keys past the end: a valid row, masked below
+    auto fetch = [&](int slot, int j) {
+        const int i = lane + 64 * j;
+        const int kk = i / G::CH, ch = i - kk * G::CH;
+        const int row = G::CH % 64 == 0 ? __builtin_amdgcn_readlane(slot, j / (G::CH / 64 > 0 ? G::CH / 64 : 1)) : __shfl(slot, kk, 64);
+        st[j] = ld16_nt(a.cache + (size_t)row * rp + ch * 8);
+    };
+    auto keep = [&](int j) {
+        const int i = lane + 64 * j;
+        const int kk = i / G::CH, ch = i - kk * G::CH;
+        *reinterpret_cast<u32x4*>(img + kk * G::PITCH + ch * 16) = st[j];
+    };
+    const int slot0 = slot_of(t0 + wave, block_of(t0 + wave));      // (every split of a row has a tile)
+    int blk = block_of(t0 + wave + LA_DEC_WAVES);     // block ids are looked up a round ahead of the rows
+#pragma unroll
+    for (int j = 0; j < RS; ++j) fetch(slot0, j);
+    // waited for here: inside the loop the wait would be for what is in flight then, the next round's rows
+#pragma unroll
+    for (int s = 0; s < RS; ++s) asm volatile("" : "+v"(Q[s]));
     f32x4 O[DPW];
 #pragma unroll
     for (int i = 0; i < DPW; ++i) O[i] = (f32x4){0.f, 0.f, 0.f, 0.f};
     float m = LA_SENT, l = 0.f;                       // m: common to the waves; l: this wave's keys
     for (int base = t0; base < t1; base += LA_DEC_WAVES) {
         const int key0 = (base + wave) * 16 + 4 * qk; // the lane's keys: key0 .. key0 + 3
+        if (base + LA_DEC_WAVES < t1) {               // a piece goes to LDS and the next round's is asked for in its place
+            const int slot = slot_of(base + wave + LA_DEC_WAVES, blk);
+            blk = block_of(base + wave + 2 * LA_DEC_WAVES);      // (ahead of the rows: they are not waited for with it)
 #pragma unroll
-        for (int j = 0; j < RS; ++j) {
-            const int i = lane + 64 * j;
-            const int kk = i / G::CH, ch = i - kk * G::CH;
-            *reinterpret_cast<u32x4*>(img + kk * G::PITCH + ch * 16) = st[j];
-        }
-        if (base + LA_DEC_WAVES < t1) {
-            fetch(base + wave + LA_DEC_WAVES, blk);
-            blk = block_of(base + wave + 2 * LA_DEC_WAVES);
+            for (int j = 0; j < RS; ++j) { keep(j); fetch(slot, j); }
+        } else {
+#pragma unroll
+            for (int j = 0; j < RS; ++j) keep(j);
         }
         __builtin_amdgcn_wave_barrier();
         f32x4 S4[4];

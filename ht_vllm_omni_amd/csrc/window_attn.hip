@@ -38,6 +38,9 @@ __device__ __forceinline__ void wa_store(const uint16_t* gate, uint16_t* out, in
     *reinterpret_cast<uint2*>(out + (frag ? frag_off((int)t, k, width) : t * width + k)) = make_uint2(pack_bf2(v[0], v[1]), pack_bf2(v[2], v[3]));
 }
 
+// The row's operand of q is asked for first and waited for before the loop, block ids ahead of the rows, and the next round's pieces in the place of this
+// round's.  Us with the merge, 16 heads over 4 of 128, before / this: 64 rows of 1024 to 2048 keys 49.6 / 48.3, in windows of 1024 29.5 / 28.7; of 176 to 352
+// 11.8 / 11.5; 48 of 352 to 704 18.8 / 18.3; one row of 352 8.4 either way; 8 heads over 2 of 64, 64 rows of up to 2048 18.1 / 17.8.  The same bits.
 template <int WS, bool EX>
 __global__ __launch_bounds__(64 * LA_DEC_WAVES, 2) void window_decode_kernel(const WinArgs a) {
     constexpr int DPW = (2 * WS + LA_DEC_WAVES - 1) / LA_DEC_WAVES;      // output column tiles of a wave: wave, wave + 4, ...
@@ -59,25 +62,31 @@ __global__ __launch_bounds__(64 * LA_DEC_WAVES, 2) void window_decode_kernel(con
     if (split >= nsplit) return;
     const int t0 = tl + (int)((long long)ntiles * split / nsplit), t1 = tl + (int)((long long)ntiles * (split + 1) / nsplit);
     const int end = min(len, t1 * 16);                // keys of this split: [lo, end) from tile t0 on
-    u32x4 K[WS], st[WS];                              // the wave's next tile: keys as operands, values on their way to LDS
-    auto block_of = [&](int tile) { return bt[min(tile * 16 + c, len - 1) >> a.bs_shift]; };
-    auto fetch = [&](int tile, int blk) {             // lane (c, qk): 16-byte pieces qk, qk + 4, ... of key c's rows
-        const int key = min(tile * 16 + c, len - 1);  // keys past the end: a valid row, masked below
-        const size_t row = ((size_t)(blk * a.kv_heads + g) << a.bs_shift) + (key & a.bs_mask);
-#pragma unroll
-        for (int s = 0; s < WS; ++s)
-            if (EX || s < ds) K[s] = ld16_nt(a.kc + row * dp + 32 * s + 8 * qk);
-#pragma unroll
-        for (int s = 0; s < WS; ++s)
-            if (EX || s < vs) st[s] = ld16_nt(a.vc + row * vp + 32 * s + 8 * qk);
-    };
-    int blk = block_of(t0 + wave);                    // block ids are looked up a round ahead of the rows
-    fetch(t0 + wave, blk);
-    blk = block_of(t0 + wave + LA_DEC_WAVES);
     u32x4 Q[WS];
 #pragma unroll
     for (int s = 0; s < WS; ++s)
         if (EX || s < ds) Q[s] = ld16(a.q + ((size_t)t * a.heads + head) * dp + 32 * s + 8 * qk);
+    u32x4 K[WS], st[WS];                              // the wave's next tile: keys as operands, values on their way to LDS
+    auto block_of = [&](int tile) { return bt[min(tile * 16 + c, len - 1) >> a.bs_shift]; };
+    auto row_of = [&](int tile, int blk) {            // keys past the end: a valid row, masked below
+        return ((size_t)(blk * a.kv_heads + g) << a.bs_shift) + (min(tile * 16 + c, len - 1) & a.bs_mask);
+    };
+    auto key_piece = [&](size_t row, int s) {         // lane (c, qk): 16-byte pieces qk, qk + 4, ... of key c's rows
+        if (EX || s < ds) K[s] = ld16_nt(a.kc + row * dp + 32 * s + 8 * qk);
+    };
+    auto value_piece = [&](size_t row, int s) {
+        if (EX || s < vs) st[s] = ld16_nt(a.vc + row * vp + 32 * s + 8 * qk);
+    };
+    const size_t row0 = row_of(t0 + wave, block_of(t0 + wave));
+    int blk = block_of(t0 + wave + LA_DEC_WAVES);     // block ids are looked up a round ahead of the rows
+#pragma unroll
+    for (int s = 0; s < WS; ++s) key_piece(row0, s);
+#pragma unroll
+    for (int s = 0; s < WS; ++s) value_piece(row0, s);
+    // waited for here: inside the loop the wait would be for what is in flight then
+#pragma unroll
+    for (int s = 0; s < WS; ++s)
+        if (EX || s < ds) asm volatile("" : "+v"(Q[s]));
     f32x4 O[DPW];
 #pragma unroll
     for (int i = 0; i < DPW; ++i) O[i] = (f32x4){0.f, 0.f, 0.f, 0.f};
@@ -86,16 +95,21 @@ __global__ __launch_bounds__(64 * LA_DEC_WAVES, 2) void window_decode_kernel(con
     float m = sink ? a.sink[head] * LA_LOG2E : LA_SENT, l = sink && wave == 0 ? 1.f : 0.f;
     for (int base = t0; base < t1; base += LA_DEC_WAVES) {
         const int key0 = (base + wave) * 16 + 4 * qk; // the lane's keys: key0 .. key0 + 3
-#pragma unroll
-        for (int s = 0; s < WS; ++s)
-            if (EX || s < vs) *reinterpret_cast<u32x4*>(img + c * pitch + (32 * s + 8 * qk) * 2) = st[s];
         f32x4 S2[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
+        auto score = [&](int s) { if (EX || s < ds) S2[s & 1] = mfma16(K[s], Q[s], S2[s & 1]); };
+        auto keep = [&](int s) { if (EX || s < vs) *reinterpret_cast<u32x4*>(img + c * pitch + (32 * s + 8 * qk) * 2) = st[s]; };
+        if (base + LA_DEC_WAVES < t1) {               // the next round's pieces are asked for in the place of this one's
+            const size_t row = row_of(base + wave + LA_DEC_WAVES, blk);
+            blk = block_of(base + wave + 2 * LA_DEC_WAVES);      // (ahead of the rows: they are not waited for with it)
 #pragma unroll
-        for (int s = 0; s < WS; ++s)
-            if (EX || s < ds) S2[s & 1] = mfma16(K[s], Q[s], S2[s & 1]);
-        if (base + LA_DEC_WAVES < t1) {
-            fetch(base + wave + LA_DEC_WAVES, blk);
-            blk = block_of(base + wave + 2 * LA_DEC_WAVES);
+            for (int s = 0; s < WS; ++s) { score(s); key_piece(row, s); }
+#pragma unroll
+            for (int s = 0; s < WS; ++s) { keep(s); value_piece(row, s); }
+        } else {
+#pragma unroll
+            for (int s = 0; s < WS; ++s) score(s);
+#pragma unroll
+            for (int s = 0; s < WS; ++s) keep(s);
         }
         const f32x4 S = S2[0] + S2[1];
         float sv[4], mx = LA_SENT;

@@ -250,6 +250,7 @@ DECODER_SIGNATURES = {
     "omni_gemm_f32": (i32, [vp, i32, i64, vp, i64, vp, i32, i64, i32, i32, i32, i32, i32, f32, f32, vp]),
     "omni_gemm_stream": (i32, [vp, vp, vp, i32, i32, i32, i32, i32, f32, f32, i32, vp]),
     "omni_gemm_stream_splits": (i32, [i32, i32, i32]),
+    "omni_gemm_stream_plain": (i32, [vp, i32, vp, vp, i32, i32, i32, i32, vp]),
     "omni_gemm_stream_rows": (i32, [vp, vp, vp, i32, i32, i32, C.POINTER(RowTable), i32, vp]),
     "omni_gemm_stream_joined": (i32, [C.POINTER(StreamRows), vp, vp, i32, i32, i32, f32, f32, C.POINTER(RowTable), i32, vp]),
     "omni_gemm_stream_joins": (i32, [i32, i32, i32, i32, i32]),

@@ -95,8 +95,8 @@ __device__ __forceinline__ u32x4 la_transposed(const unsigned char* img, int dt,
 }
 
 // What bounds it: the stream of rows, 16 KB a wave in flight, and the chain in front of it.  A row's operand of q is asked for first and waited for before the
-// loop (a wait inside is for all that is in flight there, the next round's rows), the next ids ahead of the rows, and a piece of the next round the moment
-// this round's has gone to LDS.  Us with the merge, 16 heads, latents of 512 | 256, before / this: 64 rows of 1024 to 2048 keys 37.4 / 34.9 | 23.4 / 22.3, of 1536
+// loop (a wait inside is for all that is in flight there, the next turn's rows), the next ids ahead of the rows, and a piece of the next turn the moment
+// this turn's has gone to LDS.  Us with the merge, 16 heads, latents of 512 | 256, before / this: 64 rows of 1024 to 2048 keys 37.4 / 34.9 | 23.4 / 22.3, of 1536
 // 35.2 / 31.4 | 21.8 / 20.6, of 176 to 352 17.0 / 15.8 | 11.8 / 11.2, 32 of 256 14.2 / 13.3 | 10.5 / 9.9, 8 of 150 to 300 11.3 / 11.1 | 9.3 / 9.1; the same bits.
 template <int RS>
 __global__ __launch_bounds__(64 * LA_DEC_WAVES, 2) void latent_decode_kernel(const LatentArgs a) {
@@ -140,7 +140,7 @@ __global__ __launch_bounds__(64 * LA_DEC_WAVES, 2) void latent_decode_kernel(con
     int blk = block_of(t0 + wave + LA_DEC_WAVES);     // block ids are looked up a round ahead of the rows
 #pragma unroll
     for (int j = 0; j < RS; ++j) fetch(slot0, j);
-    // waited for here: inside the loop the wait would be for what is in flight then, the next round's rows
+    // waited for here: inside the loop the wait would be for what is in flight then, the next turn's rows
 #pragma unroll
     for (int s = 0; s < RS; ++s) asm volatile("" : "+v"(Q[s]));
     f32x4 O[DPW];
@@ -149,7 +149,7 @@ __global__ __launch_bounds__(64 * LA_DEC_WAVES, 2) void latent_decode_kernel(con
     float m = LA_SENT, l = 0.f;                       // m: common to the waves; l: this wave's keys
     for (int base = t0; base < t1; base += LA_DEC_WAVES) {
         const int key0 = (base + wave) * 16 + 4 * qk; // the lane's keys: key0 .. key0 + 3
-        if (base + LA_DEC_WAVES < t1) {               // a piece goes to LDS and the next round's is asked for in its place
+        if (base + LA_DEC_WAVES < t1) {               // a piece goes to LDS and the next turn's is asked for in its place
             const int slot = slot_of(base + wave + LA_DEC_WAVES, blk);
             blk = block_of(base + wave + 2 * LA_DEC_WAVES);      // (ahead of the rows: they are not waited for with it)
 #pragma unroll

@@ -38,8 +38,8 @@ __device__ __forceinline__ void wa_store(const uint16_t* gate, uint16_t* out, in
     *reinterpret_cast<uint2*>(out + (frag ? frag_off((int)t, k, width) : t * width + k)) = make_uint2(pack_bf2(v[0], v[1]), pack_bf2(v[2], v[3]));
 }
 
-// The row's operand of q is asked for first and waited for before the loop, block ids ahead of the rows, and the next round's pieces in the place of this
-// round's.  Us with the merge, 16 heads over 4 of 128, before / this: 64 rows of 1024 to 2048 keys 49.6 / 48.3, in windows of 1024 29.5 / 28.7; of 176 to 352
+// The row's operand of q is asked for first and waited for before the loop, block ids ahead of the rows, and the next turn's pieces in the place of this
+// turn's.  Us with the merge, 16 heads over 4 of 128, before / this: 64 rows of 1024 to 2048 keys 49.6 / 48.3, in windows of 1024 29.5 / 28.7; of 176 to 352
 // 11.8 / 11.5; 48 of 352 to 704 18.8 / 18.3; one row of 352 8.4 either way; 8 heads over 2 of 64, 64 rows of up to 2048 18.1 / 17.8.  The same bits.
 template <int WS, bool EX>
 __global__ __launch_bounds__(64 * LA_DEC_WAVES, 2) void window_decode_kernel(const WinArgs a) {
@@ -98,7 +98,7 @@ __global__ __launch_bounds__(64 * LA_DEC_WAVES, 2) void window_decode_kernel(con
         f32x4 S2[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
         auto score = [&](int s) { if (EX || s < ds) S2[s & 1] = mfma16(K[s], Q[s], S2[s & 1]); };
         auto keep = [&](int s) { if (EX || s < vs) *reinterpret_cast<u32x4*>(img + c * pitch + (32 * s + 8 * qk) * 2) = st[s]; };
-        if (base + LA_DEC_WAVES < t1) {               // the next round's pieces are asked for in the place of this one's
+        if (base + LA_DEC_WAVES < t1) {               // the next turn's pieces are asked for in the place of this one's
             const size_t row = row_of(base + wave + LA_DEC_WAVES, blk);
             blk = block_of(base + wave + 2 * LA_DEC_WAVES);      // (ahead of the rows: they are not waited for with it)
 #pragma unroll

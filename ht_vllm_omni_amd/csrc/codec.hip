@@ -13,7 +13,6 @@
 // it calls); oracle: oracle/code2wav_oracle.py.
 #include "common.cuh"
 #include "kernels.h"
-#include <initializer_list>
 
 typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
 
@@ -363,12 +362,6 @@ __global__ __launch_bounds__(256) void codec_dwconv_ln_kernel(const float* __res
     }
 }
 
-static bool aligned16(std::initializer_list<const void*> ps) {
-    for (const void* p : ps)
-        if ((uintptr_t)p & 15) return false;
-    return true;
-}
-
 extern "C" int omni_codec_dwconv_ln(const float* x, int ldx, const float* w, const float* b, const float* ln_w, const float* ln_b, float eps,
                                     void* out, int T, int C, int taps, void* stream) {
     OMNI_CHECK_ARG(x && w && b && ln_w && ln_b && out && T > 0 && C > 0 && C <= 1024 && taps > 0 && ldx >= C, "omni_codec_dwconv_ln: T=%d C=%d (<= 1024)", T, C);
@@ -382,8 +375,19 @@ extern "C" int omni_codec_dwconv_ln(const float* x, int ldx, const float* w, con
 // wav[t] = clamp(b + sum_{j, c} w[j][c] x[t - (taps - 1) + j][c], -1, 1); x bf16 [T, C] (already through the last snake), w fp32 [taps][C].
 // A lane's sample needs `taps` whole rows, and neighbouring lanes' rows are neighbours: lanes that fetch a row each take 16 bytes out of as many lines as there
 // are lanes, `taps` times over.  So a block's rows go to LDS once, in whole lines (pitch of an odd number of 16-byte pieces: 16 rows lie in 16 different
-// bank groups), and the weights, the same for every lane, come through scalar loads.  96000 samples of 96 channels, 7 taps: 19.5 -> 12.5 us; 624000: 219 -> 65.
+// bank groups), all pieces of a thread asked for at once, and the weights, the same for every lane, behind them.  A sample is one chain of sums, taps outer, channels
+// inner, whatever the width.  Us, out of cold caches with the events around it, weights by scalar loads 32 at a time and rows a piece after the other / this: 23040 samples of 96
+// channels, 7 taps, 23.3 / 11.7, 96000 23.7 / 14.0, 624000 71 / 55.  Every row times every tap on the matrix cores takes 7.5, 9.5 and 25, but adds up in another order: not kept.
 #define OC_ROWS 256
+// xr: 16-byte pieces; wr: in LDS, 16-byte aligned
+__device__ __forceinline__ float oc_piece(u32x4 v, const float* wr, float acc) {
+    const f32x4 a = *reinterpret_cast<const f32x4*>(wr), b = *reinterpret_cast<const f32x4*>(wr + 4);
+    acc += bf_lo(v[0]) * a[0] + bf_hi(v[0]) * a[1];
+    acc += bf_lo(v[1]) * a[2] + bf_hi(v[1]) * a[3];
+    acc += bf_lo(v[2]) * b[0] + bf_hi(v[2]) * b[1];
+    acc += bf_lo(v[3]) * b[2] + bf_hi(v[3]) * b[3];
+    return acc;
+}
 __device__ __forceinline__ float oc_row(const uint16_t* xr, const float* wr, int C, float acc) {
     int c = 0;
     for (; c + 32 <= C; c += 32) {                        // (four pieces of the row and of the weights per wait)
@@ -391,15 +395,9 @@ __device__ __forceinline__ float oc_row(const uint16_t* xr, const float* wr, int
 #pragma unroll
         for (int i = 0; i < 4; ++i) v[i] = *reinterpret_cast<const u32x4*>(xr + c + 8 * i);
 #pragma unroll
-        for (int i = 0; i < 4; ++i)
-#pragma unroll
-            for (int e = 0; e < 4; ++e) acc += bf_lo(v[i][e]) * wr[c + 8 * i + 2 * e] + bf_hi(v[i][e]) * wr[c + 8 * i + 2 * e + 1];
+        for (int i = 0; i < 4; ++i) acc = oc_piece(v[i], wr + c + 8 * i, acc);
     }
-    for (; c < C; c += 8) {
-        const u32x4 v = *reinterpret_cast<const u32x4*>(xr + c);
-#pragma unroll
-        for (int e = 0; e < 4; ++e) acc += bf_lo(v[e]) * wr[c + 2 * e] + bf_hi(v[e]) * wr[c + 2 * e + 1];
-    }
+    for (; c < C; c += 8) acc = oc_piece(*reinterpret_cast<const u32x4*>(xr + c), wr + c, acc);
     return acc;
 }
 static inline __host__ __device__ int oc_pitch(int C) { return 16 * ((C / 8) | 1); }
@@ -408,90 +406,37 @@ __global__ __launch_bounds__(OC_ROWS) void codec_out_conv_kernel(const uint16_t*
                                                                  float* __restrict__ wav, int T, int C, int taps) {
     extern __shared__ __attribute__((aligned(16))) uint8_t rows[];
     const int t0 = blockIdx.x * OC_ROWS, r0 = t0 - (taps - 1), ch = C / 8, pitch = oc_pitch(C), total = (min(OC_ROWS, T - t0) + taps - 1) * ch;
-#pragma unroll 8
-    for (int id = threadIdx.x; id < total; id += OC_ROWS) {
-        const int lr = id / ch, lc = id - lr * ch;
-        if (r0 + lr >= 0) *reinterpret_cast<u32x4*>(rows + lr * pitch + lc * 16) = *reinterpret_cast<const u32x4*>(x + (size_t)(r0 + lr) * C + lc * 8);
+    float* wl = reinterpret_cast<float*>(rows + (OC_ROWS + taps - 1) * pitch);
+    constexpr int P = 16;                                 // pieces of a thread in flight: 7 taps of 96 channels are 13
+    for (int first = 0; first < total; first += P * OC_ROWS) {
+        const int base = first + threadIdx.x;
+        u32x4 v[P];
+#pragma unroll
+        for (int i = 0; i < P; ++i) {                     // (rows in front of the first: its first piece, not used; past the last: that one again)
+            const int64_t at = (int64_t)r0 * ch + min(base + i * OC_ROWS, total - 1);
+            v[i] = *reinterpret_cast<const u32x4*>(x + (at < 0 ? 0 : at) * 8);
+        }
+        if (first == 0)
+            for (int i = threadIdx.x; i < taps * C; i += OC_ROWS) wl[i] = w[i];
+#pragma unroll
+        for (int i = 0; i < P; ++i) {
+            const int id = base + i * OC_ROWS, lr = id / ch;
+            if (id < total) *reinterpret_cast<u32x4*>(rows + lr * pitch + (id - lr * ch) * 16) = v[i];
+        }
     }
     __syncthreads();
     const int t = t0 + threadIdx.x;
     if (t >= T) return;
     float acc = bias;
     for (int j = 0; j < taps; ++j)
-        if (t - (taps - 1) + j >= 0) acc = oc_row(reinterpret_cast<const uint16_t*>(rows + (threadIdx.x + j) * pitch), w + j * C, C, acc);
-    wav[t] = fminf(fmaxf(acc, -1.0f), 1.0f);
-}
-
-// Up to eight taps, rows of whole 32-channel steps: every row times every tap on the matrix cores, the fp32 weights as three bf16 terms whose sum they are (16 columns: the
-// taps' first terms | their second; 16 more for the third), then a sample adds up `taps` numbers out of LDS.  A lane's operand is 16 bytes of a row: rows are read once, in place,
-// and nothing waits for weights 32 at a time (21.1 us of the decode of 50 frames, 7.2 so).  Closer than a chain of 672 fp32 additions.  A sample
-// that is no finite number is added up as in the kernel above: a term of an infinite weight or row is no number here.
-#define OM_ROWS 256
-template <int KS>
-__global__ __launch_bounds__(256) void codec_out_mfma_kernel(const uint16_t* __restrict__ x, const float* __restrict__ w, float bias, float* __restrict__ wav, int T, int taps) {
-    constexpr int C = 32 * KS, TILES = OM_ROWS / 64;
-    __shared__ float part[OM_ROWS][9];
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, c = lane & 15, q = lane >> 4;
-    const int outs = OM_ROWS - (taps - 1), t0 = blockIdx.x * outs, r0 = t0 - (taps - 1);
-    u32x4 X[TILES][KS];
-#pragma unroll
-    for (int i = 0; i < TILES; ++i) {
-        const int r = r0 + (wave * TILES + i) * 16 + c;
-#pragma unroll
-        for (int k = 0; k < KS; ++k) {
-            X[i][k] = *reinterpret_cast<const u32x4*>(x + (size_t)min(max(r, 0), T - 1) * C + 32 * k + 8 * q);
-            if (r < 0) X[i][k] = u32x4{0, 0, 0, 0};
-        }
-    }
-    u32x4 W0[KS], W1[KS];
-    const int tap = c & 7;
-#pragma unroll
-    for (int k = 0; k < KS; ++k) {
-        const float* wp = w + (size_t)min(tap, taps - 1) * C + 32 * k + 8 * q;
-        const f32x4 a = *reinterpret_cast<const f32x4*>(wp), b = *reinterpret_cast<const f32x4*>(wp + 4);
-        const float v[8] = {a[0], a[1], a[2], a[3], b[0], b[1], b[2], b[3]};
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-            const float w0 = tap < taps ? v[2 * e] : 0.f, w1 = tap < taps ? v[2 * e + 1] : 0.f;
-            const uint32_t hi = pack_bf2(w0, w1);
-            const float m0 = w0 - bf_lo(hi), m1 = w1 - bf_hi(hi);
-            const uint32_t mid = pack_bf2(m0, m1);
-            W0[k][e] = c < 8 ? hi : mid;
-            W1[k][e] = c < 8 ? pack_bf2(m0 - bf_lo(mid), m1 - bf_hi(mid)) : 0u;
-        }
-    }
-    auto mul = [](u32x4 a, u32x4 b, f32x4 d) { return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, a), __builtin_bit_cast(bf16x8, b), d, 0, 0, 0); };
-#pragma unroll
-    for (int i = 0; i < TILES; ++i) {
-        f32x4 d0 = {0.f, 0.f, 0.f, 0.f}, d1 = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-        for (int k = 0; k < KS; ++k) {
-            d0 = mul(X[i][k], W0[k], d0);
-            d1 = mul(X[i][k], W1[k], d1);
-        }
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-            const float mid = __shfl_xor(d0[e], 8);
-            if (c < 8) part[(wave * TILES + i) * 16 + 4 * q + e][c] = (d1[e] + mid) + d0[e];
-        }
-    }
-    __syncthreads();
-    const int t = t0 + threadIdx.x;
-    if ((int)threadIdx.x >= outs || t >= T) return;
-    float acc = bias;
-    for (int j = 0; j < taps; ++j) acc += part[threadIdx.x + j][j];
-    if (!(fabsf(acc) < INFINITY)) {
-        acc = bias;
-        for (int j = 0; j < taps; ++j)
-            if (t - (taps - 1) + j >= 0) acc = oc_row(x + (size_t)(t - (taps - 1) + j) * C, w + j * C, C, acc);
-    }
+        if (t - (taps - 1) + j >= 0) acc = oc_row(reinterpret_cast<const uint16_t*>(rows + (threadIdx.x + j) * pitch), wl + j * C, C, acc);
     wav[t] = fminf(fmaxf(acc, -1.0f), 1.0f);
 }
 
 // rows too wide for LDS: straight from memory, the weights in LDS
 __global__ __launch_bounds__(256) void codec_out_conv_wide_kernel(const uint16_t* __restrict__ x, const float* __restrict__ w, float bias,
                                                                   float* __restrict__ wav, int T, int C, int taps) {
-    extern __shared__ float wl[];                         // [taps * C]
+    extern __shared__ __attribute__((aligned(16))) float wl[];                         // [taps * C]
     for (int i = threadIdx.x; i < taps * C; i += blockDim.x) wl[i] = w[i];
     __syncthreads();
     const int t = blockIdx.x * blockDim.x + threadIdx.x;
@@ -504,18 +449,15 @@ __global__ __launch_bounds__(256) void codec_out_conv_wide_kernel(const uint16_t
 
 extern "C" int omni_codec_out_conv(const void* x, const float* w, float bias, float* wav, int T, int C, int taps, void* stream) {
     OMNI_CHECK_ARG(x && w && wav && T > 0 && C > 0 && C % 8 == 0 && taps > 0 && taps * C * 4 <= 64 * 1024, "omni_codec_out_conv: T=%d C=%d taps=%d", T, C, taps);
-    const int64_t rows = (int64_t)(OC_ROWS + taps - 1) * oc_pitch(C);
-    if (taps <= 8 && C % 32 == 0 && C <= 256 && aligned16({x, w})) {
-        const dim3 grid((T + OM_ROWS - taps) / (OM_ROWS - taps + 1)), block(256);
-        switch (C / 32) {
-#define OM(K) case K: hipLaunchKernelGGL(codec_out_mfma_kernel<K>, grid, block, 0, (hipStream_t)stream, (const uint16_t*)x, w, bias, wav, T, taps); break;
-            OM(1) OM(2) OM(3) OM(4) OM(5) OM(6) OM(7) OM(8)
-#undef OM
+    const int rows = (OC_ROWS + taps - 1) * oc_pitch(C), weights = taps * C * (int)sizeof(float);
+    if (rows <= 64 * 1024) {
+        if (rows + weights > 64 * 1024) {
+            static const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(codec_out_conv_kernel), hipFuncAttributeMaxDynamicSharedMemorySize, 128 * 1024);
+            if (e != hipSuccess) { omni_set_error("omni_codec_out_conv: LDS attribute: %s", hipGetErrorString(e)); return OMNI_EHIP; }
         }
-    } else if (rows <= 64 * 1024)
-        hipLaunchKernelGGL(codec_out_conv_kernel, dim3((T + OC_ROWS - 1) / OC_ROWS), dim3(OC_ROWS), (size_t)rows, (hipStream_t)stream,
+        hipLaunchKernelGGL(codec_out_conv_kernel, dim3((T + OC_ROWS - 1) / OC_ROWS), dim3(OC_ROWS), (size_t)(rows + weights), (hipStream_t)stream,
                            (const uint16_t*)x, w, bias, wav, T, C, taps);
-    else
+    } else
         hipLaunchKernelGGL(codec_out_conv_wide_kernel, dim3((T + 255) / 256), dim3(256), taps * C * sizeof(float), (hipStream_t)stream,
                            (const uint16_t*)x, w, bias, wav, T, C, taps);
     OMNI_CHECK_LAUNCH("omni_codec_out_conv");

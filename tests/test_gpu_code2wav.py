@@ -326,9 +326,9 @@ def test_last_conv(C, T, taps):
 
 
 @pytest.mark.parametrize("C,T,taps", [(32, 1, 8), (32, 249, 8), (64, 251, 7), (96, 250, 7), (128, 1000, 2), (160, 255, 1), (192, 256, 3), (224, 17, 7), (256, 499, 8)])
-def test_last_conv_on_the_matrix_cores(C, T, taps):
-    """Every width that the kernel of matrix products takes, blocks of 256 - (taps - 1) samples and their edges; the bound of test_last_conv.  A row or a weight that is
-    no finite number reaches its own samples alone, as what the plain sum makes of it (an infinity times a weight is an infinity, not what its terms add up to)."""
+def test_last_conv_of_rows_that_are_no_numbers(C, T, taps):
+    """Widths of whole 32-channel steps, blocks of samples and their edges; the bound of test_last_conv.  A row or a weight that is no finite number reaches its own samples
+    alone, as what the sum makes of it, and no sample whose tap on it lies in front of the first row."""
     from ht_vllm_omni_amd import _lib as L
     g = torch.Generator().manual_seed(C + T)
     x, w = torch.randn(T, C, generator=g).to(torch.bfloat16), torch.randn(taps, C, generator=g) * (0.3 / (taps * C) ** 0.5)
@@ -361,6 +361,23 @@ def test_last_conv_on_the_matrix_cores(C, T, taps):
     ref, got = sums(x, wb), run(x, wb)
     keep = torch.isfinite(ref)
     assert torch.equal(got[~keep], torch.where(torch.isnan(ref), -torch.ones_like(ref), ref.clamp(-1, 1)).float()[~keep])
+    wf = wb.clone()
+    wf[0, 0] = 0.0                                         # (the finite samples have no tap 0)
+    assert int(keep.sum()) >= min(taps - 1, T)
+    assert bool(((got.double() - ref.clamp(-1, 1)).abs() <= sums(x, wf, True) * (taps * C * 2.0 ** -24))[keep].all())
+
+
+@pytest.mark.parametrize("C,T,taps", [(32, 249, 8), (96, 1000, 7), (256, 300, 3), (96, 5, 1)])
+def test_last_conv_adds_in_one_order_at_every_width(C, T, taps):
+    """Eight more channels of zeros change the width, and with it what a piece of a row is, but no bit of a sample."""
+    from ht_vllm_omni_amd import _lib as L
+    g = torch.Generator().manual_seed(C + T)
+    x, w, outs = torch.randn(T, C, generator=g).to(torch.bfloat16), torch.randn(taps, C, generator=g) * (0.3 / (taps * C) ** 0.5), []
+    for more in (0, 8):
+        xd, wd, wav = (torch.nn.functional.pad(x, (0, more)).cuda(), torch.nn.functional.pad(w, (0, more)).cuda(), torch.full((T + 4,), 7.0, device="cuda"))
+        L.check(L.load().omni_codec_out_conv(xd.data_ptr(), wd.data_ptr(), 0.0625, wav.data_ptr(), T, C + more, taps, L.current_stream()), "omni_codec_out_conv")
+        outs.append(wav)
+    assert torch.equal(*outs)
 
 
 @pytest.mark.parametrize("C,T,ldx,taps", [(4, 1, 4, 7), (252, 9, 256, 7), (1024, 3, 1024, 7), (1020, 40, 1028, 7), (256, 20, 257, 7), (130, 20, 130, 7), (64, 30, 64, 5)])

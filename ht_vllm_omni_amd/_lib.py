@@ -115,6 +115,7 @@ ACT_NONE, ACT_XIELU, ACT_RELU2, ACT_GELU_MUL = 0, 1, 2, 3            # OMNI_ACT_
 GATHER_ROWS = 16                                                     # rows of an omni_latent_gather item
 REC_CHUNK, REC_MAX_DIM = 128, 256                                    # OMNI_REC_*
 STREAM_MAX_SPLITS, STREAM_MAX_ROWS = 4, 64
+TILE_HINT_FEW, TILE_FEW_ROWS = 17, 64            # omni_tile_gemm.tile_hint: a wave per 16 x 16, up to so many rows
 STREAM_JOINED_ROWS = 4                                               # most rows of a product that makes them
 STREAM_LATENT_ROWS, STREAM_LATENT_WIDTH = 2, 3072                     # ... of latents
 WINDOW_MFMA_DIM = 256                                                # widest heads of omni_window_attn's matrix-core kernels
@@ -250,7 +251,6 @@ DECODER_SIGNATURES = {
     "omni_gemm_f32": (i32, [vp, i32, i64, vp, i64, vp, i32, i64, i32, i32, i32, i32, i32, f32, f32, vp]),
     "omni_gemm_stream": (i32, [vp, vp, vp, i32, i32, i32, i32, i32, f32, f32, i32, vp]),
     "omni_gemm_stream_splits": (i32, [i32, i32, i32]),
-    "omni_gemm_stream_plain": (i32, [vp, i32, vp, vp, i32, i32, i32, i32, vp]),
     "omni_gemm_stream_rows": (i32, [vp, vp, vp, i32, i32, i32, C.POINTER(RowTable), i32, vp]),
     "omni_gemm_stream_joined": (i32, [C.POINTER(StreamRows), vp, vp, i32, i32, i32, f32, f32, C.POINTER(RowTable), i32, vp]),
     "omni_gemm_stream_joins": (i32, [i32, i32, i32, i32, i32]),

@@ -36,7 +36,7 @@ BF16 = torch.bfloat16
 # Up to so many frames the transformer's products that join the stream may leave partial sums (their tiles are fewer than the compute units: 50 rows x 1024 columns
 # are 64).  Measured, us, the decode of 12 frames 890 / 870, 30 989 / 966, 50 1087 / 1062, 75 1703 / 1684, 325 4407 / 4376; of 160 and 230 the same
 SPLIT_FRAMES = 512
-STREAM_FRAMES = 32                   # ... and take the weight-streaming product (Code2WavDecoder.forward)
+FEW_FRAMES = 32                      # Code2WavDecoder.forward: products by a wave per 16 x 16
 
 
 @dataclass
@@ -118,7 +118,7 @@ class Code2WavDecoder:
                  operand_precision: str = "bf16"):
         if not torch.cuda.is_available():
             raise L.OmniError("Code2WavDecoder needs an MI355X (torch.cuda unavailable); there is no CPU fallback")
-        self.lib, self.streams = L.load(), L.load_decoder()
+        self.lib = L.load()
         self.cfg = cfg if isinstance(cfg, Code2WavConfig) else Code2WavConfig.from_dict(cfg)
         self.cfg.check()
         self.device = torch.device(device)
@@ -281,29 +281,18 @@ class Code2WavDecoder:
         few = T <= SPLIT_FRAMES and H <= 1024
         parts = torch.empty(L.STREAM_MAX_SPLITS, T, H, dtype=torch.float32, device=dev) if few else None
 
-        # Few frames: W streams past all rows at once, instead of tiles of 16 rows pulling it again.  Us, tile / streamed, frames x columns x K: 12 x 3072 x 1024
-        # 5.1 / 3.6, x 1024 x 1024 3.7 / 2.8, x 1024 x 3072 4.7 / 3.7; 25: 5.2 / 4.5, 3.8 / 3.1, 4.8 / 4.2; 33: 5.3 / 5.3, 3.9 / 3.3, 5.0 / 4.9; 50: 5.3 / 6.1,
-        # 3.9 / 3.5, 5.1 / 5.6 -- every workgroup's pull of all rows counts then, but where columns and K are both few
-        def streams(n, k):
-            return T <= STREAM_FRAMES or (T <= L.STREAM_MAX_ROWS and n * k <= 1024 * 1024)
-
-        def streamed(g, x, out, kind):
-            L.check(self.streams.omni_gemm_stream_plain(x.data_ptr(), x.stride(0), g.w.data_ptr(), out.data_ptr(), T, g.n, x.shape[1], kind, st),
-                    "omni_gemm_stream_plain", self.streams)
-            return out
+        # A product of few frames by a wave per 16 x 16, the same bits (its table is at the kernel): up to 32 frames; up to 64 where columns and K are both few, as every
+        # column's waves pull the rows again (33 frames, us, the rule's tile / this: 3072 x 1024 5.7 / 5.7, 1024 x 3072 5.3 / 5.3, 1024 x 1024 4.1 / 3.2)
+        def hint(n, k):
+            return L.TILE_HINT_FEW if T <= FEW_FRAMES or (T <= L.TILE_FEW_ROWS and n * k <= 1024 * 1024) else 0
 
         def joins(g, x):
             nonlocal behind
-            if few and streams(H, x.shape[1]):
-                n = self.streams.omni_gemm_stream_splits(T, H, x.shape[1])
-                streamed(g, x, parts[:n], L.STREAM_F32)
-                behind = n, g.scale
-                return
             n = lib.omni_gemm_tile_splits(T, H, x.shape[1]) if few else 1
             if n == 1:
                 g(x, resid=h, out_f32=h, want="f")
             else:
-                ops.gemm_tile(x, g.w, out_f32=parts[:n], want="f", splits=n)
+                ops.gemm_tile(x, g.w, out_f32=parts[:n], want="f", splits=n, tile_hint=hint(H, x.shape[1]))
                 behind = n, g.scale
 
         def norm(w):
@@ -317,8 +306,7 @@ class Code2WavDecoder:
                 behind = None
         for lw in self.layers:
             norm(lw["ln1"])
-            n = lw["qkv"].n
-            qkv = streamed(lw["qkv"], a, torch.empty(T, n, dtype=BF16, device=dev), L.STREAM_BF16) if streams(n, H) else lw["qkv"](a)
+            qkv = lw["qkv"](a, tile_hint=hint(lw["qkv"].n, H))
             self._check(lib.omni_codec_rope(qkv.data_ptr(), qkv.stride(0), T, nh, nkv, hd, float(c.rope_theta), st), "omni_codec_rope")
             self._check(lib.omni_codec_window_attn(qkv.data_ptr(), qkv.stride(0), attn.data_ptr(), attn.stride(0), T, nh, nkv, hd,
                                                    c.sliding_window, hd ** -0.5, st), "omni_codec_window_attn")

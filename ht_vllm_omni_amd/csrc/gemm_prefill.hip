@@ -893,6 +893,47 @@ static int launch_mid_of(int geom, const TileArgs& a, hipStream_t st, int groups
     return OMNI_EINVAL;
 }
 
+// ---- up to 64 rows of a plain product (tile_hint 17): a wave alone owns 16 rows x 16 columns of one run of K and takes both operands straight into registers, P steps in flight.  One
+// chain of MFMAs over K as in every tile: the same bits.  What bounds it: trips to memory, 24 KB of W a wave in flight (8 steps 5.1 of the first, 16 4.4, 32 4.3), and the rows, which
+// every wave of a column reads for itself.  Us, weights out of HBM, the rule's tile / this, rows x columns x K: 12 x 3072 x 1024 5.6 / 4.0, 12 x 1024 x 1024 in four runs of K 4.0 / 2.7,
+// 12 x 1024 x 3072 in four 5.1 / 3.8; 25 rows 5.6 / 5.1, 4.1 / 3.0, 5.3 / 4.6; 33 5.7 / 5.7, 4.1 / 3.2, 5.3 / 5.3; 64 5.8 / 6.6, 4.4 / 3.8, 5.5 / 6.9.
+template <bool F32>
+__global__ __launch_bounds__(64) void gemm_few_kernel(const TileArgs a) {
+    constexpr int P = 24;
+    const int lane = threadIdx.x, c = lane & 15, q = lane >> 4, all = a.K >> 5;
+    const int s0 = (int)blockIdx.z * all / a.splits, n = ((int)blockIdx.z + 1) * all / a.splits - s0;
+    const int m = blockIdx.y * 16 + c, col = blockIdx.x * 16 + 4 * q;
+    const u32x4* wp = reinterpret_cast<const u32x4*>(a.W + ((size_t)blockIdx.x * all + s0) * 512 + lane * 8);
+    const u32x4* xp = reinterpret_cast<const u32x4*>(a.x + (size_t)min(m, a.M - 1) * a.ldx + s0 * 32 + 8 * q);      // rows past M: the last one again, not stored
+    u32x4 W[P], X[P];
+    auto load = [&](int d, int s) {
+        W[d] = __builtin_nontemporal_load(wp + s * 64);
+        X[d] = xp[s * 4];
+    };
+#pragma unroll
+    for (int d = 0; d < P; ++d)
+        if (d < n) load(d, d);
+    f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+    for (int s = 0; s < n; s += P)
+#pragma unroll
+        for (int d = 0; d < P; ++d) {
+            if (s + d >= n) break;
+            acc = tg_mfma(W[d], X[d], acc);
+            if (s + d + P < n) load(d, s + d + P);
+        }
+    if (m >= a.M) return;
+    if (F32) *reinterpret_cast<f32x4*>(a.out_f32 + blockIdx.z * a.slab_stride + (size_t)m * a.ldf + col) = acc;
+    else *reinterpret_cast<uint2*>(a.out + (size_t)m * a.ldo + col) = make_uint2(pack_bf2(acc[0], acc[1]), pack_bf2(acc[2], acc[3]));
+}
+
+static int launch_few(const TileArgs& a, bool f32, hipStream_t st) {
+    const dim3 grid(a.N / 16, (a.M + 15) / 16, a.splits), block(64);
+    if (f32) hipLaunchKernelGGL((gemm_few_kernel<true>), grid, block, 0, st, a);
+    else hipLaunchKernelGGL((gemm_few_kernel<false>), grid, block, 0, st, a);
+    OMNI_CHECK_LAUNCH("omni_gemm_tile");
+    return OMNI_OK;
+}
+
 // ---- which tile.  Every geometry accumulates in the same order, so the choice moves time only.  A grid costs its rounds: 256 workgroups run at a time,
 // one per CU (512 where two fit), and a round costs a prologue and an epilogue (`round`) and the slices of K (`slice`, per 64-deep slice).  What a slice
 // costs is what a CU takes in -- 60 - 90 GB/s of operands in every geometry (a slice of the 32 x 64 tile is 12 KB in 0.17 us, of the 256 x 256 tile
@@ -979,7 +1020,7 @@ extern "C" int omni_gemm_tile(const omni_tile_gemm* g, void* stream) {
     OMNI_CHECK_ARG(g->act != OMNI_TILE_ACT_SILU_SIGMOID || (g->act_cols >= 0 && g->act_cols % 4 == 0), "omni_gemm_tile: act_cols=%d (%% 4)", g->act_cols);
     OMNI_CHECK_ARG(g->act != OMNI_TILE_ACT_GELU_MUL || (g->mul_table && g->mul_ids && g->mul_rows > 0 && g->mul_ld >= g->N && g->mul_ld % 8 == 0 && g->out && !g->out2 && !g->resid &&
                                                         g->groups <= 1), "omni_gemm_tile: the row table takes ids, mul_ld >= N (%% 8), a bf16 output and one group");
-    OMNI_CHECK_ARG(g->tile_hint >= 0 && g->tile_hint <= 16, "omni_gemm_tile: tile_hint=%d", g->tile_hint);
+    OMNI_CHECK_ARG(g->tile_hint >= 0 && g->tile_hint <= 17, "omni_gemm_tile: tile_hint=%d", g->tile_hint);
     OMNI_CHECK_ARG(g->tile_hint < 3 || g->tile_hint > 7 || g->N % 256 == 0, "omni_gemm_tile: tile_hint=%d needs N %% 256 == 0", g->tile_hint);
     OMNI_CHECK_ARG(!gu8 || (g->out && !g->resid && !g->out2 && !g->out_f32), "omni_gemm_tile: SiLU-mul takes out only");
     OMNI_CHECK_ARG(!g->out2 || (g->snake_alpha && g->snake_inv_beta), "omni_gemm_tile: out2 needs the snake parameters");
@@ -1020,10 +1061,16 @@ extern "C" int omni_gemm_tile(const omni_tile_gemm* g, void* stream) {
     OMNI_CHECK_ARG(g->k_splits >= 0 && g->k_splits <= 4 && (g->k_splits <= 1 || (tile_epi(a) == EPI_F32 && groups == 1 && g->k_splits <= g->K / 32 &&
                    g->slab_stride >= (int64_t)(g->M - 1) * g->ldf + N && g->slab_stride % 4 == 0)), "omni_gemm_tile: k_splits=%d (<= K / 32; one group, fp32 output alone)", g->k_splits);
     a.splits = g->k_splits > 1 ? g->k_splits : 1; a.slab_stride = g->slab_stride;
-    // tile_hint: 1 the large lockstep tiles, 2 and 8 ... 16 the mid-size ones, 3 / 4 lockstep and 5 / 6 / 7 two-group at 224 / 192 and 256 / 224 / 192 rows
+    // tile_hint: 1 the large lockstep tiles, 2 and 8 ... 16 the mid-size ones, 17 a wave per 16 x 16, 3 / 4 lockstep and 5 / 6 / 7 two-group at 224 / 192 and 256 / 224 / 192 rows
     const bool plain = groups == 1 && !g->group_rows && seg_len == g->K && g->row_off == 0;
     OMNI_CHECK_ARG(g->tile_hint < 5 || g->tile_hint > 7 || plain, "omni_gemm_tile: tile_hint=%d (two-group tile) takes a plain GEMM", g->tile_hint);
     OMNI_CHECK_ARG(a.splits == 1 || g->tile_hint == 0 || g->tile_hint == 2 || g->tile_hint >= 5, "omni_gemm_tile: tile_hint=%d takes no k_splits", g->tile_hint);
+    if (g->tile_hint == 17) {
+        const int epi = tile_epi(a);
+        OMNI_CHECK_ARG(plain && !gu8 && (epi == EPI_PLAIN || epi == EPI_F32) && g->M <= 64 && g->M <= g->x_rows && ((uintptr_t)g->x & 15) == 0,
+                       "omni_gemm_tile: tile_hint=17 takes a plain product of up to 64 rows, x aligned to 16 bytes, bf16 or fp32 output alone (M=%d)", g->M);
+        return launch_few(a, epi == EPI_F32, st);
+    }
     int kind = KIND_LARGE, geom = 256;
     switch (g->tile_hint) {
         case 0: {

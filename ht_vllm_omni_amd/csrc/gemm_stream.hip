@@ -22,7 +22,6 @@ struct StreamArgs {
     float ap, an;
     int act;
     omni_row_table rt;
-    int ldx;                                              // XR: elements from one row of x to the next
 };
 
 // the waves' sums added up in a fixed order, and out
@@ -60,9 +59,7 @@ __device__ __forceinline__ void gs_store(const StreamArgs& a, const f32x4* part,
 
 // P: k-steps in flight per wave: 2 on a grid that fills the chip (4 measured the same or slower at 1 .. 64 rows).
 // grid.z: groups of MT row tiles (more than one where the columns alone leave CUs idle)
-// XR: rows of x as they lie, 64 bytes of 16 rows a piece instead of 1 KB: dearer the more rows (us, 3072 x 1024, fragment-major / rows: 12 rows 3.6 / 3.6, 25 4.1 / 4.5,
-// 50 5.1 / 6.1), and no launch or producer has to lay them out.
-template <int MT, int NT, int KIND, int P, bool XR = false>
+template <int MT, int NT, int KIND, int P>
 __global__ __launch_bounds__(GS_THREADS) void gemm_stream_kernel(const StreamArgs a) {
     extern __shared__ __attribute__((aligned(16))) f32x4 part[];      // [wave][NT * MT][lane]
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
@@ -73,9 +70,7 @@ __global__ __launch_bounds__(GS_THREADS) void gemm_stream_kernel(const StreamArg
 #pragma unroll
     for (int j = 0; j < NT; ++j) wp[j] = a.W + ((size_t)(blockIdx.x * NT + j) * a.nsteps + k0 + wave) * 512 + lane * 8;
 #pragma unroll
-    for (int i = 0; i < MT; ++i)                          // rows and row tiles past M: re-read, discarded
-        xp[i] = a.x + (XR ? (size_t)min((m0 + i) * 16 + (lane & 15), a.M - 1) * a.ldx + (k0 + wave) * 32 + 8 * (lane >> 4)
-                          : ((size_t)min(m0 + i, ((a.M + 15) >> 4) - 1) * a.nsteps + k0 + wave) * 512 + lane * 8);
+    for (int i = 0; i < MT; ++i) xp[i] = a.x + ((size_t)min(m0 + i, ((a.M + 15) >> 4) - 1) * a.nsteps + k0 + wave) * 512 + lane * 8;      // row tiles past M: re-read, discarded
     f32x4 acc[NT][MT];
 #pragma unroll
     for (int j = 0; j < NT; ++j)
@@ -87,7 +82,7 @@ __global__ __launch_bounds__(GS_THREADS) void gemm_stream_kernel(const StreamArg
 #pragma unroll
         for (int j = 0; j < NT; ++j) W[d][j] = ld16_nt(wp[j] + (size_t)s * (GS_WAVES * 512));
 #pragma unroll
-        for (int i = 0; i < MT; ++i) X[d][i] = ld16(xp[i] + (size_t)s * (GS_WAVES * (XR ? 32 : 512)));
+        for (int i = 0; i < MT; ++i) X[d][i] = ld16(xp[i] + (size_t)s * (GS_WAVES * 512));
     };
     auto mul = [&](int d) {
 #pragma unroll
@@ -327,14 +322,14 @@ static void gs_policy(int M, int N, int nsteps, bool slabs, int* nt, int* splits
     }
 }
 
-template <int MT, int NT, int KIND, int P, bool XR = false>
+template <int MT, int NT, int KIND, int P>
 static int gs_launch(const StreamArgs& a, int splits, hipStream_t st) {
     constexpr int LDS = GS_WAVES * NT * MT * 1024;
     if (LDS > 64 * 1024) {
-        static const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(gemm_stream_kernel<MT, NT, KIND, P, XR>), hipFuncAttributeMaxDynamicSharedMemorySize, LDS);
+        static const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(gemm_stream_kernel<MT, NT, KIND, P>), hipFuncAttributeMaxDynamicSharedMemorySize, LDS);
         if (e != hipSuccess) { omni_set_error("omni_gemm_stream: LDS attribute: %s", hipGetErrorString(e)); return OMNI_EHIP; }
     }
-    hipLaunchKernelGGL((gemm_stream_kernel<MT, NT, KIND, P, XR>), dim3(a.N / (16 * NT), splits, ((a.M + 15) / 16 + MT - 1) / MT), dim3(GS_THREADS), LDS, st, a);
+    hipLaunchKernelGGL((gemm_stream_kernel<MT, NT, KIND, P>), dim3(a.N / (16 * NT), splits, ((a.M + 15) / 16 + MT - 1) / MT), dim3(GS_THREADS), LDS, st, a);
     OMNI_CHECK_LAUNCH("omni_gemm_stream");
     return OMNI_OK;
 }
@@ -345,7 +340,6 @@ extern "C" int omni_gemm_stream_splits(int M, int N, int K) {
     return s;
 }
 
-template <bool XR = false>
 static int gs_run(StreamArgs a, int kind, bool one, hipStream_t st) {
     int nt, splits;
     gs_policy(a.M, a.N, a.nsteps, kind == GS_F32 && !one, &nt, &splits);
@@ -357,15 +351,13 @@ static int gs_run(StreamArgs a, int kind, bool one, hipStream_t st) {
     while (mt > 1 && a.N / 16 / nt * splits * (((a.M + 15) / 16 + mt / 2 - 1) / (mt / 2)) <= 256) mt /= 2;
     // a narrow product (a side input's gate), more steps in flight
     if (a.N / 16 * splits <= 32) {
-        if (kind == GS_F32) return gs_launch<1, 1, GS_F32, 4, XR>(a, splits, st);
-        if (XR || kind == GS_BF16) return gs_launch<1, 1, GS_BF16, 4, XR>(a, splits, st);
-        return gs_launch<1, 1, GS_ACT, 4>(a, splits, st);
+        if (kind == GS_F32) return gs_launch<1, 1, GS_F32, 4>(a, splits, st);
+        return kind == GS_BF16 ? gs_launch<1, 1, GS_BF16, 4>(a, splits, st) : gs_launch<1, 1, GS_ACT, 4>(a, splits, st);
     }
-#define GS(MT_, NT_, K_) if (mt == MT_ && nt == NT_ && kind == K_) return gs_launch<MT_, NT_, K_, 2, XR>(a, splits, st);
+#define GS(MT_, NT_, K_) if (mt == MT_ && nt == NT_ && kind == K_) return gs_launch<MT_, NT_, K_, 2>(a, splits, st);
 #define GS_NT(NT_, K_) GS(1, NT_, K_) GS(2, NT_, K_) GS(4, NT_, K_)
 #define GS_ALL(K_) GS_NT(1, K_) GS_NT(2, K_) GS_NT(3, K_) GS_NT(4, K_)
-    GS_ALL(GS_F32) GS_ALL(GS_BF16)
-    if constexpr (!XR) { GS_ALL(GS_ACT) }
+    GS_ALL(GS_F32) GS_ALL(GS_BF16) GS_ALL(GS_ACT)
     omni_set_error("omni_gemm_stream: no tile for M=%d N=%d", a.M, a.N);
     return OMNI_EINVAL;
 }
@@ -380,14 +372,6 @@ extern "C" int omni_gemm_stream(const void* x, const void* w, void* out, int M, 
     OMNI_CHECK_ARG(kind >= 0 && kind <= 3 && (!out_frag || kind != GS_F32), "omni_gemm_stream: kind=%d out_frag=%d", kind, out_frag);
     StreamArgs a{(const uint16_t*)x, (const uint16_t*)w, out, M, N, K / 32, 0, out_frag, act_p, act_n, kind == 3 ? OMNI_ACT_RELU2 : OMNI_ACT_XIELU, {}};
     return gs_run(a, kind == 3 ? (int)GS_ACT : kind, one != 0, (hipStream_t)stream);
-}
-
-extern "C" int omni_gemm_stream_plain(const void* x, int ldx, const void* w, void* out, int M, int N, int K, int kind, void* stream) {
-    constexpr int out_frag = 0;
-    GS_CHECK("omni_gemm_stream_plain");
-    OMNI_CHECK_ARG((kind == GS_F32 || kind == GS_BF16) && ldx >= K && ldx % 8 == 0 && ((uintptr_t)x & 15) == 0, "omni_gemm_stream_plain: kind=%d ldx=%d (rows of 16-byte pieces)", kind, ldx);
-    StreamArgs a{(const uint16_t*)x, (const uint16_t*)w, out, M, N, K / 32, 0, 0, 0.f, 0.f, OMNI_ACT_XIELU, {}, ldx};
-    return gs_run<true>(a, kind, false, (hipStream_t)stream);
 }
 
 extern "C" int omni_gemm_stream_rows(const void* x, const void* w, void* out, int M, int N, int K, const omni_row_table* rt, int out_frag, void* stream) {

@@ -109,8 +109,6 @@ int omni_gemm_f32_rows(const float* x, int ldx, const float* w, float* out, int 
 int omni_gemm_stream(const void* x, const void* w, void* out, int M, int N, int K, int kind, int one, float act_p, float act_n, int out_frag, void* stream);
 int omni_gemm_stream_rows(const void* x, const void* w, void* out, int M, int N, int K, const omni_row_table* rt, int out_frag, void* stream);
 int omni_gemm_stream_splits(int M, int N, int K);
-/* ... of x row-major, ldx elements a row, 16-byte aligned: kind 0 (all of its partial sums) or 1, the same sums bit for bit */
-int omni_gemm_stream_plain(const void* x, int ldx, const void* w, void* out, int M, int N, int K, int kind, void* stream);
 /* omni_gemm_stream of a few rows that it makes itself, in one launch, bit for bit:
  *   _joined:  the rows omni_stream_rows_run would leave in h_out (not written here; x_out is), K = wp: up to OMNI_STREAM_JOINED_ROWS of wp <= 1024, 2 of wp <=
  *             2048.  kind 0, 2 or 3; rt != NULL: the row table's activation; with mu: kind 0

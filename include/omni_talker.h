@@ -179,7 +179,7 @@ typedef struct omni_tile_gemm {
     int tile_hint;   /* 0: automatic; 1: the large output tiles (256 x 256 ...); 2: the tile of 64 rows x 128 columns;
                         3 / 4: 256 columns x 224 / 192 rows (N % 256 == 0); 5 / 6 / 7: the two-group form of the 256-column tile at
                         256 / 224 / 192 rows (plain GEMMs only); 8 ... 13: 32 x 32, 32 x 64, 64 x 64, 128 x 128, 256 x 128, 128 x 256; 14 ... 16: 96 x 64, 192 x 128, 96 x 128
-                        rows x columns.  Same results whatever the tile */
+                        rows x columns; 17: up to 64 rows, a wave per 16 x 16 (plain GEMMs, x 16-byte aligned, bf16 or fp32 out alone).  Same results whatever the tile */
     /* grouped (batched) launch, groups > 1: group g computes out rows [g * out_group_rows, + M) from x rows [g * x_group_rows, + M)
      * and the matrix w + g * w_group_elems (elements) -- the expert-sorted [E, cap, H] batch of the MoE prefill against the
      * decode step's per-expert fragment-major weights (replaces the batched GEMMs vLLM's FusedMoE issues under

@@ -235,6 +235,32 @@ def test_a_waveform_is_the_same_with_and_without_the_streams(T):
     assert torch.equal(dec.forward(codes), dec.forward(codes, {}))
 
 
+@pytest.mark.parametrize("T,more", [(1, 9), (12, 20), (32, 48), (50, 59)])
+def test_few_frames_are_the_first_of_more(T, more):
+    """Every product adds up K in one order at any number of rows, so the samples of T frames are the first of a longer signal's, bit for bit, as long as the products that leave
+    partial sums leave as many for both."""
+    from ht_vllm_omni_amd import _lib as L
+    H, lib = FULL_CODEC["hidden_size"], L.load()
+    assert all(lib.omni_gemm_tile_splits(T, H, k) == lib.omni_gemm_tile_splits(more, H, k) for k in (H, FULL_CODEC["intermediate_size"]))
+    dec = _decoder(FULL_CODEC, make_codec_state(FULL_CODEC, 11, device="cuda"))
+    codes = torch.randint(0, 2048, (1, 16, more), generator=torch.Generator().manual_seed(T)).cuda()
+    long = dec(codes)
+    assert torch.equal(dec(codes[..., :T]), long[..., :T * dec.total_upsample])
+
+
+@pytest.mark.parametrize("precision", ["bf16", "fp32"])
+def test_the_vocoder_opens_the_talkers_library_alone(monkeypatch, precision):
+    from ht_vllm_omni_amd import _lib as L
+    from ht_vllm_omni_amd.code2wav import Code2WavDecoder
+
+    def absent():
+        raise L.OmniError("no language models' library")
+    monkeypatch.setattr(L, "load_decoder", absent)
+    dec = Code2WavDecoder(TINY_CODEC, make_codec_state(TINY_CODEC, 1), operand_precision=precision)
+    for T in (1, 33):
+        assert torch.isfinite(dec(torch.zeros(1, 4, T, dtype=torch.long, device="cuda"))).all()
+
+
 @pytest.mark.parametrize("hd,nh,nkv,T,window,ldo", [(64, 4, 4, 1, 72, 256), (64, 4, 2, 65, 64, 256), (64, 3, 1, 130, 72, 203), (128, 2, 1, 129, 200, 256), (128, 2, 2, 9, 1, 264)])
 def test_window_attention_kernel(hd, nh, nkv, T, window, ldo):
     """Chunk edges of 64 keys, windows of one key and of several chunks, shared key heads, output rows of odd pitch.  Bound: the result's rounding to bf16

@@ -304,27 +304,6 @@ def test_gemm_stream(M, N, K):
         close(unfrag(b, M, N), ref, 8e-3)
 
 
-@pytest.mark.parametrize("M", [1, 15, 16, 17, 32, 33, 48, 64])
-@pytest.mark.parametrize("N,K,pad", [(16, 32, 0), (96, 64, 8), (224, 288, 24), (1024, 3072, 0), (3072, 1024, 8), (512, 4640, 0)])
-def test_gemm_stream_of_rows_as_they_lie(M, N, K, pad):
-    """Row-major x, with and without a pitch: the bits of the fragment-major product, nothing past the rows or between them read into a sum."""
-    g = gen(M * N)
-    x, w = torch.randn(M, K, generator=g).bfloat16(), dev(torch.randn(N, K, generator=g).bfloat16())
-    xf, wf = frag_rows(x), frag_shuffle(w)
-    xr = torch.full((M, K + pad), float("nan"), dtype=torch.bfloat16)
-    xr[:, :K] = x
-    xr, S = dev(xr), L.load_decoder().omni_gemm_stream_splits(M, N, K)
-    for kind, shape, dt in ((L.STREAM_F32, (S, M, N), torch.float32), (L.STREAM_BF16, (1, M, N), torch.bfloat16)):
-        a, b = (torch.full((shape[0] + 1, *shape[1:]), 7.0, dtype=dt, device="cuda") for _ in range(2))
-        call("omni_gemm_stream", xf, wf, a, M, N, K, kind, 0, 0.0, 0.0, 0)
-        call("omni_gemm_stream_plain", xr, K + pad, wf, b, M, N, K, kind)
-        assert torch.equal(a, b) and bool((b[-1] == 7.0).all())
-    lib = L.load_decoder()
-    bad = lambda x_, ldx, m, kind: lib.omni_gemm_stream_plain(x_, ldx, wf.data_ptr(), b.data_ptr(), m, N, K, kind, L.current_stream()) != 0  # noqa: E731
-    assert bad(xr.data_ptr() + 2, K + pad, M, 1) and bad(xr.data_ptr(), K - 8, M, 1) and bad(xr.data_ptr(), K + 4, M, 1) and bad(xr.data_ptr(), K + pad, 65, 1)
-    assert bad(xr.data_ptr(), K + pad, M, 2)
-
-
 @pytest.mark.parametrize("T", [17, 32, 33, 48, 64, 70])
 @pytest.mark.parametrize("heads,n,k", [(1, 64, 64), (16, 512, 128), (16, 128, 512), (16, 128, 256), (40, 256, 128)])
 def test_head_products_dealt_out_by_rows(T, heads, n, k):

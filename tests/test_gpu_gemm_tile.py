@@ -98,6 +98,34 @@ def test_fp32_output_alone_at_every_tiles_edges(M, N, K):
         assert torch.equal(out[:M, :N], ref) and bool((out[M:] == 7.0).all()) and bool((out[:, N:] == 7.0).all()), hint
 
 
+@pytest.mark.parametrize("M", [1, 15, 16, 17, 33, 64])
+@pytest.mark.parametrize("N,K,pad", [(16, 32, 0), (96, 64, 8), (224, 288, 24), (1024, 3072, 0), (3072, 1024, 8), (512, 4640, 0)])
+def test_few_rows_a_wave_per_piece(M, N, K, pad):
+    """tile_hint 17: the tiles' bits, whole and in runs of K shorter and longer than what a wave has in flight, at rows inside, on and one past a piece; a pitch that holds no
+    numbers, nothing of the outputs' rest.  What it does not take it refuses."""
+    ops, L, frag_shuffle, gu8_shuffle = _ops()
+    g = torch.Generator().manual_seed(M * 19 + K)
+    x = torch.full((M, K + pad), float("nan"), dtype=BF16, device="cuda")
+    x[:, :K] = torch.randn(M, K, generator=g).to(BF16)
+    x, w = x[:, :K], frag_shuffle((torch.randn(N, K, generator=g) * 0.05).to(BF16)).cuda()
+    out = torch.full((M + 3, N + 8), 7.0, dtype=BF16, device="cuda")
+    ops.gemm_tile(x, w, out=out[:M, :N], tile_hint=17)
+    assert torch.equal(out[:M, :N], ops.gemm_tile(x, w)) and bool((out[M:] == 7.0).all()) and bool((out[:, N:] == 7.0).all())
+    for splits in range(1, min(4, K // 32) + 1):
+        got, ref = (torch.full((splits, M + 1, N + 4), 7.0, device="cuda") for _ in range(2))
+        for o, h in ((got, 17), (ref, 0)):
+            ops.gemm_tile(x, w, want="f", out_f32=o[:, :M, :N] if splits > 1 else o[0, :M, :N], splits=splits, tile_hint=h)
+        assert torch.equal(got, ref) and bool((got[:, M] == 7.0).all()) and bool((got[..., N:] == 7.0).all()), splits
+    b = torch.zeros(N, device="cuda")
+    for bad in (dict(bias=b), dict(want="fb"), dict(want="f", resid=torch.zeros(M, N, device="cuda")), dict(act=L.TILE_ACT_RELU2), dict(M=M + 1)):
+        with pytest.raises(L.OmniError):
+            ops.gemm_tile(x, w, tile_hint=17, **bad)
+    with pytest.raises(L.OmniError):                   # rows of 65, and rows that start inside 16 bytes
+        ops.gemm_tile(torch.zeros(65, K, dtype=BF16, device="cuda"), w, tile_hint=17)
+    with pytest.raises(L.OmniError):
+        ops.gemm_tile(torch.zeros(M * (K + 8) + 4, dtype=BF16, device="cuda")[4:].view(M, K + 8)[:, :K], w, tile_hint=17)
+
+
 @pytest.mark.parametrize("M,K,splits", [(33, 32, 1), (70, 96, 3), (129, 160, 4), (65, 64, 1)])
 def test_rows_that_end_an_array(M, K, splits):
     """x is the last columns of a wider array and a run of K steps is a single one: what a tile fetches ahead of its last step lies past the last row."""

@@ -325,24 +325,27 @@ __global__ __launch_bounds__(256) void latent_values_kernel(const float* __restr
     *reinterpret_cast<uint2*>(out + (frag ? frag_off(c, col, heads * n) : (size_t)c * heads * n + col)) = make_uint2(pack_bf2(v[0], v[1]), pack_bf2(v[2], v[3]));
 }
 
-// The same for more rows: a workgroup merges `rows` rows of one head (128 threads each, eight records in flight) and multiplies them by all of the head's
-// columns, its waves taking K's steps in turn as head_gemm's do: the same sums.  A merge of its own and the product behind it are two launches and a round trip of the rows: with
+#define LA_VALUE_TILES 8                               // column tiles of a workgroup
+// The same for more rows: a workgroup merges `rows` rows of one head (128 threads each, eight records in flight; fewer than eight rows: idle
+// threads ask for the last one's again) and multiplies them by up to 128 of the head's columns -- more of them are further workgroups, which merge once more.  Its waves take K's steps
+// in turn where head_gemm's do (KSPLIT, from 256 on), else a column tile each: the same sums at every width.  A merge of its own and the product behind it are two launches and a round trip of the rows: with
 // the attention in front, us a layer, two launches / one, 16 heads of 128 by latents of 512 (256): 64 rows of up to 2048 keys 41.4 / 38.8 (27.1 / 24.4), 64 of up to 352 21.2 / 19.0
 // (15.1 / 13.9), 16 of up to 2048 24.2 / 21.9 (18.2 / 16.5), 3 of up to 352 14.3 / 12.8 (11.8 / 10.3), 20 of 40 keys, nothing to merge, 12.0 / 11.8 (9.3 / 9.1); 64 heads, 64 rows 99 / 92.5.
 // By four waves, two rows at a time and all columns to each, 39.3 of the first and 12.4 of the last but one.  What bounds it now: the records, 2 KB a split and row out of the last-level cache, and the head's weights, which stay in one XCD's L2 (heads are the grid's x).
-template <int NT>                                     // column tiles of a wave; two groups of four waves
+template <bool KSPLIT>                                // two groups of four waves, four column tiles each
 __global__ __launch_bounds__(512) void latent_rows_values_kernel(const float* __restrict__ partial, const float* __restrict__ gate, const uint16_t* __restrict__ merged,
                                                                  const int32_t* __restrict__ positions, const uint16_t* __restrict__ w, uint16_t* __restrict__ out, int T, int heads,
                                                                  int max_split, int per, int rp, int n, int frag, int rows) {
-    constexpr int P = 4, WAVES = 4, S = 8;
+    constexpr int P = 4, WAVES = 4, S = 8, NT = KSPLIT ? LA_VALUE_TILES / 2 : 1, STRIDE = KSPLIT ? WAVES : 1;
     extern __shared__ __attribute__((aligned(16))) uint16_t xs[];      // [rows][rp + 8]
-    __shared__ f32x4 part[2 * WAVES][NT][64];
+    __shared__ f32x4 part[KSPLIT ? 2 * WAVES : 1][NT][64];
     const int lane = threadIdx.x & 63, id = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), wave = id & 3, group = id >> 2, c = lane & 15, q = lane >> 4;
-    const int h = blockIdx.x, t0 = blockIdx.y * rows, n0 = (blockIdx.z * 2 + group) * NT, ntiles = n >> 4, nsteps = rp >> 5, mine = nsteps > wave ? (nsteps - wave + WAVES - 1) / WAVES : 0;
+    const int h = blockIdx.x, t0 = blockIdx.y * rows, ntiles = n >> 4, nsteps = rp >> 5;
+    const int n0 = (blockIdx.z * 2 + group) * WAVES + (KSPLIT ? 0 : wave), first = KSPLIT ? wave : 0, mine = nsteps > first ? (nsteps - first + STRIDE - 1) / STRIDE : 0;
     u32x4 W[P][NT];
     auto load = [&](int d, int s) {                       // (past the last step or tile: that one again, not used)
 #pragma unroll
-        for (int j = 0; j < NT; ++j) W[d][j] = ld16(w + (((size_t)h * ntiles + min(n0 + j, ntiles - 1)) * nsteps + min(wave + s * WAVES, nsteps - 1)) * 512 + lane * 8);
+        for (int j = 0; j < NT; ++j) W[d][j] = ld16(w + (((size_t)h * ntiles + min(n0 + j, ntiles - 1)) * nsteps + min(first + s * STRIDE, nsteps - 1)) * 512 + lane * 8);
     };
 #pragma unroll
     for (int d = 0; d < P; ++d) load(d, d);
@@ -384,7 +387,7 @@ __global__ __launch_bounds__(512) void latent_rows_values_kernel(const float* __
         }
     }
     __syncthreads();
-    const uint16_t* xp = xs + (size_t)min(c, rows - 1) * (rp + 8) + wave * 32 + 8 * q;
+    const uint16_t* xp = xs + (size_t)min(c, rows - 1) * (rp + 8) + first * 32 + 8 * q;
     f32x4 acc[NT];
 #pragma unroll
     for (int j = 0; j < NT; ++j) acc[j] = (f32x4){0.f, 0.f, 0.f, 0.f};
@@ -392,22 +395,29 @@ __global__ __launch_bounds__(512) void latent_rows_values_kernel(const float* __
 #pragma unroll
         for (int d = 0; d < P; ++d) {
             if (s + d >= mine) break;
-            const u32x4 X = *reinterpret_cast<const u32x4*>(xp + (size_t)(s + d) * (WAVES * 32));
+            const u32x4 X = *reinterpret_cast<const u32x4*>(xp + (size_t)(s + d) * (STRIDE * 32));
 #pragma unroll
             for (int j = 0; j < NT; ++j) acc[j] = mfma16(W[d][j], X, acc[j]);
             if (s + d + P < mine) load(d, s + d + P);
         }
-#pragma unroll
-    for (int j = 0; j < NT; ++j) part[id][j][lane] = acc[j];
-    __syncthreads();
     const int t = t0 + c;
-    if (c >= rows || t >= T) return;
-    for (int j = wave; j < min(NT, ntiles - n0); j += WAVES) {
-        f32x4 v = part[group * WAVES][j][lane];
-#pragma unroll
-        for (int u = 1; u < WAVES; ++u) v += part[group * WAVES + u][j][lane];
-        const int col = h * n + (n0 + j) * 16 + 4 * q;
+    auto store = [&](int tile, f32x4 v) {
+        const int col = h * n + tile * 16 + 4 * q;
         *reinterpret_cast<uint2*>(out + (frag ? frag_off(t, col, heads * n) : (size_t)t * heads * n + col)) = make_uint2(pack_bf2(v[0], v[1]), pack_bf2(v[2], v[3]));
+    };
+    if constexpr (!KSPLIT) {
+        if (c < rows && t < T && n0 < ntiles) store(n0, acc[0]);
+    } else {
+#pragma unroll
+        for (int j = 0; j < NT; ++j) part[id][j][lane] = acc[j];
+        __syncthreads();
+        if (c >= rows || t >= T) return;
+        for (int j = wave; j < min(NT, ntiles - n0); j += WAVES) {
+            f32x4 v = part[group * WAVES][j][lane];
+#pragma unroll
+            for (int u = 1; u < WAVES; ++u) v += part[group * WAVES + u][j][lane];
+            store(n0 + j, v);
+        }
     }
 }
 
@@ -608,7 +618,6 @@ static int la_lds(K kernel, int bytes) {
 
 // the per-head product behind decode tokens; w NULL: none.  rows: of a workgroup of latent_rows_values_kernel; 0: latent_values_kernel
 struct LatentValues { const uint16_t* w; uint16_t* out; int n, frag, rows; };
-#define LA_VALUE_TILES 8
 template <int RS>
 static int la_run(const omni_latent_attn& p, LatentArgs a, const LatentValues& then, hipStream_t st) {
     using G = LatentGeom<RS>;
@@ -624,7 +633,7 @@ static int la_run(const omni_latent_attn& p, LatentArgs a, const LatentValues& t
         hipLaunchKernelGGL(latent_decode_kernel<RS>, dim3((p.heads + 15) / 16, p.n_decode, a.nsplit), dim3(64 * LA_DEC_WAVES), LDS, st, a);
         OMNI_CHECK_LAUNCH("omni_latent_attn(decode)");
         if (then.w && then.rows) {
-            hipLaunchKernelGGL(latent_rows_values_kernel<LA_VALUE_TILES / 2>, dim3(p.heads, (p.n_decode + then.rows - 1) / then.rows, (then.n / 16 + LA_VALUE_TILES - 1) / LA_VALUE_TILES), dim3(512),
+            hipLaunchKernelGGL(latent_rows_values_kernel<(RS >= 8)>, dim3(p.heads, (p.n_decode + then.rows - 1) / then.rows, (then.n / 16 + LA_VALUE_TILES - 1) / LA_VALUE_TILES), dim3(512),
                                then.rows * (p.rp + 8) * 2, st, (const float*)a.partial, a.gate, (const uint16_t*)a.out, a.positions, then.w, then.out, p.n_decode, p.heads, a.nsplit, a.per, p.rp,
                                then.n, then.frag, then.rows);
             OMNI_CHECK_LAUNCH("omni_latent_attn(values)");

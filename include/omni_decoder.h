@@ -135,10 +135,11 @@ typedef struct omni_latent_attn {
 } omni_latent_attn;
 int omni_latent_attn_run(const omni_latent_attn* a, void* stream);
 /* Decode tokens alone (T = n_decode <= OMNI_STREAM_LATENT_ROWS, bf16, a width of omni_latent_attn_mfma, rp <= 512) and the per-head product behind it:
- * out[t, h] = (what omni_latent_attn_run leaves in a->out) . w[h]^T as omni_head_gemm, in one launch less where heads * n / 16 <= 256; a->out is
- * scratch                                                                                                                                            */
+ * out[t, h] = (what omni_latent_attn_run leaves in a->out) . w[h]^T as omni_head_gemm, in one launch less where heads * n / 16 <= 256 (bit for bit from
+ * rp = 256 on); a->out is scratch                                                                                                                     */
 int omni_latent_attn_values(const omni_latent_attn* a, const void* w, void* out, int n, int frag, void* stream);
-/* ... for any number of decode tokens (T = n_decode): merged splits and product in one launch where 16 rows of a head to a workgroup make no more than 256 of them */
+/* ... for any number of decode tokens (T = n_decode): merged splits and product in one launch where 16 rows of a head to a workgroup make no more than 256 of them; bit for bit
+ * at every width */
 int omni_latent_attn_products(const omni_latent_attn* a, const void* w, void* out, int n, int frag, void* stream);
 int64_t omni_latent_attn_workspace_bytes(int n_decode, int heads, int rp);
 int omni_latent_attn_tile_rows(int rp);

@@ -61,16 +61,13 @@ extern "C" int omni_codec_rvq_embed(const int64_t* codes, int ld_codes, const fl
 // The row and the weights are asked for at once and stay in registers (PIECES of 256 columns; the row was walked twice, a wait per piece).  Measured in the
 // decode of 50 frames, 17 of these launches over 50 rows of 1024: 1158 -> 1143 us.  Wider rows take the kernel that walks them.
 // ADD: what the sublayer in front left joins the row first: partial sums of a product whose few tiles would each walk all of K alone (omni_gemm_tile k_splits).
-// A few rows are dealt out a wave to a workgroup: with partial sums a row is 28 KB, and four of them on one CU wait for its intake
-// (the 17 norms of 50 frames, all together 15 us less).
-static int norm_rows(int T) { return T <= 1024 ? 1 : 4; }
+// A row to a workgroup: four of them on one CU wait for its intake (with four partial sums a row is 28 KB).  Us, four rows / one of 1024, behind the kernel that wrote them, without partial
+// sums, with one, with four: 50 rows 2.0 / 1.8, 3.6 / 2.0, 3.4 / 2.6; 325 2.5 / 2.0, 3.9 / 2.6, 5.8 / 4.1; 1024 3.9 / 2.6, 7.9 / 3.9, 11.5 / 3.5; 8192 12.2 / 8.5, 18.6 / 16.9.
 struct CodecAdd { float* x; const float* y; const float* scale; int slabs; long long stride; };
 template <int PIECES, bool ADD>
-__global__ __launch_bounds__(256) void codec_rmsnorm_kernel(const float* x, int ldx, const float* __restrict__ w, float eps,
-                                                            uint16_t* __restrict__ out, int T, int H, const CodecAdd add) {
-    const int lane = threadIdx.x & 63;
-    const int t = blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6);
-    if (t >= T) return;
+__global__ __launch_bounds__(64) void codec_rmsnorm_kernel(const float* x, int ldx, const float* __restrict__ w, float eps,
+                                                           uint16_t* __restrict__ out, int H, const CodecAdd add) {
+    const int lane = threadIdx.x, t = blockIdx.x;
     const float* xr = x + (size_t)t * ldx;
     f32x4 v[PIECES], g[PIECES];
 #pragma unroll
@@ -137,11 +134,10 @@ __global__ __launch_bounds__(256) void codec_rmsnorm_wide_kernel(const float* __
 
 extern "C" int omni_codec_rmsnorm(const float* x, int ldx, const float* w, float eps, void* out, int T, int H, void* stream) {
     OMNI_CHECK_ARG(x && w && out && T > 0 && H > 0 && H % 4 == 0 && ldx >= H && ldx % 4 == 0, "omni_codec_rmsnorm: T=%d H=%d ldx=%d", T, H, ldx);
-    const int per = H <= 1024 ? norm_rows(T) : 4;
-    const dim3 grid((T + per - 1) / per), block(64 * per);
-    if (H <= 512) hipLaunchKernelGGL((codec_rmsnorm_kernel<2, false>), grid, block, 0, (hipStream_t)stream, x, ldx, w, eps, (uint16_t*)out, T, H, CodecAdd{});
-    else if (H <= 1024) hipLaunchKernelGGL((codec_rmsnorm_kernel<4, false>), grid, block, 0, (hipStream_t)stream, x, ldx, w, eps, (uint16_t*)out, T, H, CodecAdd{});
-    else hipLaunchKernelGGL(codec_rmsnorm_wide_kernel, grid, block, 0, (hipStream_t)stream, x, ldx, w, eps, (uint16_t*)out, T, H);
+    const dim3 grid(T), block(64);
+    if (H <= 512) hipLaunchKernelGGL((codec_rmsnorm_kernel<2, false>), grid, block, 0, (hipStream_t)stream, x, ldx, w, eps, (uint16_t*)out, H, CodecAdd{});
+    else if (H <= 1024) hipLaunchKernelGGL((codec_rmsnorm_kernel<4, false>), grid, block, 0, (hipStream_t)stream, x, ldx, w, eps, (uint16_t*)out, H, CodecAdd{});
+    else hipLaunchKernelGGL(codec_rmsnorm_wide_kernel, dim3((T + 3) / 4), dim3(256), 0, (hipStream_t)stream, x, ldx, w, eps, (uint16_t*)out, T, H);
     OMNI_CHECK_LAUNCH("omni_codec_rmsnorm");
     return OMNI_OK;
 }
@@ -149,11 +145,10 @@ extern "C" int omni_codec_rmsnorm(const float* x, int ldx, const float* w, float
 extern "C" int omni_codec_add_rmsnorm(float* x, int ldx, const float* y, int slabs, int64_t slab_stride, const float* scale, const float* w, float eps, void* out, int T, int H, void* stream) {
     OMNI_CHECK_ARG(x && y && scale && w && out && T > 0 && H > 0 && H % 4 == 0 && H <= 1024 && ldx >= H && ldx % 4 == 0 && slabs >= 1 && slabs <= 4 &&
                    (slabs == 1 || slab_stride >= (int64_t)T * H) && slab_stride % 4 == 0, "omni_codec_add_rmsnorm: T=%d H=%d (<= 1024) ldx=%d slabs=%d (<= 4)", T, H, ldx, slabs);
-    const int per = norm_rows(T);
-    const dim3 grid((T + per - 1) / per), block(64 * per);
+    const dim3 grid(T), block(64);
     const CodecAdd add{x, y, scale, slabs, slab_stride};
-    if (H <= 512) hipLaunchKernelGGL((codec_rmsnorm_kernel<2, true>), grid, block, 0, (hipStream_t)stream, x, ldx, w, eps, (uint16_t*)out, T, H, add);
-    else hipLaunchKernelGGL((codec_rmsnorm_kernel<4, true>), grid, block, 0, (hipStream_t)stream, x, ldx, w, eps, (uint16_t*)out, T, H, add);
+    if (H <= 512) hipLaunchKernelGGL((codec_rmsnorm_kernel<2, true>), grid, block, 0, (hipStream_t)stream, x, ldx, w, eps, (uint16_t*)out, H, add);
+    else hipLaunchKernelGGL((codec_rmsnorm_kernel<4, true>), grid, block, 0, (hipStream_t)stream, x, ldx, w, eps, (uint16_t*)out, H, add);
     OMNI_CHECK_LAUNCH("omni_codec_add_rmsnorm");
     return OMNI_OK;
 }

@@ -425,7 +425,7 @@ def test_depthwise_conv_and_layer_norm(C, T, ldx, taps):
 
 @pytest.mark.parametrize("T", [1024, 1025, 1030])
 def test_norm_of_many_rows(T):
-    """A wave to a workgroup up to 1024 rows, four behind: the same bits."""
+    """The last rows of many alone: the same bits."""
     from ht_vllm_omni_amd import _lib as L
     g, H = torch.Generator().manual_seed(T), 260
     x, w = torch.randn(T, H, generator=g).cuda(), torch.randn(H, generator=g).cuda()

@@ -57,8 +57,9 @@ const char* omni_last_error(void);
 int omni_abi_version(void);   /* 8: omni_tile_gemm.k_splits / slab_stride, omni_gemm_tile_splits, omni_res_unit.row_tiles, omni_window_attn.key_base / k_row /
                                  v_row / head_gate, omni_latent_gather; an attention workspace may hold anything (7: omni_tile_gemm activations RELU2, SILU_SIGMOID,
                                  GELU_MUL; 6: column groups, xIELU; 5: omni_ar_peers.tile_flags, omni_talker_set_chains modes 2 / 3).  A library reads whole structs of
-                                 its own version: a caller compares this with the header it was built against.  Added within 8, no struct moved: tile_hint 14 ... 16,
-                                 omni_codec_add_rmsnorm, omni_gemm_stream_joined / _joins / _latents, omni_latent_attn_values, omni_window_attn.prompt_keys */
+                                 its own version: a caller compares this with the header it was built against.  Added within 8, no struct moved: tile_hint 14 ... 17,
+                                 omni_codec_add_rmsnorm, omni_codec_res_unit_last, omni_gemm_stream_joined / _joins / _latents, omni_latent_attn_values / _products,
+                                 omni_latent_write_rows, omni_window_attn.prompt_keys */
 
 /* ------------------------------------------------------------------ per-op entry points */
 

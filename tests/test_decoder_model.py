@@ -153,8 +153,8 @@ def test_items_of_a_batch_are_those_its_mixers_will_walk():
     m.tiles, m.head_tiles = ("tiles", 16, 128), ("tiles", 1, 128)
     m.work = (m.tiles,)
     batch = lambda segs, n_decode=0: SimpleNamespace(T=n_decode + sum(n for n, _ in segs), n_decode=n_decode, segs=segs)  # noqa: E731
-    assert m.work_for(batch([(2000, 0)])) == (m.head_tiles, ("cached_rows",), ("first_rows",))
-    assert m.work_for(batch([(251, 512)] * 2, 48)) == (m.head_tiles, ("cached_rows",), ("first_rows",))
+    assert m.work_for(batch([(2000, 0)])) == (m.head_tiles, ("earlier_rows",), ("first_rows",))
+    assert m.work_for(batch([(251, 512)] * 2, 48)) == (m.head_tiles, ("earlier_rows",), ("first_rows",))
     assert m.work_for(batch([(32, 8000)] * 60)) == m.work_for(batch([(3, 900)], 2)) == m.work_for(batch([], 3)) == (m.tiles,)
     m.ukv = None
     assert m.work_for(batch([(2000, 0)])) == (m.tiles,)

@@ -409,7 +409,8 @@ def test_last_conv_adds_in_one_order_at_every_width(C, T, taps):
 @pytest.mark.parametrize("C,T,ldx,taps", [(4, 1, 4, 7), (252, 9, 256, 7), (1024, 3, 1024, 7), (1020, 40, 1028, 7), (256, 20, 257, 7), (130, 20, 130, 7), (64, 30, 64, 5)])
 def test_depthwise_conv_and_layer_norm(C, T, ldx, taps):
     """Seven taps, and the general kernel of other counts; channels that end inside a round of threads, frames before the first whole window.  Bound:
-    one rounding to bf16, and fp32 sums whose errors a small variance enlarges: 2^-20 of the largest gain."""
+    one rounding to bf16, and fp32 sums: a conv's taps + 1 roundings of its magnitudes, twice (a value and the mean), the mean's own and the difference's, some 15 -- no more than
+    4 (taps + 3) of 2^-24 -- which the norm enlarges by gain and 1 / deviation, and once more by the value's distance from the mean (the variance)."""
     from ht_vllm_omni_amd import _lib as L
     g = torch.Generator().manual_seed(C + T)
     x, w, b = torch.randn(T, ldx, generator=g), torch.randn(C, taps, generator=g) * 0.4, torch.randn(C, generator=g) * 0.1
@@ -420,7 +421,11 @@ def test_depthwise_conv_and_layer_norm(C, T, ldx, taps):
     xp = torch.cat([torch.zeros(taps - 1, C), x[:, :C]]).double()
     y = b.double() + sum(xp[j:j + T] * w[:, j].double() for j in range(taps))
     ref = torch.nn.functional.layer_norm(y, (C,), lw.double(), lb.double(), 1e-6)
-    assert bool(((out[:T].cpu().double() - ref).abs() <= ref.abs() * 2.0 ** -8 + 2.0 ** -18).all()) and bool((out[T:] == 7.0).all())
+    mag = b.double().abs() + sum((xp[j:j + T] * w[:, j].double()).abs() for j in range(taps))
+    rstd = 1 / torch.sqrt(y.var(-1, unbiased=False, keepdim=True) + 1e-6)
+    far = 1 + (y - y.mean(-1, keepdim=True)).abs() * rstd
+    bound = ref.abs() * 2.0 ** -8 + lw.double().abs() * rstd * far * 4 * (taps + 3) * 2.0 ** -24 * mag.amax(-1, keepdim=True)
+    assert bool(((out[:T].cpu().double() - ref).abs() <= bound).all()) and bool((out[T:] == 7.0).all())
 
 
 @pytest.mark.parametrize("T", [1024, 1025, 1030])

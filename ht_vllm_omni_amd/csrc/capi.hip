@@ -104,6 +104,7 @@ struct omni_talker {
     float* kv_scale_dev;                // fp8 KV: device [layers][2] = {k_scale, v_scale} per layer, read by the decode step's attention launches
     std::vector<float> ksc_h, vsc_h;    // the same on the host (arguments of the eager prefill launches)
     void* bb_table;                     // device table of the backbone layers' pointers (bb_all.hip)
+    char* cp_flow;                      // hand-off buffers of the predictor's all-pass launch (cp_chain.hip)
     uint32_t* chain_flags;              // stage flags of the persistent chains: OMNI_FLAG_REPLICAS copies of [256] (coherent.cuh) + the error word at [320]
     omni_ar_peers ar_attn, ar_mlp;      // copies of desc.ar_* (has_ar)
     bool has_ar;
@@ -168,6 +169,7 @@ static int carve(omni_talker* t, char* base, size_t* total) {
     t->cp_slots = c.take<int64_t>((Q + 1) * B);
     t->pf_seq = c.take<int32_t>(8);
     t->chain_flags = c.take<uint32_t>(OMNI_FLAG_WORDS);
+    t->cp_flow = c.take<char>(k_cp_flow_bytes());
     t->kv_scale_dev = c.take<float>(2 * (size_t)(d.layers > 0 ? d.layers : 1));
 #ifdef OMNI_DEBUG_HOOKS
     t->bb_table = c.take<char>(k_bb_all_table_bytes(d.layers > 0 ? d.layers : 1));
@@ -620,8 +622,8 @@ static int run_code_predictor(omni_talker* t, const int32_t* layer0_ids, const v
                 hd.greedy = greedy; hd.top_k = top_k; hd.temperature = temperature; hd.top_p = top_p; hd.seed = seed;
                 hd.steps = steps; hd.row_seed = row_seed; hd.codes = t->codes;
                 hd.tail = (tail && k_cp_chain_tail_supported(d, B)) ? tail : nullptr;
-                TRY(k_cp_chain(d, t->cp_layer.data(), t->cp_k.data(), t->cp_v.data(), B, g, Q, np, t->cp_resid, t->cp_part, t->cp_qkv,
-                               t->cp_attn, t->cp_act, cflags, cerr, &hd, st));
+                TRY(k_cp_chain(d, t->cp_layer.data(), t->cp_k.data(), t->cp_v.data(), B, g, Q, np, t->cp_resid, t->cp_part, cflags,
+                               cerr, t->cp_flow, &hd, st));
                 t->ran |= 1;
                 t->tail_fused = hd.tail != nullptr;
                 break;
@@ -629,8 +631,8 @@ static int run_code_predictor(omni_talker* t, const int32_t* layer0_ids, const v
             if (!in_pair) {
                 if (d.cp_chain && !t->chain_half && k_cp_chain_supported(d, g)) {
                     // the layer stack of this pass as one persistent launch: 25 stages behind flag hand-offs
-                    TRY(k_cp_chain(d, t->cp_layer.data(), t->cp_k.data(), t->cp_v.data(), B, g, g + 1, np, t->cp_resid, t->cp_part, t->cp_qkv,
-                                   t->cp_attn, t->cp_act, cflags, cerr, nullptr, st));
+                    TRY(k_cp_chain(d, t->cp_layer.data(), t->cp_k.data(), t->cp_v.data(), B, g, g + 1, np, t->cp_resid, t->cp_part, cflags,
+                                   cerr, t->cp_flow, nullptr, st));
                     t->ran |= 1;
                     np = Hc / 16;
                 } else {

@@ -15,13 +15,15 @@
 #define CH_NSTAMP 8
 #define CH_STAMP_PASS (40 * CH_NSTAMP * OMNI_CHAIN_WGS)      // stamp words of one predictor pass (cp_chain.hip: block `pass` of the buffer)
 #ifdef OMNI_DEBUG_HOOKS
-#define CH_STAMP(buf, sidx, k)                                                                                          \
+#define CH_STAMP(buf, sidx, k) CH_STAMP_BY(buf, sidx, k, 0)
+#define CH_STAMP_BY(buf, sidx, k, thread)                                                                               \
     do {                                                                                                                \
-        if ((buf) != nullptr && threadIdx.x == 0)                                                                       \
+        if ((buf) != nullptr && threadIdx.x == (thread))                                                                \
             (buf)[((size_t)(sidx) * CH_NSTAMP + (k)) * OMNI_CHAIN_WGS + blockIdx.x] = __builtin_amdgcn_s_memrealtime(); \
     } while (0)
 #else
 #define CH_STAMP(buf, sidx, k) do { (void)(buf); (void)(sidx); } while (0)
+#define CH_STAMP_BY(buf, sidx, k, thread) do { (void)(buf); (void)(sidx); } while (0)
 #endif
 
 // PRO 3 (round 4: an A/B arm; round 6: the product form of every norm-fused stage whose normalised rows are nobody's output -- qkv, gate_up --

@@ -4,14 +4,16 @@
 // Launch-per-op, a predictor pass is 25 dependent launches (5 layers x { qkv, attention, o_proj, gate_up, down_proj }) of
 // ~5.5 us each although a workgroup's share of a GEMM is 16-48 KB of weights and a few MFMAs: a dependent launch pays the
 // kernel boundary (1.65 us), a cold weight fetch, a cold activation fetch and a store drain, one after the other.
-// Here the 25 stages run inside one grid of 256 co-resident workgroups (one per CU):
-//   * a stage's WEIGHT slice does not depend on its predecessor: every wave loads its whole slice (4-12 k-steps, 32-64 VGPRs)
-//     before it looks at the stage flags, so the weight latency overlaps the predecessor's tail;
-//   * stages hand activations over "coherent by access" (coherent.cuh): sc1 write-through stores, one flag word per
-//     workgroup, sc1 loads behind the flag poll -- no cache write-back / invalidate, no kernel boundary;
-//   * what a stage may read BEFORE the flags (besides weights): bytes that were final two or more stages earlier -- the
-//     K / V history of the private cache, the old residual values of a residual epilogue.
-// Tiles, k-step ownership of the 8 waves, accumulation order, LDS combine order and every rounding point are those of
+// Here the stages run inside one grid of 256 co-resident workgroups (one per CU):
+//   * a stage's WEIGHT slice does not depend on its predecessor: every wave loads its whole slice before it looks for its operands;
+//   * cp_chain_kernel (passes 2 .. 15, their heads and samplers) hands activations over by content: an operand is there when none of its words
+//     is EMPTY (chain_flow.cuh).  No drain, no flag, no barrier between a stage's last store and its successor's first MFMA.  What bounds it is
+//     that chain of dependent trips: 27 stages a pass of about 2.7 us (5 rows: 73 us a pass; 64 rows: 90), of which 0.6 to 1.6 us are a stage's own
+//     arithmetic, LDS combine and epilogue and the rest the operands' way.  Behind flags (coherent.cuh) a pass took 104 / 110 us;
+//   * cp_pair_kernel (positions 0 and 1) hands over behind flag words ("coherent by access", coherent.cuh);
+//   * what a stage may read without waiting (besides weights): bytes that were final two or more stages earlier -- the K / V history of the
+//     private cache, the old residual values of a residual epilogue.
+// K-step ownership of the 8 waves, accumulation order, LDS combine order and every rounding point are those of
 // gemm_skinny_kernel / attn_tiny_dense_kernel: the chain is bit-identical to the launch-per-op path (tests/test_gpu_chain.py).
 // Bounded spins: a grid that is not co-resident times out into an error word (never a hang).
 #include "attn_common.cuh"
@@ -19,6 +21,7 @@
 #include "common.cuh"
 #include "gemm_frag.cuh"
 #include "chain_gemm.cuh"
+#include "chain_flow.cuh"
 #include "kernels.h"
 #include "sampler_body.cuh"
 
@@ -38,7 +41,7 @@ struct ChainArgs {
     float eps, sm_scale;
     uint16_t* resid;                      // fragment-major residual stream [64][Hc]
     float* part;                          // sum(r^2) slabs [np][64]
-    uint16_t *qkv, *attn, *act;           // stage outputs: row-major [B][4096], fragment-major [64][2048], fragment-major [64][3072]
+    uint16_t *qkv, *attn, *act;           // pair kernel: stage outputs, row-major [B][4096], fragment-major [64][2048], fragment-major [64][3072]
     const uint16_t* cos_sin;
     // head + sampler of pass g (group g): logits row b at logits + b * logits_ld + (g - 1) * logits_pass
     const uint16_t *cp_norm, *lm_head;    // lm_head: [Q - 1][codebook][Hc] fragment-major per group
@@ -56,116 +59,11 @@ struct ChainArgs {
         const uint16_t* wqkv; const uint16_t* ln1; uint16_t* qkv; int NQ;
         int enabled;
     } tail;
+    char* flow;                           // the all-pass launch's hand-off buffers: FLOW_COPIES copies of CP_COPY bytes
     int Bp;                               // pair kernel: rows of position 1 start at Bp (B rounded up to 16) in the 128-row stream
-    int skip;                             // debug library: ingest experiment (coherent.cuh ChainGate::skip)
-    int dom, gu_narrow, nap;              // policy (run-time knobs in the debug library): flag domain (coherent.cuh), gate_up on the launch path's 32 x 24 tile, poll pause
+    int nap;                              // pair kernel: poll pause (coherent.cuh; a run-time knob in the debug library)
     unsigned long long* stamps;           // debug library only: [stage][CH_NSTAMP][256] s_memrealtime ticks (100 MHz) of wave 0, or NULL
 };
-
-// ---- attention stage at buffer position pos <= 15 (dense private cache: row b owns block b): one wave per (row, q head),
-// the work layout of attn_tiny_dense_kernel (paged_attn.hip).  Waves 0-3 of workgroup w take pairs 4 w .. 4 w + 3.
-__device__ __forceinline__ void chain_attn(const ChainArgs& a, const ChainLayer& L, int pos, float* lds, ChainGate& g, int code,
-                                           unsigned long long* stamps) {
-    const int sidx = ((code & 255) >> 4) * 5 + (code & 15) - 1;
-    CH_STAMP(stamps, sidx, 0);
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    const int q_heads = a.q_heads, kv_heads = a.kv_heads, bs = a.bs;
-    if ((int)blockIdx.x * 4 >= a.B * q_heads) {                 // none of this workgroup's four pairs is a live row
-        chain_gate_skip(g);
-        return;
-    }
-    const int pair = blockIdx.x * 4 + (wave & 3);               // waves 4-7 do the work: wave 0 polls the flags, and a wave's
-    const bool active = wave >= 4 && pair < a.B * q_heads;      // loads return in order -- history loads ahead of a poll delay it
-    const int row = pair / q_heads, h = pair - row * q_heads;
-    const int ratio = q_heads / kv_heads, kvh = h / ratio;
-    const int nslots = q_heads + 2 * kv_heads;
-    const int t = lane >> 2, qd = lane & 3;
-    const coh_rsrc_t krs = coh_rsrc(L.kc), vrs = coh_rsrc(L.vc), qrs = coh_rsrc(a.qkv), ars = coh_rsrc(a.attn);
-    // ---- before the flags: the history rows (written by earlier passes; rows >= pos hold stale bytes and are masked)
-    u32x4 kq[4];
-    uint32_t vq[16];
-    if (active) {
-        const uint32_t hrow = ((uint32_t)(row * bs + t) * kv_heads + kvh) * 128;
-#pragma unroll
-        for (int j = 0; j < 4; ++j) kq[j] = coh_ld16(krs, (hrow + qd * 32 + j * 8) * 2);
-#pragma unroll
-        for (int u = 0; u < 16; ++u) vq[u] = coh_ld4(vrs, (((uint32_t)(row * bs + u) * kv_heads + kvh) * 128 + 2 * lane) * 2);
-    }
-    CH_STAMP(stamps, sidx, 1);
-    chain_gate_wait(g, code);
-    CH_STAMP(stamps, sidx, 2);
-    if (active) {
-        // ---- behind the flags: this row's q / k / v heads out of the qkv GEMM's output, one dword per lane each; the
-        // (l, l + 64) pairing of the norm + RoPE is restored through LDS
-        const uint32_t qoff = ((uint32_t)row * nslots + h) * 128, koff = ((uint32_t)row * nslots + q_heads + kvh) * 128,
-                       voff = ((uint32_t)row * nslots + q_heads + kv_heads + kvh) * 128;
-        const uint32_t qw = coh_ld4(qrs, (qoff + 2 * lane) * 2), kw = coh_ld4(qrs, (koff + 2 * lane) * 2);
-        const uint32_t vnew = coh_ld4(qrs, (voff + 2 * lane) * 2);
-        float* sq = lds + (wave & 3) * 256;                   // [0,128): q in the score layout; [128,256): raw q | k dwords
-        uint32_t* raw = reinterpret_cast<uint32_t*>(sq + 128);
-        raw[lane] = qw;
-        raw[64 + lane] = kw;
-        __builtin_amdgcn_wave_barrier();
-        const uint16_t* rq = reinterpret_cast<const uint16_t*>(raw);
-        const uint16_t* rk = rq + 128;
-        const uint16_t* cs = a.cos_sin + (size_t)pos * 128;
-        float q0, q1, k0, k1;
-        head_norm_rope_vals(bf2f(rq[lane]), bf2f(rq[lane + 64]), L.qnorm, cs, a.eps, lane, q0, q1);
-        head_norm_rope_vals(bf2f(rk[lane]), bf2f(rk[lane + 64]), L.knorm, cs, a.eps, lane, k0, k1);
-        if (h % ratio == 0) {
-            // the new token's K / V into the private cache: one dword per lane (even lanes elements l, l + 1 of the first
-            // half, odd lanes l + 63, l + 64 of the second), written through for the later passes
-            const uint32_t crow = ((uint32_t)(row * bs + pos) * kv_heads + kvh) * 128;
-            const uint32_t kb0 = f2bf(k0), kb1 = f2bf(k1);
-            const uint32_t n0 = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)kb0, OMNI_DPP_XOR1, 0xF, 0xF, true);
-            const uint32_t n1 = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)kb1, OMNI_DPP_XOR1, 0xF, 0xF, true);
-            const bool odd = (lane & 1) != 0;
-            const uint32_t word = odd ? (n1 | (kb1 << 16)) : (kb0 | (n0 << 16));
-            const uint32_t elem = odd ? 64 + lane - 1 : lane;
-            coh_st4(krs, (crow + elem) * 2, word);
-            coh_st4(vrs, (crow + 2 * lane) * 2, vnew);
-        }
-        const float qs = a.sm_scale * LOG2E;
-        const float s_new = wave_sum(fmaf(q0 * qs, k0, (q1 * qs) * k1));
-        sq[lane] = q0 * qs;
-        sq[lane + 64] = q1 * qs;
-        __builtin_amdgcn_wave_barrier();
-        float d = 0.f;
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-            const f32x4 qa = *reinterpret_cast<const f32x4*>(&sq[qd * 32 + j * 8]);
-            const f32x4 qb = *reinterpret_cast<const f32x4*>(&sq[qd * 32 + j * 8 + 4]);
-            d = fmaf(qa[0], bf_lo(kq[j][0]), d); d = fmaf(qa[1], bf_hi(kq[j][0]), d);
-            d = fmaf(qa[2], bf_lo(kq[j][1]), d); d = fmaf(qa[3], bf_hi(kq[j][1]), d);
-            d = fmaf(qb[0], bf_lo(kq[j][2]), d); d = fmaf(qb[1], bf_hi(kq[j][2]), d);
-            d = fmaf(qb[2], bf_lo(kq[j][3]), d); d = fmaf(qb[3], bf_hi(kq[j][3]), d);
-        }
-        d += dpp_f<OMNI_DPP_XOR1>(d);
-        d += dpp_f<OMNI_DPP_XOR2>(d);
-        const float s = t < pos ? d : -INFINITY;
-        float m = fmaxf(s, dpp_f<OMNI_DPP_HALF_MIRROR>(s));
-        m = fmaxf(m, dpp_f<OMNI_DPP_MIRROR>(m));
-        m = xor32_max(xor16_max(m));
-        m = fmaxf(m, s_new);
-        const float p = exp2f(s - m);
-        const float p_new = exp2f(s_new - m);
-        float lsum = p + dpp_f<OMNI_DPP_HALF_MIRROR>(p);
-        lsum += dpp_f<OMNI_DPP_MIRROR>(lsum);
-        lsum = xor32_sum(xor16_sum(lsum));
-        const float inv = 1.0f / (lsum + p_new);
-        float o0 = p_new * bf_lo(vnew), o1 = p_new * bf_hi(vnew);
-#pragma unroll
-        for (int u = 0; u < 16; ++u) {
-            const float pu = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(p), 4 * u));
-            o0 = fmaf(pu, bf_lo(vq[u]), o0);
-            o1 = fmaf(pu, bf_hi(vq[u]), o1);
-        }
-        coh_st4(ars, (uint32_t)frag_off(row, h * 128 + 2 * lane, q_heads * 128) * 2, pack_bf2(o0 * inv, o1 * inv));
-    }
-    CH_STAMP(stamps, sidx, 6);
-    chain_gate_arrive(g);
-    CH_STAMP(stamps, sidx, 7);
-}
 
 // ---- the backbone's input row of batch row b (mtp_finalize_kernel, capi.hip: x[t+1] = bf16(bf16(sum_fp32(e0, emb_1 .. emb_{Q-1})) + text_step), an
 // invalid layer-0 id -> a frame of zeros; qwen3_tts_talker.py:1630-1641) by the workgroup that just drew the row's last code: the same 256 threads,
@@ -461,9 +359,278 @@ __global__ __launch_bounds__(CH_THREADS) void cp_pair_kernel(const ChainArgs a) 
     chain_sample(a, 1, lds, g, 0x01F2, a.stamps);
 }
 
-// DEFER: rstd of the qkv / gate_up stages applied in their epilogues (chain_gemm PRO 3; the head GEMM keeps the exact norm) -- round 4's
-// A/B arm of VERDICT r3 item 1b, the product form since round 6 (the launch path's gemm_skinny_kernel takes it for the same GEMMs: same bits);
-// <.., false> = round 5's exact-rstd stages, debug library only
+// ---- the all-pass launch: passes 2 .. 15 of every row, hand-offs by content (chain_flow.cuh)
+// hand-off buffers of one copy, bytes from its base (64 rows)
+enum : uint32_t {
+    CP_QKV = 0,                           // 4096 columns, 16 x 16 tiles
+    CP_ATT = CP_QKV + 64 * 4096 * 2,      // fragment-major, 2048 columns
+    CP_RA = CP_ATT + 64 * 2048 * 2,       // residual stream behind o_proj, fragment-major, + its slabs
+    CP_PA = CP_RA + 64 * 1024 * 2,
+    CP_ACT = CP_PA + 64 * 64 * 4,         // fragment-major, 3072 columns
+    CP_RB = CP_ACT + 64 * 3072 * 2,       // residual stream behind down_proj + its slabs
+    CP_PB = CP_RB + 64 * 1024 * 2,
+    CP_R0 = CP_PB + 64 * 64 * 4,          // a pass's input rows (the sampler's gather) + their one slab
+    CP_P0 = CP_R0 + 64 * 1024 * 2,
+    CP_LOG = CP_P0 + 1024,                // 2048 logits a row, 16 x 16 tiles
+    CP_COPY = CP_LOG + 64 * 2048 * 4
+};
+#define CP_FLOW_BYTES ((size_t)FLOW_COPIES * CP_COPY)
+size_t k_cp_flow_bytes() { return CP_FLOW_BYTES; }
+
+// LDS of the launch: two combine halves, a KB per wave for the attention, the sampler's working set, one word
+#define CPF_ATTN_FLOATS (2 * FLOW_HALF_FLOATS)
+#define CPF_SMP_FLOATS (CPF_ATTN_FLOATS + CH_WAVES * 256)
+#define CPF_LAST_FLOATS (CPF_SMP_FLOATS + (SMP_LDS_BYTES(8) + 15) / 16 * 4)
+#define CPF_LDS_BYTES ((CPF_LAST_FLOATS + 4) * 4)
+
+// attention at buffer position pos <= 15 (dense private cache: row b owns block b): one wave per (row, q head), the work layout of
+// attn_tiny_dense_kernel (paged_attn.hip).  A kv head's q heads are waves of ONE workgroup, in every pass the same one: the K / V rows that the
+// first of them writes are read, passes later, behind that workgroup's own barriers.
+struct FlowHist { u32x4 k[4]; uint32_t v[16]; };        // a wave's history rows: lane = (token lane / 4, quarter lane % 4) of K, a dword of every token of V
+__device__ __forceinline__ void flow_history(const ChainArgs& a, const ChainLayer& L, int pair, FlowHist& hist) {
+    int lane = threadIdx.x & 63;
+    asm volatile("" : "+v"(lane));
+    const int row = pair / a.q_heads, kvh = (pair - row * a.q_heads) / (a.q_heads / a.kv_heads);
+    const coh_rsrc_t krs = coh_rsrc(L.kc), vrs = coh_rsrc(L.vc);
+    const uint32_t hrow = ((uint32_t)(row * a.bs + (lane >> 2)) * a.kv_heads + kvh) * 128;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) hist.k[j] = coh_ld16(krs, (hrow + (lane & 3) * 32 + j * 8) * 2);
+#pragma unroll
+    for (int u = 0; u < 16; ++u) hist.v[u] = coh_ld4(vrs, (((uint32_t)(row * a.bs + u) * a.kv_heads + kvh) * 128 + 2 * lane) * 2);
+}
+__device__ __forceinline__ void flow_attn(const ChainArgs& a, const ChainLayer& L, int pos, int pair, float* sq, const char* in, char* out, char* clr,
+                                          const FlowHist& hist, FlowWait& fw, int code, unsigned long long* stamps) {
+    const int sidx = ((code & 255) >> 4) * 5 + (code & 15) - 1;
+    CH_STAMP_BY(stamps, sidx, 0, 256);
+    int lane = threadIdx.x & 63;
+    asm volatile("" : "+v"(lane));      // opaque per call (flow_gemm)
+    const int q_heads = a.q_heads, kv_heads = a.kv_heads, bs = a.bs;
+    const int row = pair / q_heads, h = pair - row * q_heads;
+    const int ratio = q_heads / kv_heads, kvh = h / ratio;
+    const int tiles = (q_heads + 2 * kv_heads) * 8;
+    const int t = lane >> 2, qd = lane & 3;
+    const coh_rsrc_t krs = coh_rsrc(L.kc), vrs = coh_rsrc(L.vc), qrs = coh_rsrc(in + CP_QKV), ars = coh_rsrc(out + CP_ATT);
+    if (lane < 16) flow_clear16(coh_rsrc(clr + CP_ATT), (uint32_t)frag_off(row, h * 128 + 8 * lane, q_heads * 128) * 2);
+    const u32x4 (&kq)[4] = hist.k;
+    const uint32_t (&vq)[16] = hist.v;
+    CH_STAMP_BY(stamps, sidx, 1, 256);
+    // ---- this row's q / k / v heads out of the qkv stage's tiles, one dword per lane each; the (l, l + 64) pairing of the norm + RoPE is
+    // restored through LDS
+    const uint32_t base = (uint32_t)(row >> 4) * tiles * 512 + (row & 15) * 32 + (lane >> 3) * 512 + (lane & 7) * 4;
+    uint32_t qw, kw, vnew;
+    {
+        unsigned spins = 0;
+        unsigned long long t0 = 0;
+        bool go = true;
+        do {
+            qw = coh_ld4(qrs, base + h * 4096);
+            kw = coh_ld4(qrs, base + (q_heads + kvh) * 4096);
+            vnew = coh_ld4(qrs, base + (q_heads + kv_heads + kvh) * 4096);
+        } while (__builtin_amdgcn_ballot_w64(max(max(qw, kw), vnew) == FLOW_EMPTY) != 0 && go && (go = flow_again(fw, code, spins, t0)));
+    }
+    if (fw.dead) { qw = flow_or0(qw); kw = flow_or0(kw); vnew = flow_or0(vnew); }
+    CH_STAMP_BY(stamps, sidx, 2, 256);
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");      // the clearing is complete before this use's rows go out (chain_flow.cuh)
+    uint32_t* raw = reinterpret_cast<uint32_t*>(sq + 128);        // sq: [0, 128) q in the score layout; [128, 256) raw q | k dwords
+    raw[lane] = qw;
+    raw[64 + lane] = kw;
+    __builtin_amdgcn_wave_barrier();
+    const uint16_t* rq = reinterpret_cast<const uint16_t*>(raw);
+    const uint16_t* rk = rq + 128;
+    const uint16_t* cs = a.cos_sin + (size_t)pos * 128;
+    float q0, q1, k0, k1;
+    head_norm_rope_vals(bf2f(rq[lane]), bf2f(rq[lane + 64]), L.qnorm, cs, a.eps, lane, q0, q1);
+    head_norm_rope_vals(bf2f(rk[lane]), bf2f(rk[lane + 64]), L.knorm, cs, a.eps, lane, k0, k1);
+    if (h % ratio == 0) {
+        // the new token's K / V into the private cache: one dword per lane (even lanes elements l, l + 1 of the first half, odd lanes l + 63,
+        // l + 64 of the second), written through for the later passes
+        const uint32_t crow = ((uint32_t)(row * bs + pos) * kv_heads + kvh) * 128;
+        const uint32_t kb0 = f2bf(k0), kb1 = f2bf(k1);
+        const uint32_t n0 = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)kb0, OMNI_DPP_XOR1, 0xF, 0xF, true);
+        const uint32_t n1 = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)kb1, OMNI_DPP_XOR1, 0xF, 0xF, true);
+        const bool odd = (lane & 1) != 0;
+        const uint32_t word = odd ? (n1 | (kb1 << 16)) : (kb0 | (n0 << 16));
+        const uint32_t elem = odd ? 64 + lane - 1 : lane;
+        coh_st4(krs, (crow + elem) * 2, word);
+        coh_st4(vrs, (crow + 2 * lane) * 2, vnew);
+    }
+    const float qs = a.sm_scale * LOG2E;
+    const float s_new = wave_sum(fmaf(q0 * qs, k0, (q1 * qs) * k1));
+    sq[lane] = q0 * qs;
+    sq[lane + 64] = q1 * qs;
+    __builtin_amdgcn_wave_barrier();
+    float d = 0.f;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+        const f32x4 qa = *reinterpret_cast<const f32x4*>(&sq[qd * 32 + j * 8]);
+        const f32x4 qb = *reinterpret_cast<const f32x4*>(&sq[qd * 32 + j * 8 + 4]);
+        d = fmaf(qa[0], bf_lo(kq[j][0]), d); d = fmaf(qa[1], bf_hi(kq[j][0]), d);
+        d = fmaf(qa[2], bf_lo(kq[j][1]), d); d = fmaf(qa[3], bf_hi(kq[j][1]), d);
+        d = fmaf(qb[0], bf_lo(kq[j][2]), d); d = fmaf(qb[1], bf_hi(kq[j][2]), d);
+        d = fmaf(qb[2], bf_lo(kq[j][3]), d); d = fmaf(qb[3], bf_hi(kq[j][3]), d);
+    }
+    d += dpp_f<OMNI_DPP_XOR1>(d);
+    d += dpp_f<OMNI_DPP_XOR2>(d);
+    const float s = t < pos ? d : -INFINITY;
+    float m = fmaxf(s, dpp_f<OMNI_DPP_HALF_MIRROR>(s));
+    m = fmaxf(m, dpp_f<OMNI_DPP_MIRROR>(m));
+    m = xor32_max(xor16_max(m));
+    m = fmaxf(m, s_new);
+    const float p = exp2f(s - m);
+    const float p_new = exp2f(s_new - m);
+    float lsum = p + dpp_f<OMNI_DPP_HALF_MIRROR>(p);
+    lsum += dpp_f<OMNI_DPP_MIRROR>(lsum);
+    lsum = xor32_sum(xor16_sum(lsum));
+    const float inv = 1.0f / (lsum + p_new);
+    float o0 = p_new * bf_lo(vnew), o1 = p_new * bf_hi(vnew);
+#pragma unroll
+    for (int u = 0; u < 16; ++u) {
+        const float pu = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(p), 4 * u));
+        o0 = fmaf(pu, bf_lo(vq[u]), o0);
+        o1 = fmaf(pu, bf_hi(vq[u]), o1);
+    }
+    coh_st4(ars, (uint32_t)frag_off(row, h * 128 + 2 * lane, q_heads * 128) * 2, flow_word(pack_bf2(o0 * inv, o1 * inv)));
+    CH_STAMP_BY(stamps, sidx, 6, 256);
+    CH_STAMP_BY(stamps, sidx, 7, 256);
+}
+
+// the sampler stage of pass g by the workgroup that owns batch row b: draws code g of row b from the head stage's logits and, unless this was the
+// last group, gathers the folded embedding -> projection row of the drawn code as the next pass's input (slab 0 = its sum of squares).  The pick
+// is wave 0's alone (sampler_body.cuh smp_pick_wave); rows that ask for top-p take the four-wave pick
+template <bool TAIL>
+__device__ __forceinline__ void flow_sample(const ChainArgs& a, int g, int b, float* lds, const char* in, char* out, char* clr, FlowWait& fw, int code,
+                                            unsigned long long* stamps) {
+    const int sidx = 26;
+    int* const last_code = reinterpret_cast<int*>(lds + CPF_LAST_FLOATS);
+    CH_STAMP(stamps, sidx, 0);
+    int tid = threadIdx.x;
+    asm volatile("" : "+v"(tid));       // opaque per call (flow_gemm)
+    const int lane = tid & 63;
+    const bool more = g < a.Q - 1 && a.ptab != nullptr;
+    const int V = a.codebook, Hc = 1024;
+    const coh_rsrc_t lrs = coh_rsrc(in + CP_LOG), rrs = coh_rsrc(out + CP_R0), prs = coh_rsrc(out + CP_P0);
+    const uint32_t base = (uint32_t)(b >> 4) * 128 * 1024 + (b & 15) * 64;        // logit i of the row: base + (i / 16) * 1024 + (i % 16) * 4
+    if (tid < 64) {
+        const coh_rsrc_t c0 = coh_rsrc(clr + CP_R0), cl = coh_rsrc(clr + CP_P0);
+        flow_clear16(c0, (uint32_t)frag_off(b, lane * 8, Hc) * 2);
+        flow_clear16(c0, (uint32_t)frag_off(b, (lane + 64) * 8, Hc) * 2);
+        if (lane == 0) coh_st4(cl, (uint32_t)b * 4, FLOW_EMPTY);
+    }
+    const uint32_t seed = a.row_seed ? a.row_seed[b] : a.seed;
+    const uint32_t step = (uint32_t)(a.steps ? a.steps[b] * a.Q + g : g);
+    CH_STAMP(stamps, sidx, 1);
+    // workgroup-uniform: kernel arguments only
+    const bool wave_path = a.greedy || !(a.top_p > 0.f && a.top_p < 1.f);
+    const SmpLds S = smp_carve<8>(lds + CPF_SMP_FLOATS);
+    int pick = 0;
+    if (wave_path) {
+        if (tid < 64) {
+            // a moderate temperature keeps the head GEMM's bf16-exact logits strictly ordered under the division: select first, divide the kept
+            const bool late = !a.greedy && a.temperature >= 1.0f / 64 && a.temperature <= 64.0f;
+            float xr[32];
+            unsigned spins = 0;
+            unsigned long long t0 = 0;
+            for (;;) {
+                uint32_t w = 0;
+#pragma unroll
+                for (int j8 = 0; j8 < 8; ++j8) {
+                    const u32x4 v4 = coh_ld16(lrs, base + (j8 * 16 + (lane >> 2)) * 1024 + (lane & 3) * 16);
+                    w = max(w, flow_max(v4));
+#pragma unroll
+                    for (int c = 0; c < 4; ++c) xr[j8 * 4 + c] = __uint_as_float(v4[c]);
+                }
+                if (__builtin_amdgcn_ballot_w64(w == FLOW_EMPTY) == 0 || !flow_again(fw, code, spins, t0)) break;
+            }
+            if (fw.dead) {
+#pragma unroll
+                for (int e = 0; e < 32; ++e) xr[e] = flow_or0(xr[e]);
+            }
+            CH_STAMP(stamps, sidx, 2);
+            // (both fix-ups behind wave-uniform branches the optimiser cannot turn into 32 selects: as straight-line code they were 32 IEEE
+            //  divisions on every pick)
+            if (V < 2048) {
+                asm volatile("" ::: "memory");
+#pragma unroll
+                for (int e = 0; e < 32; ++e)
+                    if ((e >> 2) * 256 + 4 * lane + (e & 3) >= V) xr[e] = -INFINITY;
+            }
+            if (!a.greedy && !late) {
+                asm volatile("" ::: "memory");
+#pragma unroll
+                for (int e = 0; e < 32; ++e) xr[e] = xr[e] / a.temperature;
+            }
+            pick = smp_pick_wave<32>(xr, V, a.greedy, a.top_k, late, a.temperature, seed, step, S.ckey);
+        }
+    } else {
+        constexpr int NPT = 8;
+        const bool live = tid < SMP_THREADS;
+        float xr[NPT];
+        unsigned spins = 0;
+        unsigned long long t0 = 0;
+        for (;;) {
+            uint32_t w = 0;
+#pragma unroll
+            for (int e = 0; e < NPT; ++e) {
+                const int i = tid + e * SMP_THREADS;
+                uint32_t v = __float_as_uint(-INFINITY);
+                if (live && i < V) v = coh_ld4(lrs, base + (i >> 4) * 1024 + (i & 15) * 4);
+                w = max(w, v);
+                xr[e] = __uint_as_float(v);
+            }
+            if (__builtin_amdgcn_ballot_w64(w == FLOW_EMPTY) == 0 || !flow_again(fw, code, spins, t0)) break;
+        }
+        if (fw.dead) {
+#pragma unroll
+            for (int e = 0; e < NPT; ++e) xr[e] = flow_or0(xr[e]);
+        }
+        if (!a.greedy) {
+#pragma unroll
+            for (int e = 0; e < NPT; ++e) {
+                const int i = tid + e * SMP_THREADS;
+                if (live && i < V) xr[e] = xr[e] / a.temperature;
+            }
+        }
+        pick = smp_pick<NPT>(xr, V, a.greedy, a.top_k, a.top_p, seed, step, S, live, stamps);
+    }
+    CH_STAMP(stamps, sidx, 4);
+    if (tid < 64) {
+        if (more) {
+            // the folded embedding -> projection row of the drawn code: lane l moves 16-byte pieces l and l + 64 of the 2 KB row; the slab value in
+            // sample_kernel's order of additions (piece sums, one wave_sum per 64 pieces, then the two halves)
+            const uint16_t* tab = a.ptab + ((size_t)(g - 1) * a.codebook + pick) * Hc;
+            float ss2[2];
+            u32x4 w4[2];
+#pragma unroll
+            for (int h2 = 0; h2 < 2; ++h2) w4[h2] = ld16(tab + (lane + 64 * h2) * 8);
+            asm volatile("s_waitcnt vmcnt(0)" ::: "memory");      // the clearing is complete (chain_flow.cuh)
+#pragma unroll
+            for (int h2 = 0; h2 < 2; ++h2) {
+                u32x4 o;
+#pragma unroll
+                for (int j = 0; j < 4; ++j) o[j] = flow_word(w4[h2][j]);
+                coh_st16(rrs, (uint32_t)frag_off(b, (lane + 64 * h2) * 8, Hc) * 2, o);
+                float ss = 0.f;
+#pragma unroll
+                for (int j = 0; j < 4; ++j) ss += bf_lo(w4[h2][j]) * bf_lo(w4[h2][j]) + bf_hi(w4[h2][j]) * bf_hi(w4[h2][j]);
+                ss2[h2] = wave_sum(ss);
+            }
+            if (lane == 0) coh_st4(prs, (uint32_t)b * 4, flow_word(__float_as_uint(((ss2[0] + ss2[1]) + 0.f) + 0.f)));
+        }
+        if (lane == 0) {
+            coh_st4(coh_rsrc(a.codes), ((uint32_t)b * a.Q + g) * 4, (uint32_t)pick);
+            last_code[0] = pick;
+        }
+    }
+    if (TAIL && g == a.Q - 1 && a.tail.enabled) {
+        // the row's frame is complete: its owner assembles the backbone's input row right here (no hand-off: the last code is its own)
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        __syncthreads();
+        chain_finalize_row(ChainFinArgs{a.tail, a.codes, a.Q, a.codebook}, b, last_code[0], lds);
+    }
+    CH_STAMP(stamps, sidx, 6);
+    CH_STAMP(stamps, sidx, 7);
+}
+
 // the tail's qkv stage as a real call on a copy of the gate (the launch ends behind it: nothing reads the gate afterwards)
 template <int KHT>
 __device__ __attribute__((noinline)) void chain_tail_qkv(const ChainArgs::Tail T, int B, float eps, float* lds, ChainGate g, int code) {
@@ -473,84 +640,177 @@ __device__ __attribute__((noinline)) void chain_tail_qkv(const ChainArgs::Tail T
                                                true, code, nullptr);
 }
 
-// KHT: 0, or hidden / 256 of the backbone whose first qkv stage closes the launch (the tail: round 6)
-template <bool GU_NARROW, bool DEFER = true, int KHT = 0>
+// ROWS: the most rows the launch's split of a stage over the 256 workgroups is for
+//   16   every stage but o_proj / down_proj over (nearly) all workgroups: qkv 16 columns each, gate_up 16 activation columns on 192, head 16 on
+//        128; o_proj / down_proj (64 tiles of 16 columns) on the other 64, whose weights then wait in registers before gate_up has begun.  (64
+//        workgroups for everything, the other 192 idle, pull four times as much each: a pass 104 us behind flags)
+//   32   qkv 16 columns x 32 rows each; o_proj / down_proj on 128 workgroups, gate_up (24 activation columns x 32 rows) and head on the others
+//   48, 64  a row group of 16 owns 64 workgroups (gate_up at 64: 24 activation columns x 32 rows): three row groups divide no better, four fill the
+//        chip
+// KHT: 0, or hidden / 256 of the backbone whose first qkv stage closes the launch (the tail)
+template <int ROWS, int KHT = 0>
 __global__ __launch_bounds__(CH_THREADS) void cp_chain_kernel(const ChainArgs a) {
-    __shared__ __attribute__((aligned(16))) float lds[CH_LDS_FLOATS];
-    static_assert(CH_LDS_FLOATS * 4 >= SMP_LDS_BYTES(8), "sampler working set must fit the chain's LDS");
+    extern __shared__ __attribute__((aligned(16))) float lds[];
+    static_assert(KHT == 0 || ROWS == 64, "the tail needs every row group live");
     ChainGate g;
     chain_gate_init(g, a.flags, a.err);
-    g.dom = a.dom;
-    g.nap = a.nap & 31;
-    if (a.nap >> 5) g.skip_units = (a.nap >> 5) - 1;      // debug library: nap + 32 (units + 1) selects the run-ahead sleep (coherent.cuh)
-    g.skip = a.skip;
-    const int wg = blockIdx.x;
-    {
-        // a partly filled batch: a workgroup that owns no live row in ANY stage of the launch (its 16-row group, its 32-row gate_up
-        // pair, its four attention pairs, its sampler row) publishes the launch's final stage count at once and leaves -- the others
-        // find its flag ahead of every stage they wait for, and it never polls
-        const int rows_per_dom = 16 << (a.dom - 6), wi = wg & ((1 << a.dom) - 1);
-        const bool gemm16 = (wg >> 6) * 16 < a.B, gemm32 = GU_NARROW && (wg >> 7) * 32 < a.B, attn_ = wg * 4 < a.B * a.q_heads;
-        const bool smp = a.with_head && wi < rows_per_dom && (wg >> a.dom) * rows_per_dom + wi < a.B;
-        if (!(gemm16 || gemm32 || attn_ || smp)) {
-            const uint32_t total = (uint32_t)(a.g1 - a.g0) * (uint32_t)(a.layers * 5 + (a.with_head ? 2 : 0)) + ((KHT > 0 && a.tail.enabled) ? 1u : 0u);
-            if (threadIdx.x < 64) chain_flag_publish(g.frs, wg, g.epoch + total);
-            return;
+    const int Hc = 1024, NQ = 4096, NI = 3072, B = a.B;
+    const int wg0 = blockIdx.x, wave = threadIdx.x >> 6;
+    constexpr bool SPLIT = ROWS <= 32;
+    constexpr int NO = ROWS == 16 ? 64 : 128;                    // SPLIT: workgroups of o_proj / down_proj; the others do gate_up
+    if (!SPLIT && (wg0 >> 6) * 16 >= B) {                        // a row group without rows: nobody waits for it beyond the launch's first gate
+        if (threadIdx.x < 64) chain_flag_publish(g.frs, wg0, g.epoch + 1u);
+        return;
+    }
+    FlowWait fw{a.err, g.dead ? 1 : 0};
+    float* const attn_lds = lds + CPF_ATTN_FLOATS + wave * 256;
+    // ---- this workgroup's part of each stage
+    const bool does_o = !SPLIT || wg0 < NO, does_gu = !SPLIT || wg0 >= NO;
+    const bool does_head = a.with_head && (!SPLIT || wg0 >= 128);
+    const int smp_row = ROWS == 16 ? wg0 - 64 : (ROWS == 32 ? wg0 : ((wg0 & 63) < 16 ? (wg0 >> 6) * 16 + (wg0 & 63) : 64));
+    const bool does_smp = a.with_head && smp_row >= 0 && smp_row < B;
+    constexpr int PPW = SPLIT ? 2 : 4;                           // (row, q head) pairs per workgroup: waves 4 .. 4 + PPW - 1
+    const int pair = (ROWS == 16 ? wg0 - 64 : wg0) * PPW + wave - 4;
+    const bool does_attn = wave >= 4 && wave < 4 + PPW && pair >= 0 && pair < B * a.q_heads;
+    // ---- empty this workgroup's tiles of every copy; the launch's first gate tells the others (chain_flow.cuh)
+    for (int c = 0; c < FLOW_COPIES; ++c) {
+        char* const cb = a.flow + (size_t)c * CP_COPY;
+        const int tid = threadIdx.x;
+        auto fill = [&](uint32_t off, int pieces) {
+            const coh_rsrc_t rs = coh_rsrc(cb + off);
+            for (int i = tid; i < pieces; i += CH_THREADS) flow_clear16(rs, i * 16);
+        };
+        if (ROWS == 16) fill(CP_QKV + wg0 * 512, 32);
+        else if (ROWS == 32) { fill(CP_QKV + wg0 * 512, 32); fill(CP_QKV + 256 * 512 + wg0 * 512, 32); }
+        else fill(CP_QKV + (wg0 >> 6) * 256 * 512 + (wg0 & 63) * 2048, 128);
+        if (does_attn && (tid & 63) < 16) flow_clear16(coh_rsrc(cb + CP_ATT), (uint32_t)frag_off(pair / a.q_heads, (pair % a.q_heads) * 128 + 8 * (tid & 15), a.q_heads * 128) * 2);
+        if (does_o) {
+            const int bx = wg0 & 63, by = wg0 >> 6;
+            fill(CP_RA + by * 32768 + bx * 512, 32); fill(CP_RB + by * 32768 + bx * 512, 32);
+            fill(CP_PA + (bx * 64 + by * 16) * 4, 4); fill(CP_PB + (bx * 64 + by * 16) * 4, 4);
+        }
+        if (does_gu) {
+            if (ROWS == 16) fill(CP_ACT + (wg0 - NO) * 512, 32);
+            else if (ROWS == 48) fill(CP_ACT + (wg0 >> 6) * 98304 + (wg0 & 63) * 1536, 96);
+            else {
+                const int bx = ROWS == 32 ? wg0 - NO : wg0 & 127, by = ROWS == 32 ? 0 : wg0 >> 7;
+                fill(CP_ACT + by * 196608 + bx * 768, 48); fill(CP_ACT + by * 196608 + 98304 + bx * 768, 48);
+            }
+        }
+        if (does_head) {
+            if (ROWS == 16) fill(CP_LOG + (wg0 - 128) * 1024, 64);
+            else if (ROWS == 32) { fill(CP_LOG + (wg0 - 128) * 1024, 64); fill(CP_LOG + 131072 + (wg0 - 128) * 1024, 64); }
+            else fill(CP_LOG + (wg0 >> 6) * 131072 + (wg0 & 63) * 2048, 128);
+        }
+        if (does_smp && tid < 128) {
+            flow_clear16(coh_rsrc(cb + CP_R0), (uint32_t)frag_off(smp_row, tid * 8, Hc) * 2);
+            if (tid == 0) coh_st4(coh_rsrc(cb + CP_P0), smp_row * 4, FLOW_EMPTY);
         }
     }
-    int np = a.np_in;
-    const int Hc = 1024, NQ = 4096, NI = 3072;
+    chain_gate_arrive(g);
+
+    int cl = 0, cp = 0, half = 0;                                // copies of this layer's and this pass's hand-offs; LDS half of the next combine
+    bool open = false;                                           // the launch's first gate is behind us
+    u32x2 res = (u32x2){0u, 0u}, none = res;
     for (int pass = a.g0; pass < a.g1; ++pass) {
-        const int pc = pass << 8;            // error-word stage codes: (pass << 8) | (16 * layer + stage + 1); head 0xF1, sampler 0xF2
-        // debug library: every pass stamps its own block of CH_STAMP_PASS words (round 6: the cold tail of the passes in the real step)
+        const int pc = pass << 8;            // error-word stage codes: (pass << 8) | (16 * layer + stage + 1); head 0x56, sampler 0xF2
+        // debug library: every pass stamps its own block of CH_STAMP_PASS words
         unsigned long long* const st = a.stamps ? a.stamps + (size_t)pass * CH_STAMP_PASS : nullptr;
+        const int cpn = cp == FLOW_COPIES - 1 ? 0 : cp + 1, cpl = cp == 0 ? FLOW_COPIES - 1 : cp - 1;
+        char *const pb = a.flow + (size_t)cp * CP_COPY, *const pbn = a.flow + (size_t)cpn * CP_COPY, *const pbl = a.flow + (size_t)cpl * CP_COPY;
+        const bool first = pass == a.g0;
+        char* last = nullptr;                                    // copy of the previous layer
         for (int l = 0; l < a.layers; ++l) {
             const ChainLayer& L = a.layer[l];
             // the workgroup index, opaque per layer: hipcc otherwise hoists every tile / k-step offset of every stage (they depend on
-            // blockIdx only) out of both loops and parks ~450 of them in VGPR lanes for the whole launch (v_writelane / v_readlane)
+            // blockIdx only) out of both loops and parks them in VGPR lanes for the whole launch (v_writelane / v_readlane)
             int wg = blockIdx.x;
             asm volatile("" : "+s"(wg));
-            chain_gemm<1, 4, 4, DEFER ? 3 : 2, OMNI_EPI_BF16>(L.wqkv, L.ln1, a.resid, a.part, np, a.qkv, NQ, nullptr, a.B, NQ, a.eps, wg & 63, wg >> 6, lds, g,
-                                                              l > 0 || pass > a.g0, pc | (16 * l + 1), st);
-            chain_attn(a, L, pass, lds, g, pc | (16 * l + 2), st);
-            chain_gemm<1, 1, 8, 0, OMNI_EPI_RESID>(L.wo, nullptr, a.attn, nullptr, 0, a.resid, 0, a.part, a.B, Hc, a.eps, wg & 63, wg >> 6, lds, g,
-                                                   true, pc | (16 * l + 3), st);
-            np = Hc / 16;
-            if (GU_NARROW)
-                chain_gemm<2, 3, 4, DEFER ? 3 : 2, OMNI_EPI_SILU_MUL_GU8>(L.wgu, L.ln2, a.resid, a.part, np, a.act, 0, nullptr, a.B, NI, a.eps, wg & 127, wg >> 7,
-                                                                          lds, g, true, pc | (16 * l + 4), st);
-            else   // 16 rows x 48 act columns: half the in-register RMSNorm per workgroup, a weight slice twice as wide (prefetched)
-                chain_gemm<1, 6, 4, DEFER ? 3 : 2, OMNI_EPI_SILU_MUL_GU8>(L.wgu, L.ln2, a.resid, a.part, np, a.act, 0, nullptr, a.B, NI, a.eps, wg & 63, wg >> 6,
-                                                                          lds, g, true, pc | (16 * l + 4), st);
-            chain_gemm<1, 1, 12, 0, OMNI_EPI_RESID>(L.wdown, nullptr, a.act, nullptr, 0, a.resid, 0, a.part, a.B, Hc, a.eps, wg & 63, wg >> 6, lds, g,
-                                                    true, pc | (16 * l + 5), st);
+            const int cn = cl == FLOW_COPIES - 1 ? 0 : cl + 1;
+            char *const lb = a.flow + (size_t)cl * CP_COPY, *const nb = a.flow + (size_t)cn * CP_COPY;
+            auto area = [&]() -> float* { half ^= 1; return lds + half * FLOW_HALF_FLOATS; };
+            // the pass's own input: raw rows; behind o_proj and down_proj the stream travels as bf16(w r) of the norm in front of its consumer
+            const void* xin = first ? (const void*)a.resid : (const void*)(pbl + CP_R0);
+            const float* pin = first ? a.part : (const float*)(pbl + CP_P0);
+            const int np = first ? a.np_in : 1;
+            const bool given = first;
+            constexpr int QMT = ROWS == 32 ? 2 : 1, QNT = SPLIT ? 1 : 4;
+            // the attention's history (written by earlier passes, rows >= pass hold stale bytes and are masked): there before its q / k / v
+            FlowHist hist;
+            if (does_attn) flow_history(a, L, pair, hist);
+            if (l == 0)
+                flow_gemm<QMT, QNT, 4, 3, OMNI_EPI_BF16>(L.wqkv, L.ln1, xin, pin, np, lb + CP_QKV, nullptr, nb + CP_QKV, nullptr, B, NQ, a.eps,
+                                                         SPLIT ? wg : wg & 63, SPLIT ? 0 : wg >> 6, area(), none, fw, pc | (16 * l + 1), st, given);
+            else
+                flow_gemm<QMT, QNT, 4, 4, OMNI_EPI_BF16>(L.wqkv, nullptr, last + CP_RB, (const float*)(last + CP_PB), Hc / 16, lb + CP_QKV, nullptr, nb + CP_QKV,
+                                                         nullptr, B, NQ, a.eps, SPLIT ? wg : wg & 63, SPLIT ? 0 : wg >> 6, area(), none, fw, pc | (16 * l + 1), st);
+            if (!open) {                                         // everybody's tiles are empty: the first content that is waited for lies behind this
+                chain_gate_wait(g, pc | (16 * l + 2));
+                fw.dead = flow_failed(a.err);
+                open = true;
+            }
+            if (does_attn) flow_attn(a, L, pass, pair, attn_lds, lb, lb, nb, hist, fw, pc | (16 * l + 2), st);
+            const bool to_plain = !a.with_head && l == a.layers - 1;       // the stream leaves the launch
+            if (does_o) {
+                const int bx = wg & 63, by = wg >> 6;
+                // this thread's residual values: kept in registers from stage to stage, the pass's own from its input rows
+                if (l == 0 && threadIdx.x < 64 && by * 16 + (threadIdx.x & 15) < B) {
+                    res = coh_ld8(coh_rsrc(xin), (uint32_t)frag_off(by * 16 + (threadIdx.x & 15), bx * 16 + 4 * (threadIdx.x >> 4), Hc) * 2);
+                    if (fw.dead) res = (u32x2){flow_or0(res[0]), flow_or0(res[1])};
+                }
+                flow_gemm<1, 1, 8, 0, OMNI_EPI_RESID>(L.wo, L.ln2, lb + CP_ATT, nullptr, 0, lb + CP_RA, (float*)(lb + CP_PA), nb + CP_RA, (float*)(nb + CP_PA), B,
+                                                      Hc, a.eps, bx, by, area(), res, fw, pc | (16 * l + 3), st);
+            }
+            if (does_gu) {
+                if (ROWS == 16)
+                    flow_gemm<1, 2, 4, 4, OMNI_EPI_SILU_MUL_GU8>(L.wgu, nullptr, lb + CP_RA, (const float*)(lb + CP_PA), Hc / 16, lb + CP_ACT, nullptr, nb + CP_ACT,
+                                                                 nullptr, B, NI, a.eps, wg - NO, 0, area(), none, fw, pc | (16 * l + 4), st);
+                else if (ROWS == 48)
+                    flow_gemm<1, 6, 4, 4, OMNI_EPI_SILU_MUL_GU8>(L.wgu, nullptr, lb + CP_RA, (const float*)(lb + CP_PA), Hc / 16, lb + CP_ACT, nullptr, nb + CP_ACT,
+                                                                 nullptr, B, NI, a.eps, wg & 63, wg >> 6, area(), none, fw, pc | (16 * l + 4), st);
+                else
+                    flow_gemm<2, 3, 4, 4, OMNI_EPI_SILU_MUL_GU8>(L.wgu, nullptr, lb + CP_RA, (const float*)(lb + CP_PA), Hc / 16, lb + CP_ACT, nullptr, nb + CP_ACT,
+                                                                 nullptr, B, NI, a.eps, ROWS == 32 ? wg - NO : wg & 127, ROWS == 32 ? 0 : wg >> 7, area(), none, fw,
+                                                                 pc | (16 * l + 4), st);
+            }
+            if (does_o)
+                flow_gemm<1, 1, 12, 0, OMNI_EPI_RESID>(L.wdown, l < a.layers - 1 ? a.layer[l + 1].ln1 : nullptr, lb + CP_ACT, nullptr, 0, to_plain ? (void*)a.resid : lb + CP_RB,
+                                                       to_plain ? a.part : (float*)(lb + CP_PB), nb + CP_RB, (float*)(nb + CP_PB), B, Hc, a.eps, wg & 63, wg >> 6,
+                                                       area(), res, fw, pc | (16 * l + 5), st);
+            last = lb;
+            cl = cn;
         }
         if (!a.with_head) continue;
         int wg = blockIdx.x;
         asm volatile("" : "+s"(wg));
         // group `pass`: final norm folded into the head GEMM (2048 logits per row), then one workgroup per row samples
-        chain_gemm<1, 2, 4, 2, OMNI_EPI_F32_BF16RND>(a.lm_head + (size_t)(pass - 1) * a.codebook * Hc, a.cp_norm, a.resid, a.part, np,
-                                                     a.logits + (size_t)(pass - 1) * a.logits_pass, a.logits_ld, nullptr, a.B, a.codebook, a.eps,
-                                                     wg & 63, wg >> 6, lds, g, true, pc | 0x56, st);
-        chain_sample<(KHT > 0)>(a, pass, lds, g, pc | 0xF2, st);
-        np = 1;
+        if (does_head) {
+            half ^= 1;
+            constexpr int HMT = ROWS == 32 ? 2 : 1, HNT = SPLIT ? 1 : 2;
+            flow_gemm<HMT, HNT, 4, 2, OMNI_EPI_F32_BF16RND>(a.lm_head + (size_t)(pass - 1) * a.codebook * Hc, a.cp_norm, last + CP_RB, (const float*)(last + CP_PB),
+                                                            Hc / 16, pb + CP_LOG, nullptr, pbn + CP_LOG, nullptr, B, a.codebook, a.eps, SPLIT ? wg - 128 : wg & 63,
+                                                            SPLIT ? 0 : wg >> 6, lds + half * FLOW_HALF_FLOATS, none, fw, pc | 0x56, st, false,
+                                                            a.logits_pass ? a.logits + (size_t)(pass - 1) * a.logits_pass : nullptr, a.logits_ld);
+        }
+        if (does_smp) flow_sample<(KHT > 0)>(a, pass, smp_row, lds, pb, pb, pbn, fw, pc | 0xF2, st);
+        cp = cpn;
     }
     if constexpr (KHT > 0) {
         if (a.tail.enabled) {
             // layer 0's qkv rows of the backbone, behind EVERY row's input assembly (flag domain: all 256 workgroups); gemm_skinny_kernel's
             // norm-fused arithmetic on 32 x 32 tiles (the bits do not depend on the tile shape: gemm_frag.cuh SlabOrder)
-            chain_tail_qkv<KHT>(a.tail, a.B, a.eps, lds, g, ((a.g1 - 1) << 8) | 0x62);
+            chain_gate_arrive(g);
+            chain_tail_qkv<KHT>(a.tail, B, a.eps, lds, g, ((a.g1 - 1) << 8) | 0x62);
         }
     }
 }
 
 // ---- host
-OMNI_KNOB g_cp_chain = 1, g_chain_dom = 7, g_chain_gu_narrow = 1, g_chain_nap = 1, g_chain_span = 2, g_chain_skip = 0, g_chain_defer = 1, g_chain_pair = 1;
+OMNI_KNOB g_cp_chain = 1, g_chain_wide = 0, g_chain_nap = 1, g_chain_span = 2, g_chain_pair = 1;
 #ifdef OMNI_DEBUG_HOOKS
-extern "C" void omni_debug_chain_mode(int dom, int gu_narrow, int nap) { g_chain_dom = dom; g_chain_gu_narrow = gu_narrow; g_chain_nap = nap; }
-extern "C" void omni_debug_chain_skip(int mode) { g_chain_skip = mode; }
-extern "C" void omni_debug_chain_defer(int on) { g_chain_defer = on; }
-extern "C" void omni_debug_chain_pair(int on) { g_chain_pair = on; }            // positions 0 / 1 + group 1 as a persistent launch (0: the launch path's pair pass)          // timing arm: rstd in the epilogues (not the reference's rounding)      // timing experiment: 1 = half the weight bytes, 2 = half the activation bytes (results garbage)
+// gu_narrow 0: above 32 rows always the 48-row split of the stages (16-row gate_up tiles); nap: the pair launch's poll pause
+extern "C" void omni_debug_chain_mode(int, int gu_narrow, int nap) { g_chain_wide = gu_narrow == 0; g_chain_nap = nap; }
+extern "C" void omni_debug_chain_pair(int on) { g_chain_pair = on; }            // positions 0 / 1 + group 1 as a persistent launch (0: the launch path's pair pass)
 static unsigned long long* g_chain_stamps = nullptr;
 // 0: launch per op; 1: one persistent launch per pass (layer stack only); 2: one persistent launch for all passes incl. heads + samplers
 extern "C" void omni_debug_cp_chain(int on) { g_cp_chain = on != 0; g_chain_span = on; }
@@ -606,7 +866,7 @@ int k_cp_pair(const omni_talker_desc& d, const omni_layer_weights* layers, uint1
     a.temperature = head->temperature; a.top_p = head->top_p; a.seed = head->seed;
     a.steps = head->steps; a.row_seed = head->row_seed; a.codes = head->codes;
     a.ptab = (const uint16_t*)d.cp_proj_table;
-    a.dom = 8; a.nap = g_chain_nap;
+    a.nap = g_chain_nap;
 #ifdef OMNI_DEBUG_HOOKS
     a.stamps = g_chain_stamps;            // block 0 of the stamp buffer (the chain's passes 2 .. 15 stamp blocks 2 .. 15)
 #endif
@@ -629,13 +889,13 @@ bool k_cp_chain_tail_supported(const omni_talker_desc& d, int B) {
     const int NQ = (d.q_heads + 2 * d.kv_heads) * 128;
     // every row group live (B > 48: no workgroup leaves at launch start, all of them own a qkv tile with rows), the norm-free stream, the
     // qkv stage's 32 x 32 tile grid inside the 256 workgroups
-    return g_chain_tail && g_chain_defer && g_chain_gu_narrow && g_cp_chain && g_chain_span >= 2 && listed && B > 48 && B <= 64 && d.fused_norm && d.frag_layout && d.moe_experts == 0 && d.head_dim == 128 &&
+    return g_chain_tail && !g_chain_wide && g_cp_chain && g_chain_span >= 2 && listed && B > 48 && B <= 64 && d.fused_norm && d.frag_layout && d.moe_experts == 0 && d.head_dim == 128 &&
            NQ % 32 == 0 && (NQ / 32) * 2 <= OMNI_CHAIN_WGS && d.hidden % 8 == 0;
 }
 
 int k_cp_chain(const omni_talker_desc& d, const omni_layer_weights* layers, uint16_t* const* k_cache, uint16_t* const* v_cache, int B,
-               int g0, int g1, int np_in, uint16_t* resid, float* part, uint16_t* qkv, uint16_t* attn, uint16_t* act, uint32_t* flags,
-               int32_t* err, const omni_chain_head* head, void* stream) {
+               int g0, int g1, int np_in, uint16_t* resid, float* part, uint32_t* flags,
+               int32_t* err, void* flow, const omni_chain_head* head, void* stream) {
     ChainArgs a{};
     for (int l = 0; l < d.cp_layers; ++l) {
         const omni_layer_weights& w = layers[l];
@@ -646,7 +906,7 @@ int k_cp_chain(const omni_talker_desc& d, const omni_layer_weights* layers, uint
     a.layers = d.cp_layers; a.B = B; a.g0 = g0; a.g1 = g1; a.bs = d.num_code_groups + 1; a.np_in = np_in;
     a.q_heads = d.cp_q_heads; a.kv_heads = d.cp_kv_heads;
     a.eps = d.eps; a.sm_scale = 1.0f / sqrtf((float)d.cp_head_dim);
-    a.resid = resid; a.part = part; a.qkv = qkv; a.attn = attn; a.act = act;
+    a.resid = resid; a.part = part; a.flow = (char*)flow;
     a.cos_sin = (const uint16_t*)d.cp_cos_sin;
     a.flags = flags; a.err = err;
     if (head) {
@@ -658,39 +918,39 @@ int k_cp_chain(const omni_talker_desc& d, const omni_layer_weights* layers, uint
         a.steps = head->steps; a.row_seed = head->row_seed; a.codes = head->codes;
         a.ptab = (const uint16_t*)d.cp_proj_table;
     }
-    a.dom = g_chain_dom < 6 ? 6 : (g_chain_dom > 8 ? 8 : g_chain_dom);
-    // (32-row gate_up tiles from 49 rows: at 33-48 rows the launch path takes 16-row tiles too since round 5 -- gemm.hip pick_tile -- so
-    //  that the fourth row group has no work in any stage and its workgroups leave at the start of the launch)
-    const bool narrow = g_chain_gu_narrow == 2 || (g_chain_gu_narrow && B > 48);      // 2 (debug): the 32-row tile at any batch size
-    if (narrow && a.dom < 7) a.dom = 7;  // the 32-row tile ties two row groups together
-    a.skip = g_chain_skip;
-    // gate_up's RMSNorm statistics are summed in an order that depends on the rows per tile: follow the launch path's tile
-    // policy (32-row tiles only above 32 rows) so that both schedules produce the same bits
-    a.gu_narrow = narrow;
-    a.nap = g_chain_nap;
 #ifdef OMNI_DEBUG_HOOKS
     a.stamps = g_chain_stamps;
 #endif
-#ifdef OMNI_DEBUG_HOOKS
-    if (!g_chain_defer) {      // timing arm: round 5's exact rstd (its bits are no longer the launch path's)
-        if (a.gu_narrow) hipLaunchKernelGGL((cp_chain_kernel<true, false>), dim3(OMNI_CHAIN_WGS), dim3(CH_THREADS), 0, (hipStream_t)stream, a);
-        else hipLaunchKernelGGL((cp_chain_kernel<false, false>), dim3(OMNI_CHAIN_WGS), dim3(CH_THREADS), 0, (hipStream_t)stream, a);
-        OMNI_CHECK_LAUNCH("cp_chain(exact rstd)");
-        return OMNI_OK;
+    static bool attr = false;
+    if (!attr) {
+        (void)hipFuncSetAttribute((const void*)cp_chain_kernel<16>, hipFuncAttributeMaxDynamicSharedMemorySize, CPF_LDS_BYTES);
+        (void)hipFuncSetAttribute((const void*)cp_chain_kernel<32>, hipFuncAttributeMaxDynamicSharedMemorySize, CPF_LDS_BYTES);
+        (void)hipFuncSetAttribute((const void*)cp_chain_kernel<48>, hipFuncAttributeMaxDynamicSharedMemorySize, CPF_LDS_BYTES);
+        (void)hipFuncSetAttribute((const void*)cp_chain_kernel<64>, hipFuncAttributeMaxDynamicSharedMemorySize, CPF_LDS_BYTES);
+#define X(KH_) (void)hipFuncSetAttribute((const void*)cp_chain_kernel<64, KH_>, hipFuncAttributeMaxDynamicSharedMemorySize, CPF_LDS_BYTES);
+        CP_TAIL_WIDTHS(X)
+#undef X
+        attr = true;
     }
-#endif
-    if (head && head->tail && g1 == d.num_code_groups && a.gu_narrow && k_cp_chain_tail_supported(d, B)) {
+#define CP_LAUNCH(...)                                                                                                                              \
+    do {                                                                                                                                             \
+        hipLaunchKernelGGL((cp_chain_kernel<__VA_ARGS__>), dim3(OMNI_CHAIN_WGS), dim3(CH_THREADS), CPF_LDS_BYTES, (hipStream_t)stream, a);           \
+        OMNI_CHECK_LAUNCH("cp_chain");                                                                                                               \
+        return OMNI_OK;                                                                                                                              \
+    } while (0)
+    if (head && head->tail && g1 == d.num_code_groups && k_cp_chain_tail_supported(d, B)) {
         // the launch ends in the step's input assembly + layer 0's qkv (instantiated per backbone width: CP_TAIL_WIDTHS)
         const omni_chain_tail& T = *head->tail;
         a.tail = ChainArgs::Tail{T.input_ids, (const uint16_t*)T.embed, T.vocab, (const uint16_t*)T.cp_embed, (const uint16_t*)T.text_step,
                                  (uint16_t*)T.x_out, (uint16_t*)T.resid, T.part, T.audio_codes, T.H,
                                  (const uint16_t*)T.wqkv, (const uint16_t*)T.ln1, (uint16_t*)T.qkv, T.NQ, 1};
-#define X(KH_) if (d.hidden == KH_ * 256) { hipLaunchKernelGGL((cp_chain_kernel<true, true, KH_>), dim3(OMNI_CHAIN_WGS), dim3(CH_THREADS), 0, (hipStream_t)stream, a); OMNI_CHECK_LAUNCH("cp_chain(tail)"); return OMNI_OK; }
+#define X(KH_) if (d.hidden == KH_ * 256) CP_LAUNCH(64, KH_);
         CP_TAIL_WIDTHS(X)
 #undef X
     }
-    if (a.gu_narrow) hipLaunchKernelGGL(cp_chain_kernel<true>, dim3(OMNI_CHAIN_WGS), dim3(CH_THREADS), 0, (hipStream_t)stream, a);
-    else hipLaunchKernelGGL(cp_chain_kernel<false>, dim3(OMNI_CHAIN_WGS), dim3(CH_THREADS), 0, (hipStream_t)stream, a);
-    OMNI_CHECK_LAUNCH("cp_chain");
-    return OMNI_OK;
+    if (B <= 16) CP_LAUNCH(16);
+    if (B <= 32) CP_LAUNCH(32);
+    if (B <= 48 || g_chain_wide) CP_LAUNCH(48);
+    CP_LAUNCH(64);
+#undef CP_LAUNCH
 }

@@ -96,9 +96,10 @@ int k_cp_pair(const omni_talker_desc& d, const omni_layer_weights* layers, uint1
               void* stream);
 bool k_cp_chain_supported(const omni_talker_desc& d, int pos);
 bool k_cp_chain_all_supported(const omni_talker_desc& d, int g0, int greedy, int top_k, float top_p);
+size_t k_cp_flow_bytes();                               // the all-pass launch's hand-off buffers (`flow`)
 int k_cp_chain(const omni_talker_desc& d, const omni_layer_weights* layers, uint16_t* const* k_cache, uint16_t* const* v_cache, int B,
-               int g0, int g1, int np_in, uint16_t* resid, float* part, uint16_t* qkv, uint16_t* attn, uint16_t* act, uint32_t* flags,
-               int32_t* err, const omni_chain_head* head, void* stream);
+               int g0, int g1, int np_in, uint16_t* resid, float* part, uint32_t* flags, int32_t* err, void* flow, const omni_chain_head* head,
+               void* stream);
 // the backbone between two attention launches (o_proj -> gate_up -> down_proj -> next layer's qkv) as one persistent launch
 // (bb_chain.hip); supported = a dense shape whose (q width, hidden, intermediate) triple is instantiated there (BB_SHAPES) and whose tile
 // grids fit 256 workgroups, at 1-64 rows on a single rank; or the 0.6B shape (bb_chain_small_kernel)

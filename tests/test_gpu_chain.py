@@ -69,6 +69,32 @@ def test_chain_is_bit_identical_to_the_launch_chain(model, B, mode):
     assert torch.equal(res[1][2], res[0][2]), "sampled codes differ between the persistent chain and the launch chain"
 
 
+@pytest.mark.parametrize("top_p", [0.0, 0.9], ids=["top-k", "top-p"])
+@pytest.mark.parametrize("B", [1, 15, 31, 33, 49, 63])
+def test_all_pass_chain_at_the_edges_of_its_row_splits(B, top_p):
+    """The all-pass launch splits its stages over the workgroups by rows (up to 16, 32, 48, 64): at the edges of each, sampled codes (both picks: one
+    wave a row, four waves with top-p), greedy codes and logits are the launch path's."""
+    d = get_dims("tts-1.7b").with_(layers=1, max_model_len=256)
+    w = make_weights(d, seed=12, std=0.02)
+    code0, e0, lh = (t.cuda() for t in _inputs(d, w, B, 7 * B))
+    res = {}
+    with L.debug_library() as lib:
+        lib.omni_debug_cp_chain.argtypes = [C.c_int]; lib.omni_debug_cp_chain.restype = None
+        try:
+            for on in (0, 2):
+                lib.omni_debug_cp_chain(on)
+                eng = _engine(d, w, kv_dtype="bf16", num_blocks=8, max_batch=64)
+                steps = torch.full((B,), 5, dtype=torch.int32, device="cuda")
+                sampled = [eng.code_predictor(code0.to(torch.int32), e0, lh, greedy=False, temperature=0.9, top_k=50, top_p=top_p, seed=3, steps=steps) for _ in range(2)]
+                codes, lg = eng.code_predictor(code0.to(torch.int32), e0, lh, greedy=True, return_logits=True)
+                assert eng.chain_error() == 0
+                res[on] = [t.cpu() for t in (*sampled, codes, lg)]
+        finally:
+            lib.omni_debug_cp_chain(2)
+    for x, y in zip(res[0], res[2]):
+        assert torch.equal(x, y)
+
+
 def test_chain_matches_oracle_at_full_predictor_depth():
     """Product library, chain on (the default): greedy codes / logits of the 5-layer, 16-group predictor vs the oracle."""
     d = get_dims("tts-1.7b").with_(layers=1, max_model_len=256)

@@ -1,20 +1,20 @@
 // The talker backbone between two attention launches as ONE persistent launch per decoder layer:
 //     o_proj(l) -> gate_up(l) -> down_proj(l) -> qkv_proj(l + 1)
 // (reference: the vLLM Qwen3 decoder layer reached through qwen3_tts_talker.py:341,414-422; four of the five launches of
-// a layer on the launch-per-op path).  Same protocol as the code-predictor chain (cp_chain.hip, chain_gemm.cuh): a stage's
-// weight slice -- 64-196 KB per workgroup, 32-96 VGPRs per lane -- goes out before the stage's flags, so the HBM stream keeps
-// running through the hand-off instead of stopping for a kernel boundary (1.65 us) plus a cold first fetch; activations
-// cross behind the flags with sc1 accesses.  Tiles = the launch path's (pick_tile at 64 rows), so results are bit-identical.
-// Shapes (round 6: parameters, not literals -- the checkpoint decides them, configuration_qwen3_tts.py:192-216): the stage set is a template
+// a layer on the launch-per-op path).  A stage's weight slice -- 64-196 KB per workgroup, 32-96 VGPRs per lane -- goes out before the
+// stage looks for its operands, so the HBM stream keeps running through the hand-off instead of stopping for a kernel boundary (1.65 us)
+// plus a cold first fetch.
+//   bb_flow_kernel, bb_flow_small_kernel   one rank, the whole chip: activations cross by content (chain_flow.cuh)
+//   bb_chain_kernel                        a tensor-parallel rank (AR), the half grid (HALF), the debug library's arms: behind flags (chain_gemm.cuh)
+// K-step ownership, combine order and rounding points are the launch path's: results are bit-identical.
+// A decode step, behind flags and by content, one box: 64 rows of the 1.7B shape 3050 -> 2886 us, 5 rows of the 0.6B one 2091 -> 1859.
+// Shapes are parameters, not literals (the checkpoint decides them, configuration_qwen3_tts.py:192-216): the stage set is a template
 // on the k-steps per wave of its three reduction widths -- KO = q_heads * 128 / 256 (o_proj), KH = hidden / 256 (gate_up, qkv), KI =
-// intermediate / 256 (down_proj) -- and reads the output widths (hidden, intermediate, qkv) from its arguments; BB_SHAPES lists the
-// instantiated triples: the released 1.7B shape (8, 8, 24) and (6, 6, 18) = hidden 1536 / intermediate 4608 / 12 q heads, a shape no released
-// checkpoint has (tests/test_gpu_chain.py).  A shape runs here when its triple is listed and every stage's tile grid fits the 256
-// workgroups (k_bb_chain_supported); since the rstd moved into the epilogues (PRO 3) and the slab order is canonical (gemm_frag.cuh) the
-// bits no longer depend on which row tiles the launch path picks for the same GEMM.  33-64 rows: bb_chain_kernel (33-48 rows run the 64-row
-// stage set with their last row tile partly filled), 1-32 rows: bb_chain_b32_kernel, the 0.6B shape (hidden 1024 = the code predictor's
-// layer dimensions, 16-row tiles): bb_chain_small_kernel; every other configuration stays on the launch path.
-#include "chain_gemm.cuh"
+// intermediate / 256 (down_proj); BB_SHAPES lists the instantiated triples: the released 1.7B shape (8, 8, 24) and (6, 6, 18) = hidden 1536 /
+// intermediate 4608 / 12 q heads, a shape no released checkpoint has (tests/test_gpu_chain.py).  A shape runs here when its triple is listed
+// and every stage's tile grid fits the 256 workgroups (k_bb_chain_supported); the 0.6B shape has the code predictor's layer dimensions and its
+// split of the stages; every other configuration stays on the launch path.
+#include "chain_flow.cuh"
 #include "common.cuh"
 #include "kernels.h"
 
@@ -38,7 +38,13 @@ struct BbArgs {
     // (chain_gemm AR).  ar_epoch = allreduce.hip's epoch / ticket words: this launch makes calls epoch + 1 (o_proj) and epoch + 2 (down_proj)
     ChainAr ar_o, ar_dn;
     uint32_t* ar_epoch;
+    // hand-offs by content: this launch's buffers, the ones it empties for the next layer's launch (NULL: none behind it), 1: the step's first launch
+    char *flow, *flow_next;
+    int first;
 };
+// LDS of a stage's combine with `tiles` tiles, in floats; a launch's stages take turns: o_proj | gate_up | down_proj, and the last stage over the first
+// two's (their readers are behind down_proj's barrier)
+#define BB_AREA(tiles) (CH_WAVES * (tiles) * 256 + CH_WAVES * 64)
 
 // (Round 3 also tried a ninth wave that warms the XCD's L2 with the next stage's slice -- one dword per 64 bytes, nothing
 // depending on it: +0.10 ms per step, removed; and the loader / consumer split of bb_engine.hip.  What is kept is below:
@@ -185,73 +191,160 @@ __global__ __launch_bounds__(CH_THREADS) void bb_chain_kernel(const BbArgs a) {
     }
 }
 
-// ---- the 0.6B backbone shape (hidden 1024, 16 x 128 attention width over 8 kv heads, intermediate 3072: BASELINE config #2) --
-// the dimensions of the code predictor's layers, so the segment runs on the stage set of cp_chain.hip: 16-row tiles, four
-// independent row groups of 64 workgroups (gate_up on 32-row tiles above 32 rows, as the launch path picks them: same bits), any
-// batch size 1..64; a workgroup without rows in any stage publishes the launch's stage count and leaves.  Launch-per-op this
-// layer is five launches of 7-11 us for 25 MB of weights (profiles/r03_other_configs.txt: 56 us per layer).
-#define BBS_LDS_FLOATS ((CH_WAVES * 6 * 4 * 64) + CH_WAVES * 64)
-template <bool GU_NARROW>
-__global__ __launch_bounds__(CH_THREADS) void bb_chain_small_kernel(const BbArgs a) {
-    __shared__ __attribute__((aligned(16))) float lds[BBS_LDS_FLOATS];
+// ---- the single-rank launches: hand-offs by content (chain_flow.cuh).  What bounds a stage here is the trip from its predecessor's last store to its
+// own operands and what a CU can take in (wide shape, 64 rows: 0.2 to 0.6 MB of weights and activations a stage); behind flags every stage paid a
+// drain, a barrier, a flag, a poll and another barrier on top.
+// Two copies of the hand-off buffers: a launch uses one, empty when it starts, and empties its own tiles of the other for the launch behind it (the
+// last layer's has none).  The first layer's launch empties its own copy itself and is the only one that meets at a gate: whatever an earlier, broken
+// off step left there does not matter.
+struct BbFlowMap {                          // byte offsets within a copy (64 rows)
+    uint32_t ra, pa, act, rb, pb, copy;
+    __host__ __device__ constexpr BbFlowMap(int H, int I)
+        : ra(0), pa(64 * H * 2), act(pa + H / 16 * 64 * 4), rb(act + 64 * I * 2), pb(rb + 64 * H * 2), copy(pb + H / 16 * 64 * 4) {}
+};
+// the attention's rows are the launch's input: taken as they are
+#define BB_GIVEN true
+
+// ROWS: 64 (33 to 64 rows: o_proj / down_proj 16 columns x 32 rows a workgroup, gate_up 24 activation columns x 64, qkv 32 x 32), 32 (o_proj / down_proj
+// 16 x 16, qkv 16 x 32) or 16 (one row tile: o_proj / down_proj on half of the workgroups); gate_up takes 24 activation columns of all rows
+template <int KO, int KH, int KI, int ROWS, bool HEAD>
+__global__ __launch_bounds__(CH_THREADS) void bb_flow_kernel(const BbArgs a) {
+    extern __shared__ __attribute__((aligned(16))) float lds[];
+    constexpr int H = KH * 256, I = KI * 256, MO = ROWS == 64 ? 2 : 1, MG = ROWS / 16, NQT = ROWS == 64 ? 2 : 1, MQ = ROWS == 16 ? 1 : 2;
+    constexpr BbFlowMap F(H, I);
+    constexpr int nc_h = H / 16, nc_gu = I / 24;
+    static_assert(nc_h * (ROWS == 16 ? 1 : 2) <= OMNI_CHAIN_WGS && nc_gu <= OMNI_CHAIN_WGS && I % 24 == 0, "bb_flow: tiles");
+    const int B = a.B, wg = blockIdx.x;
+    const int bxo = wg % nc_h, byo = wg / nc_h;
+    const bool does_o = byo < (ROWS == 16 ? 1 : 2) && byo * MO * 16 < B, does_gu = wg < nc_gu;
+    char *const fl = a.flow, *const nx = a.flow_next;
     ChainGate g;
-    chain_gate_init(g, a.flags, a.err);
-    g.dom = GU_NARROW ? 7 : 6;          // 32-row gate_up tiles tie two 16-row groups together
-    g.nap = a.nap;
-    const int wg = blockIdx.x;
-    constexpr int H = 1024, I = 3072, NQ = 4096, KO = 2048;
-    if (!((wg >> 6) * 16 < a.B || (GU_NARROW && (wg >> 7) * 32 < a.B))) {
-        if (threadIdx.x < 64) chain_flag_publish(g.frs, wg, g.epoch + (a.wqkv_next ? 4u : 3u));
-        return;
+    FlowWait fw{a.err, 0};
+    u32x2 res = (u32x2){0u, 0u}, none = res;
+    if (a.first) {
+        chain_gate_init(g, a.flags, a.err);
+        fw.dead = g.dead;
+        auto fill = [&](uint32_t off, int pieces) {
+            const coh_rsrc_t rs = coh_rsrc(fl + off);
+            for (int i = threadIdx.x; i < pieces; i += CH_THREADS) flow_clear16(rs, i * 16);
+        };
+        if (does_o) {
+            for (int i = 0; i < MO; ++i) {
+                fill(F.ra + (byo * MO + i) * 32 * H + bxo * 512, 32);
+                fill(F.rb + (byo * MO + i) * 32 * H + bxo * 512, 32);
+            }
+            fill(F.pa + (bxo * 64 + byo * MO * 16) * 4, MO * 4);
+            fill(F.pb + (bxo * 64 + byo * MO * 16) * 4, MO * 4);
+        }
+        if (does_gu)
+            for (int i = 0; i < MG; ++i) fill(F.act + i * 32 * I + wg * 768, 48);
+        chain_gate_arrive(g);
     }
-    static_assert(KO == 8 * 256 && H == 4 * 256 && I == 12 * 256, "bb_chain_small: k-steps per wave");
-    chain_gemm<1, 1, 8, 0, OMNI_EPI_RESID>(a.wo, nullptr, a.attn, nullptr, 0, a.resid, 0, a.part, a.B, H, a.eps, wg & 63, wg >> 6, lds, g, false, 0x1001,
-                                           a.stamps);
-    if (GU_NARROW)
-        chain_gemm<2, 3, 4, 3, OMNI_EPI_SILU_MUL_GU8>(a.wgu, a.ln2, a.resid, a.part, H / 16, a.act, 0, nullptr, a.B, I, a.eps, wg & 127, wg >> 7, lds, g,
-                                                      true, 0x1002, a.stamps);
-    else
-        chain_gemm<1, 6, 4, 3, OMNI_EPI_SILU_MUL_GU8>(a.wgu, a.ln2, a.resid, a.part, H / 16, a.act, 0, nullptr, a.B, I, a.eps, wg & 63, wg >> 6, lds, g,
-                                                      true, 0x1002, a.stamps);
-    chain_gemm<1, 1, 12, 0, OMNI_EPI_RESID>(a.wdown, nullptr, a.act, nullptr, 0, a.resid, 0, a.part, a.B, H, a.eps, wg & 63, wg >> 6, lds, g, true, 0x1003,
-                                            a.stamps);
-    if (a.wqkv_next)
-        chain_gemm<1, 4, 4, 3, OMNI_EPI_BF16>(a.wqkv_next, a.ln1_next, a.resid, a.part, H / 16, a.qkv, NQ, nullptr, a.B, NQ, a.eps, wg & 63, wg >> 6, lds, g,
-                                              true, 0x1004, a.stamps);
+    auto next = [&](uint32_t off) -> char* { return nx != nullptr ? nx + off : nullptr; };
+    float *const lo = lds, *const lg = lo + BB_AREA(MO), *const ld = lg + BB_AREA(3 * MG);
+    if (does_o) {
+        if (threadIdx.x < MO * 64 && byo * MO * 16 + (int)threadIdx.x / 64 * 16 + (threadIdx.x & 15) < B)
+            res = coh_ld8(coh_rsrc(a.resid), (uint32_t)frag_off(byo * MO * 16 + threadIdx.x / 64 * 16 + (threadIdx.x & 15), bxo * 16 + 4 * ((threadIdx.x & 63) >> 4), H) * 2);
+        flow_gemm<MO, 1, KO, 0, OMNI_EPI_RESID>(a.wo, a.ln2, a.attn, nullptr, 0, fl + F.ra, (float*)(fl + F.pa), next(F.ra), (float*)next(F.pa), B, H, a.eps, bxo,
+                                                byo, lo, res, fw, 0x1001, a.stamps, BB_GIVEN);
+    }
+    if (a.first) {
+        chain_gate_wait(g, 0x1002);
+        fw.dead = flow_failed(a.err);
+    }
+    if (does_gu)
+        flow_gemm<MG, 3, KH, 4, OMNI_EPI_SILU_MUL_GU8, ROWS == 64 ? 4 : 0>(a.wgu, nullptr, fl + F.ra, (const float*)(fl + F.pa), H / 16, fl + F.act, nullptr, next(F.act),
+                                                                          nullptr, B, I, a.eps, wg, 0, lg, none, fw, 0x1002, a.stamps);
+    const bool qkv = a.wqkv_next != nullptr, head = HEAD && !qkv && a.lm_head != nullptr;
+    if (does_o)
+        // raw values for the next launch; bf16(w r) for the qkv stage, the values themselves for the head (its norm is exact)
+        flow_gemm<MO, 1, KI, 0, OMNI_EPI_RESID, ROWS == 64 ? 8 : 12>(a.wdown, qkv ? a.ln1_next : nullptr, fl + F.act, nullptr, 0, qkv || head ? fl + F.rb : nullptr,
+                                                                    (float*)(fl + F.pb), next(F.rb), (float*)next(F.pb), B, H, a.eps, bxo, byo, ld, res, fw, 0x1003,
+                                                                    a.stamps, false, nullptr, 0, FlowPlain{nullptr, a.resid, a.part});
+    if (qkv) {
+        const int nc_q = a.NQ / (16 * NQT), bx = wg % nc_q, by = wg / nc_q;
+        if (by * MQ * 16 < B && by < 4 / MQ)
+            flow_gemm<MQ, NQT, KH, 4, OMNI_EPI_BF16, 0, true>(a.wqkv_next, nullptr, fl + F.rb, (const float*)(fl + F.pb), H / 16, nullptr, nullptr, nullptr, nullptr, B,
+                                                              a.NQ, a.eps, bx, by, lds, none, fw, 0x1004, a.stamps, false, nullptr, a.NQ, FlowPlain{a.qkv});
+    } else if (head) {
+        const int nc_v = a.V / (16 * NQT), bx = wg % nc_v, by = wg / nc_v;
+        if (by * MQ * 16 < B && by < 4 / MQ)
+            flow_gemm<MQ, NQT, KH, 2, OMNI_EPI_F32_BF16RND, 0, true>(a.lm_head, a.final_norm, fl + F.rb, (const float*)(fl + F.pb), H / 16, nullptr, nullptr, nullptr,
+                                                                     nullptr, B, a.V, a.eps, bx, by, lds, none, fw, 0x1005, a.stamps, false, a.logits, a.V,
+                                                                     FlowPlain{nullptr, nullptr, nullptr, a.last_hidden, a.num_live, a.mask, a.mask_fill});
+    }
 }
 
-// ---- the 1.7B shape at 1-32 rows (round 4): the launch path's tiles at those batch sizes -- 16-row tiles for qkv / o_proj / down_proj
-// (128 column tiles x 2 row tiles), gate_up on 16 rows x 24 columns up to 16 rows and 32 x 24 above (the rstd summation order follows the
-// rows per tile: same bits as the launch path).  33-48 rows: bb_chain_kernel (the 64-row stage set).
-template <int KO, int KH, int KI, int GU_MT, bool HEAD = false>
-__global__ __launch_bounds__(CH_THREADS) void bb_chain_b32_kernel(const BbArgs a) {
+// ---- the 0.6B backbone shape (hidden 1024, 16 x 128 attention width over 8 kv heads, intermediate 3072): the dimensions of the code predictor's
+// layers, and its split of the stages over the 256 workgroups by rows (cp_chain.hip cp_chain_kernel).
+template <int ROWS>
+__global__ __launch_bounds__(CH_THREADS) void bb_flow_small_kernel(const BbArgs a) {
     extern __shared__ __attribute__((aligned(16))) float lds[];
+    constexpr int H = 1024, I = 3072, NQ = 4096;
+    constexpr BbFlowMap F(H, I);
+    constexpr bool SPLIT = ROWS <= 32;
+    constexpr int NO = ROWS == 16 ? 64 : 128;                    // SPLIT: workgroups of o_proj / down_proj; the others do gate_up
+    const int B = a.B, wg = blockIdx.x;
+    if (!SPLIT && (wg >> 6) * 16 >= B) {                         // a row group without rows: nobody waits for it beyond the first launch's gate
+        if (a.first && threadIdx.x < 64) {
+            ChainGate g;
+            chain_gate_init(g, a.flags, a.err);
+            chain_flag_publish(g.frs, wg, g.epoch + 1u);
+        }
+        return;
+    }
+    const bool does_o = (!SPLIT || wg < NO) && (wg >> 6) * 16 < B, does_gu = !SPLIT || wg >= NO;
+    const int bxo = wg & 63, byo = wg >> 6;
+    char *const fl = a.flow, *const nx = a.flow_next;
     ChainGate g;
-    chain_gate_init(g, a.flags, a.err);
-    g.dom = 8;
-    g.nap = a.nap;
-    const int wg = blockIdx.x;
-    const int H = a.H, I = a.I, NQ = a.NQ;
-    const int nc_h = H >> 4, nc_gu = I / 24, nc_q = NQ >> 5;        // 16-row tiles: two row tiles of each column tile cover the 32 rows
-    chain_gemm<1, 1, KO, 0, OMNI_EPI_RESID, 0>(a.wo, nullptr, a.attn, nullptr, 0, a.resid, 0, a.part, a.B, H, a.eps, wg % nc_h, wg / nc_h, lds, g, false, 0x1001,
-                                               a.stamps);
-    if (wg < nc_gu)
-        chain_gemm<GU_MT, 3, KH, 3, OMNI_EPI_SILU_MUL_GU8, 2, 1>(a.wgu, a.ln2, a.resid, a.part, H / 16, a.act, 0, nullptr, a.B, I, a.eps, wg, 0, lds, g, true, 0x1002,
-                                                                 a.stamps);
-    else
-        chain_gate_skip(g);
-    chain_gemm<1, 1, KI, 0, OMNI_EPI_RESID, 4>(a.wdown, nullptr, a.act, nullptr, 0, a.resid, 0, a.part, a.B, H, a.eps, wg % nc_h, wg / nc_h, lds, g, true, 0x1003,
-                                               a.stamps);
-    if (a.wqkv_next)
-        chain_gemm<1, 2, KH, 3, OMNI_EPI_BF16, 4>(a.wqkv_next, a.ln1_next, a.resid, a.part, H / 16, a.qkv, NQ, nullptr, a.B, NQ, a.eps, wg % nc_q, wg / nc_q, lds, g,
-                                                  true, 0x1004, a.stamps);
-    else if (HEAD && a.lm_head) {
-        const int nc_v = a.V >> 5;
-        chain_gemm<1, 2, KH, 2, OMNI_EPI_F32_BF16RND, 4>(a.lm_head, a.final_norm, a.resid, a.part, H / 16, a.logits, a.V, nullptr, a.B, a.V, a.eps, wg % nc_v,
-                                                         wg / nc_v, lds, g, true, 0x1005, a.stamps, nullptr, ChainNoPrefetch(), a.last_hidden, a.mask,
-                                                         a.mask_fill, a.num_live);
+    FlowWait fw{a.err, 0};
+    u32x2 res = (u32x2){0u, 0u}, none = res;
+    constexpr int GM = ROWS == 16 || ROWS == 48 ? 1 : 2, GN = ROWS == 16 ? 2 : (ROWS == 48 ? 6 : 3);       // gate_up's tiles
+    const int bxg = SPLIT ? wg - NO : (ROWS == 48 ? wg & 63 : wg & 127), byg = SPLIT ? 0 : (ROWS == 48 ? wg >> 6 : wg >> 7);
+    if (a.first) {
+        chain_gate_init(g, a.flags, a.err);
+        fw.dead = g.dead;
+        auto fill = [&](uint32_t off, int pieces) {
+            const coh_rsrc_t rs = coh_rsrc(fl + off);
+            for (int i = threadIdx.x; i < pieces; i += CH_THREADS) flow_clear16(rs, i * 16);
+        };
+        if (does_o) {
+            fill(F.ra + byo * 32 * H + bxo * 512, 32); fill(F.rb + byo * 32 * H + bxo * 512, 32);
+            fill(F.pa + (bxo * 64 + byo * 16) * 4, 4); fill(F.pb + (bxo * 64 + byo * 16) * 4, 4);
+        }
+        if (does_gu)
+            for (int i = 0; i < GM; ++i) fill(F.act + (byg * GM + i) * 32 * I + bxg * GN * 256, GN * 16);
+        chain_gate_arrive(g);
+    }
+    auto next = [&](uint32_t off) -> char* { return nx != nullptr ? nx + off : nullptr; };
+    float *const lo = lds, *const lg = lo + BB_AREA(1), *const ld = lg + BB_AREA(GM * GN);
+    if (does_o) {
+        if (threadIdx.x < 64 && byo * 16 + (int)(threadIdx.x & 15) < B)
+            res = coh_ld8(coh_rsrc(a.resid), (uint32_t)frag_off(byo * 16 + (threadIdx.x & 15), bxo * 16 + 4 * (threadIdx.x >> 4), H) * 2);
+        flow_gemm<1, 1, 8, 0, OMNI_EPI_RESID>(a.wo, a.ln2, a.attn, nullptr, 0, fl + F.ra, (float*)(fl + F.pa), next(F.ra), (float*)next(F.pa), B, H, a.eps, bxo, byo,
+                                              lo, res, fw, 0x1001, a.stamps, BB_GIVEN);
+    }
+    if (a.first) {
+        chain_gate_wait(g, 0x1002);
+        fw.dead = flow_failed(a.err);
+    }
+    if (does_gu)
+        flow_gemm<GM, GN, 4, 4, OMNI_EPI_SILU_MUL_GU8>(a.wgu, nullptr, fl + F.ra, (const float*)(fl + F.pa), H / 16, fl + F.act, nullptr, next(F.act), nullptr, B, I,
+                                                       a.eps, bxg, byg, lg, none, fw, 0x1002, a.stamps);
+    const bool qkv = a.wqkv_next != nullptr;
+    if (does_o)
+        flow_gemm<1, 1, 12, 0, OMNI_EPI_RESID>(a.wdown, qkv ? a.ln1_next : nullptr, fl + F.act, nullptr, 0, qkv ? fl + F.rb : nullptr, (float*)(fl + F.pb), next(F.rb),
+                                               (float*)next(F.pb), B, H, a.eps, bxo, byo, ld, res, fw, 0x1003, a.stamps, false, nullptr, 0,
+                                               FlowPlain{nullptr, a.resid, a.part});
+    if (qkv) {
+        constexpr int QM = ROWS == 32 ? 2 : 1, QN = SPLIT ? 1 : 4;
+        flow_gemm<QM, QN, 4, 4, OMNI_EPI_BF16, 0, true>(a.wqkv_next, nullptr, fl + F.rb, (const float*)(fl + F.pb), H / 16, nullptr, nullptr, nullptr, nullptr, B, NQ,
+                                                        a.eps, SPLIT ? wg : wg & 63, SPLIT ? 0 : wg >> 6, lds, none, fw, 0x1004, a.stamps, false, nullptr, NQ,
+                                                        FlowPlain{a.qkv});
     }
 }
+
+size_t k_bb_flow_bytes(const omni_talker_desc& d) { return 2 * (size_t)BbFlowMap(d.hidden, d.inter).copy; }
 
 OMNI_KNOB g_bb_chain = 1, g_bb_nap = 1, g_bb_prefetch = 0, g_bb_deep = 0, g_bb_min_rows = 33, g_bb_b32 = 1, g_bb_ar = 1;      // cross-stage prefetch: measured +0.4 ms per step, off
 #ifdef OMNI_DEBUG_HOOKS
@@ -302,34 +395,31 @@ bool k_bb_chain_small(const omni_talker_desc& d) {
     return d.hidden == 1024 && d.inter == 3072 && d.q_heads * 128 == 2048 && (d.q_heads + 2 * d.kv_heads) * 128 == 4096;
 }
 
-// one shape's launches: the 64-row stage set (33-64 rows) or the 16-row one (1-32 rows); the debug library's A/B arms exist for the 1.7B triple
+// one shape's launches, by rows; the step's head rides along where the last layer's launch brings one
+template <int KO, int KH, int KI, int ROWS, bool HEAD>
+static int bb_launch_rows(const BbArgs& a, hipStream_t stream) {
+    constexpr int MO = ROWS == 64 ? 2 : 1;
+    constexpr int bytes = (BB_AREA(MO) + BB_AREA(3 * ROWS / 16) + BB_AREA(MO)) * 4;
+    static const hipError_t attr = hipFuncSetAttribute((const void*)bb_flow_kernel<KO, KH, KI, ROWS, HEAD>, hipFuncAttributeMaxDynamicSharedMemorySize, bytes);
+    (void)attr;
+    hipLaunchKernelGGL((bb_flow_kernel<KO, KH, KI, ROWS, HEAD>), dim3(OMNI_CHAIN_WGS), dim3(CH_THREADS), bytes, stream, a);
+    OMNI_CHECK_LAUNCH("bb_flow");
+    return OMNI_OK;
+}
 template <int KO, int KH, int KI>
 static int bb_launch_shape(const BbArgs& a, int B, hipStream_t stream) {
-    static bool attr = false;
-    if (!attr) {
-        (void)hipFuncSetAttribute((const void*)bb_chain_b32_kernel<KO, KH, KI, 1>, hipFuncAttributeMaxDynamicSharedMemorySize, BB_LDS_BYTES);
-        (void)hipFuncSetAttribute((const void*)bb_chain_b32_kernel<KO, KH, KI, 2>, hipFuncAttributeMaxDynamicSharedMemorySize, BB_LDS_BYTES);
-        (void)hipFuncSetAttribute((const void*)bb_chain_b32_kernel<KO, KH, KI, 1, true>, hipFuncAttributeMaxDynamicSharedMemorySize, BB_LDS_BYTES);
-        (void)hipFuncSetAttribute((const void*)bb_chain_b32_kernel<KO, KH, KI, 2, true>, hipFuncAttributeMaxDynamicSharedMemorySize, BB_LDS_BYTES);
-        (void)hipFuncSetAttribute((const void*)bb_chain_kernel<KO, KH, KI, 2, 4, 4, false>, hipFuncAttributeMaxDynamicSharedMemorySize, BB_LDS_BYTES);
-        (void)hipFuncSetAttribute((const void*)bb_chain_kernel<KO, KH, KI, 2, 4, 4, false, true, false, true, 0, true>, hipFuncAttributeMaxDynamicSharedMemorySize, BB_LDS_BYTES);
-        attr = true;
-    }
     const bool head = a.lm_head != nullptr;
-    if (B <= 32) {
-        if (B <= 16) {
-            if (head) hipLaunchKernelGGL((bb_chain_b32_kernel<KO, KH, KI, 1, true>), dim3(OMNI_CHAIN_WGS), dim3(CH_THREADS), BB_LDS_BYTES, stream, a);
-            else hipLaunchKernelGGL((bb_chain_b32_kernel<KO, KH, KI, 1>), dim3(OMNI_CHAIN_WGS), dim3(CH_THREADS), BB_LDS_BYTES, stream, a);
-        } else {
-            if (head) hipLaunchKernelGGL((bb_chain_b32_kernel<KO, KH, KI, 2, true>), dim3(OMNI_CHAIN_WGS), dim3(CH_THREADS), BB_LDS_BYTES, stream, a);
-            else hipLaunchKernelGGL((bb_chain_b32_kernel<KO, KH, KI, 2>), dim3(OMNI_CHAIN_WGS), dim3(CH_THREADS), BB_LDS_BYTES, stream, a);
-        }
-        OMNI_CHECK_LAUNCH("bb_chain_b32");
-        return OMNI_OK;
-    }
-    if (head) hipLaunchKernelGGL((bb_chain_kernel<KO, KH, KI, 2, 4, 4, false, true, false, true, 0, true>), dim3(OMNI_CHAIN_WGS), dim3(CH_THREADS), BB_LDS_BYTES, stream, a);
-    else hipLaunchKernelGGL((bb_chain_kernel<KO, KH, KI, 2, 4, 4, false>), dim3(OMNI_CHAIN_WGS), dim3(CH_THREADS), BB_LDS_BYTES, stream, a);
-    OMNI_CHECK_LAUNCH("bb_chain");
+    if (B <= 16) return head ? bb_launch_rows<KO, KH, KI, 16, true>(a, stream) : bb_launch_rows<KO, KH, KI, 16, false>(a, stream);
+    if (B <= 32) return head ? bb_launch_rows<KO, KH, KI, 32, true>(a, stream) : bb_launch_rows<KO, KH, KI, 32, false>(a, stream);
+    return head ? bb_launch_rows<KO, KH, KI, 64, true>(a, stream) : bb_launch_rows<KO, KH, KI, 64, false>(a, stream);
+}
+template <int ROWS>
+static int bb_launch_small(const BbArgs& a, hipStream_t stream) {
+    constexpr int bytes = (BB_AREA(1) + BB_AREA(ROWS == 16 ? 2 : 6) + BB_AREA(1)) * 4;
+    static const hipError_t attr = hipFuncSetAttribute((const void*)bb_flow_small_kernel<ROWS>, hipFuncAttributeMaxDynamicSharedMemorySize, bytes);
+    (void)attr;
+    hipLaunchKernelGGL(bb_flow_small_kernel<ROWS>, dim3(OMNI_CHAIN_WGS), dim3(CH_THREADS), bytes, stream, a);
+    OMNI_CHECK_LAUNCH("bb_flow_small");
     return OMNI_OK;
 }
 
@@ -371,7 +461,7 @@ bool k_bb_chain_head_supported(const omni_talker_desc& d) {      // the lm_head 
 
 int k_bb_chain(const omni_talker_desc& d, const omni_layer_weights& w, const omni_layer_weights* next, const void* attn, void* resid, float* part,
                void* act, void* qkv, int B, float eps, uint32_t* flags, int32_t* err, void* stream, bool small, const omni_bb_head* head,
-               const omni_bb_ar* ar, bool half) {
+               const omni_bb_ar* ar, bool half, char* flow, int layer) {
     BbArgs a{};
     a.wo = (const uint16_t*)w.wo; a.ln2 = (const uint16_t*)w.ln2; a.wgu = (const uint16_t*)w.wgu; a.wdown = (const uint16_t*)w.wdown;
     a.ln1_next = next ? (const uint16_t*)next->ln1 : nullptr;
@@ -386,13 +476,17 @@ int k_bb_chain(const omni_talker_desc& d, const omni_layer_weights& w, const omn
 #ifdef OMNI_DEBUG_HOOKS
     a.stamps = g_bb_stamps;
 #endif
+    if (flow != nullptr) {
+        const size_t copy = BbFlowMap(a.H, a.I).copy;
+        a.flow = flow + (layer & 1) * copy;
+        a.flow_next = next ? flow + ((layer + 1) & 1) * copy : nullptr;
+        a.first = layer == 0;
+    }
     if (small) {
-        // (gate_up on 32-row tiles above 48 rows, on 16-row tiles below: the row group without rows then leaves at launch start -- round 5;
-        //  the bits do not depend on the choice since round 6)
-        if (B > 48) hipLaunchKernelGGL(bb_chain_small_kernel<true>, dim3(OMNI_CHAIN_WGS), dim3(CH_THREADS), 0, (hipStream_t)stream, a);
-        else hipLaunchKernelGGL(bb_chain_small_kernel<false>, dim3(OMNI_CHAIN_WGS), dim3(CH_THREADS), 0, (hipStream_t)stream, a);
-        OMNI_CHECK_LAUNCH("bb_chain_small");
-        return OMNI_OK;
+        if (B <= 16) return bb_launch_small<16>(a, (hipStream_t)stream);
+        if (B <= 32) return bb_launch_small<32>(a, (hipStream_t)stream);
+        if (B <= 48) return bb_launch_small<48>(a, (hipStream_t)stream);
+        return bb_launch_small<64>(a, (hipStream_t)stream);
     }
     const int ko = d.q_heads * 128 / 256, kh = d.hidden / 256, ki = d.inter / 256;
     if (ar != nullptr || half) {

@@ -104,6 +104,7 @@ struct omni_talker {
     float* kv_scale_dev;                // fp8 KV: device [layers][2] = {k_scale, v_scale} per layer, read by the decode step's attention launches
     std::vector<float> ksc_h, vsc_h;    // the same on the host (arguments of the eager prefill launches)
     void* bb_table;                     // device table of the backbone layers' pointers (bb_all.hip)
+    char* bb_flow;                      // hand-off buffers of the backbone's layer launches (bb_chain.hip)
     char* cp_flow;                      // hand-off buffers of the predictor's all-pass launch (cp_chain.hip)
     uint32_t* chain_flags;              // stage flags of the persistent chains: OMNI_FLAG_REPLICAS copies of [256] (coherent.cuh) + the error word at [320]
     omni_ar_peers ar_attn, ar_mlp;      // copies of desc.ar_* (has_ar)
@@ -170,6 +171,7 @@ static int carve(omni_talker* t, char* base, size_t* total) {
     t->pf_seq = c.take<int32_t>(8);
     t->chain_flags = c.take<uint32_t>(OMNI_FLAG_WORDS);
     t->cp_flow = c.take<char>(k_cp_flow_bytes());
+    t->bb_flow = c.take<char>(k_bb_flow_bytes(d));
     t->kv_scale_dev = c.take<float>(2 * (size_t)(d.layers > 0 ? d.layers : 1));
 #ifdef OMNI_DEBUG_HOOKS
     t->bb_table = c.take<char>(k_bb_all_table_bytes(d.layers > 0 ? d.layers : 1));
@@ -982,7 +984,7 @@ static int run_backbone(omni_talker* t, const omni_step_io* io, void* stream, in
                 const bool with_head = last && fuse_head && !t->chain_half && g_bb_head && k_bb_chain_head_supported(d);      // (the half grid has no head stage)
                 TRY(k_bb_chain(d, w, last ? nullptr : &t->layer[l + 1], t->attn, t->resid, t->part, t->act, t->qkv, B, d.eps,
                                t->chain_flags, reinterpret_cast<int32_t*>(t->chain_flags + 320), stream, plain && k_bb_chain_small(d), with_head ? &hd : nullptr,
-                               t->has_ar ? &bar : nullptr, t->chain_half));
+                               t->has_ar ? &bar : nullptr, t->chain_half, t->bb_flow, l));
                 if (with_head) t->head_fused = true;
             }
         }

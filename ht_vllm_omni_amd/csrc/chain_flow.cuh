@@ -1,4 +1,5 @@
-// Hand-offs between the stages of a persistent launch in which the DATA is the flag (cp_chain.hip: the code predictor).
+// Hand-offs between the stages of a persistent launch in which the DATA is the flag (cp_chain.hip: the code predictor; bb_chain.hip: the
+// backbone's layer segment).
 //
 // The flag protocol of coherent.cuh puts five dependent trips between a stage's last store and its successor's first MFMA: the stores'
 // drain, a workgroup barrier, the flag's write-through, a poll that sees it, another barrier, and only then the activations' own fetch
@@ -17,6 +18,7 @@
 //               - who polls use c + 1 has seen use c of the same tiles before, whose stores came behind the clearing: it never meets the
 //                 bytes of use c - 2.
 //             The first polls of a launch wait once for all workgroups' flags: each has cleared its tiles of all three copies by then.
+//             (A launch that uses each buffer once needs two copies: it clears the one that the launch behind it will use: bb_chain.hip.)
 //   order     loads and stores of handed-off bytes carry sc1 (coherent.cuh): a completed store is what every later load returns
 //   end       a wait is bounded by wall clock (coherent.cuh) and by the launch's error word: a wave that gives up records its stage code and
 //             never waits again; the launch runs to its end on whatever it has loaded
@@ -75,18 +77,30 @@ __device__ __forceinline__ int flow_slot(int row, int piece) { return (row * 4 +
 //   BF16          16 x 16 bf16 tiles, 512 B: tile t of row group r at (r * (N / 16) + t) * 512, rows of 32 B
 //   F32_BF16RND   16 x 16 fp32 tiles, 1 KB:  tile t of row group r at (r * (N / 16) + t) * 1024, rows of 64 B
 // res: the residual values of this thread's item (RESID: threads < 64 MT), kept in registers from one residual stage to the next
-template <int MT, int NT, int NTW, int PRO, int EPI>
+// G: k-steps of x in flight (0: the wave's whole share).  A ring looks for EMPTY words step by step, in front of the step's MFMAs
+// pl: what leaves the launch, by plain stores (FlowPlain); ROWS: the output goes there only (BF16 / F32 rows)
+struct FlowPlain {
+    uint16_t* rows;                       // BF16: row-major output, row m at rows + m * ldo
+    uint16_t* resid; float* part;         // RESID: the residual values themselves (fragment-major) and their slabs
+    uint16_t* normed; const int32_t* num_live;        // PRO 2: the normalised rows below *num_live, row-major
+    const uint8_t* mask; float mask_fill;             // F32: logit n is mask_fill where mask[n] == 0
+};
+template <int MT, int NT, int NTW, int PRO, int EPI, int G = 0, bool ROWS = false>
 __device__ __forceinline__ void flow_gemm(const uint16_t* __restrict__ W, const uint16_t* __restrict__ norm_w, const void* x, const float* part_in,
                                           int np_in, void* out, float* part_out, void* clr, float* clr_part, int M, int N, float eps, int bx, int by,
                                           float* lds, u32x2& res, FlowWait& fw, int code, unsigned long long* stamps,
                                           bool given = false /* x and the slabs were there before the launch: taken as they are, whatever their words */,
-                                          float* logits_rows = nullptr /* F32: also row-major, row m at logits_rows + m * ldo */, int ldo = 0) {
+                                          float* logits_rows = nullptr /* F32: also row-major, row m at logits_rows + m * ldo */, int ldo = 0,
+                                          const FlowPlain pl = FlowPlain{}) {
     const int sidx = ((code & 255) >> 4) * 5 + (code & 15) - 1;
     constexpr bool NORM = PRO == 2 || PRO == 3 || PRO == 4, DEFER = PRO == 3 || PRO == 4, NW = PRO == 2 || PRO == 3;
     constexpr bool GU8 = EPI == OMNI_EPI_SILU_MUL_GU8, RESID = EPI == OMNI_EPI_RESID, F32 = EPI == OMNI_EPI_F32_BF16RND;
     constexpr int K = NTW * CH_WAVES * 32, nsteps = K / 32;
     static_assert(EPI == OMNI_EPI_BF16 || RESID || F32 || GU8, "flow_gemm: epilogue");
-    static_assert(NT * MT <= FLOW_TILES && (!RESID || (NT == 1 && PRO == 0)), "flow_gemm: tiles");
+    constexpr int XG = (G == 0 || G > NTW) ? NTW : G;
+    constexpr bool RING = XG < NTW;
+    static_assert((NT * MT <= FLOW_TILES || RING) && (!RESID || (NT == 1 && PRO == 0)), "flow_gemm: tiles");
+    static_assert(!RING || PRO == 0 || PRO == 4, "flow_gemm: a ring's x is multiplied as it is");
     // opaque per stage: hipcc otherwise hoists every stage's lane-dependent offsets out of the caller's loops and keeps them in scratch
     int tid = threadIdx.x;
     asm volatile("" : "+v"(tid));
@@ -134,14 +148,14 @@ __device__ __forceinline__ void flow_gemm(const uint16_t* __restrict__ W, const 
     constexpr int XROWS = MT * 16;
     typedef SlabOrder<XROWS> SO;
     float pv[SO::PE];
-    u32x4 Xq[NTW][MT];
+    u32x4 Xq[XG][MT];
     const coh_rsrc_t prs = coh_rsrc(NORM ? (const void*)part_in : x);
     const int prow = lane % XROWS, psub = lane / XROWS;
     const uint32_t poff = (uint32_t)(m_base + prow) * 4;
 #pragma unroll
     for (int e = 0; e < SO::PE; ++e) pv[e] = 0.f;
 #pragma unroll
-    for (int d = 0; d < NTW; ++d)
+    for (int d = 0; d < XG; ++d)
 #pragma unroll
         for (int i = 0; i < MT; ++i) Xq[d][i] = (u32x4){0u, 0u, 0u, 0u};
     auto load_p = [&]() {
@@ -156,7 +170,7 @@ __device__ __forceinline__ void flow_gemm(const uint16_t* __restrict__ W, const 
             if (i * 16 + (lane & 15) < Mloc) {
 #pragma unroll
                 for (int d = d0; d < d1; ++d)
-                    Xq[d][i] = __builtin_amdgcn_raw_buffer_load_b128(xrs, lane16, (uint32_t)((((m_base >> 4) + i) * nsteps + wave + d * CH_WAVES) * 1024), OMNI_AUX_SC1);
+                    Xq[d % XG][i] = __builtin_amdgcn_raw_buffer_load_b128(xrs, lane16, (uint32_t)((((m_base >> 4) + i) * nsteps + wave + d * CH_WAVES) * 1024), OMNI_AUX_SC1);
             }
     };
     // Waiting looks at ONE line, the first of the wave's first k-step; when that has come, at everything.  Waiting eats the bandwidth of those who
@@ -173,37 +187,38 @@ __device__ __forceinline__ void flow_gemm(const uint16_t* __restrict__ W, const 
     while (go && peek()) go = flow_again(fw, code, spins, t0);
     CH_STAMP(stamps, sidx, 2);                                           // 2: something is there
     if (NORM) load_p();
-    load_x(0, NTW);
-    while (go) {
+    load_x(0, XG);
+    while (!RING && go) {
         uint32_t w = 0;
         if (NORM) {
 #pragma unroll
             for (int e = 0; e < SO::PE; ++e) w = max(w, __float_as_uint(pv[e]));
         }
 #pragma unroll
-        for (int d = 0; d < NTW; ++d)
+        for (int d = 0; d < XG; ++d)
 #pragma unroll
             for (int i = 0; i < MT; ++i) w = max(w, flow_max(Xq[d][i]));
         if (__builtin_amdgcn_ballot_w64(w == FLOW_EMPTY) == 0 || !(go = flow_again(fw, code, spins, t0))) break;
         if (NORM) load_p();
-        load_x(0, NTW);
+        load_x(0, XG);
     }
-    if (fw.dead) {                                                       // (see FlowWait)
+    if (!RING && fw.dead) {                                                     // (see FlowWait)
 #pragma unroll
         for (int e = 0; e < SO::PE; ++e) pv[e] = flow_or0(pv[e]);
 #pragma unroll
-        for (int d = 0; d < NTW; ++d)
+        for (int d = 0; d < XG; ++d)
 #pragma unroll
             for (int i = 0; i < MT; ++i)
 #pragma unroll
                 for (int c = 0; c < 4; ++c) Xq[d][i][c] = flow_or0(Xq[d][i][c]);
     }
-    CH_STAMP(stamps, sidx, 3);                                           // 3: operands complete
-    if (NORM) {
+    CH_STAMP(stamps, sidx, 3);                                           // 3: operands complete (a ring: asked for)
+    auto short_p = [&]() {               // slabs past the last one
 #pragma unroll
         for (int e = 0; e < SO::PE; ++e)
             if (SO::index(wave, psub, e) >= np_in) pv[e] = 0.f;
-    }
+    };
+    if (NORM && !RING) short_p();
     float* red = lds + CH_WAVES * NT * MT * 256;
     float rstd[MT];
     if (PRO == 2) {
@@ -221,15 +236,67 @@ __device__ __forceinline__ void flow_gemm(const uint16_t* __restrict__ W, const 
     for (int j = 0; j < NT; ++j)
 #pragma unroll
         for (int i = 0; i < MT; ++i) acc[j][i] = (f32x4){0.f, 0.f, 0.f, 0.f};
+    if constexpr (RING) {
+#pragma unroll
+        for (int d = 0; d < NTW; ++d) {
+            u32x4 (&X)[MT] = Xq[d % XG];
+            auto empty = [&]() -> bool {
+                uint32_t w = 0;
+#pragma unroll
+                for (int i = 0; i < MT; ++i) w = max(w, flow_max(X[i]));
+                return __builtin_amdgcn_ballot_w64(w == FLOW_EMPTY) != 0;
+            };
+            if (!given && empty()) {
+                while (flow_again(fw, code, spins, t0)) {
+                    load_x(d, d + 1);
+                    if (!empty()) break;
+                }
+                if (fw.dead) {
+#pragma unroll
+                    for (int i = 0; i < MT; ++i)
+#pragma unroll
+                        for (int c = 0; c < 4; ++c) X[i][c] = flow_or0(X[i][c]);
+                }
+            }
+#pragma unroll
+            for (int j = 0; j < NT; ++j)
+#pragma unroll
+                for (int i = 0; i < MT; ++i) acc[j][i] = mfma16(Wq[d][j], X[i], acc[j][i]);
+            if (d + XG < NTW) load_x(d + XG, d + XG + 1);
+        }
+        if (NORM) {
+            for (;;) {
+                uint32_t w = 0;
+#pragma unroll
+                for (int e = 0; e < SO::PE; ++e) w = max(w, __float_as_uint(pv[e]));
+                if (given || __builtin_amdgcn_ballot_w64(w == FLOW_EMPTY) == 0 || !flow_again(fw, code, spins, t0)) break;
+                load_p();
+            }
+            if (fw.dead) {
+#pragma unroll
+                for (int e = 0; e < SO::PE; ++e) pv[e] = flow_or0(pv[e]);
+            }
+            short_p();
+        }
+    } else {
 #pragma unroll
     for (int d = 0; d < NTW; ++d) {
         u32x4 Xn[MT];
 #pragma unroll
         for (int i = 0; i < MT; ++i) Xn[i] = PRO == 2 ? xnorm_frag(Xq[d][i], NWq[NW ? d : 0], rstd[i]) : (PRO == 3 ? xw_frag(Xq[d][i], NWq[NW ? d : 0]) : Xq[d][i]);
+        if (PRO == 2 && pl.normed != nullptr && bx < CH_WAVES && wave == bx) {
+            // k-steps bx, bx + 8, ... leave through workgroup column bx (gemm_skinny_kernel)
+            const int live = pl.num_live ? min(*pl.num_live, M) - m_base : Mloc;
+#pragma unroll
+            for (int i = 0; i < MT; ++i)
+                if (i * 16 + (lane & 15) < min(Mloc, live))
+                    *reinterpret_cast<u32x4*>(pl.normed + (size_t)(m_base + i * 16 + (lane & 15)) * K + (wave + d * CH_WAVES) * 32 + 8 * q) = Xn[i];
+        }
 #pragma unroll
         for (int j = 0; j < NT; ++j)
 #pragma unroll
             for (int i = 0; i < MT; ++i) acc[j][i] = mfma16(Wq[d][j], Xn[i], acc[j][i]);
+    }
     }
     if (DEFER) red[wave * 64 + lane] = SO::reduce(pv);
     const int wslot = flow_slot(lane & 15, q);
@@ -259,7 +326,11 @@ __device__ __forceinline__ void flow_gemm(const uint16_t* __restrict__ W, const 
             res = (u32x2){pack_bf2(rv[0], rv[1]), pack_bf2(rv[2], rv[3])};
             float ss = sq4_sum(rv[0], rv[1], rv[2], rv[3]);
             ss = xor32_sum(xor16_sum(ss));
-            if (ml < Mloc) {
+            if (ml < Mloc && pl.resid != nullptr) {
+                *reinterpret_cast<u32x2*>(reinterpret_cast<char*>(pl.resid) + tile_off(i, 0) + (q >> 1) * 256 + r * 16 + (q & 1) * 8) = res;
+                if (lane < 16) pl.part[bx * 64 + m_base + ml] = ss;
+            }
+            if (ml < Mloc && out != nullptr) {
                 // what the next norm's product takes: bf16(w r) (gemm_frag.cuh xw_frag); the residual values themselves stay here
                 const u32x2 o = (u32x2){flow_word(pack_bf2(bf_lo(res[0]) * bf_lo(nwn[0]), bf_hi(res[0]) * bf_hi(nwn[0]))),
                                         flow_word(pack_bf2(bf_lo(res[1]) * bf_lo(nwn[1]), bf_hi(res[1]) * bf_hi(nwn[1])))};
@@ -304,9 +375,16 @@ __device__ __forceinline__ void flow_gemm(const uint16_t* __restrict__ W, const 
                 coh_st4(ors, tile_off(i, j) + k * 4, flow_word(pack_bf2(silu_mul_bf16(sum[0], sum2[0]), silu_mul_bf16(sum[1], sum2[1]))));
             } else if (F32) {
                 // logits: fp32 cells holding bf16-rounded values (the reference's bf16 head output)
-                const float y0 = bfround(sum[0]), y1 = bfround(sum[1]);
-                coh_st8(ors, tile_off(i, j) + k * 8, (u32x2){flow_word(__float_as_uint(y0)), flow_word(__float_as_uint(y1))});
+                float y0 = bfround(sum[0]), y1 = bfround(sum[1]);
+                if (ROWS && pl.mask != nullptr) {
+                    const int n = (bx * NT + j) * 16 + 2 * c2;
+                    if (!pl.mask[n]) y0 = pl.mask_fill;
+                    if (!pl.mask[n + 1]) y1 = pl.mask_fill;
+                }
+                if (!ROWS) coh_st8(ors, tile_off(i, j) + k * 8, (u32x2){flow_word(__float_as_uint(y0)), flow_word(__float_as_uint(y1))});
                 if (logits_rows != nullptr) *reinterpret_cast<f32x2*>(logits_rows + (size_t)(m_base + ml) * ldo + (bx * NT + j) * 16 + 2 * c2) = (f32x2){y0, y1};
+            } else if (ROWS) {
+                *reinterpret_cast<uint32_t*>(pl.rows + (size_t)(m_base + ml) * ldo + (bx * NT + j) * 16 + 2 * c2) = pack_bf2(sum[0], sum[1]);
             } else {
                 coh_st4(ors, tile_off(i, j) + k * 4, flow_word(pack_bf2(sum[0], sum[1])));
             }

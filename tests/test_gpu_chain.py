@@ -240,6 +240,33 @@ def test_backbone_segment_chain_at_the_0p6b_shape_against_the_launch_path(B):
         assert torch.equal(x, y), f"KV cache of layer {l} differs"
 
 
+@pytest.mark.parametrize("model,shape", [("tts-0.6b", None), ("tts-1.7b", None), ("tts-1.7b", UNRELEASED)], ids=["0.6b", "1.7b", "unreleased"])
+@pytest.mark.parametrize("layers", [1, 4])
+def test_backbone_launches_of_changing_batches(model, shape, layers):
+    """One engine, steps of batches on either side of every row split (16, 32, 48, 64) in turn: a layer's launch empties the hand-off buffers of the next
+    one's, the first layer's its own, so what a batch of another size left there must not matter.  Bits of the launch path throughout."""
+    d = get_dims(model).with_(layers=layers, max_model_len=256, **(shape or {}))
+    w = make_weights(d, seed=9, std=0.02)
+    res = {}
+    with L.debug_library() as lib:
+        lib.omni_debug_bb_chain.argtypes = [C.c_int]; lib.omni_debug_bb_chain.restype = None
+        try:
+            for on in (0, 1):
+                lib.omni_debug_bb_chain(on)
+                eng = _decode_engine(d, w, 64, "bf16")
+                outs = []
+                for B in (64, 16, 33, 1, 49, 17, 48, 32, 15, 64):
+                    eng.decode_step(B)
+                    outs += [eng.logits[:B].clone(), eng.last_hidden[:B].clone(), eng.audio_codes[:B].clone()]
+                torch.cuda.synchronize()
+                assert eng.chain_error() == 0
+                res[on] = outs + [c.view(torch.uint8).clone() for c in eng.kv_caches]
+        finally:
+            lib.omni_debug_bb_chain(1)
+    for i, (x, y) in enumerate(zip(res[1], res[0])):
+        assert torch.equal(x, y), i
+
+
 @pytest.mark.parametrize("B,kv,base", [(64, "fp8", "launch-path"), (49, "bf16", "layer-chain"), (57, "int8", "launch-path"), (51, "fp16", "layer-chain")])
 def test_whole_backbone_launch_against_the_launch_path(B, kv, base):
     """The whole decoder stack -- qkv(0), then attention -> o_proj -> gate_up -> down_proj -> next qkv per layer -- as ONE persistent

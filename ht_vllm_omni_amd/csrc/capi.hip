@@ -593,8 +593,8 @@ static int run_code_predictor(omni_talker* t, const int32_t* layer0_ids, const v
                 hd.logits_pass = cp_logits_out ? d.codebook : 0;
                 hd.greedy = greedy; hd.top_k = top_k; hd.temperature = temperature; hd.top_p = top_p; hd.seed = seed;
                 hd.steps = steps; hd.row_seed = row_seed; hd.codes = t->codes;
-                TRY(k_cp_pair(d, t->cp_layer.data(), t->cp_k.data(), t->cp_v.data(), B, np, t->cp_resid, t->cp_part, t->cp_qkv, t->cp_attn, t->cp_act,
-                              t->chain_flags, reinterpret_cast<int32_t*>(t->chain_flags + 320), &hd, st));
+                TRY(k_cp_pair(d, t->cp_layer.data(), t->cp_k.data(), t->cp_v.data(), B, np, t->cp_resid, t->cp_part,
+                              t->chain_flags, reinterpret_cast<int32_t*>(t->chain_flags + 320), t->cp_flow, &hd, st));
                 t->ran |= 1;
                 pair_chain = true;
                 np = 1;

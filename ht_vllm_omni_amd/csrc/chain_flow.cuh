@@ -78,6 +78,7 @@ __device__ __forceinline__ int flow_slot(int row, int piece) { return (row * 4 +
 //   F32_BF16RND   16 x 16 fp32 tiles, 1 KB:  tile t of row group r at (r * (N / 16) + t) * 1024, rows of 64 B
 // res: the residual values of this thread's item (RESID: threads < 64 MT), kept in registers from one residual stage to the next
 // G: k-steps of x in flight (0: the wave's whole share).  A ring looks for EMPTY words step by step, in front of the step's MFMAs
+// PS: rows per slab of sums of squares
 // pl: what leaves the launch, by plain stores (FlowPlain); ROWS: the output goes there only (BF16 / F32 rows)
 struct FlowPlain {
     uint16_t* rows;                       // BF16: row-major output, row m at rows + m * ldo
@@ -85,7 +86,7 @@ struct FlowPlain {
     uint16_t* normed; const int32_t* num_live;        // PRO 2: the normalised rows below *num_live, row-major
     const uint8_t* mask; float mask_fill;             // F32: logit n is mask_fill where mask[n] == 0
 };
-template <int MT, int NT, int NTW, int PRO, int EPI, int G = 0, bool ROWS = false>
+template <int MT, int NT, int NTW, int PRO, int EPI, int G = 0, bool ROWS = false, int PS = 64>
 __device__ __forceinline__ void flow_gemm(const uint16_t* __restrict__ W, const uint16_t* __restrict__ norm_w, const void* x, const float* part_in,
                                           int np_in, void* out, float* part_out, void* clr, float* clr_part, int M, int N, float eps, int bx, int by,
                                           float* lds, u32x2& res, FlowWait& fw, int code, unsigned long long* stamps,
@@ -99,7 +100,7 @@ __device__ __forceinline__ void flow_gemm(const uint16_t* __restrict__ W, const 
     static_assert(EPI == OMNI_EPI_BF16 || RESID || F32 || GU8, "flow_gemm: epilogue");
     constexpr int XG = (G == 0 || G > NTW) ? NTW : G;
     constexpr bool RING = XG < NTW;
-    static_assert((NT * MT <= FLOW_TILES || RING) && (!RESID || (NT == 1 && PRO == 0)), "flow_gemm: tiles");
+    static_assert(NT * MT <= 12 && (!RESID || (NT == 1 && PRO == 0)), "flow_gemm: tiles");
     static_assert(!RING || PRO == 0 || PRO == 4, "flow_gemm: a ring's x is multiplied as it is");
     // opaque per stage: hipcc otherwise hoists every stage's lane-dependent offsets out of the caller's loops and keeps them in scratch
     int tid = threadIdx.x;
@@ -128,7 +129,7 @@ __device__ __forceinline__ void flow_gemm(const uint16_t* __restrict__ W, const 
             const int t = it / TP16;
             flow_clear16(crs, tile_off(t % MT, t / MT) + (it % TP16) * 16);
         }
-        if (RESID && tid >= 256 && tid < 256 + MT * 4) flow_clear16(coh_rsrc(clr_part), (uint32_t)(bx * 64 + m_base + (tid - 256) * 4) * 4);
+        if (RESID && tid >= 256 && tid < 256 + MT * 4) flow_clear16(coh_rsrc(clr_part), (uint32_t)(bx * PS + m_base + (tid - 256) * 4) * 4);
     }
 
     // ---- what does not depend on the predecessor: the weight slice, the norm weights
@@ -161,7 +162,7 @@ __device__ __forceinline__ void flow_gemm(const uint16_t* __restrict__ W, const 
     auto load_p = [&]() {
         if (prow < Mloc) {
 #pragma unroll
-            for (int e = 0; e < SO::PE; ++e) pv[e] = coh_ldf(prs, (uint32_t)(min(SO::index(wave, psub, e), np_in - 1) * 256) + poff);
+            for (int e = 0; e < SO::PE; ++e) pv[e] = coh_ldf(prs, (uint32_t)(min(SO::index(wave, psub, e), np_in - 1) * (PS * 4)) + poff);
         }
     };
     auto load_x = [&](int d0, int d1) {
@@ -328,14 +329,14 @@ __device__ __forceinline__ void flow_gemm(const uint16_t* __restrict__ W, const 
             ss = xor32_sum(xor16_sum(ss));
             if (ml < Mloc && pl.resid != nullptr) {
                 *reinterpret_cast<u32x2*>(reinterpret_cast<char*>(pl.resid) + tile_off(i, 0) + (q >> 1) * 256 + r * 16 + (q & 1) * 8) = res;
-                if (lane < 16) pl.part[bx * 64 + m_base + ml] = ss;
+                if (lane < 16) pl.part[bx * PS + m_base + ml] = ss;
             }
             if (ml < Mloc && out != nullptr) {
                 // what the next norm's product takes: bf16(w r) (gemm_frag.cuh xw_frag); the residual values themselves stay here
                 const u32x2 o = (u32x2){flow_word(pack_bf2(bf_lo(res[0]) * bf_lo(nwn[0]), bf_hi(res[0]) * bf_hi(nwn[0]))),
                                         flow_word(pack_bf2(bf_lo(res[1]) * bf_lo(nwn[1]), bf_hi(res[1]) * bf_hi(nwn[1])))};
                 coh_st8(ors, tile_off(i, 0) + (q >> 1) * 256 + r * 16 + (q & 1) * 8, o);
-                if (lane < 16) coh_st4(coh_rsrc(part_out), (uint32_t)(bx * 64 + m_base + ml) * 4, flow_word(__float_as_uint(ss)));
+                if (lane < 16) coh_st4(coh_rsrc(part_out), (uint32_t)(bx * PS + m_base + ml) * 4, flow_word(__float_as_uint(ss)));
             }
         }
     } else {

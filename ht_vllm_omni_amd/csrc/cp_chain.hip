@@ -10,7 +10,8 @@
 //     is EMPTY (chain_flow.cuh).  No drain, no flag, no barrier between a stage's last store and its successor's first MFMA.  What bounds it is
 //     that chain of dependent trips: 27 stages a pass of about 2.7 us (5 rows: 73 us a pass; 64 rows: 90), of which 0.6 to 1.6 us are a stage's own
 //     arithmetic, LDS combine and epilogue and the rest the operands' way.  Behind flags (coherent.cuh) a pass took 104 / 110 us;
-//   * cp_pair_kernel (positions 0 and 1) hands over behind flag words ("coherent by access", coherent.cuh);
+//   * cp_pair_kernel (positions 0 and 1, group 1) likewise, over both positions' rows; a decode step of 64 / of 5 rows, us, behind flags 2886 / 1859, by
+//     content 2860 / 1784 (the stages of up to 16 rows over all 256 workgroups: 64 of them owned every column of qkv);
 //   * what a stage may read without waiting (besides weights): bytes that were final two or more stages earlier -- the K / V history of the
 //     private cache, the old residual values of a residual epilogue.
 // K-step ownership of the 8 waves, accumulation order, LDS combine order and every rounding point are those of
@@ -41,7 +42,6 @@ struct ChainArgs {
     float eps, sm_scale;
     uint16_t* resid;                      // fragment-major residual stream [64][Hc]
     float* part;                          // sum(r^2) slabs [np][64]
-    uint16_t *qkv, *attn, *act;           // pair kernel: stage outputs, row-major [B][4096], fragment-major [64][2048], fragment-major [64][3072]
     const uint16_t* cos_sin;
     // head + sampler of pass g (group g): logits row b at logits + b * logits_ld + (g - 1) * logits_pass
     const uint16_t *cp_norm, *lm_head;    // lm_head: [Q - 1][codebook][Hc] fragment-major per group
@@ -59,9 +59,8 @@ struct ChainArgs {
         const uint16_t* wqkv; const uint16_t* ln1; uint16_t* qkv; int NQ;
         int enabled;
     } tail;
-    char* flow;                           // the all-pass launch's hand-off buffers: FLOW_COPIES copies of CP_COPY bytes
+    char* flow;                           // hand-off buffers: FLOW_COPIES copies of CP_COPY (all-pass launch) or PP_COPY bytes (pair launch)
     int Bp;                               // pair kernel: rows of position 1 start at Bp (B rounded up to 16) in the 128-row stream
-    int nap;                              // pair kernel: poll pause (coherent.cuh; a run-time knob in the debug library)
     unsigned long long* stamps;           // debug library only: [stage][CH_NSTAMP][256] s_memrealtime ticks (100 MHz) of wave 0, or NULL
 };
 
@@ -120,245 +119,6 @@ __device__ __attribute__((noinline)) void chain_finalize_row(const ChainFinArgs 
     if (tid == 0) coh_st4(coh_rsrc(T.part), (uint32_t)b * 4, __float_as_uint(red[0] + red[1] + red[2] + red[3]));
 }
 
-// ---- sampler stage of pass g: the workgroup that owns batch row b (inside b's flag domain) draws code g of row b from the
-// head GEMM's logits and, unless this was the last group, gathers the folded embedding -> projection row of the drawn code
-// into the residual stream as the next pass's input (slab 0 = its sum of squares).  sample_kernel's arithmetic (sampler_body.cuh):
-// waves 0-3 are the row's 256 threads, waves 4-7 only keep the barriers.
-template <bool TAIL = false>
-__device__ __forceinline__ void chain_sample(const ChainArgs& a, int g, float* lds, ChainGate& gate, int code, unsigned long long* stamps) {
-    const int sidx = 26;
-    int* const last_code = reinterpret_cast<int*>(lds + CH_LDS_FLOATS - 136);      // the drawn code, for the whole workgroup (tail: chain_finalize_row)
-    CH_STAMP(stamps, sidx, 0);
-    const int rows_per_dom = 16 << (gate.dom - 6);
-    const int wi = blockIdx.x & ((1 << gate.dom) - 1);
-    const int b = (blockIdx.x >> gate.dom) * rows_per_dom + wi;
-    const bool has_row = wi < rows_per_dom && b < a.B;              // workgroup-uniform
-    const bool live = threadIdx.x < SMP_THREADS;
-    const bool more = g < a.Q - 1 && a.ptab != nullptr;
-    if (!has_row) {
-        chain_gate_skip(gate);
-        return;
-    }
-    CH_STAMP(stamps, sidx, 1);
-    chain_gate_wait(gate, code);
-    CH_STAMP(stamps, sidx, 2);
-    // the pick is wave 0's alone, without a workgroup barrier (sampler_body.cuh smp_pick_wave: round 6, 8.4 -> ~2.5 us per pass); rows that ask
-    // for top-p keep the 4-wave pick.  Workgroup-uniform: kernel arguments only
-    const bool wave_path = a.greedy || !(a.top_p > 0.f && a.top_p < 1.f);
-    if (wave_path) {
-        if (threadIdx.x < 64) {
-            const int lane = threadIdx.x;
-            const SmpLds S = smp_carve<8>(lds);
-            const coh_rsrc_t lrs = coh_rsrc(a.logits);
-            const int V = a.codebook;
-            const uint32_t base = (uint32_t)b * a.logits_ld + (uint32_t)(g - 1) * a.logits_pass;
-            // a moderate temperature keeps the head GEMM's bf16-exact logits strictly ordered under the division: select first, divide the kept
-            const bool late = !a.greedy && a.temperature >= 1.0f / 64 && a.temperature <= 64.0f;
-            float xr[32];
-#pragma unroll
-            for (int j8 = 0; j8 < 8; ++j8) {
-                const u32x4 v4 = coh_ld16(lrs, (base + j8 * 256 + 4 * lane) * 4);
-#pragma unroll
-                for (int c = 0; c < 4; ++c) xr[j8 * 4 + c] = __uint_as_float(v4[c]);
-            }
-            // (both fix-ups behind wave-uniform branches the optimiser cannot turn into 32 selects: as straight-line code they were 32 IEEE
-            //  divisions on every pick)
-            if (V < 2048) {
-                asm volatile("" ::: "memory");
-#pragma unroll
-                for (int e = 0; e < 32; ++e)
-                    if ((e >> 2) * 256 + 4 * lane + (e & 3) >= V) xr[e] = -INFINITY;
-            }
-            if (!a.greedy && !late) {
-                asm volatile("" ::: "memory");
-#pragma unroll
-                for (int e = 0; e < 32; ++e) xr[e] = xr[e] / a.temperature;
-            }
-            const uint32_t seed = a.row_seed ? a.row_seed[b] : a.seed;
-            const uint32_t step = (uint32_t)(a.steps ? a.steps[b] * a.Q + g : g);
-            const int pick = smp_pick_wave<32>(xr, V, a.greedy, a.top_k, late, a.temperature, seed, step, S.ckey);
-            CH_STAMP(stamps, sidx, 4);
-            if (more) {
-                // the folded embedding -> projection row of the drawn code: lane l moves 16-byte pieces l and l + 64 of the 2 KB row; the
-                // slab value in sample_kernel's order of additions (piece sums, one wave_sum per 64 pieces, then the two halves)
-                const int Hc = 1024;
-                const uint16_t* tab = a.ptab + ((size_t)(g - 1) * a.codebook + pick) * Hc;
-                const coh_rsrc_t rrs = coh_rsrc(a.resid);
-                float ss2[2];
-#pragma unroll
-                for (int h2 = 0; h2 < 2; ++h2) {
-                    const int v = lane + 64 * h2;
-                    const u32x4 w4 = ld16(tab + v * 8);
-                    float ss = 0.f;
-#pragma unroll
-                    for (int j = 0; j < 4; ++j) ss += bf_lo(w4[j]) * bf_lo(w4[j]) + bf_hi(w4[j]) * bf_hi(w4[j]);
-                    coh_st16(rrs, (uint32_t)frag_off(b, v * 8, Hc) * 2, w4);
-                    ss2[h2] = wave_sum(ss);
-                }
-                if (lane == 0) coh_st4(coh_rsrc(a.part), (uint32_t)b * 4, __float_as_uint(((ss2[0] + ss2[1]) + 0.f) + 0.f));
-            }
-            if (lane == 0) coh_st4(coh_rsrc(a.codes), ((uint32_t)b * a.Q + g) * 4, (uint32_t)pick);
-            if (lane == 0) last_code[0] = pick;
-        }
-    } else {
-        constexpr int NPT = 8;
-        const SmpLds S = smp_carve<NPT>(lds);
-        const coh_rsrc_t lrs = coh_rsrc(a.logits);
-        const int V = a.codebook;
-        const uint32_t base = (uint32_t)b * a.logits_ld + (uint32_t)(g - 1) * a.logits_pass;
-        float xr[NPT];
-#pragma unroll
-        for (int e = 0; e < NPT; ++e) {
-            const int i = threadIdx.x + e * SMP_THREADS;
-            float x = -INFINITY;
-            if (live && i < V) {
-                x = coh_ldf(lrs, (base + i) * 4);
-                if (!a.greedy) x = x / a.temperature;
-            }
-            xr[e] = x;
-        }
-        const uint32_t seed = a.row_seed ? a.row_seed[b] : a.seed;
-        const uint32_t step = (uint32_t)(a.steps ? a.steps[b] * a.Q + g : g);
-        const int pick = smp_pick<NPT>(xr, V, a.greedy, a.top_k, a.top_p, seed, step, S, live, stamps);
-        CH_STAMP(stamps, sidx, 4);
-        if (more) {
-            const int Hc = 1024;
-            const uint16_t* tab = a.ptab + ((size_t)(g - 1) * a.codebook + pick) * Hc;
-            const coh_rsrc_t rrs = coh_rsrc(a.resid);
-            float ss = 0.f;
-            if (live) {
-                for (int v = threadIdx.x; v < Hc / 8; v += SMP_THREADS) {
-                    const u32x4 w4 = ld16(tab + v * 8);
-#pragma unroll
-                    for (int j = 0; j < 4; ++j) ss += bf_lo(w4[j]) * bf_lo(w4[j]) + bf_hi(w4[j]) * bf_hi(w4[j]);
-                    coh_st16(rrs, (uint32_t)frag_off(b, v * 8, Hc) * 2, w4);
-                }
-            }
-            ss = wave_sum(ss);
-            if ((threadIdx.x & 63) == 0) S.sval[threadIdx.x >> 6] = ss;
-            __syncthreads();
-            if (threadIdx.x == 0) {
-                float t = 0.f;
-#pragma unroll
-                for (int w = 0; w < SMP_WAVES; ++w) t += S.sval[w];
-                coh_st4(coh_rsrc(a.part), (uint32_t)b * 4, __float_as_uint(t));
-            }
-        }
-        if (threadIdx.x == 0) coh_st4(coh_rsrc(a.codes), ((uint32_t)b * a.Q + g) * 4, (uint32_t)pick);
-        if (threadIdx.x == 0) last_code[0] = pick;
-    }
-    if (TAIL && g == a.Q - 1 && a.tail.enabled) {
-        // the row's frame is complete: its owner assembles the backbone's input row right here (no hand-off: the last code is its own)
-        __syncthreads();
-        chain_finalize_row(ChainFinArgs{a.tail, a.codes, a.Q, a.codebook}, b, last_code[0], lds);
-    }
-    CH_STAMP(stamps, sidx, 6);
-    chain_gate_arrive(gate);
-    CH_STAMP(stamps, sidx, 7);
-}
-
-// ---- positions 0 and 1 of the predictor as stages too (round 4; they were 25 launches + the group-1 head and sampler launches):
-// the two-block stream of cp_forward_pair01 (capi.hip) -- rows [0, B) = position 0 (the talker's last hidden state), rows [Bp, Bp + B)
-// = position 1 (the layer-0 code embedding), slabs 128 rows wide -- through 5 x { qkv, pair attention, o_proj, gate_up, down_proj },
-// then the group-1 head GEMM on the position-1 rows and the sampler (which gathers the input of pass 2 into rows [0, B)).  Tiles =
-// the launch path's at 128 rows (pick_tile: qkv 32 x 64, o / down 32 x 16, gate_up 64 x 24): same bits.
-// The pair attention: one wave per (row, q head) as attn_pair01_kernel (paged_attn.hip) -- position 0 attends to itself (output = its
-// V row), position 1 to both; q / k / v cross from the qkv stage with sc1 dword loads (elements 2 l, 2 l + 1 per lane: V needs no
-// other layout; the (l, l + 64) pairing of the norm + RoPE is restored through LDS), K / V of both positions go to the private cache.
-__device__ __forceinline__ void chain_attn_pair(const ChainArgs& a, const ChainLayer& L, float* lds, ChainGate& g, int code,
-                                                unsigned long long* stamps) {
-    const int sidx = ((code & 255) >> 4) * 5 + (code & 15) - 1;
-    CH_STAMP(stamps, sidx, 0);
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    const int q_heads = a.q_heads, kv_heads = a.kv_heads, bs = a.bs;
-    if ((int)blockIdx.x * 4 >= a.B * q_heads) {
-        chain_gate_skip(g);
-        return;
-    }
-    const int pair = blockIdx.x * 4 + (wave & 3);               // waves 4-7 work, wave 0 polls (chain_attn)
-    const bool active = wave >= 4 && pair < a.B * q_heads;
-    const int row = pair / q_heads, h = pair - row * q_heads;
-    const int ratio = q_heads / kv_heads, kvh = h / ratio;
-    const int nslots = q_heads + 2 * kv_heads;
-    const coh_rsrc_t krs = coh_rsrc(L.kc), vrs = coh_rsrc(L.vc), qrs = coh_rsrc(a.qkv), ars = coh_rsrc(a.attn);
-    CH_STAMP(stamps, sidx, 1);
-    chain_gate_wait(g, code);
-    CH_STAMP(stamps, sidx, 2);
-    if (active) {
-        const uint32_t r0 = (uint32_t)row * nslots * 128, r1 = (uint32_t)(a.Bp + row) * nslots * 128;
-        const uint32_t ko = (uint32_t)(q_heads + kvh) * 128, vo = (uint32_t)(q_heads + kv_heads + kvh) * 128;
-        const uint32_t k0w = coh_ld4(qrs, (r0 + ko + 2 * lane) * 2), k1w = coh_ld4(qrs, (r1 + ko + 2 * lane) * 2);
-        const uint32_t q1w = coh_ld4(qrs, (r1 + (uint32_t)h * 128 + 2 * lane) * 2);
-        const uint32_t v0w = coh_ld4(qrs, (r0 + vo + 2 * lane) * 2), v1w = coh_ld4(qrs, (r1 + vo + 2 * lane) * 2);
-        uint32_t* raw = reinterpret_cast<uint32_t*>(lds + (wave & 3) * 256);        // three heads of raw dwords: k(pos 0) | k(pos 1) | q(pos 1)
-        raw[lane] = k0w; raw[64 + lane] = k1w; raw[128 + lane] = q1w;
-        __builtin_amdgcn_wave_barrier();
-        const uint16_t* rh = reinterpret_cast<const uint16_t*>(raw);
-        float k00, k01, k10, k11, q0, q1;
-        head_norm_rope_vals(bf2f(rh[lane]), bf2f(rh[lane + 64]), L.knorm, a.cos_sin, a.eps, lane, k00, k01);
-        head_norm_rope_vals(bf2f(rh[128 + lane]), bf2f(rh[128 + lane + 64]), L.knorm, a.cos_sin + 128, a.eps, lane, k10, k11);
-        head_norm_rope_vals(bf2f(rh[256 + lane]), bf2f(rh[256 + lane + 64]), L.qnorm, a.cos_sin + 128, a.eps, lane, q0, q1);
-        if (h % ratio == 0) {
-            // K / V of both positions into the private cache, one dword per lane (chain_attn's pairing of the two halves)
-            const bool odd = (lane & 1) != 0;
-            const uint32_t elem = odd ? 64 + lane - 1 : lane;
-#pragma unroll
-            for (int pz = 0; pz < 2; ++pz) {
-                const uint32_t crow = ((uint32_t)(row * bs + pz) * kv_heads + kvh) * 128;
-                const uint32_t kb0 = f2bf(pz ? k10 : k00), kb1 = f2bf(pz ? k11 : k01);
-                const uint32_t n0 = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)kb0, OMNI_DPP_XOR1, 0xF, 0xF, true);
-                const uint32_t n1 = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)kb1, OMNI_DPP_XOR1, 0xF, 0xF, true);
-                coh_st4(krs, (crow + elem) * 2, odd ? (n1 | (kb1 << 16)) : (kb0 | (n0 << 16)));
-                coh_st4(vrs, (crow + 2 * lane) * 2, pz ? v1w : v0w);
-            }
-        }
-        const float qs = a.sm_scale * LOG2E;
-        const float s0 = wave_sum(fmaf(q0 * qs, k00, (q1 * qs) * k01));
-        const float s1 = wave_sum(fmaf(q0 * qs, k10, (q1 * qs) * k11));
-        const float m = fmaxf(s0, s1);
-        const float p0 = exp2f(s0 - m), p1 = exp2f(s1 - m);
-        const float inv = 1.0f / (p0 + p1);
-        const int width = q_heads * 128, col = h * 128 + 2 * lane;
-        coh_st4(ars, (uint32_t)frag_off(row, col, width) * 2, v0w);
-        coh_st4(ars, (uint32_t)frag_off(a.Bp + row, col, width) * 2,
-                pack_bf2(fmaf(p1, bf_lo(v1w), p0 * bf_lo(v0w)) * inv, fmaf(p1, bf_hi(v1w), p0 * bf_hi(v0w)) * inv));
-    }
-    CH_STAMP(stamps, sidx, 6);
-    chain_gate_arrive(g);
-    CH_STAMP(stamps, sidx, 7);
-}
-
-__global__ __launch_bounds__(CH_THREADS) void cp_pair_kernel(const ChainArgs a) {
-    __shared__ __attribute__((aligned(16))) float lds[CH_LDS_FLOATS];
-    ChainGate g;
-    chain_gate_init(g, a.flags, a.err);
-    g.dom = 8;                            // 64-row gate_up tiles and the (row, head) pairs tie every row together
-    g.nap = a.nap & 31;
-    if (a.nap >> 5) g.skip_units = (a.nap >> 5) - 1;
-    const int wg = blockIdx.x;
-    const int Hc = 1024, NQ = 4096, NI = 3072;
-    const int M2 = a.Bp + a.B;
-    int np = a.np_in;
-    for (int l = 0; l < a.layers; ++l) {
-        const ChainLayer& L = a.layer[l];
-        chain_gemm<2, 4, 4, 3, OMNI_EPI_BF16, 0, 0, ChainNoPrefetch, false, 128>(L.wqkv, L.ln1, a.resid, a.part, np, a.qkv, NQ, nullptr, M2, NQ, a.eps, wg & 63,
-                                                                                 wg >> 6, lds, g, l > 0, 0x0100 | (16 * l + 1), a.stamps);
-        chain_attn_pair(a, L, lds, g, 0x0100 | (16 * l + 2), a.stamps);
-        chain_gemm<2, 1, 8, 0, OMNI_EPI_RESID, 0, 0, ChainNoPrefetch, false, 128>(L.wo, nullptr, a.attn, nullptr, 0, a.resid, 0, a.part, M2, Hc, a.eps, wg & 63,
-                                                                                  wg >> 6, lds, g, true, 0x0100 | (16 * l + 3), a.stamps);
-        np = Hc / 16;
-        chain_gemm<4, 3, 4, 3, OMNI_EPI_SILU_MUL_GU8, 0, 0, ChainNoPrefetch, false, 128>(L.wgu, L.ln2, a.resid, a.part, np, a.act, 0, nullptr, M2, NI, a.eps,
-                                                                                         wg & 127, wg >> 7, lds, g, true, 0x0100 | (16 * l + 4), a.stamps);
-        chain_gemm<2, 1, 12, 0, OMNI_EPI_RESID, 0, 0, ChainNoPrefetch, false, 128>(L.wdown, nullptr, a.act, nullptr, 0, a.resid, 0, a.part, M2, Hc, a.eps,
-                                                                                   wg & 63, wg >> 6, lds, g, true, 0x0100 | (16 * l + 5), a.stamps);
-    }
-    // group 1: head GEMM on the position-1 rows (fragment-major tiles Bp / 16 onwards; their slabs start at row Bp), then the sampler
-    chain_gemm<1, 2, 4, 2, OMNI_EPI_F32_BF16RND, 0, 0, ChainNoPrefetch, false, 128>(a.lm_head, a.cp_norm, a.resid + (size_t)a.Bp * Hc, a.part + a.Bp, np,
-                                                                                    a.logits, a.logits_ld, nullptr, a.B, a.codebook, a.eps, wg & 63, wg >> 6,
-                                                                                    lds, g, true, 0x0156, a.stamps);
-    chain_sample(a, 1, lds, g, 0x01F2, a.stamps);
-}
-
 // ---- the all-pass launch: passes 2 .. 15 of every row, hand-offs by content (chain_flow.cuh)
 // hand-off buffers of one copy, bytes from its base (64 rows)
 enum : uint32_t {
@@ -375,13 +135,25 @@ enum : uint32_t {
     CP_COPY = CP_LOG + 64 * 2048 * 4
 };
 #define CP_FLOW_BYTES ((size_t)FLOW_COPIES * CP_COPY)
-size_t k_cp_flow_bytes() { return CP_FLOW_BYTES; }
+// ... and of one copy of the pair launch: the same for 128 rows; its logits, written once, lie behind the copies
+enum : uint32_t {
+    PP_QKV = 0,
+    PP_ATT = PP_QKV + 128 * 4096 * 2,
+    PP_RA = PP_ATT + 128 * 2048 * 2,
+    PP_PA = PP_RA + 128 * 1024 * 2,
+    PP_ACT = PP_PA + 64 * 128 * 4,
+    PP_RB = PP_ACT + 128 * 3072 * 2,
+    PP_PB = PP_RB + 128 * 1024 * 2,
+    PP_COPY = PP_PB + 64 * 128 * 4
+};
+#define PP_FLOW_BYTES ((size_t)FLOW_COPIES * PP_COPY + 64 * 2048 * 4)
+size_t k_cp_flow_bytes() { return CP_FLOW_BYTES > PP_FLOW_BYTES ? CP_FLOW_BYTES : PP_FLOW_BYTES; }       // (the two launches run one behind the other)
 
 // LDS of the launch: two combine halves, a KB per wave for the attention, the sampler's working set, one word
 #define CPF_ATTN_FLOATS (2 * FLOW_HALF_FLOATS)
 #define CPF_SMP_FLOATS (CPF_ATTN_FLOATS + CH_WAVES * 256)
-#define CPF_LAST_FLOATS (CPF_SMP_FLOATS + (SMP_LDS_BYTES(8) + 15) / 16 * 4)
-#define CPF_LDS_BYTES ((CPF_LAST_FLOATS + 4) * 4)
+#define CPF_LAST ((SMP_LDS_BYTES(8) + 15) / 16 * 4)                  // the drawn code's word, floats behind the sampler's working set
+#define CPF_LDS_BYTES ((CPF_SMP_FLOATS + CPF_LAST + 4) * 4)
 
 // attention at buffer position pos <= 15 (dense private cache: row b owns block b): one wave per (row, q head), the work layout of
 // attn_tiny_dense_kernel (paged_attn.hip).  A kv head's q heads are waves of ONE workgroup, in every pass the same one: the K / V rows that the
@@ -497,31 +269,32 @@ __device__ __forceinline__ void flow_attn(const ChainArgs& a, const ChainLayer& 
 // the sampler stage of pass g by the workgroup that owns batch row b: draws code g of row b from the head stage's logits and, unless this was the
 // last group, gathers the folded embedding -> projection row of the drawn code as the next pass's input (slab 0 = its sum of squares).  The pick
 // is wave 0's alone (sampler_body.cuh smp_pick_wave); rows that ask for top-p take the four-wave pick
+// logits: 16 x 16 fp32 tiles; r0, p0: where the next pass's input rows and their slab go; c0, cl: the same places in the copy to clear, NULL: none
 template <bool TAIL>
-__device__ __forceinline__ void flow_sample(const ChainArgs& a, int g, int b, float* lds, const char* in, char* out, char* clr, FlowWait& fw, int code,
-                                            unsigned long long* stamps) {
+__device__ __forceinline__ void flow_sample(const ChainArgs& a, int g, int b, float* lds, float* smp, const void* logits, void* r0, void* p0, void* c0, void* cl,
+                                            FlowWait& fw, int code, unsigned long long* stamps) {
     const int sidx = 26;
-    int* const last_code = reinterpret_cast<int*>(lds + CPF_LAST_FLOATS);
+    int* const last_code = reinterpret_cast<int*>(smp + CPF_LAST);
     CH_STAMP(stamps, sidx, 0);
     int tid = threadIdx.x;
     asm volatile("" : "+v"(tid));       // opaque per call (flow_gemm)
     const int lane = tid & 63;
     const bool more = g < a.Q - 1 && a.ptab != nullptr;
     const int V = a.codebook, Hc = 1024;
-    const coh_rsrc_t lrs = coh_rsrc(in + CP_LOG), rrs = coh_rsrc(out + CP_R0), prs = coh_rsrc(out + CP_P0);
+    const coh_rsrc_t lrs = coh_rsrc(logits), rrs = coh_rsrc(r0), prs = coh_rsrc(p0);
     const uint32_t base = (uint32_t)(b >> 4) * 128 * 1024 + (b & 15) * 64;        // logit i of the row: base + (i / 16) * 1024 + (i % 16) * 4
-    if (tid < 64) {
-        const coh_rsrc_t c0 = coh_rsrc(clr + CP_R0), cl = coh_rsrc(clr + CP_P0);
-        flow_clear16(c0, (uint32_t)frag_off(b, lane * 8, Hc) * 2);
-        flow_clear16(c0, (uint32_t)frag_off(b, (lane + 64) * 8, Hc) * 2);
-        if (lane == 0) coh_st4(cl, (uint32_t)b * 4, FLOW_EMPTY);
+    if (tid < 64 && c0 != nullptr) {
+        const coh_rsrc_t crs = coh_rsrc(c0);
+        flow_clear16(crs, (uint32_t)frag_off(b, lane * 8, Hc) * 2);
+        flow_clear16(crs, (uint32_t)frag_off(b, (lane + 64) * 8, Hc) * 2);
+        if (lane == 0) coh_st4(coh_rsrc(cl), (uint32_t)b * 4, FLOW_EMPTY);
     }
     const uint32_t seed = a.row_seed ? a.row_seed[b] : a.seed;
     const uint32_t step = (uint32_t)(a.steps ? a.steps[b] * a.Q + g : g);
     CH_STAMP(stamps, sidx, 1);
     // workgroup-uniform: kernel arguments only
     const bool wave_path = a.greedy || !(a.top_p > 0.f && a.top_p < 1.f);
-    const SmpLds S = smp_carve<8>(lds + CPF_SMP_FLOATS);
+    const SmpLds S = smp_carve<8>(smp);
     int pick = 0;
     if (wave_path) {
         if (tid < 64) {
@@ -629,6 +402,206 @@ __device__ __forceinline__ void flow_sample(const ChainArgs& a, int g, int b, fl
     }
     CH_STAMP(stamps, sidx, 6);
     CH_STAMP(stamps, sidx, 7);
+}
+
+// ---- positions 0 and 1 of the predictor: the two-block stream of cp_forward_pair01 (capi.hip) -- rows [0, B) = position 0 (the talker's last hidden
+// state), rows [Bp, Bp + B) = position 1 (the layer-0 code embedding), slabs 128 rows wide -- through the layers { qkv, pair attention, o_proj, gate_up,
+// down_proj }, then the group-1 head GEMM on the position-1 rows and the sampler, which gathers the input of pass 2 into rows [0, B).
+// The pair attention: a wave per (row, q head) as attn_pair01_kernel (paged_attn.hip) -- position 0 attends to itself (output = its V row), position 1
+// to both; K / V of both positions go to the private cache.  The rows between B and Bp pass through the stages of position 0 like the others (their
+// consumers wait for whole tiles); nothing of them is kept.
+__device__ __forceinline__ void flow_attn_pair(const ChainArgs& a, const ChainLayer& L, int pair, float* sq, char* buf, char* clr, FlowWait& fw, int code,
+                                               unsigned long long* stamps) {
+    const int sidx = ((code & 255) >> 4) * 5 + (code & 15) - 1;
+    CH_STAMP_BY(stamps, sidx, 0, 256);
+    int lane = threadIdx.x & 63;
+    asm volatile("" : "+v"(lane));      // opaque per call (flow_gemm)
+    const int q_heads = a.q_heads, kv_heads = a.kv_heads, bs = a.bs, width = q_heads * 128;
+    const int row = pair / q_heads, h = pair - row * q_heads;
+    const int ratio = q_heads / kv_heads, kvh = h / ratio;
+    const int tiles = (q_heads + 2 * kv_heads) * 8;
+    const bool both = row < a.B;
+    const coh_rsrc_t krs = coh_rsrc(L.kc), vrs = coh_rsrc(L.vc), qrs = coh_rsrc(buf + PP_QKV), ars = coh_rsrc(buf + PP_ATT), crs = coh_rsrc(clr + PP_ATT);
+    if (lane < 16) flow_clear16(crs, (uint32_t)frag_off(row, h * 128 + 8 * lane, width) * 2);
+    else if (lane < 32 && both) flow_clear16(crs, (uint32_t)frag_off(a.Bp + row, h * 128 + 8 * (lane - 16), width) * 2);
+    CH_STAMP_BY(stamps, sidx, 1, 256);
+    // elements 2 l, 2 l + 1 of the heads out of the qkv stage's tiles
+    auto at = [&](int m, int head) -> uint32_t { return (uint32_t)((m >> 4) * tiles * 512 + (m & 15) * 32 + (lane >> 3) * 512 + (lane & 7) * 4 + head * 4096); };
+    uint32_t k0w = 0, k1w = 0, q1w = 0, v0w, v1w = 0;
+    {
+        unsigned spins = 0;
+        unsigned long long t0 = 0;
+        for (;;) {
+            v0w = coh_ld4(qrs, at(row, q_heads + kv_heads + kvh));
+            if (both) {
+                k0w = coh_ld4(qrs, at(row, q_heads + kvh));
+                k1w = coh_ld4(qrs, at(a.Bp + row, q_heads + kvh));
+                q1w = coh_ld4(qrs, at(a.Bp + row, h));
+                v1w = coh_ld4(qrs, at(a.Bp + row, q_heads + kv_heads + kvh));
+            }
+            if (__builtin_amdgcn_ballot_w64(max(max(max(k0w, k1w), max(q1w, v0w)), v1w) == FLOW_EMPTY) == 0 || !flow_again(fw, code, spins, t0)) break;
+        }
+    }
+    if (fw.dead) { k0w = flow_or0(k0w); k1w = flow_or0(k1w); q1w = flow_or0(q1w); v0w = flow_or0(v0w); v1w = flow_or0(v1w); }
+    CH_STAMP_BY(stamps, sidx, 2, 256);
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");      // the clearing is complete before this use's rows go out (chain_flow.cuh)
+    const int col = h * 128 + 2 * lane;
+    coh_st4(ars, (uint32_t)frag_off(row, col, width) * 2, v0w);
+    if (both) {
+        uint32_t* raw = reinterpret_cast<uint32_t*>(sq);        // three heads of raw dwords: k(pos 0) | k(pos 1) | q(pos 1); the (l, l + 64) pairing through LDS
+        raw[lane] = k0w; raw[64 + lane] = k1w; raw[128 + lane] = q1w;
+        __builtin_amdgcn_wave_barrier();
+        const uint16_t* rh = reinterpret_cast<const uint16_t*>(raw);
+        float k00, k01, k10, k11, q0, q1;
+        head_norm_rope_vals(bf2f(rh[lane]), bf2f(rh[lane + 64]), L.knorm, a.cos_sin, a.eps, lane, k00, k01);
+        head_norm_rope_vals(bf2f(rh[128 + lane]), bf2f(rh[128 + lane + 64]), L.knorm, a.cos_sin + 128, a.eps, lane, k10, k11);
+        head_norm_rope_vals(bf2f(rh[256 + lane]), bf2f(rh[256 + lane + 64]), L.qnorm, a.cos_sin + 128, a.eps, lane, q0, q1);
+        __builtin_amdgcn_wave_barrier();
+        const float qs = a.sm_scale * LOG2E;
+        const float s0 = wave_sum(fmaf(q0 * qs, k00, (q1 * qs) * k01));
+        const float s1 = wave_sum(fmaf(q0 * qs, k10, (q1 * qs) * k11));
+        const float m = fmaxf(s0, s1);
+        const float p0 = exp2f(s0 - m), p1 = exp2f(s1 - m);
+        const float inv = 1.0f / (p0 + p1);
+        coh_st4(ars, (uint32_t)frag_off(a.Bp + row, col, width) * 2,
+                flow_word(pack_bf2(fmaf(p1, bf_lo(v1w), p0 * bf_lo(v0w)) * inv, fmaf(p1, bf_hi(v1w), p0 * bf_hi(v0w)) * inv)));
+        if (h % ratio == 0) {
+            // K / V of both positions into the private cache, one dword per lane (flow_attn's pairing of the two halves)
+            const bool odd = (lane & 1) != 0;
+            const uint32_t elem = odd ? 64 + lane - 1 : lane;
+#pragma unroll
+            for (int pz = 0; pz < 2; ++pz) {
+                const uint32_t crow = ((uint32_t)(row * bs + pz) * kv_heads + kvh) * 128;
+                const uint32_t kb0 = f2bf(pz ? k10 : k00), kb1 = f2bf(pz ? k11 : k01);
+                const uint32_t n0 = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)kb0, OMNI_DPP_XOR1, 0xF, 0xF, true);
+                const uint32_t n1 = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)kb1, OMNI_DPP_XOR1, 0xF, 0xF, true);
+                coh_st4(krs, (crow + elem) * 2, odd ? (n1 | (kb1 << 16)) : (kb0 | (n0 << 16)));
+                coh_st4(vrs, (crow + 2 * lane) * 2, pz ? v1w : v0w);
+            }
+        }
+    }
+    CH_STAMP_BY(stamps, sidx, 6, 256);
+    CH_STAMP_BY(stamps, sidx, 7, 256);
+}
+
+// combine areas of the pair launch, in floats: o_proj | down_proj | qkv, gate_up and head.  A workgroup's o_proj and down_proj barriers stand between two uses
+// of the last; one without o_proj rows meets once more in front of each
+#define PP_AREA(tiles) (CH_WAVES * (tiles) * 256 + CH_WAVES * 64)
+#define PP_BIG_FLOATS (2 * PP_AREA(2))
+#define PP_ATTN_FLOATS (PP_BIG_FLOATS + PP_AREA(12))
+#define PP_LDS_BYTES ((PP_ATTN_FLOATS + CH_WAVES * 256) * 4)
+static_assert((CPF_LAST + 4) <= PP_ATTN_FLOATS, "the sampler's working set lies over the combine areas");
+
+// R: the most stream rows (both positions) of the launch's split of a stage over the 256 workgroups
+//   32   qkv 16 columns x 32 rows each; o_proj / down_proj 16 x 16 on 128 workgroups, gate_up 24 activation columns x 32 rows on the others
+//   64   qkv 32 x 32, o_proj / down_proj 16 x 16, gate_up 24 x 32
+//   128  qkv 64 x 32, o_proj / down_proj 16 x 32, gate_up 24 x 64
+template <int R>
+__global__ __launch_bounds__(CH_THREADS) void cp_pair_kernel(const ChainArgs a) {
+    extern __shared__ __attribute__((aligned(16))) float lds[];
+    ChainGate g;
+    chain_gate_init(g, a.flags, a.err);
+    constexpr int Hc = 1024, NQ = 4096, NI = 3072;
+    constexpr bool SPLIT = R == 32;
+    constexpr int QM = 2, QN = R == 32 ? 1 : R / 32, OM = R == 128 ? 2 : 1, GM = R == 128 ? 4 : 2, QC = NQ / 16 / QN;
+    const int B = a.B, Bp = a.Bp, M2 = Bp + B;
+    const int wg0 = blockIdx.x, wave = threadIdx.x >> 6;
+    FlowWait fw{a.err, g.dead ? 1 : 0};
+    // ---- this workgroup's part of each stage
+    const bool does_q = (wg0 / QC) * QM * 16 < M2;
+    const bool does_o = (!SPLIT || wg0 < 128) && (wg0 >> 6) * OM * 16 < M2;
+    const bool does_gu = SPLIT ? wg0 >= 128 : (wg0 >> 7) * GM * 16 < M2;
+    constexpr int HM = R == 64 ? 2 : 1, HN = R == 128 ? 2 : 1;
+    const int hbx = R == 128 ? wg0 & 63 : wg0 - 128, hby = R == 128 ? wg0 >> 6 : 0;
+    const bool does_head = hbx >= 0 && hby * HM * 16 < B;
+    const int smp_row = R == 128 ? ((wg0 & 63) < 16 ? (wg0 >> 6) * 16 + (wg0 & 63) : 64) : wg0;
+    constexpr int PPW = R == 128 ? 4 : 2;                        // (row, q head) pairs per workgroup: waves 4 .. 4 + PPW - 1
+    const int pair = (SPLIT ? wg0 - 128 : wg0) * PPW + wave - 4;
+    const bool does_attn = wave >= 4 && wave < 4 + PPW && pair >= 0 && pair < Bp * a.q_heads;
+    char* const logits = a.flow + (size_t)FLOW_COPIES * PP_COPY;
+    float *const lo = lds, *const ld = lds + PP_AREA(2), *const big = lds + PP_BIG_FLOATS;
+    // ---- empty this workgroup's tiles of every copy; the launch's first gate tells the others (chain_flow.cuh)
+    auto fill = [&](char* p, int pieces) {
+        const coh_rsrc_t rs = coh_rsrc(p);
+        for (int i = threadIdx.x; i < pieces; i += CH_THREADS) flow_clear16(rs, i * 16);
+    };
+    for (int c = 0; c < FLOW_COPIES; ++c) {
+        char* const cb = a.flow + (size_t)c * PP_COPY;
+        if (does_q)
+            for (int i = 0; i < QM; ++i) fill(cb + PP_QKV + ((wg0 / QC) * QM + i) * (NQ / 16 * 512) + (wg0 % QC) * QN * 512, QN * 32);
+        if (does_attn && (threadIdx.x & 63) < 32) {
+            const int row = pair / a.q_heads, m = (threadIdx.x & 16) ? Bp + row : row;
+            if (m == row || row < B)
+                flow_clear16(coh_rsrc(cb + PP_ATT), (uint32_t)frag_off(m, (pair % a.q_heads) * 128 + 8 * (threadIdx.x & 15), a.q_heads * 128) * 2);
+        }
+        if (does_o) {
+            const int bx = wg0 & 63, by = wg0 >> 6;
+            for (int i = 0; i < OM; ++i) { fill(cb + PP_RA + (by * OM + i) * 32768 + bx * 512, 32); fill(cb + PP_RB + (by * OM + i) * 32768 + bx * 512, 32); }
+            fill(cb + PP_PA + (bx * 128 + by * OM * 16) * 4, OM * 4);
+            fill(cb + PP_PB + (bx * 128 + by * OM * 16) * 4, OM * 4);
+        }
+        if (does_gu)
+            for (int i = 0; i < GM; ++i) fill(cb + PP_ACT + ((SPLIT ? 0 : wg0 >> 7) * GM + i) * 98304 + (wg0 & 127) * 768, 48);
+    }
+    if (does_head)
+        for (int i = 0; i < HM; ++i) fill(logits + (hby * HM + i) * 131072 + hbx * HN * 1024, HN * 64);
+    chain_gate_arrive(g);
+
+    u32x2 res = (u32x2){0u, 0u}, none = res;
+    char *last = nullptr, *lb = a.flow;
+    for (int l = 0; l < a.layers; ++l) {
+        const ChainLayer& L = a.layer[l];
+        int wg = blockIdx.x;                 // opaque per layer (cp_chain_kernel)
+        asm volatile("" : "+s"(wg));
+        char* const nb = l % FLOW_COPIES == FLOW_COPIES - 1 ? a.flow : lb + PP_COPY;
+        if (does_q) {
+            if (!does_o) __syncthreads();
+            if (l == 0)
+                flow_gemm<QM, QN, 4, 3, OMNI_EPI_BF16, 0, false, 128>(L.wqkv, L.ln1, a.resid, a.part, a.np_in, lb + PP_QKV, nullptr, nb + PP_QKV, nullptr, M2, NQ, a.eps,
+                                                                      wg % QC, wg / QC, big, none, fw, 0x0100 | (16 * l + 1), a.stamps, true);
+            else
+                flow_gemm<QM, QN, 4, 4, OMNI_EPI_BF16, 0, false, 128>(L.wqkv, nullptr, last + PP_RB, (const float*)(last + PP_PB), Hc / 16, lb + PP_QKV, nullptr,
+                                                                      nb + PP_QKV, nullptr, M2, NQ, a.eps, wg % QC, wg / QC, big, none, fw, 0x0100 | (16 * l + 1),
+                                                                      a.stamps);
+        }
+        if (l == 0) {                        // everybody's tiles are empty: the first content that is waited for lies behind this
+            chain_gate_wait(g, 0x0102);
+            fw.dead = flow_failed(a.err);
+        }
+        if (does_attn) flow_attn_pair(a, L, pair, lds + PP_ATTN_FLOATS + wave * 256, lb, nb, fw, 0x0100 | (16 * l + 2), a.stamps);
+        const int bx = wg & 63, by = wg >> 6;
+        if (does_o) {
+            if (l == 0) {
+                const int m = by * OM * 16 + (threadIdx.x >> 6) * 16 + (threadIdx.x & 15);
+                if (threadIdx.x < OM * 64 && m < M2) res = coh_ld8(coh_rsrc(a.resid), (uint32_t)frag_off(m, bx * 16 + 4 * ((threadIdx.x & 63) >> 4), Hc) * 2);
+            }
+            flow_gemm<OM, 1, 8, 0, OMNI_EPI_RESID, 0, false, 128>(L.wo, L.ln2, lb + PP_ATT, nullptr, 0, lb + PP_RA, (float*)(lb + PP_PA), nb + PP_RA, (float*)(nb + PP_PA),
+                                                                  M2, Hc, a.eps, bx, by, lo, res, fw, 0x0100 | (16 * l + 3), a.stamps);
+        }
+        if (does_gu) {
+            if (!does_o) __syncthreads();
+            flow_gemm<GM, 3, 4, 4, OMNI_EPI_SILU_MUL_GU8, 0, false, 128>(L.wgu, nullptr, lb + PP_RA, (const float*)(lb + PP_PA), Hc / 16, lb + PP_ACT, nullptr, nb + PP_ACT,
+                                                                         nullptr, M2, NI, a.eps, wg & 127, SPLIT ? 0 : wg >> 7, big, none, fw,
+                                                                         0x0100 | (16 * l + 4), a.stamps);
+        }
+        if (does_o)
+            flow_gemm<OM, 1, 12, 0, OMNI_EPI_RESID, 0, false, 128>(L.wdown, l < a.layers - 1 ? a.layer[l + 1].ln1 : nullptr, lb + PP_ACT, nullptr, 0, lb + PP_RB,
+                                                                   (float*)(lb + PP_PB), nb + PP_RB, (float*)(nb + PP_PB), M2, Hc, a.eps, bx, by, ld, res, fw,
+                                                                   0x0100 | (16 * l + 5), a.stamps);
+        last = lb;
+        lb = nb;
+    }
+    // group 1 on the position-1 rows (tiles Bp / 16 onwards; their slabs start at row Bp)
+    if (does_head) {
+        if (!does_o) __syncthreads();
+        flow_gemm<HM, HN, 4, 2, OMNI_EPI_F32_BF16RND, 0, false, 128>(a.lm_head, a.cp_norm, last + PP_RB + (size_t)Bp * Hc * 2, (const float*)(last + PP_PB) + Bp, Hc / 16,
+                                                                     logits, nullptr, nullptr, nullptr, B, a.codebook, a.eps, hbx, hby, big, none, fw, 0x0156, a.stamps,
+                                                                     false, a.logits_pass ? a.logits : nullptr, a.logits_ld);
+    }
+    if (smp_row < B) {
+        __syncthreads();                     // the combine areas are read
+        flow_sample<false>(a, 1, smp_row, lds, lds, logits, a.resid, a.part, nullptr, nullptr, fw, 0x01F2, a.stamps);
+    }
 }
 
 // the tail's qkv stage as a real call on a copy of the gate (the launch ends behind it: nothing reads the gate afterwards)
@@ -792,7 +765,7 @@ __global__ __launch_bounds__(CH_THREADS) void cp_chain_kernel(const ChainArgs a)
                                                             SPLIT ? 0 : wg >> 6, lds + half * FLOW_HALF_FLOATS, none, fw, pc | 0x56, st, false,
                                                             a.logits_pass ? a.logits + (size_t)(pass - 1) * a.logits_pass : nullptr, a.logits_ld);
         }
-        if (does_smp) flow_sample<(KHT > 0)>(a, pass, smp_row, lds, pb, pb, pbn, fw, pc | 0xF2, st);
+        if (does_smp) flow_sample<(KHT > 0)>(a, pass, smp_row, lds, lds + CPF_SMP_FLOATS, pb + CP_LOG, pb + CP_R0, pb + CP_P0, pbn + CP_R0, pbn + CP_P0, fw, pc | 0xF2, st);
         cp = cpn;
     }
     if constexpr (KHT > 0) {
@@ -806,10 +779,10 @@ __global__ __launch_bounds__(CH_THREADS) void cp_chain_kernel(const ChainArgs a)
 }
 
 // ---- host
-OMNI_KNOB g_cp_chain = 1, g_chain_wide = 0, g_chain_nap = 1, g_chain_span = 2, g_chain_pair = 1;
+OMNI_KNOB g_cp_chain = 1, g_chain_wide = 0, g_chain_span = 2, g_chain_pair = 1;
 #ifdef OMNI_DEBUG_HOOKS
-// gu_narrow 0: above 32 rows always the 48-row split of the stages (16-row gate_up tiles); nap: the pair launch's poll pause
-extern "C" void omni_debug_chain_mode(int, int gu_narrow, int nap) { g_chain_wide = gu_narrow == 0; g_chain_nap = nap; }
+// gu_narrow 0: above 32 rows always the 48-row split of the stages (16-row gate_up tiles)
+extern "C" void omni_debug_chain_mode(int, int gu_narrow, int) { g_chain_wide = gu_narrow == 0; }
 extern "C" void omni_debug_chain_pair(int on) { g_chain_pair = on; }            // positions 0 / 1 + group 1 as a persistent launch (0: the launch path's pair pass)
 static unsigned long long* g_chain_stamps = nullptr;
 // 0: launch per op; 1: one persistent launch per pass (layer stack only); 2: one persistent launch for all passes incl. heads + samplers
@@ -843,9 +816,16 @@ bool k_cp_chain_all_supported(const omni_talker_desc& d, int g0, int greedy, int
 bool k_cp_pair_supported(const omni_talker_desc& d, int B, int greedy, int top_k, float top_p) {
     return g_chain_pair && k_cp_chain_all_supported(d, 1, greedy, top_k, top_p) && d.cp_layers <= CH_MAX_LAYERS && B >= 1 && ((B + 15) & ~15) + B <= 128;
 }
+template <int R>
+static int cp_pair_launch(const ChainArgs& a, hipStream_t stream) {
+    static const hipError_t attr = hipFuncSetAttribute((const void*)cp_pair_kernel<R>, hipFuncAttributeMaxDynamicSharedMemorySize, PP_LDS_BYTES);
+    (void)attr;
+    hipLaunchKernelGGL(cp_pair_kernel<R>, dim3(OMNI_CHAIN_WGS), dim3(CH_THREADS), PP_LDS_BYTES, stream, a);
+    OMNI_CHECK_LAUNCH("cp_pair");
+    return OMNI_OK;
+}
 int k_cp_pair(const omni_talker_desc& d, const omni_layer_weights* layers, uint16_t* const* k_cache, uint16_t* const* v_cache, int B, int np_in,
-              uint16_t* resid, float* part, uint16_t* qkv, uint16_t* attn, uint16_t* act, uint32_t* flags, int32_t* err, const omni_chain_head* head,
-              void* stream) {
+              uint16_t* resid, float* part, uint32_t* flags, int32_t* err, void* flow, const omni_chain_head* head, void* stream) {
     ChainArgs a{};
     for (int l = 0; l < d.cp_layers; ++l) {
         const omni_layer_weights& w = layers[l];
@@ -856,7 +836,7 @@ int k_cp_pair(const omni_talker_desc& d, const omni_layer_weights* layers, uint1
     a.layers = d.cp_layers; a.B = B; a.Bp = (B + 15) & ~15; a.g0 = 0; a.g1 = 2; a.bs = d.num_code_groups + 1; a.np_in = np_in;
     a.q_heads = d.cp_q_heads; a.kv_heads = d.cp_kv_heads;
     a.eps = d.eps; a.sm_scale = 1.0f / sqrtf((float)d.cp_head_dim);
-    a.resid = resid; a.part = part; a.qkv = qkv; a.attn = attn; a.act = act;
+    a.resid = resid; a.part = part; a.flow = (char*)flow;
     a.cos_sin = (const uint16_t*)d.cp_cos_sin;
     a.flags = flags; a.err = err;
     a.with_head = 1;
@@ -866,13 +846,13 @@ int k_cp_pair(const omni_talker_desc& d, const omni_layer_weights* layers, uint1
     a.temperature = head->temperature; a.top_p = head->top_p; a.seed = head->seed;
     a.steps = head->steps; a.row_seed = head->row_seed; a.codes = head->codes;
     a.ptab = (const uint16_t*)d.cp_proj_table;
-    a.nap = g_chain_nap;
 #ifdef OMNI_DEBUG_HOOKS
     a.stamps = g_chain_stamps;            // block 0 of the stamp buffer (the chain's passes 2 .. 15 stamp blocks 2 .. 15)
 #endif
-    hipLaunchKernelGGL(cp_pair_kernel, dim3(OMNI_CHAIN_WGS), dim3(CH_THREADS), 0, (hipStream_t)stream, a);
-    OMNI_CHECK_LAUNCH("cp_pair");
-    return OMNI_OK;
+    const int rows = a.Bp + B;
+    if (rows <= 32) return cp_pair_launch<32>(a, (hipStream_t)stream);
+    if (rows <= 64) return cp_pair_launch<64>(a, (hipStream_t)stream);
+    return cp_pair_launch<128>(a, (hipStream_t)stream);
 }
 
 // backbone widths (hidden / 256) the tail's qkv stage is instantiated for: those of bb_chain.hip's BB_SHAPES

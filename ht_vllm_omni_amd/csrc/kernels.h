@@ -92,8 +92,7 @@ struct omni_chain_tail {
 bool k_cp_chain_tail_supported(const omni_talker_desc& d, int B);
 bool k_cp_pair_supported(const omni_talker_desc& d, int B, int greedy, int top_k, float top_p);
 int k_cp_pair(const omni_talker_desc& d, const omni_layer_weights* layers, uint16_t* const* k_cache, uint16_t* const* v_cache, int B, int np_in,
-              uint16_t* resid, float* part, uint16_t* qkv, uint16_t* attn, uint16_t* act, uint32_t* flags, int32_t* err, const omni_chain_head* head,
-              void* stream);
+              uint16_t* resid, float* part, uint32_t* flags, int32_t* err, void* flow, const omni_chain_head* head, void* stream);
 bool k_cp_chain_supported(const omni_talker_desc& d, int pos);
 bool k_cp_chain_all_supported(const omni_talker_desc& d, int g0, int greedy, int top_k, float top_p);
 size_t k_cp_flow_bytes();                               // the all-pass launch's hand-off buffers (`flow`)

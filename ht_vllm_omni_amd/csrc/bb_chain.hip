@@ -8,6 +8,11 @@
 //   bb_chain_kernel                        a tensor-parallel rank (AR), the half grid (HALF), the debug library's arms: behind flags (chain_gemm.cuh)
 // K-step ownership, combine order and rounding points are the launch path's: results are bit-identical.
 // A decode step, behind flags and by content, one box: 64 rows of the 1.7B shape 3050 -> 2886 us, 5 rows of the 0.6B one 2091 -> 1859.
+// Of a 64-row launch (34 us, 100 MB) gate_up is half: its 50 MB come out of HBM at 5.5 TB/s, and a wave's loads return in order, so half of a wave's
+// slice goes out in front of the first look at the operands and half behind the first of them (down_proj: half of its 24 k-steps, x twelve deep): 2866 ->
+// 2837 us a step.  Slices with a single reader are loaded past the caches, which leaves the last-level cache to the predictor's weights (157 MB): 64 rows
+// 2837 -> 2805, 24 rows 2409 -> 2371, 7 rows 2112 -> 2065, 0.6B, 5 rows 1772 -> 1744; those that the two row halves share are not (64 rows 2817 -> 2839).
+// Tried: gate_up's slice asked for by o_proj's waves (their combine waits for the queue: the same), half of qkv's behind the look (64 rows + 10 us).
 // Shapes are parameters, not literals (the checkpoint decides them, configuration_qwen3_tts.py:192-216): the stage set is a template
 // on the k-steps per wave of its three reduction widths -- KO = q_heads * 128 / 256 (o_proj), KH = hidden / 256 (gate_up, qkv), KI =
 // intermediate / 256 (down_proj); BB_SHAPES lists the instantiated triples: the released 1.7B shape (8, 8, 24) and (6, 6, 18) = hidden 1536 /
@@ -213,6 +218,8 @@ __global__ __launch_bounds__(CH_THREADS) void bb_flow_kernel(const BbArgs a) {
     constexpr int H = KH * 256, I = KI * 256, MO = ROWS == 64 ? 2 : 1, MG = ROWS / 16, NQT = ROWS == 64 ? 2 : 1, MQ = ROWS == 16 ? 1 : 2;
     constexpr BbFlowMap F(H, I);
     constexpr int nc_h = H / 16, nc_gu = I / 24;
+    // weight slices that one workgroup alone reads go past the caches (a step's weights do not fit them, the predictor's do)
+    constexpr int NO = ROWS == 16 ? OMNI_AUX_NT : 0, NQA = ROWS <= 32 ? OMNI_AUX_NT : 0;
     static_assert(nc_h * (ROWS == 16 ? 1 : 2) <= OMNI_CHAIN_WGS && nc_gu <= OMNI_CHAIN_WGS && I % 24 == 0, "bb_flow: tiles");
     const int B = a.B, wg = blockIdx.x;
     const int bxo = wg % nc_h, byo = wg / nc_h;
@@ -245,7 +252,7 @@ __global__ __launch_bounds__(CH_THREADS) void bb_flow_kernel(const BbArgs a) {
     if (does_o) {
         if (threadIdx.x < MO * 64 && byo * MO * 16 + (int)threadIdx.x / 64 * 16 + (threadIdx.x & 15) < B)
             res = coh_ld8(coh_rsrc(a.resid), (uint32_t)frag_off(byo * MO * 16 + threadIdx.x / 64 * 16 + (threadIdx.x & 15), bxo * 16 + 4 * ((threadIdx.x & 63) >> 4), H) * 2);
-        flow_gemm<MO, 1, KO, 0, OMNI_EPI_RESID>(a.wo, a.ln2, a.attn, nullptr, 0, fl + F.ra, (float*)(fl + F.pa), next(F.ra), (float*)next(F.pa), B, H, a.eps, bxo,
+        flow_gemm<MO, 1, KO, 0, OMNI_EPI_RESID, 0, false, 64, 0, NO>(a.wo, a.ln2, a.attn, nullptr, 0, fl + F.ra, (float*)(fl + F.pa), next(F.ra), (float*)next(F.pa), B, H, a.eps, bxo,
                                                 byo, lo, res, fw, 0x1001, a.stamps, BB_GIVEN);
     }
     if (a.first) {
@@ -253,18 +260,18 @@ __global__ __launch_bounds__(CH_THREADS) void bb_flow_kernel(const BbArgs a) {
         fw.dead = flow_failed(a.err);
     }
     if (does_gu)
-        flow_gemm<MG, 3, KH, 4, OMNI_EPI_SILU_MUL_GU8, ROWS == 64 ? 4 : 0>(a.wgu, nullptr, fl + F.ra, (const float*)(fl + F.pa), H / 16, fl + F.act, nullptr, next(F.act),
+        flow_gemm<MG, 3, KH, 4, OMNI_EPI_SILU_MUL_GU8, ROWS == 64 ? 4 : 0, false, 64, 4, OMNI_AUX_NT>(a.wgu, nullptr, fl + F.ra, (const float*)(fl + F.pa), H / 16, fl + F.act, nullptr, next(F.act),
                                                                           nullptr, B, I, a.eps, wg, 0, lg, none, fw, 0x1002, a.stamps);
     const bool qkv = a.wqkv_next != nullptr, head = HEAD && !qkv && a.lm_head != nullptr;
     if (does_o)
         // raw values for the next launch; bf16(w r) for the qkv stage, the values themselves for the head (its norm is exact)
-        flow_gemm<MO, 1, KI, 0, OMNI_EPI_RESID, ROWS == 64 ? 8 : 12>(a.wdown, qkv ? a.ln1_next : nullptr, fl + F.act, nullptr, 0, qkv || head ? fl + F.rb : nullptr,
+        flow_gemm<MO, 1, KI, 0, OMNI_EPI_RESID, ROWS == 64 ? 12 : 8, false, 64, ROWS == 64 ? 12 : 0, NO>(a.wdown, qkv ? a.ln1_next : nullptr, fl + F.act, nullptr, 0, qkv || head ? fl + F.rb : nullptr,
                                                                     (float*)(fl + F.pb), next(F.rb), (float*)next(F.pb), B, H, a.eps, bxo, byo, ld, res, fw, 0x1003,
                                                                     a.stamps, false, nullptr, 0, FlowPlain{nullptr, a.resid, a.part});
     if (qkv) {
         const int nc_q = a.NQ / (16 * NQT), bx = wg % nc_q, by = wg / nc_q;
         if (by * MQ * 16 < B && by < 4 / MQ)
-            flow_gemm<MQ, NQT, KH, 4, OMNI_EPI_BF16, 0, true>(a.wqkv_next, nullptr, fl + F.rb, (const float*)(fl + F.pb), H / 16, nullptr, nullptr, nullptr, nullptr, B,
+            flow_gemm<MQ, NQT, KH, 4, OMNI_EPI_BF16, 0, true, 64, 0, NQA>(a.wqkv_next, nullptr, fl + F.rb, (const float*)(fl + F.pb), H / 16, nullptr, nullptr, nullptr, nullptr, B,
                                                               a.NQ, a.eps, bx, by, lds, none, fw, 0x1004, a.stamps, false, nullptr, a.NQ, FlowPlain{a.qkv});
     } else if (head) {
         const int nc_v = a.V / (16 * NQT), bx = wg % nc_v, by = wg / nc_v;
@@ -321,7 +328,7 @@ __global__ __launch_bounds__(CH_THREADS) void bb_flow_small_kernel(const BbArgs 
     if (does_o) {
         if (threadIdx.x < 64 && byo * 16 + (int)(threadIdx.x & 15) < B)
             res = coh_ld8(coh_rsrc(a.resid), (uint32_t)frag_off(byo * 16 + (threadIdx.x & 15), bxo * 16 + 4 * (threadIdx.x >> 4), H) * 2);
-        flow_gemm<1, 1, 8, 0, OMNI_EPI_RESID>(a.wo, a.ln2, a.attn, nullptr, 0, fl + F.ra, (float*)(fl + F.pa), next(F.ra), (float*)next(F.pa), B, H, a.eps, bxo, byo,
+        flow_gemm<1, 1, 8, 0, OMNI_EPI_RESID, 0, false, 64, 0, ROWS == 16 ? OMNI_AUX_NT : 0>(a.wo, a.ln2, a.attn, nullptr, 0, fl + F.ra, (float*)(fl + F.pa), next(F.ra), (float*)next(F.pa), B, H, a.eps, bxo, byo,
                                               lo, res, fw, 0x1001, a.stamps, BB_GIVEN);
     }
     if (a.first) {
@@ -329,16 +336,16 @@ __global__ __launch_bounds__(CH_THREADS) void bb_flow_small_kernel(const BbArgs 
         fw.dead = flow_failed(a.err);
     }
     if (does_gu)
-        flow_gemm<GM, GN, 4, 4, OMNI_EPI_SILU_MUL_GU8>(a.wgu, nullptr, fl + F.ra, (const float*)(fl + F.pa), H / 16, fl + F.act, nullptr, next(F.act), nullptr, B, I,
+        flow_gemm<GM, GN, 4, 4, OMNI_EPI_SILU_MUL_GU8, 0, false, 64, 0, SPLIT ? OMNI_AUX_NT : 0>(a.wgu, nullptr, fl + F.ra, (const float*)(fl + F.pa), H / 16, fl + F.act, nullptr, next(F.act), nullptr, B, I,
                                                        a.eps, bxg, byg, lg, none, fw, 0x1002, a.stamps);
     const bool qkv = a.wqkv_next != nullptr;
     if (does_o)
-        flow_gemm<1, 1, 12, 0, OMNI_EPI_RESID>(a.wdown, qkv ? a.ln1_next : nullptr, fl + F.act, nullptr, 0, qkv ? fl + F.rb : nullptr, (float*)(fl + F.pb), next(F.rb),
+        flow_gemm<1, 1, 12, 0, OMNI_EPI_RESID, 0, false, 64, 0, ROWS == 16 ? OMNI_AUX_NT : 0>(a.wdown, qkv ? a.ln1_next : nullptr, fl + F.act, nullptr, 0, qkv ? fl + F.rb : nullptr, (float*)(fl + F.pb), next(F.rb),
                                                (float*)next(F.pb), B, H, a.eps, bxo, byo, ld, res, fw, 0x1003, a.stamps, false, nullptr, 0,
                                                FlowPlain{nullptr, a.resid, a.part});
     if (qkv) {
         constexpr int QM = ROWS == 32 ? 2 : 1, QN = SPLIT ? 1 : 4;
-        flow_gemm<QM, QN, 4, 4, OMNI_EPI_BF16, 0, true>(a.wqkv_next, nullptr, fl + F.rb, (const float*)(fl + F.pb), H / 16, nullptr, nullptr, nullptr, nullptr, B, NQ,
+        flow_gemm<QM, QN, 4, 4, OMNI_EPI_BF16, 0, true, 64, 0, SPLIT ? OMNI_AUX_NT : 0>(a.wqkv_next, nullptr, fl + F.rb, (const float*)(fl + F.pb), H / 16, nullptr, nullptr, nullptr, nullptr, B, NQ,
                                                         a.eps, SPLIT ? wg : wg & 63, SPLIT ? 0 : wg >> 6, lds, none, fw, 0x1004, a.stamps, false, nullptr, NQ,
                                                         FlowPlain{a.qkv});
     }

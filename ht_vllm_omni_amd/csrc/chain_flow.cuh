@@ -78,6 +78,8 @@ __device__ __forceinline__ int flow_slot(int row, int piece) { return (row * 4 +
 //   F32_BF16RND   16 x 16 fp32 tiles, 1 KB:  tile t of row group r at (r * (N / 16) + t) * 1024, rows of 64 B
 // res: the residual values of this thread's item (RESID: threads < 64 MT), kept in registers from one residual stage to the next
 // G: k-steps of x in flight (0: the wave's whole share).  A ring looks for EMPTY words step by step, in front of the step's MFMAs
+// WA: k-steps of weights that go out in front of the first look at the operands (0: all); the others go out behind the first k-steps of x
+// WAUX: cache policy of the weights
 // PS: rows per slab of sums of squares
 // pl: what leaves the launch, by plain stores (FlowPlain); ROWS: the output goes there only (BF16 / F32 rows)
 struct FlowPlain {
@@ -86,7 +88,7 @@ struct FlowPlain {
     uint16_t* normed; const int32_t* num_live;        // PRO 2: the normalised rows below *num_live, row-major
     const uint8_t* mask; float mask_fill;             // F32: logit n is mask_fill where mask[n] == 0
 };
-template <int MT, int NT, int NTW, int PRO, int EPI, int G = 0, bool ROWS = false, int PS = 64>
+template <int MT, int NT, int NTW, int PRO, int EPI, int G = 0, bool ROWS = false, int PS = 64, int WA = 0, int WAUX = 0>
 __device__ __forceinline__ void flow_gemm(const uint16_t* __restrict__ W, const uint16_t* __restrict__ norm_w, const void* x, const float* part_in,
                                           int np_in, void* out, float* part_out, void* clr, float* clr_part, int M, int N, float eps, int bx, int by,
                                           float* lds, u32x2& res, FlowWait& fw, int code, unsigned long long* stamps,
@@ -134,13 +136,16 @@ __device__ __forceinline__ void flow_gemm(const uint16_t* __restrict__ W, const 
 
     // ---- what does not depend on the predecessor: the weight slice, the norm weights
     u32x4 Wq[NTW][NT], NWq[NW ? NTW : 1];
+    auto load_w = [&](int d0, int d1) {
 #pragma unroll
-    for (int d = 0; d < NTW; ++d) {
-        const int ks = wave + d * CH_WAVES;
+        for (int d = d0; d < d1; ++d) {
+            const int ks = wave + d * CH_WAVES;
 #pragma unroll
-        for (int j = 0; j < NT; ++j) Wq[d][j] = __builtin_amdgcn_raw_buffer_load_b128(wrs, lane16, (uint32_t)(((bx * NT + j) * nsteps + ks) * 1024), 0);
-        if (NW) NWq[d] = __builtin_amdgcn_raw_buffer_load_b128(nrs, q * 16, ks * 64, 0);
-    }
+            for (int j = 0; j < NT; ++j) Wq[d][j] = __builtin_amdgcn_raw_buffer_load_b128(wrs, lane16, (uint32_t)(((bx * NT + j) * nsteps + ks) * 1024), WAUX);
+            if (NW) NWq[d] = __builtin_amdgcn_raw_buffer_load_b128(nrs, q * 16, ks * 64, 0);
+        }
+    };
+    load_w(0, WA > 0 ? WA : NTW);
     u32x2 nwn = (u32x2){0x3f803f80u, 0x3f803f80u};                       // RESID: the next norm's weights of this thread's columns (1: none)
     if (RESID && norm_w != nullptr) nwn = __builtin_amdgcn_raw_buffer_load_b64(nrs, (bx * 16 + 4 * q) * 2, 0, 0);
     CH_STAMP(stamps, sidx, 1);                                           // 1: weight loads issued
@@ -189,6 +194,7 @@ __device__ __forceinline__ void flow_gemm(const uint16_t* __restrict__ W, const 
     CH_STAMP(stamps, sidx, 2);                                           // 2: something is there
     if (NORM) load_p();
     load_x(0, XG);
+    if (WA > 0) load_w(WA, NTW);
     while (!RING && go) {
         uint32_t w = 0;
         if (NORM) {

@@ -69,6 +69,20 @@ __device__ __forceinline__ void flow_barrier() { asm volatile("s_waitcnt vmcnt(0
 #define FLOW_HALF_FLOATS (CH_WAVES * FLOW_TILES * 256 + CH_WAVES * 64)
 __device__ __forceinline__ int flow_slot(int row, int piece) { return (row * 4 + (piece ^ ((row >> 2) & 3))) * 4; }        // in floats
 
+// a later stage's weight slice, asked for ahead of it
+template <int NT, int NTW>
+__device__ __forceinline__ void flow_ask(const uint16_t* W, int bx, u32x4 (&Wq)[NTW][NT]) {
+    int tid = threadIdx.x;
+    asm volatile("" : "+v"(tid));      // opaque per call (flow_gemm)
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const coh_rsrc_t rs = coh_rsrc(W);
+#pragma unroll
+    for (int d = 0; d < NTW; ++d)
+#pragma unroll
+        for (int j = 0; j < NT; ++j)
+            Wq[d][j] = __builtin_amdgcn_raw_buffer_load_b128(rs, (tid & 63) * 16, (uint32_t)(((bx * NT + j) * NTW * CH_WAVES + wave + d * CH_WAVES) * 1024), 0);
+}
+
 // One skinny-GEMM stage: chain_gemm's k-steps per wave, accumulation, combine order and rounding points (the launch path's bits), its x and
 // slabs awaited by content.  x: fragment-major, 32-column k-steps; `x` / `part_in` / `out` / `part_out` lie in this use's copy (or, the launch's
 // first input, in the plain buffers its predecessor filled: never EMPTY).  clr / clr_part: the same places in the copy to clear, NULL: none.
@@ -79,6 +93,7 @@ __device__ __forceinline__ int flow_slot(int row, int piece) { return (row * 4 +
 // res: the residual values of this thread's item (RESID: threads < 64 MT), kept in registers from one residual stage to the next
 // G: k-steps of x in flight (0: the wave's whole share).  A ring looks for EMPTY words step by step, in front of the step's MFMAs
 // WA: k-steps of weights that go out in front of the first look at the operands (0: all); the others go out behind the first k-steps of x
+// WP: the weight slice is in Wp already (flow_ask)
 // WAUX: cache policy of the weights
 // PS: rows per slab of sums of squares
 // pl: what leaves the launch, by plain stores (FlowPlain); ROWS: the output goes there only (BF16 / F32 rows)
@@ -88,13 +103,13 @@ struct FlowPlain {
     uint16_t* normed; const int32_t* num_live;        // PRO 2: the normalised rows below *num_live, row-major
     const uint8_t* mask; float mask_fill;             // F32: logit n is mask_fill where mask[n] == 0
 };
-template <int MT, int NT, int NTW, int PRO, int EPI, int G = 0, bool ROWS = false, int PS = 64, int WA = 0, int WAUX = 0>
+template <int MT, int NT, int NTW, int PRO, int EPI, int G = 0, bool ROWS = false, int PS = 64, int WA = 0, int WAUX = 0, bool WP = false>
 __device__ __forceinline__ void flow_gemm(const uint16_t* __restrict__ W, const uint16_t* __restrict__ norm_w, const void* x, const float* part_in,
                                           int np_in, void* out, float* part_out, void* clr, float* clr_part, int M, int N, float eps, int bx, int by,
                                           float* lds, u32x2& res, FlowWait& fw, int code, unsigned long long* stamps,
                                           bool given = false /* x and the slabs were there before the launch: taken as they are, whatever their words */,
                                           float* logits_rows = nullptr /* F32: also row-major, row m at logits_rows + m * ldo */, int ldo = 0,
-                                          const FlowPlain pl = FlowPlain{}) {
+                                          const FlowPlain pl = FlowPlain{}, const u32x4 (*Wp)[NT] = nullptr) {
     const int sidx = ((code & 255) >> 4) * 5 + (code & 15) - 1;
     constexpr bool NORM = PRO == 2 || PRO == 3 || PRO == 4, DEFER = PRO == 3 || PRO == 4, NW = PRO == 2 || PRO == 3;
     constexpr bool GU8 = EPI == OMNI_EPI_SILU_MUL_GU8, RESID = EPI == OMNI_EPI_RESID, F32 = EPI == OMNI_EPI_F32_BF16RND;
@@ -141,7 +156,7 @@ __device__ __forceinline__ void flow_gemm(const uint16_t* __restrict__ W, const 
         for (int d = d0; d < d1; ++d) {
             const int ks = wave + d * CH_WAVES;
 #pragma unroll
-            for (int j = 0; j < NT; ++j) Wq[d][j] = __builtin_amdgcn_raw_buffer_load_b128(wrs, lane16, (uint32_t)(((bx * NT + j) * nsteps + ks) * 1024), WAUX);
+            for (int j = 0; j < NT; ++j) Wq[d][j] = WP ? Wp[d][j] : __builtin_amdgcn_raw_buffer_load_b128(wrs, lane16, (uint32_t)(((bx * NT + j) * nsteps + ks) * 1024), WAUX);
             if (NW) NWq[d] = __builtin_amdgcn_raw_buffer_load_b128(nrs, q * 16, ks * 64, 0);
         }
     };

@@ -158,13 +158,21 @@ size_t k_cp_flow_bytes() { return CP_FLOW_BYTES > PP_FLOW_BYTES ? CP_FLOW_BYTES 
 // attention at buffer position pos <= 15 (dense private cache: row b owns block b): one wave per (row, q head), the work layout of
 // attn_tiny_dense_kernel (paged_attn.hip).  A kv head's q heads are waves of ONE workgroup, in every pass the same one: the K / V rows that the
 // first of them writes are read, passes later, behind that workgroup's own barriers.
-struct FlowHist { u32x4 k[4]; uint32_t v[16]; };        // a wave's history rows: lane = (token lane / 4, quarter lane % 4) of K, a dword of every token of V
-__device__ __forceinline__ void flow_history(const ChainArgs& a, const ChainLayer& L, int pair, FlowHist& hist) {
+// a wave's history rows: lane = (token lane / 4, quarter lane % 4) of K, a dword of every token of V; and what the norm and the rotation multiply by (asked for
+// behind the wait, the trip stood between q and the scores: a decode step of 64 rows 2817 -> 2787 us, of 5 rows 1739 -> 1720)
+struct FlowHist { u32x4 k[4]; uint32_t v[16]; uint16_t qn[2], kn[2], cs[2]; };
+__device__ __forceinline__ void flow_history(const ChainArgs& a, const ChainLayer& L, int pos, int pair, FlowHist& hist) {
     int lane = threadIdx.x & 63;
     asm volatile("" : "+v"(lane));
     const int row = pair / a.q_heads, kvh = (pair - row * a.q_heads) / (a.q_heads / a.kv_heads);
     const coh_rsrc_t krs = coh_rsrc(L.kc), vrs = coh_rsrc(L.vc);
     const uint32_t hrow = ((uint32_t)(row * a.bs + (lane >> 2)) * a.kv_heads + kvh) * 128;
+#pragma unroll
+    for (int e = 0; e < 2; ++e) {
+        hist.qn[e] = L.qnorm[lane + 64 * e];
+        hist.kn[e] = L.knorm[lane + 64 * e];
+        hist.cs[e] = a.cos_sin[(size_t)pos * 128 + lane + 64 * e];
+    }
 #pragma unroll
     for (int j = 0; j < 4; ++j) hist.k[j] = coh_ld16(krs, (hrow + (lane & 3) * 32 + j * 8) * 2);
 #pragma unroll
@@ -209,10 +217,10 @@ __device__ __forceinline__ void flow_attn(const ChainArgs& a, const ChainLayer& 
     __builtin_amdgcn_wave_barrier();
     const uint16_t* rq = reinterpret_cast<const uint16_t*>(raw);
     const uint16_t* rk = rq + 128;
-    const uint16_t* cs = a.cos_sin + (size_t)pos * 128;
     float q0, q1, k0, k1;
-    head_norm_rope_vals(bf2f(rq[lane]), bf2f(rq[lane + 64]), L.qnorm, cs, a.eps, lane, q0, q1);
-    head_norm_rope_vals(bf2f(rk[lane]), bf2f(rk[lane + 64]), L.knorm, cs, a.eps, lane, k0, k1);
+    const float co = bf2f(hist.cs[0]), si = bf2f(hist.cs[1]);
+    head_norm_rope_with(bf2f(rq[lane]), bf2f(rq[lane + 64]), bf2f(hist.qn[0]), bf2f(hist.qn[1]), co, si, a.eps, q0, q1);
+    head_norm_rope_with(bf2f(rk[lane]), bf2f(rk[lane + 64]), bf2f(hist.kn[0]), bf2f(hist.kn[1]), co, si, a.eps, k0, k1);
     if (h % ratio == 0) {
         // the new token's K / V into the private cache: one dword per lane (even lanes elements l, l + 1 of the first half, odd lanes l + 63,
         // l + 64 of the second), written through for the later passes
@@ -424,6 +432,15 @@ __device__ __forceinline__ void flow_attn_pair(const ChainArgs& a, const ChainLa
     const coh_rsrc_t krs = coh_rsrc(L.kc), vrs = coh_rsrc(L.vc), qrs = coh_rsrc(buf + PP_QKV), ars = coh_rsrc(buf + PP_ATT), crs = coh_rsrc(clr + PP_ATT);
     if (lane < 16) flow_clear16(crs, (uint32_t)frag_off(row, h * 128 + 8 * lane, width) * 2);
     else if (lane < 32 && both) flow_clear16(crs, (uint32_t)frag_off(a.Bp + row, h * 128 + 8 * (lane - 16), width) * 2);
+    // what the norm and the rotation multiply by, ahead of the wait (FlowHist)
+    uint16_t qn[2], kn[2], cs[4];
+#pragma unroll
+    for (int e = 0; e < 2; ++e) {
+        qn[e] = L.qnorm[lane + 64 * e];
+        kn[e] = L.knorm[lane + 64 * e];
+    }
+#pragma unroll
+    for (int e = 0; e < 4; ++e) cs[e] = a.cos_sin[lane + 64 * e];
     CH_STAMP_BY(stamps, sidx, 1, 256);
     // elements 2 l, 2 l + 1 of the heads out of the qkv stage's tiles
     auto at = [&](int m, int head) -> uint32_t { return (uint32_t)((m >> 4) * tiles * 512 + (m & 15) * 32 + (lane >> 3) * 512 + (lane & 7) * 4 + head * 4096); };
@@ -453,9 +470,10 @@ __device__ __forceinline__ void flow_attn_pair(const ChainArgs& a, const ChainLa
         __builtin_amdgcn_wave_barrier();
         const uint16_t* rh = reinterpret_cast<const uint16_t*>(raw);
         float k00, k01, k10, k11, q0, q1;
-        head_norm_rope_vals(bf2f(rh[lane]), bf2f(rh[lane + 64]), L.knorm, a.cos_sin, a.eps, lane, k00, k01);
-        head_norm_rope_vals(bf2f(rh[128 + lane]), bf2f(rh[128 + lane + 64]), L.knorm, a.cos_sin + 128, a.eps, lane, k10, k11);
-        head_norm_rope_vals(bf2f(rh[256 + lane]), bf2f(rh[256 + lane + 64]), L.qnorm, a.cos_sin + 128, a.eps, lane, q0, q1);
+        const float w0 = bf2f(kn[0]), w1 = bf2f(kn[1]), c1 = bf2f(cs[2]), s1_ = bf2f(cs[3]);
+        head_norm_rope_with(bf2f(rh[lane]), bf2f(rh[lane + 64]), w0, w1, bf2f(cs[0]), bf2f(cs[1]), a.eps, k00, k01);
+        head_norm_rope_with(bf2f(rh[128 + lane]), bf2f(rh[128 + lane + 64]), w0, w1, c1, s1_, a.eps, k10, k11);
+        head_norm_rope_with(bf2f(rh[256 + lane]), bf2f(rh[256 + lane + 64]), bf2f(qn[0]), bf2f(qn[1]), c1, s1_, a.eps, q0, q1);
         __builtin_amdgcn_wave_barrier();
         const float qs = a.sm_scale * LOG2E;
         const float s0 = wave_sum(fmaf(q0 * qs, k00, (q1 * qs) * k01));
@@ -685,6 +703,12 @@ __global__ __launch_bounds__(CH_THREADS) void cp_chain_kernel(const ChainArgs a)
     int cl = 0, cp = 0, half = 0;                                // copies of this layer's and this pass's hand-offs; LDS half of the next combine
     bool open = false;                                           // the launch's first gate is behind us
     u32x2 res = (u32x2){0u, 0u}, none = res;
+    constexpr int QMT = ROWS == 32 ? 2 : 1, QNT = SPLIT ? 1 : 4;
+    // Up to 16 rows the workgroups of o_proj / down_proj ask for their qkv slice ahead of down_proj, not behind it: the heads they own were the last that
+    // the attention waited for.  A decode step, 5 rows of the 0.6B talker 1720 -> 1702 us, 7 of the 1.7B one 2067 -> 2049; at up to 32 rows, where all
+    // of down_proj's operands queue behind it, 2362 -> 2373.
+    constexpr bool ASK = ROWS == 16;
+    u32x4 Wn[4][QNT];
     for (int pass = a.g0; pass < a.g1; ++pass) {
         const int pc = pass << 8;            // error-word stage codes: (pass << 8) | (16 * layer + stage + 1); head 0x56, sampler 0xF2
         // debug library: every pass stamps its own block of CH_STAMP_PASS words
@@ -707,16 +731,17 @@ __global__ __launch_bounds__(CH_THREADS) void cp_chain_kernel(const ChainArgs a)
             const float* pin = first ? a.part : (const float*)(pbl + CP_P0);
             const int np = first ? a.np_in : 1;
             const bool given = first;
-            constexpr int QMT = ROWS == 32 ? 2 : 1, QNT = SPLIT ? 1 : 4;
             // the attention's history (written by earlier passes, rows >= pass hold stale bytes and are masked): there before its q / k / v
+            if (ASK && (!does_o || (first && l == 0))) flow_ask<QNT, 4>(L.wqkv, wg, Wn);
             FlowHist hist;
-            if (does_attn) flow_history(a, L, pair, hist);
+            if (does_attn) flow_history(a, L, pass, pair, hist);
             if (l == 0)
-                flow_gemm<QMT, QNT, 4, 3, OMNI_EPI_BF16>(L.wqkv, L.ln1, xin, pin, np, lb + CP_QKV, nullptr, nb + CP_QKV, nullptr, B, NQ, a.eps,
-                                                         SPLIT ? wg : wg & 63, SPLIT ? 0 : wg >> 6, area(), none, fw, pc | (16 * l + 1), st, given);
+                flow_gemm<QMT, QNT, 4, 3, OMNI_EPI_BF16, 0, false, 64, 0, 0, ASK>(L.wqkv, L.ln1, xin, pin, np, lb + CP_QKV, nullptr, nb + CP_QKV, nullptr, B, NQ, a.eps,
+                                                         SPLIT ? wg : wg & 63, SPLIT ? 0 : wg >> 6, area(), none, fw, pc | (16 * l + 1), st, given, nullptr, 0, FlowPlain{}, Wn);
             else
-                flow_gemm<QMT, QNT, 4, 4, OMNI_EPI_BF16>(L.wqkv, nullptr, last + CP_RB, (const float*)(last + CP_PB), Hc / 16, lb + CP_QKV, nullptr, nb + CP_QKV,
-                                                         nullptr, B, NQ, a.eps, SPLIT ? wg : wg & 63, SPLIT ? 0 : wg >> 6, area(), none, fw, pc | (16 * l + 1), st);
+                flow_gemm<QMT, QNT, 4, 4, OMNI_EPI_BF16, 0, false, 64, 0, 0, ASK>(L.wqkv, nullptr, last + CP_RB, (const float*)(last + CP_PB), Hc / 16, lb + CP_QKV, nullptr, nb + CP_QKV,
+                                                         nullptr, B, NQ, a.eps, SPLIT ? wg : wg & 63, SPLIT ? 0 : wg >> 6, area(), none, fw, pc | (16 * l + 1), st, false, nullptr, 0, FlowPlain{},
+                                                         Wn);
             if (!open) {                                         // everybody's tiles are empty: the first content that is waited for lies behind this
                 chain_gate_wait(g, pc | (16 * l + 2));
                 fw.dead = flow_failed(a.err);
@@ -746,6 +771,7 @@ __global__ __launch_bounds__(CH_THREADS) void cp_chain_kernel(const ChainArgs a)
                                                                  nullptr, B, NI, a.eps, ROWS == 32 ? wg - NO : wg & 127, ROWS == 32 ? 0 : wg >> 7, area(), none, fw,
                                                                  pc | (16 * l + 4), st);
             }
+            if (ASK && does_o) flow_ask<QNT, 4>(a.layer[l < a.layers - 1 ? l + 1 : 0].wqkv, wg, Wn);
             if (does_o)
                 flow_gemm<1, 1, 12, 0, OMNI_EPI_RESID>(L.wdown, l < a.layers - 1 ? a.layer[l + 1].ln1 : nullptr, lb + CP_ACT, nullptr, 0, to_plain ? (void*)a.resid : lb + CP_RB,
                                                        to_plain ? a.part : (float*)(lb + CP_PB), nb + CP_RB, (float*)(nb + CP_PB), B, Hc, a.eps, wg & 63, wg >> 6,

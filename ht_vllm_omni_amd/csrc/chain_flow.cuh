@@ -39,15 +39,19 @@ __device__ __forceinline__ float flow_or0(float w) { return __uint_as_float(flow
 struct FlowWait {
     int32_t* err;
     int dead;              // this wave gave up once (or the launch began with the error word set); wave-uniform
+    int calm;              // looks further apart (constant: a launch's split of its stages)
 };
 __device__ __forceinline__ int flow_failed(const int32_t* err) {
     return __builtin_amdgcn_readfirstlane(__hip_atomic_load(err, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) != 0;
 }
 // another look at the operands is due: false = carry on with what is there.  (Looks at lines nobody has written since are served by the XCD's
-// own L2; a pause of 0, 64 or 256 clocks costs 0.3 to 0.7 % of a step against these 128)
+// own L2.  The predictor's launch, pauses of 0 / 64 / 128 / 256 / 384 clocks: 64 rows 2807 / 2810 / 2781 / 2770 / 2785 us a step, 40 rows of the 0.6B talker
+// 2208 / 2204 / 2214 (128 / 256 / 384), 24 rows 1992 / 2002 / 2006, 5 rows 1719 / 1717 / 1719 / 1722 and, on another box, 1697 / 1700 / 1705 (128 / 256 / 384): twice as long above 32 rows, where every
+// workgroup waits in every stage.  The backbone's layers: no difference.)
 __device__ __forceinline__ bool flow_again(FlowWait& f, int code, unsigned& spins, unsigned long long& t0) {
     if (f.dead) return false;
-    __builtin_amdgcn_s_sleep(2);
+    if (f.calm) __builtin_amdgcn_s_sleep(4);
+    else __builtin_amdgcn_s_sleep(2);
     if (chain_wait_expired(++spins, t0)) {
         if ((threadIdx.x & 63) == 0) atomicCAS(f.err, 0, code);
         f.dead = 1;

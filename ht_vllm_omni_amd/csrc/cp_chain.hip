@@ -653,7 +653,7 @@ __global__ __launch_bounds__(CH_THREADS) void cp_chain_kernel(const ChainArgs a)
         if (threadIdx.x < 64) chain_flag_publish(g.frs, wg0, g.epoch + 1u);
         return;
     }
-    FlowWait fw{a.err, g.dead ? 1 : 0};
+    FlowWait fw{a.err, g.dead ? 1 : 0, !SPLIT};
     float* const attn_lds = lds + CPF_ATTN_FLOATS + wave * 256;
     // ---- this workgroup's part of each stage
     const bool does_o = !SPLIT || wg0 < NO, does_gu = !SPLIT || wg0 >= NO;

@@ -7,8 +7,8 @@
 //   bb_flow_kernel, bb_flow_small_kernel   one rank, the whole chip: activations cross by content (chain_flow.cuh)
 //   bb_chain_kernel                        a tensor-parallel rank (AR), the half grid (HALF), the debug library's arms: behind flags (chain_gemm.cuh)
 // K-step ownership, combine order and rounding points are the launch path's: results are bit-identical.
-// A decode step, behind flags and by content, one box: 64 rows of the 1.7B shape 3050 -> 2886 us, 5 rows of the 0.6B one 2091 -> 1859.
-// Of a 64-row launch (34 us, 100 MB) gate_up is half: its 50 MB come out of HBM at 5.5 TB/s, and a wave's loads return in order, so half of a wave's
+// A decode step, behind flags and by content, one card: 64 rows of the 1.7B shape 3050 -> 2886 us, 5 rows of the 0.6B one 2091 -> 1859.
+// Of a 64-row launch (32 us, 100 MB) gate_up is half: its 50 MB come out of HBM at 5.5 TB/s, and a wave's loads return in order, so half of a wave's
 // slice goes out in front of the first look at the operands and half behind the first of them (down_proj: half of its 24 k-steps, x twelve deep): 2866 ->
 // 2837 us a step.  Slices with a single reader are loaded past the caches, which leaves the last-level cache to the predictor's weights (157 MB): 64 rows
 // 2837 -> 2805, 24 rows 2409 -> 2371, 7 rows 2112 -> 2065, 0.6B, 5 rows 1772 -> 1744; those that the two row halves share are not (64 rows 2817 -> 2839).

@@ -46,7 +46,7 @@ __device__ __forceinline__ int flow_failed(const int32_t* err) {
 }
 // another look at the operands is due: false = carry on with what is there.  (Looks at lines nobody has written since are served by the XCD's
 // own L2.  The predictor's launch, pauses of 0 / 64 / 128 / 256 / 384 clocks: 64 rows 2807 / 2810 / 2781 / 2770 / 2785 us a step, 40 rows of the 0.6B talker
-// 2208 / 2204 / 2214 (128 / 256 / 384), 24 rows 1992 / 2002 / 2006, 5 rows 1719 / 1717 / 1719 / 1722 and, on another box, 1697 / 1700 / 1705 (128 / 256 / 384): twice as long above 32 rows, where every
+// 2208 / 2204 / 2214 (128 / 256 / 384), 24 rows 1992 / 2002 / 2006, 5 rows 1719 / 1717 / 1719 / 1722 and, on another card, 1697 / 1700 / 1705 (128 / 256 / 384): twice as long above 32 rows, where every
 // workgroup waits in every stage.  The backbone's layers: no difference.)
 __device__ __forceinline__ bool flow_again(FlowWait& f, int code, unsigned& spins, unsigned long long& t0) {
     if (f.dead) return false;

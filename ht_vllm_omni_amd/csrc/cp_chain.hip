@@ -8,7 +8,7 @@
 //   * a stage's WEIGHT slice does not depend on its predecessor: every wave loads its whole slice before it looks for its operands;
 //   * cp_chain_kernel (passes 2 .. 15, their heads and samplers) hands activations over by content: an operand is there when none of its words
 //     is EMPTY (chain_flow.cuh).  No drain, no flag, no barrier between a stage's last store and its successor's first MFMA.  What bounds it is
-//     that chain of dependent trips: 27 stages a pass of about 2.7 us (5 rows: 73 us a pass; 64 rows: 90), of which 0.6 to 1.6 us are a stage's own
+//     that chain of dependent trips: 27 stages a pass of about 2.6 us (5 rows: 69 us a pass; 64 rows: 89), of which 0.6 to 1.6 us are a stage's own
 //     arithmetic, LDS combine and epilogue and the rest the operands' way.  Behind flags (coherent.cuh) a pass took 104 / 110 us;
 //   * cp_pair_kernel (positions 0 and 1, group 1) likewise, over both positions' rows; a decode step of 64 / of 5 rows, us, behind flags 2886 / 1859, by
 //     content 2860 / 1784 (the stages of up to 16 rows over all 256 workgroups: 64 of them owned every column of qkv);

@@ -97,7 +97,6 @@ struct ChainGate {
     int nap;               // s_sleep units (64 clocks) between two polls: 0, 1, 2, 4, 8
     int ahead;             // stages this workgroup has passed without rows since it last waited (chain_gate_skip)
     int skip_units;        // sleep per skipped stage before the first poll, in units of 32 x 64 clocks (3 = ~2.9 us; A/B knob)
-    int skip;              // debug library only (timing experiments, results garbage): 1 = fetch half of every weight slice, 2 = half of the activations
     unsigned long long* stamps;   // debug library only: timeline stamps of the attention stage (pa_body.cuh, CHAIN), or NULL
     // engine mode (NULL / unused in the plain chains): barriers among the 8 compute waves only, weights from the LDS FIFO
     EngSync* es;
@@ -162,7 +161,6 @@ __device__ __forceinline__ void chain_gate_init(ChainGate& g, uint32_t* flags, i
     g.dom = 8;
     g.nap = 1;
     g.skip_units = 3;
-    g.skip = 0;
     g.stamps = nullptr;
     g.ahead = 0;
     g.es = nullptr; g.bgen = 0; g.fifo = nullptr; g.piece_base = 0; g.ready = 0;

@@ -13,15 +13,13 @@ void omni_debug_tile(int nt, int mt);                       /* force the GEMM ti
 void omni_debug_int8_max_g(int g);                         /* int8-KV decode attention: q heads per workgroup (2 | 4) */
 void omni_debug_cp_pair01(int on);                         /* code predictor: positions 0 and 1 as one two-block pass */
 void omni_debug_cp_chain(int on);                          /* code predictor: the layer stack of a pass as one persistent launch */
-void omni_debug_chain_mode(int dom, int gu_narrow, int nap); /* chain A/B: log2 flag domain (6 | 7 | 8); gate_up on the 32 x 24 tile; s_sleep units between polls */
+void omni_debug_chain_mode(int, int wide, int);            /* predictor chain: wide 0 = above 32 rows always the 48-row split of its stages (the other arguments are of earlier forms) */
 void omni_debug_chain_stamps(void* buf);                   /* device uint64 [16 passes][40][8][256]: per-stage timeline stamps of every chain launch, one block per predictor pass, block 0 = the pair kernel (NULL: off) */
 void omni_debug_bb_chain(int on);                          /* backbone: o_proj -> gate_up -> down_proj -> next qkv as one persistent launch per layer */
 void omni_debug_bb_all(int on);                            /* backbone: the whole decoder stack, attention included, as ONE persistent launch (bb_all.hip) */
 void omni_debug_bb_all_stamps(void* buf, int layer);       /* uint64 [8][8][256] timeline stamps of one layer's stages of that launch (NULL: off) */
-void omni_debug_chain_defer(int on);                       /* code-predictor chain A/B arm: RMSNorm rstd applied in the qkv / gate_up epilogues (another rounding point than the reference's; timing + accuracy experiments) */
 void omni_debug_chain_pair(int on);                        /* code predictor: positions 0 / 1 + group 1's head and sampler as one persistent launch (cp_pair_kernel) */
 void omni_debug_chain_tail(int on);                         /* 1 (default): the step's input assembly + layer 0's qkv as the tail of the predictor's all-pass launch; 0: launches of their own (round 5) */
-void omni_debug_chain_skip(int mode);                      /* code-predictor chain timing experiment: 1 = fetch half of every weight slice, 2 = half of the activations, 4 = the polling wave fetches no weights, 5 = no wave does (garbage results) */
 void omni_debug_bb_min_rows(int rows);                     /* backbone chain: smallest batch the 64-row stage set takes (33 since round 5; 49: round 4's policy, 33-48 rows launch per op) */
 void omni_debug_moe_chain(int on);                         /* sparse-MoE layer: o_proj -> router | shared gate_up -> shared down + routing as one persistent launch (moe_chain.hip) */
 void omni_debug_pa_tail(int on);                           /* decode attention: the last, partial 128-token round as contiguous 32-token chunks per wave (0: interleaved groups) */

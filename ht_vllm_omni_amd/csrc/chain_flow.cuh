@@ -32,8 +32,8 @@ __device__ __forceinline__ uint32_t flow_word(uint32_t w) { return w == FLOW_EMP
 __device__ __forceinline__ uint32_t flow_max(u32x4 v) { return max(max(v[0], v[1]), max(v[2], v[3])); }
 __device__ __forceinline__ void flow_clear16(coh_rsrc_t rs, uint32_t off) { coh_st16(rs, off, (u32x4){FLOW_EMPTY, FLOW_EMPTY, FLOW_EMPTY, FLOW_EMPTY}); }
 
-// A wave that does not wait (any more) takes 0 for a word that is EMPTY: a step that is thrown away may hold anything but NaNs, which the private
-// K / V cache would keep -- rows past the position are masked by a weight of 0
+// A wave that does not wait (any more) takes 0 for a word that is EMPTY, so a step that is thrown away computes on zeros and not on NaNs.  Nothing depends
+// on it: what such a step leaves in a cache is written again before it is read
 __device__ __forceinline__ uint32_t flow_or0(uint32_t w) { return w == FLOW_EMPTY ? 0u : w; }
 __device__ __forceinline__ float flow_or0(float w) { return __uint_as_float(flow_or0(__float_as_uint(w))); }
 struct FlowWait {
@@ -228,7 +228,7 @@ __device__ __forceinline__ void flow_gemm(const uint16_t* __restrict__ W, const 
         if (NORM) load_p();
         load_x(0, XG);
     }
-    if (!RING && fw.dead) {                                                     // (see FlowWait)
+    if (!RING && fw.dead) {                                                     // (see flow_or0)
 #pragma unroll
         for (int e = 0; e < SO::PE; ++e) pv[e] = flow_or0(pv[e]);
 #pragma unroll

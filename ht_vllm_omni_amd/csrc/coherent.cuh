@@ -27,9 +27,9 @@
 
 typedef __amdgpu_buffer_rsrc_t coh_rsrc_t;
 
-__device__ __forceinline__ coh_rsrc_t coh_rsrc(const void* base) {
-    // stride 0 (raw), num_records = max, flags: DATA_FORMAT = 32 (bits 12-18 of dword 3: 0x00020000)
-    return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(base), 0, 0x7fffffff, 0x00020000);
+__device__ __forceinline__ coh_rsrc_t coh_rsrc(const void* base, int bytes = 0x7fffffff) {
+    // stride 0 (raw), num_records = bytes (past them a load returns 0), flags: DATA_FORMAT = 32 (bits 12-18 of dword 3: 0x00020000)
+    return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(base), 0, bytes, 0x00020000);
 }
 __device__ __forceinline__ u32x4 coh_ld16(coh_rsrc_t rs, uint32_t byte_off) {
     return __builtin_amdgcn_raw_buffer_load_b128(rs, byte_off, 0, OMNI_AUX_SC1);

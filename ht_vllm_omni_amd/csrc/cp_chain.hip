@@ -159,13 +159,15 @@ size_t k_cp_flow_bytes() { return CP_FLOW_BYTES > PP_FLOW_BYTES ? CP_FLOW_BYTES 
 // attn_tiny_dense_kernel (paged_attn.hip).  A kv head's q heads are waves of ONE workgroup, in every pass the same one: the K / V rows that the
 // first of them writes are read, passes later, behind that workgroup's own barriers.
 // a wave's history rows: lane = (token lane / 4, quarter lane % 4) of K, a dword of every token of V; and what the norm and the rotation multiply by (asked for
-// behind the wait, the trip stood between q and the scores: a decode step of 64 rows 2817 -> 2787 us, of 5 rows 1739 -> 1720)
+// behind the wait, the trip stood between q and the scores: a decode step of 64 rows 2817 -> 2787 us, of 5 rows 1739 -> 1720).
+// Rows from pos on hold what an earlier step left there, possibly NaN or infinity, which a weight of 0 does not mask: V's descriptor ends at row pos,
+// past which a load returns 0 (K's scores are replaced)
 struct FlowHist { u32x4 k[4]; uint32_t v[16]; uint16_t qn[2], kn[2], cs[2]; };
 __device__ __forceinline__ void flow_history(const ChainArgs& a, const ChainLayer& L, int pos, int pair, FlowHist& hist) {
     int lane = threadIdx.x & 63;
     asm volatile("" : "+v"(lane));
-    const int row = pair / a.q_heads, kvh = (pair - row * a.q_heads) / (a.q_heads / a.kv_heads);
-    const coh_rsrc_t krs = coh_rsrc(L.kc), vrs = coh_rsrc(L.vc);
+    const int row = __builtin_amdgcn_readfirstlane(pair / a.q_heads), kvh = (pair - row * a.q_heads) / (a.q_heads / a.kv_heads);
+    const coh_rsrc_t krs = coh_rsrc(L.kc), vrs = coh_rsrc(L.vc + (size_t)row * a.bs * a.kv_heads * 128, pos * a.kv_heads * 256);
     const uint32_t hrow = ((uint32_t)(row * a.bs + (lane >> 2)) * a.kv_heads + kvh) * 128;
 #pragma unroll
     for (int e = 0; e < 2; ++e) {
@@ -176,7 +178,7 @@ __device__ __forceinline__ void flow_history(const ChainArgs& a, const ChainLaye
 #pragma unroll
     for (int j = 0; j < 4; ++j) hist.k[j] = coh_ld16(krs, (hrow + (lane & 3) * 32 + j * 8) * 2);
 #pragma unroll
-    for (int u = 0; u < 16; ++u) hist.v[u] = coh_ld4(vrs, (((uint32_t)(row * a.bs + u) * a.kv_heads + kvh) * 128 + 2 * lane) * 2);
+    for (int u = 0; u < 16; ++u) hist.v[u] = coh_ld4(vrs, ((uint32_t)(u * a.kv_heads + kvh) * 128 + 2 * lane) * 2);
 }
 __device__ __forceinline__ void flow_attn(const ChainArgs& a, const ChainLayer& L, int pos, int pair, float* sq, const char* in, char* out, char* clr,
                                           const FlowHist& hist, FlowWait& fw, int code, unsigned long long* stamps) {

@@ -287,8 +287,9 @@ __global__ __launch_bounds__(256) void attn_tiny_dense_kernel(const uint16_t* __
 #pragma unroll
     for (int u = 0; u < 16; ++u) {
         const float pu = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(p), 4 * u));
-        o0 = fmaf(pu, bf_lo(vq[u]), o0);
-        o1 = fmaf(pu, bf_hi(vq[u]), o1);
+        const uint32_t vu = u < pos ? vq[u] : 0u;          // rows from pos on: an earlier step's, possibly NaN, which a weight of 0 does not mask
+        o0 = fmaf(pu, bf_lo(vu), o0);
+        o1 = fmaf(pu, bf_hi(vu), o1);
     }
     const int col = h * 128 + 2 * lane;
     uint16_t* op = out_frag ? out + frag_off(row, col, q_heads * 128) : out + (size_t)row * q_heads * 128 + col;

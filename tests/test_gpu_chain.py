@@ -95,6 +95,33 @@ def test_all_pass_chain_at_the_edges_of_its_row_splits(B, top_p):
         assert torch.equal(x, y)
 
 
+@pytest.mark.parametrize("chain", [0, 2], ids=["launches", "chain"])
+@pytest.mark.parametrize("B", [5, 24, 40, 64])
+def test_a_row_of_nans_leaves_nothing_behind(B, chain):
+    """One row's input is NaN for one call.  What the private K / V cache keeps of it lies past the position of every later pass that has not written
+    there again yet: the row's next call, with finite inputs, gives what it gave before."""
+    d = get_dims("tts-1.7b").with_(layers=1, max_model_len=256)
+    w = make_weights(d, seed=12, std=0.02)
+    code0, e0, lh = (t.cuda() for t in _inputs(d, w, B, 3 * B))
+    bad = lh.clone()
+    bad[B // 2] = float("nan")
+    with L.debug_library() as lib:
+        lib.omni_debug_cp_chain.argtypes = [C.c_int]; lib.omni_debug_cp_chain.restype = None
+        try:
+            lib.omni_debug_cp_chain(chain)
+            eng = _engine(d, w, kv_dtype="bf16", num_blocks=8, max_batch=64)
+            outs = [eng.code_predictor(code0.to(torch.int32), e0, x, greedy=True, return_logits=True) for x in (lh, bad, lh)]
+            assert eng.chain_error() == 0
+            assert eng.chains_ran() == (1 if chain else 0)
+        finally:
+            lib.omni_debug_cp_chain(2)
+    other = [b for b in range(B) if b != B // 2]
+    assert outs[1][1][B // 2].isnan().all(), "the NaN row's logits"
+    for first, poisoned, again in zip(*outs):
+        assert torch.equal(poisoned[other], first[other]), "another row changed"
+        assert torch.equal(again, first), "the NaN row's next call differs"
+
+
 def test_chain_matches_oracle_at_full_predictor_depth():
     """Product library, chain on (the default): greedy codes / logits of the 5-layer, 16-group predictor vs the oracle."""
     d = get_dims("tts-1.7b").with_(layers=1, max_model_len=256)

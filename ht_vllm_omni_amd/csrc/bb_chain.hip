@@ -19,6 +19,7 @@
 // intermediate 4608 / 12 q heads, a shape no released checkpoint has (tests/test_gpu_chain.py).  A shape runs here when its triple is listed
 // and every stage's tile grid fits the 256 workgroups (k_bb_chain_supported); the 0.6B shape has the code predictor's layer dimensions and its
 // split of the stages; every other configuration stays on the launch path.
+#include "bb_areas.h"
 #include "chain_flow.cuh"
 #include "common.cuh"
 #include "kernels.h"
@@ -47,9 +48,7 @@ struct BbArgs {
     char *flow, *flow_next;
     int first;
 };
-// LDS of a stage's combine with `tiles` tiles, in floats; a launch's stages take turns: o_proj | gate_up | down_proj, and the last stage over the first
-// two's (their readers are behind down_proj's barrier)
-#define BB_AREA(tiles) (CH_WAVES * (tiles) * 256 + CH_WAVES * 64)
+static_assert(BB_WAVES == CH_WAVES, "bb_areas.h");
 
 // (Round 3 also tried a ninth wave that warms the XCD's L2 with the next stage's slice -- one dword per 64 bytes, nothing
 // depending on it: +0.10 ms per step, removed; and the loader / consumer split of bb_engine.hip.  What is kept is below:
@@ -217,7 +216,10 @@ __global__ __launch_bounds__(CH_THREADS) void bb_flow_kernel(const BbArgs a) {
     extern __shared__ __attribute__((aligned(16))) float lds[];
     constexpr int H = KH * 256, I = KI * 256, MO = ROWS == 64 ? 2 : 1, MG = ROWS / 16, NQT = ROWS == 64 ? 2 : 1, MQ = ROWS == 16 ? 1 : 2;
     constexpr BbFlowMap F(H, I);
+    constexpr BbAreas A = bb_areas_wide(ROWS);
     constexpr int nc_h = H / 16, nc_gu = I / 24;
+    static_assert(ROWS == 16 || nc_gu <= 2 * nc_h, "bb_areas_wide: whoever runs gate_up runs down_proj");
+    static_assert(A.gate_up == bb_area(MO) && A.down == A.gate_up + bb_area(3 * MG) && A.last + bb_area(MQ * NQT) <= A.total, "bb_areas_wide: tiles");
     // weight slices that one workgroup alone reads go past the caches (a step's weights do not fit them, the predictor's do)
     constexpr int NO = ROWS == 16 ? OMNI_AUX_NT : 0, NQA = ROWS <= 32 ? OMNI_AUX_NT : 0;
     static_assert(nc_h * (ROWS == 16 ? 1 : 2) <= OMNI_CHAIN_WGS && nc_gu <= OMNI_CHAIN_WGS && I % 24 == 0, "bb_flow: tiles");
@@ -248,7 +250,7 @@ __global__ __launch_bounds__(CH_THREADS) void bb_flow_kernel(const BbArgs a) {
         chain_gate_arrive(g);
     }
     auto next = [&](uint32_t off) -> char* { return nx != nullptr ? nx + off : nullptr; };
-    float *const lo = lds, *const lg = lo + BB_AREA(MO), *const ld = lg + BB_AREA(3 * MG);
+    float *const lo = lds + A.o, *const lg = lds + A.gate_up, *const ld = lds + A.down, *const ll = lds + A.last;
     if (does_o) {
         if (threadIdx.x < MO * 64 && byo * MO * 16 + (int)threadIdx.x / 64 * 16 + (threadIdx.x & 15) < B)
             res = coh_ld8(coh_rsrc(a.resid), (uint32_t)frag_off(byo * MO * 16 + threadIdx.x / 64 * 16 + (threadIdx.x & 15), bxo * 16 + 4 * ((threadIdx.x & 63) >> 4), H) * 2);
@@ -272,12 +274,12 @@ __global__ __launch_bounds__(CH_THREADS) void bb_flow_kernel(const BbArgs a) {
         const int nc_q = a.NQ / (16 * NQT), bx = wg % nc_q, by = wg / nc_q;
         if (by * MQ * 16 < B && by < 4 / MQ)
             flow_gemm<MQ, NQT, KH, 4, OMNI_EPI_BF16, 0, true, 64, 0, NQA>(a.wqkv_next, nullptr, fl + F.rb, (const float*)(fl + F.pb), H / 16, nullptr, nullptr, nullptr, nullptr, B,
-                                                              a.NQ, a.eps, bx, by, lds, none, fw, 0x1004, a.stamps, false, nullptr, a.NQ, FlowPlain{a.qkv});
+                                                              a.NQ, a.eps, bx, by, ll, none, fw, 0x1004, a.stamps, false, nullptr, a.NQ, FlowPlain{a.qkv});
     } else if (head) {
         const int nc_v = a.V / (16 * NQT), bx = wg % nc_v, by = wg / nc_v;
         if (by * MQ * 16 < B && by < 4 / MQ)
             flow_gemm<MQ, NQT, KH, 2, OMNI_EPI_F32_BF16RND, 0, true>(a.lm_head, a.final_norm, fl + F.rb, (const float*)(fl + F.pb), H / 16, nullptr, nullptr, nullptr,
-                                                                     nullptr, B, a.V, a.eps, bx, by, lds, none, fw, 0x1005, a.stamps, false, a.logits, a.V,
+                                                                     nullptr, B, a.V, a.eps, bx, by, ll, none, fw, 0x1005, a.stamps, false, a.logits, a.V,
                                                                      FlowPlain{nullptr, nullptr, nullptr, a.last_hidden, a.num_live, a.mask, a.mask_fill});
     }
 }
@@ -289,6 +291,7 @@ __global__ __launch_bounds__(CH_THREADS) void bb_flow_small_kernel(const BbArgs 
     extern __shared__ __attribute__((aligned(16))) float lds[];
     constexpr int H = 1024, I = 3072, NQ = 4096;
     constexpr BbFlowMap F(H, I);
+    constexpr BbAreas A = bb_areas_small(ROWS);
     constexpr bool SPLIT = ROWS <= 32;
     constexpr int NO = ROWS == 16 ? 64 : 128;                    // SPLIT: workgroups of o_proj / down_proj; the others do gate_up
     const int B = a.B, wg = blockIdx.x;
@@ -307,6 +310,8 @@ __global__ __launch_bounds__(CH_THREADS) void bb_flow_small_kernel(const BbArgs 
     FlowWait fw{a.err, 0};
     u32x2 res = (u32x2){0u, 0u}, none = res;
     constexpr int GM = ROWS == 16 || ROWS == 48 ? 1 : 2, GN = ROWS == 16 ? 2 : (ROWS == 48 ? 6 : 3);       // gate_up's tiles
+    constexpr int QM = ROWS == 32 ? 2 : 1, QN = SPLIT ? 1 : 4;
+    static_assert(A.gate_up == bb_area(1) && A.down == A.gate_up + bb_area(ROWS == 16 ? 2 : 6) && GM * GN <= 6 && A.last + bb_area(QM * QN) <= A.total, "bb_areas_small: tiles");
     const int bxg = SPLIT ? wg - NO : (ROWS == 48 ? wg & 63 : wg & 127), byg = SPLIT ? 0 : (ROWS == 48 ? wg >> 6 : wg >> 7);
     if (a.first) {
         chain_gate_init(g, a.flags, a.err);
@@ -324,7 +329,7 @@ __global__ __launch_bounds__(CH_THREADS) void bb_flow_small_kernel(const BbArgs 
         chain_gate_arrive(g);
     }
     auto next = [&](uint32_t off) -> char* { return nx != nullptr ? nx + off : nullptr; };
-    float *const lo = lds, *const lg = lo + BB_AREA(1), *const ld = lg + BB_AREA(GM * GN);
+    float *const lo = lds + A.o, *const lg = lds + A.gate_up, *const ld = lds + A.down, *const ll = lds + A.last;
     if (does_o) {
         if (threadIdx.x < 64 && byo * 16 + (int)(threadIdx.x & 15) < B)
             res = coh_ld8(coh_rsrc(a.resid), (uint32_t)frag_off(byo * 16 + (threadIdx.x & 15), bxo * 16 + 4 * (threadIdx.x >> 4), H) * 2);
@@ -344,9 +349,8 @@ __global__ __launch_bounds__(CH_THREADS) void bb_flow_small_kernel(const BbArgs 
                                                (float*)next(F.pb), B, H, a.eps, bxo, byo, ld, res, fw, 0x1003, a.stamps, false, nullptr, 0,
                                                FlowPlain{nullptr, a.resid, a.part});
     if (qkv) {
-        constexpr int QM = ROWS == 32 ? 2 : 1, QN = SPLIT ? 1 : 4;
         flow_gemm<QM, QN, 4, 4, OMNI_EPI_BF16, 0, true, 64, 0, SPLIT ? OMNI_AUX_NT : 0>(a.wqkv_next, nullptr, fl + F.rb, (const float*)(fl + F.pb), H / 16, nullptr, nullptr, nullptr, nullptr, B, NQ,
-                                                        a.eps, SPLIT ? wg : wg & 63, SPLIT ? 0 : wg >> 6, lds, none, fw, 0x1004, a.stamps, false, nullptr, NQ,
+                                                        a.eps, SPLIT ? wg : wg & 63, SPLIT ? 0 : wg >> 6, ll, none, fw, 0x1004, a.stamps, false, nullptr, NQ,
                                                         FlowPlain{a.qkv});
     }
 }
@@ -405,8 +409,7 @@ bool k_bb_chain_small(const omni_talker_desc& d) {
 // one shape's launches, by rows; the step's head rides along where the last layer's launch brings one
 template <int KO, int KH, int KI, int ROWS, bool HEAD>
 static int bb_launch_rows(const BbArgs& a, hipStream_t stream) {
-    constexpr int MO = ROWS == 64 ? 2 : 1;
-    constexpr int bytes = (BB_AREA(MO) + BB_AREA(3 * ROWS / 16) + BB_AREA(MO)) * 4;
+    constexpr int bytes = bb_areas_wide(ROWS).total * 4;
     static const hipError_t attr = hipFuncSetAttribute((const void*)bb_flow_kernel<KO, KH, KI, ROWS, HEAD>, hipFuncAttributeMaxDynamicSharedMemorySize, bytes);
     (void)attr;
     hipLaunchKernelGGL((bb_flow_kernel<KO, KH, KI, ROWS, HEAD>), dim3(OMNI_CHAIN_WGS), dim3(CH_THREADS), bytes, stream, a);
@@ -422,7 +425,7 @@ static int bb_launch_shape(const BbArgs& a, int B, hipStream_t stream) {
 }
 template <int ROWS>
 static int bb_launch_small(const BbArgs& a, hipStream_t stream) {
-    constexpr int bytes = (BB_AREA(1) + BB_AREA(ROWS == 16 ? 2 : 6) + BB_AREA(1)) * 4;
+    constexpr int bytes = bb_areas_small(ROWS).total * 4;
     static const hipError_t attr = hipFuncSetAttribute((const void*)bb_flow_small_kernel<ROWS>, hipFuncAttributeMaxDynamicSharedMemorySize, bytes);
     (void)attr;
     hipLaunchKernelGGL(bb_flow_small_kernel<ROWS>, dim3(OMNI_CHAIN_WGS), dim3(CH_THREADS), bytes, stream, a);

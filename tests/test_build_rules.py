@@ -71,3 +71,25 @@ def test_no_kernel_of_runs_that_nothing_reaches():
     code = open(B.LIB_DECODER, "rb").read()
     assert b"rec_run_kernelILi8ELi16E" in code and b"rec_run_kernelILi16ELi32E" in code
     assert b"rec_run_kernelILi8ELi32E" not in code
+
+
+# (kernel, rows, tiles of a workgroup in o_proj, gate_up and the last stage, a workgroup may run gate_up without down_proj)
+LAYER_LAUNCHES = [("wide", 16, 1, 3, 1, True), ("wide", 32, 1, 6, 2, False), ("wide", 64, 2, 12, 4, False), ("small", 16, 1, 2, 1, True),
+                  ("small", 32, 1, 6, 2, True), ("small", 48, 1, 6, 4, False), ("small", 64, 1, 6, 4, False)]
+
+
+@pytest.mark.parametrize("kernel,rows,o,gu,last,alone", LAYER_LAUNCHES)
+def test_a_layer_launch_combines_over_nothing_that_is_still_read(tmp_path, kernel, rows, o, gu, last, alone):
+    """LDS of the backbone's layer launches: the three areas of o_proj, gate_up and down_proj do not meet; the last stage's never meets down_proj's, and
+    where a workgroup runs gate_up and no down_proj -- no barrier between -- it does not meet gate_up's."""
+    src = tmp_path / "areas.cpp"
+    src.write_text(f"""
+#include "bb_areas.h"
+constexpr BbAreas a = bb_areas_{kernel}({rows});
+constexpr bool apart(int x, int nx, int y, int ny) {{ return x + bb_area(nx) <= y || y + bb_area(ny) <= x; }}
+static_assert(apart(a.o, {o}, a.gate_up, {gu}) && apart(a.o, {o}, a.down, {o}) && apart(a.gate_up, {gu}, a.down, {o}), "three areas");
+static_assert(apart(a.last, {last}, a.down, {o}), "the last stage over down_proj's");
+static_assert({str(not alone).lower()} || apart(a.last, {last}, a.gate_up, {gu}), "the last stage over gate_up's");
+static_assert(a.down + bb_area({o}) <= a.total && a.last + bb_area({last}) <= a.total && a.total * 4 <= 160 * 1024, "total");
+""")
+    subprocess.run(["g++", "-std=c++17", "-fsyntax-only", "-I", CSRC, str(src)], check=True, timeout=60)

@@ -81,6 +81,13 @@ __device__ __forceinline__ int block_argmax(float v, int idx, float* sval, int* 
     return bi;
 }
 
+// the thread's index, opaque to the optimiser: inside a persistent kernel's pass loop hipcc otherwise computes whatever follows from it -- 64 lane masks,
+// the elements' and candidates' indices -- ahead of the loop and keeps it in scratch (cp_chain_kernel<16>: 42 VGPRs)
+__device__ __forceinline__ int smp_opaque(int i) {
+    asm volatile("" : "+v"(i));
+    return i;
+}
+
 // The pick of one row.  xr[e] = element threadIdx.x + 256 e of the row AFTER penalty / temperature (-inf beyond V and in every
 // passive thread); live = threadIdx.x < 256; step = the RNG counter of this draw.  EVERY thread of the workgroup calls this
 // (workgroup barriers inside, under workgroup-uniform conditions only).
@@ -185,12 +192,13 @@ __device__ __forceinline__ int smp_pick(float (&xr)[NPT], int V, int greedy, int
                 total += coff[w];
             }
             int o = base + inc - cnt;
+            const int tid = smp_opaque(threadIdx.x);
             if (total <= SMP_PCAP || !fast) {
 #pragma unroll
                 for (int e = 0; e < NPT; ++e)
                     if (xr[e] >= thr && xr[e] > -INFINITY) {
                         if (o < SMP_PCAP) {
-                            ckey[o] = ((unsigned long long)ord_key(xr[e]) << 32) | (uint32_t)(~(uint32_t)(threadIdx.x + e * SMP_THREADS));
+                            ckey[o] = ((unsigned long long)ord_key(xr[e]) << 32) | (uint32_t)(~(uint32_t)(tid + e * SMP_THREADS));
                             if (want_p) cexp[o] = expf(xr[e] - mx);
                         }
                         ++o;
@@ -198,7 +206,7 @@ __device__ __forceinline__ int smp_pick(float (&xr)[NPT], int V, int greedy, int
             }
             // pad to a multiple of 8 with keys that sort after everything (the rank loop runs 8 entries per trip)
             const int nn = min(total, SMP_PCAP);
-            if (threadIdx.x < 8 && nn + (int)threadIdx.x < ((nn + 7) & ~7)) { ckey[nn + threadIdx.x] = 0ull; cexp[nn + threadIdx.x] = 0.f; }
+            if (tid < 8 && nn + tid < ((nn + 7) & ~7)) { ckey[nn + tid] = 0ull; cexp[nn + tid] = 0.f; }
             __syncthreads();
             return total;
         };
@@ -212,11 +220,12 @@ __device__ __forceinline__ int smp_pick(float (&xr)[NPT], int V, int greedy, int
 #pragma unroll
                 for (int e = 0; e < NPT; ++e) lm = fmaxf(lm, xr[e]);
                 const int q = (top_k + SMP_THREADS / 64 - 1) / (SMP_THREADS / 64);
+                const int ln = smp_opaque(lane);
                 int rk = 0;
 #pragma unroll
                 for (int j = 0; j < 64; ++j) {
                     const float o = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(lm), j));
-                    rk += (o > lm || (o == lm && j < lane)) ? 1 : 0;
+                    rk += (o > lm || (o == lm && j < ln)) ? 1 : 0;
                 }
                 if (rk == q - 1) wq[wave] = lm;
                 const float wm = wave_max(lm);
@@ -284,11 +293,12 @@ __device__ __forceinline__ int smp_pick(float (&xr)[NPT], int V, int greedy, int
         }
         float bv = -INFINITY;
         int bi = 0x7FFFFFFF;
+        const int tid = smp_opaque(threadIdx.x);
         if (have_list) {
             // D: the kept candidates are the only elements with a finite score
 #pragma unroll
             for (int sl = 0; sl < SLOTS; ++sl) {
-                const int c = threadIdx.x + sl * SMP_THREADS;
+                const int c = tid + sl * SMP_THREADS;
                 if (live && c < n) {
                     const unsigned long long me = ckey[c];
                     const float x = key_val((uint32_t)(me >> 32));
@@ -303,7 +313,7 @@ __device__ __forceinline__ int smp_pick(float (&xr)[NPT], int V, int greedy, int
         } else {
 #pragma unroll
             for (int e = 0; e < NPT; ++e) {
-                const int i = threadIdx.x + e * SMP_THREADS;
+                const int i = tid + e * SMP_THREADS;
                 const float x = xr[e];
                 if (x >= kth && x > -INFINITY) {
                     const float u = hash_uniform(seed, step, (uint32_t)i);

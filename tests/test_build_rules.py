@@ -5,8 +5,9 @@ float code, and the forms that read the high dword of a VGPR src1 pair in the lo
 SIMD issues MFMAs (profiles/r04_pkfma_probe.txt) -- parity-green and bit-stable alone, wrong beside a neighbour.  The libraries are built
 with the feature off (build.FLAGS); this test compiles with the same flags and looks at what came out.
 
-Rule 2: no scratch memory in the kernels of the language models' library.  A tile kernel whose epilogue outgrew the compiler's unrolling kept its
-accumulators there -- right results, 25 us more per launch."""
+Rule 2: no scratch memory in the kernels of the language models' library and in the talker's persistent launches.  A tile kernel whose epilogue outgrew the
+compiler's unrolling kept its accumulators there -- right results, 25 us more per launch.  The all-pass launch that ends in the step's tail is the one
+exception: its two calls that are not inlined have a stack, once a launch."""
 import os
 import re
 import shutil
@@ -37,6 +38,18 @@ def scratch_bytes(lines):
     return [int(m.group(1)) for m in (re.match(r"^; ScratchSize: (\d+)", l) for l in lines) if m]
 
 
+def kernel_scratch(lines):
+    """{kernel: scratch bytes a lane}: the first size behind each kernel's label"""
+    out, name = {}, None
+    for l in lines:
+        m = re.match(r"^(_Z\w+):", l)
+        name = m.group(1) if m else name
+        m = re.match(r"^; ScratchSize: (\d+)", l)
+        if m and "_kernel" in name:
+            out.setdefault(name, int(m.group(1)))
+    return out
+
+
 def test_the_scanner_sees_the_form():
     got = packed_fp32(["_Zk:", "\tv_pk_fma_f32 v[0:1], v[2:3], v[4:5], v[0:1] op_sel:[0,1,0]", "\tv_pk_mul_f32 v[0:1], v[2:3], v[4:5]",
                        "\tv_pk_add_f32 v[0:1], v[2:3], s[4:5]", "\tv_pk_fma_f16 v0, v1, v2, v3", "\tv_fma_f32 v0, v1, v2, v3"])
@@ -60,6 +73,12 @@ def test_no_kernel_holds_a_packed_fp32_op(tmp_path, defines):
     assert sum(len(a) for a in asms) > 10000
     assert not bad, f"{len(bad)} packed fp32 ops, e.g. {bad[:4]}"
     if not defines:
+        chains = {}
+        for n in ("cp_chain.hip", "bb_chain.hip"):
+            chains |= kernel_scratch(asms[names.index(n)])
+        tail = {k for k in chains if "cp_chain_kernelILi64ELi" in k and "ELi0E" not in k}
+        assert len(chains) > 20 and len(tail) == 2
+        assert all(chains[k] <= 352 for k in tail) and not any(v for k, v in chains.items() if k not in tail), {k: v for k, v in chains.items() if v}
         scratch = {n: scratch_bytes(lines) for n, lines in zip(names, asms) if n in B.DECODER_SOURCES}
         assert sum(map(len, scratch.values())) > 50
         assert not any(map(any, scratch.values())), {n: v for n, v in scratch.items() if any(v)}

@@ -807,10 +807,10 @@ __global__ __launch_bounds__(CH_THREADS) void cp_chain_kernel(const ChainArgs a)
 }
 
 // ---- host
-OMNI_KNOB g_cp_chain = 1, g_chain_wide = 0, g_chain_span = 2, g_chain_pair = 1;
+OMNI_KNOB g_cp_chain = 1, g_chain_split48 = 0, g_chain_span = 2, g_chain_pair = 1;
 #ifdef OMNI_DEBUG_HOOKS
-// wide 0: above 32 rows always the 48-row split of the stages (16-row gate_up tiles)
-extern "C" void omni_debug_chain_mode(int, int wide, int) { g_chain_wide = wide == 0; }
+// above 48 rows too the 48-row split of the stages (16-row gate_up tiles)
+extern "C" void omni_debug_chain_split48(int on) { g_chain_split48 = on; }
 extern "C" void omni_debug_chain_pair(int on) { g_chain_pair = on; }            // positions 0 / 1 + group 1 as a persistent launch (0: the launch path's pair pass)
 static unsigned long long* g_chain_stamps = nullptr;
 // 0: launch per op; 1: one persistent launch per pass (layer stack only); 2: one persistent launch for all passes incl. heads + samplers
@@ -897,7 +897,7 @@ bool k_cp_chain_tail_supported(const omni_talker_desc& d, int B) {
     const int NQ = (d.q_heads + 2 * d.kv_heads) * 128;
     // every row group live (B > 48: no workgroup leaves at launch start, all of them own a qkv tile with rows), the norm-free stream, the
     // qkv stage's 32 x 32 tile grid inside the 256 workgroups
-    return g_chain_tail && !g_chain_wide && g_cp_chain && g_chain_span >= 2 && listed && B > 48 && B <= 64 && d.fused_norm && d.frag_layout && d.moe_experts == 0 && d.head_dim == 128 &&
+    return g_chain_tail && !g_chain_split48 && g_cp_chain && g_chain_span >= 2 && listed && B > 48 && B <= 64 && d.fused_norm && d.frag_layout && d.moe_experts == 0 && d.head_dim == 128 &&
            NQ % 32 == 0 && (NQ / 32) * 2 <= OMNI_CHAIN_WGS && d.hidden % 8 == 0;
 }
 
@@ -958,7 +958,7 @@ int k_cp_chain(const omni_talker_desc& d, const omni_layer_weights* layers, uint
     }
     if (B <= 16) CP_LAUNCH(16);
     if (B <= 32) CP_LAUNCH(32);
-    if (B <= 48 || g_chain_wide) CP_LAUNCH(48);
+    if (B <= 48 || g_chain_split48) CP_LAUNCH(48);
     CP_LAUNCH(64);
 #undef CP_LAUNCH
 }

@@ -1,6 +1,6 @@
 """The code predictor's layer stack as persistent launches (csrc/cp_chain.hip) against the launch-per-op path of the SAME
 library: the chain keeps tiles, k-step ownership, accumulation order and rounding points, so codes AND logits must be
-bit-identical; the flag waits must never time out (error word 0).  Reference function: the decoder loop of
+bit-identical; no wait may time out (error word 0).  Reference function: the decoder loop of
 qwen3_tts_code_predictor_vllm.py:480-561 (parity of either schedule with the oracle: tests/test_gpu_engine.py)."""
 import ctypes as C
 
@@ -27,42 +27,34 @@ def _inputs(d, w, B, seed):
     return code0, w["embed"][code0], torch.randn(B, d.hidden, generator=g).to(BF16)
 
 
-@pytest.mark.parametrize("mode", [(2, 7, 1, 1), (1, 7, 1, 1), (2, 8, 1, 4), (2, 6, 0, 1)],
-                         ids=["all-passes", "per-pass", "all-passes-all-flags-nap4", "all-passes-wide-gate_up"])
-@pytest.mark.parametrize("model,B", [("tts-1.7b", 64), ("tts-1.7b", 37), ("tts-1.7b", 5), ("tts-0.6b", 16), ("tts-1.7b", 32), ("tts-1.7b", 48), ("tts-1.7b", 17)])
-def test_chain_is_bit_identical_to_the_launch_chain(model, B, mode):
-    """mode = (span, flag domain, gate_up tile, poll pause): span 1 = one persistent launch per pass (layer stack only), 2 = ONE
-    launch for every pass with its head GEMM and sampler.  The 48-column gate_up tile sums the RMSNorm statistics in the
-    16-row order, which is the launch path's order only up to 32 rows: above that the comparison is on rounding distance."""
+@pytest.mark.parametrize("model,B,span,split48",
+                         [(m, B, span, 0) for m, B in (("tts-1.7b", 64), ("tts-1.7b", 37), ("tts-1.7b", 5), ("tts-0.6b", 16), ("tts-1.7b", 32), ("tts-1.7b", 48),
+                                                       ("tts-1.7b", 17)) for span in (2, 1)] + [("tts-1.7b", 64, 2, 1), ("tts-1.7b", 53, 2, 1)])
+def test_chain_is_bit_identical_to_the_launch_chain(model, B, span, split48):
+    """span 1 = one persistent launch per pass (layer stack only), 2 = ONE launch for every pass with its head GEMM and sampler.  split48: above 48 rows
+    too the split of the stages that 33 to 48 rows have (16-row gate_up tiles): the bits do not depend on a tile's height (gemm_frag.cuh SlabOrder)."""
     d = get_dims(model).with_(layers=1, max_model_len=256)          # the released predictor: 5 layers, 16 groups
     w = make_weights(d, seed=33, std=0.02)
     code0, e0, lh = _inputs(d, w, B, B)
     res = {}
     with L.debug_library() as lib:
         lib.omni_debug_cp_chain.argtypes = [C.c_int]; lib.omni_debug_cp_chain.restype = None
-        lib.omni_debug_chain_mode.argtypes = [C.c_int, C.c_int, C.c_int]; lib.omni_debug_chain_mode.restype = None
+        lib.omni_debug_chain_split48.argtypes = [C.c_int]; lib.omni_debug_chain_split48.restype = None
         try:
             for on in (0, 1):
-                lib.omni_debug_cp_chain(mode[0] if on else 0)
-                lib.omni_debug_chain_mode(*mode[1:])
+                lib.omni_debug_cp_chain(span if on else 0)
+                lib.omni_debug_chain_split48(split48)
                 eng = _engine(d, w, kv_dtype="bf16", num_blocks=8, max_batch=64)
-                for rep in range(3):                                 # flags / epochs carry over from call to call
+                for rep in range(3):                                 # flags and hand-off buffers carry over from call to call
                     codes, lg = eng.code_predictor(code0.to(torch.int32).cuda(), e0.cuda(), lh.cuda(), greedy=True, return_logits=True)
                     steps = torch.full((B,), 3 + rep, dtype=torch.int32)
                     sampled = eng.code_predictor(code0.to(torch.int32).cuda(), e0.cuda(), lh.cuda(), greedy=False, temperature=0.9,
                                                  top_k=50, seed=7, steps=steps.cuda())
-                assert eng.chain_error() == 0
+                assert eng.chain_error() == 0 and eng.chains_ran() == on
                 res[on] = (codes.cpu(), lg.cpu(), sampled.cpu())
         finally:
             lib.omni_debug_cp_chain(2)
-            lib.omni_debug_chain_mode(7, 1, 1)
-    if mode[2] == 0 and B > 32:          # other summation order of the norm statistics: equal to rounding, not to the bit
-        # (rows whose greedy codes forked at a near-tie read other inputs from that group on: the logits are compared on the rows that stayed
-        #  together -- until round 6 no row of this seed forked and the comparison silently covered all of them)
-        same = (res[1][0] == res[0][0]).all(dim=1)
-        assert same.float().mean().item() >= 0.8
-        assert_e2e_close(res[1][1][same], res[0][1][same], mean_tol=2e-3, max_ulps=3, what="wide gate_up tile vs launch chain")
-        return
+            lib.omni_debug_chain_split48(0)
     bad = (res[1][0] != res[0][0]).any(dim=1).nonzero().flatten().tolist()
     assert torch.equal(res[1][0], res[0][0]), f"greedy codes differ between the persistent chain and the launch chain in rows {bad}: first differing group per row {[int((res[1][0][b] != res[0][0][b]).nonzero()[0]) for b in bad]}"
     assert torch.equal(res[1][1], res[0][1]), "logits differ between the persistent chain and the launch chain"
@@ -87,7 +79,7 @@ def test_all_pass_chain_at_the_edges_of_its_row_splits(B, top_p):
                 steps = torch.full((B,), 5, dtype=torch.int32, device="cuda")
                 sampled = [eng.code_predictor(code0.to(torch.int32), e0, lh, greedy=False, temperature=0.9, top_k=50, top_p=top_p, seed=3, steps=steps) for _ in range(2)]
                 codes, lg = eng.code_predictor(code0.to(torch.int32), e0, lh, greedy=True, return_logits=True)
-                assert eng.chain_error() == 0
+                assert eng.chain_error() == 0 and eng.chains_ran() == (1 if on else 0)
                 res[on] = [t.cpu() for t in (*sampled, codes, lg)]
         finally:
             lib.omni_debug_cp_chain(2)
@@ -152,8 +144,8 @@ def _decode_engine(d, w, B, kv="fp8"):
     return eng
 
 
-# the released 1.7B width, and one NO released checkpoint has (round 6: the stage sets are instantiated from the shape --
-# csrc/bb_chain.hip BB_SHAPES -- not from two literals): hidden 1536, intermediate 4608, 12 q / 6 kv heads (qkv 3072 wide)
+# the released 1.7B width, and one NO released checkpoint has (the stage sets are instantiated from the shape: csrc/bb_chain.hip BB_SHAPES): hidden 1536,
+# intermediate 4608, 12 q / 6 kv heads (qkv 3072 wide)
 UNRELEASED = dict(hidden=1536, inter=4608, q_heads=12, kv_heads=6)
 
 
@@ -199,14 +191,10 @@ def test_backbone_segment_chain_against_the_launch_path(B, kv, mode, shape):
 
 @pytest.mark.parametrize("B,kv,shape", [(32, "fp8", None), (23, "bf16", None), (16, "fp8", None), (9, "int8", None), (1, "fp8", None), (40, "fp8", None),
                                         (48, "bf16", None), (33, "int8", None), (27, "fp8", UNRELEASED), (7, "bf16", UNRELEASED)])
-def test_backbone_segment_chain_at_1_to_32_rows_against_the_launch_path(B, kv, shape):
-    """Round 5 (the hole at 33-48 rows): those batch sizes run the 64-row stage set (bb_chain_kernel) with the
-    last row tile partly filled, and the launch path picks the same tiles there (gemm.hip pick_tile) -- so the two schedules still
-    agree bit for bit, at every batch size 1..64 now.
-    Round 4: the 1.7B backbone segment as a persistent launch at 1-32 rows too (csrc/bb_chain.hip bb_chain_b32_kernel: the launch
-    path's tiles at those batch sizes -- 16-row qkv / o / down tiles, gate_up on 16 rows up to 16 and 32 rows above, so the rstd
-    summation order and with it every bit is the launch path's).  Three decode steps: logits, hidden, ids, codes, KV bytes identical;
-    both chains reported as launched.  (Round 6: and at a width no released checkpoint has.)"""
+def test_backbone_segment_chain_at_1_to_48_rows_against_the_launch_path(B, kv, shape):
+    """The backbone segment as a persistent launch at 1 to 48 rows (csrc/bb_chain.hip bb_flow_kernel, split by rows: 16, 32, 64), its last row tile
+    partly filled, at the 1.7B width and one that no released checkpoint has: logits, hidden state, ids, codes and every KV byte of three decode steps
+    are the launch path's; both chains reported as launched."""
     d = get_dims("tts-1.7b").with_(layers=3, max_model_len=256, **(shape or {}))
     w = make_weights(d, seed=8, std=0.02)
     res = {}
@@ -235,10 +223,9 @@ def test_backbone_segment_chain_at_1_to_32_rows_against_the_launch_path(B, kv, s
 
 @pytest.mark.parametrize("B", [64, 37, 32, 16, 5, 1])
 def test_backbone_segment_chain_at_the_0p6b_shape_against_the_launch_path(B):
-    """BASELINE config #2's backbone (hidden 1024, intermediate 3072: the code predictor's layer dimensions) runs the per-layer
-    segment on the code predictor's 16-row stage set (csrc/bb_chain.hip bb_chain_small_kernel) at EVERY batch size; against the
-    launch-per-op backbone of the same library: logits, hidden state, sampled ids, codes and every KV byte of three decode steps
-    identical, no flag wait times out, and the native step reports both chains as launched.
+    """The 0.6B backbone (hidden 1024, intermediate 3072: the code predictor's layer dimensions) runs the per-layer segment on the code predictor's split
+    of the stages (csrc/bb_chain.hip bb_flow_small_kernel) at EVERY batch size: logits, hidden state, sampled ids, codes and every KV byte of three decode
+    steps are the launch path's, no wait times out, and the native step reports both chains as launched.
     Reference shape: configuration_qwen3_tts.py:192-216,376-409 (read from the checkpoint, never hard-coded: the chain is chosen
     by the shape, every other shape keeps the launch path)."""
     d = get_dims("tts-0.6b").with_(layers=3, max_model_len=256)
@@ -285,6 +272,7 @@ def test_backbone_launches_of_changing_batches(model, shape, layers):
                 for B in (64, 16, 33, 1, 49, 17, 48, 32, 15, 64):
                     eng.decode_step(B)
                     outs += [eng.logits[:B].clone(), eng.last_hidden[:B].clone(), eng.audio_codes[:B].clone()]
+                    assert eng.chains_ran() == (3 if on else 1), (on, B, eng.chains_ran())
                 torch.cuda.synchronize()
                 assert eng.chain_error() == 0
                 res[on] = outs + [c.view(torch.uint8).clone() for c in eng.kv_caches]
@@ -292,6 +280,76 @@ def test_backbone_launches_of_changing_batches(model, shape, layers):
             lib.omni_debug_bb_chain(1)
     for i, (x, y) in enumerate(zip(res[1], res[0])):
         assert torch.equal(x, y), i
+
+
+def _same(x, y):
+    """equal bit for bit but for the payload of NaNs"""
+    return bool(((x == y) | (x.isnan() & y.isnan())).all()) if x.is_floating_point() else torch.equal(x, y)
+
+
+def _all_ones(t):
+    t.view(torch.int16).fill_(-1)
+
+
+@pytest.mark.parametrize("model", ["tts-1.7b", "tts-0.6b"])
+@pytest.mark.parametrize("B", [5, 24, 40, 64])
+def test_words_of_all_ones_pass_the_predictors_hand_offs(model, B):
+    """An empty word of a hand-off buffer is two bf16 NaNs, 0xffff each (csrc/chain_flow.cuh).  Such words as data -- one row's hidden state, the projected
+    row of a code that the last row draws -- are stored as other NaNs: nobody waits for them, and every output is the launch path's."""
+    d = get_dims(model).with_(layers=1, max_model_len=256)
+    w = make_weights(d, seed=12, std=0.02)
+    code0, e0, lh = (t.cuda() for t in _inputs(d, w, B, 5 * B))
+    lh = lh.clone()
+    _all_ones(lh[1])
+    res = {}
+    with L.debug_library() as lib:
+        lib.omni_debug_cp_chain.argtypes = [C.c_int]; lib.omni_debug_cp_chain.restype = None
+        try:
+            for on in (0, 2):
+                lib.omni_debug_cp_chain(on)
+                eng = _engine(d, w, kv_dtype="bf16", num_blocks=8, max_batch=64)
+                clean = eng.code_predictor(code0.to(torch.int32), e0, lh, greedy=True)
+                g = d.num_code_groups // 2
+                _all_ones(eng.cp_proj_table[g - 1, clean[B - 1, g]])
+                codes, lg = eng.code_predictor(code0.to(torch.int32), e0, lh, greedy=True, return_logits=True)
+                assert eng.chain_error() == 0 and eng.chains_ran() == (1 if on else 0)
+                assert lg[1].isnan().all() and lg[B - 1, g:].isnan().all() and lg[B - 1, :g].isfinite().all()
+                res[on] = (clean, codes, lg)
+        finally:
+            lib.omni_debug_cp_chain(2)
+    for x, y in zip(res[2], res[0]):
+        assert _same(x, y)
+
+
+@pytest.mark.parametrize("model", ["tts-1.7b", "tts-0.6b"])
+@pytest.mark.parametrize("B", [5, 24, 40, 64])
+def test_words_of_all_ones_pass_the_backbones_hand_offs(model, B):
+    """The same words in one row's input of the backbone: a step, and the next one, in which the predictor gets that row's hidden state."""
+    d = get_dims(model).with_(layers=3, max_model_len=256)
+    w = make_weights(d, seed=8, std=0.02)
+    res = {}
+    with L.debug_library() as lib:
+        for fn in (lib.omni_debug_bb_chain, lib.omni_debug_cp_chain):
+            fn.argtypes = [C.c_int]; fn.restype = None
+        try:
+            for on in (0, 1):
+                lib.omni_debug_bb_chain(on)
+                lib.omni_debug_cp_chain(2 * on)
+                eng = _decode_engine(d, w, B, "bf16")
+                _all_ones(eng.text_step[1])
+                outs = []
+                for _ in range(2):
+                    eng.decode_step(B)
+                    assert eng.chains_ran() == (3 if on else 0), (on, eng.chains_ran())
+                    assert eng.last_hidden[1].isnan().all() and eng.last_hidden[:1].isfinite().all() and eng.last_hidden[2:B].isfinite().all()
+                    outs += [eng.logits[:B].clone(), eng.last_hidden[:B].clone(), eng.input_ids[:B].clone(), eng.audio_codes[:B].clone()]
+                assert eng.chain_error() == 0
+                res[on] = outs
+        finally:
+            lib.omni_debug_bb_chain(1)
+            lib.omni_debug_cp_chain(2)
+    for i, (x, y) in enumerate(zip(res[1], res[0])):
+        assert _same(x, y), i
 
 
 @pytest.mark.parametrize("B,kv,base", [(64, "fp8", "launch-path"), (49, "bf16", "layer-chain"), (57, "int8", "launch-path"), (51, "fp16", "layer-chain")])

@@ -37,7 +37,7 @@ struct BbAllArgs {
     uint16_t* resid; float* part;       // fragment-major residual stream [64][2048] + sum(r^2) slabs [128][64]
     uint16_t* act;                      // fragment-major [64][6144]
     uint16_t* qkv;                      // row-major [B][4096]
-    int B, nap; float eps;
+    int B; float eps;
     uint32_t* flags; int32_t* err;
     unsigned long long* stamps; int stamp_layer;
 };
@@ -90,7 +90,6 @@ __global__ __launch_bounds__(CH_THREADS) void bb_all_kernel(const BbAllArgs a) {
     ChainGate g;
     chain_gate_init(g, a.flags, a.err);
     g.dom = 8;                          // gate_up's 64-row tiles and the attention's (row, head) pairs tie every row group together
-    g.nap = a.nap;
     const int wg = blockIdx.x;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     constexpr int H = 2048, I = 6144, NQ = 4096;
@@ -127,7 +126,7 @@ __global__ __launch_bounds__(CH_THREADS) void bb_all_kernel(const BbAllArgs a) {
         set_layer(Ly, 0);
         if (PRE)
             chain_gemm<2, 2, 8, 3, OMNI_EPI_BF16, 4, 0>(Ly.wqkv, Ly.ln1, a.resid, a.part, 1, a.qkv, NQ, nullptr, a.B, NQ, a.eps, wg & 127, wg >> 7, lds, g,
-                                                        false, 0x20001, a.stamp_layer == 0 ? a.stamps : nullptr, nullptr, pf);
+                                                        false, 0x20001, a.stamp_layer == 0 ? a.stamps : nullptr, pf);
         else
             chain_gemm<2, 2, 8, 3, OMNI_EPI_BF16, 4>(Ly.wqkv, Ly.ln1, a.resid, a.part, 1, a.qkv, NQ, nullptr, a.B, NQ, a.eps, wg & 127, wg >> 7, lds, g,
                                                      false, 0x20001, a.stamp_layer == 0 ? a.stamps : nullptr);
@@ -150,7 +149,7 @@ __global__ __launch_bounds__(CH_THREADS) void bb_all_kernel(const BbAllArgs a) {
             set_layer(Ln, l + 1);
             if (PRE)
                 chain_gemm<2, 2, 8, 3, OMNI_EPI_BF16, 4, 0>(Ln.wqkv, Ln.ln1, a.resid, a.part, H / 16, a.qkv, NQ, nullptr, a.B, NQ, a.eps, wg & 127, wg >> 7,
-                                                            lds, g, true, lc | 1, a.stamp_layer == l + 1 ? a.stamps : nullptr, nullptr, pf);
+                                                            lds, g, true, lc | 1, a.stamp_layer == l + 1 ? a.stamps : nullptr, pf);
             else
                 chain_gemm<2, 2, 8, 3, OMNI_EPI_BF16, 4>(Ln.wqkv, Ln.ln1, a.resid, a.part, H / 16, a.qkv, NQ, nullptr, a.B, NQ, a.eps, wg & 127, wg >> 7,
                                                          lds, g, true, lc | 1, a.stamp_layer == l + 1 ? a.stamps : nullptr);
@@ -158,7 +157,7 @@ __global__ __launch_bounds__(CH_THREADS) void bb_all_kernel(const BbAllArgs a) {
     }
 }
 
-OMNI_KNOB g_bb_all = 0, g_bb_all_nap = 1;      // off: measured +0.09 .. +0.12 ms per step against round 3's two launches per layer (profiles/r04_ab_table.txt)
+OMNI_KNOB g_bb_all = 0;      // off: measured +0.09 .. +0.12 ms per step against round 3's two launches per layer (profiles/r04_ab_table.txt)
 #ifdef OMNI_DEBUG_HOOKS
 static int g_bb_all_bal = 1, g_bb_all_pre = 1;
 #endif
@@ -220,7 +219,7 @@ int k_bb_all(const omni_talker_desc& d, const void* table_dev, const omni_step_i
     p.nsplit = 1; p.out_frag = 1; p.kv_rep = 1; p.dense_pos = -1; p.num_live = io->num_live;
     p.rope_rows = io->rope_delta ? (d.rope_rows > 0 ? d.rope_rows : d.max_model_len) : 0;
     a.attn = (uint16_t*)attn; a.resid = (uint16_t*)resid; a.part = part; a.act = (uint16_t*)act; a.qkv = (uint16_t*)qkv;
-    a.B = io->B; a.nap = g_bb_all_nap; a.eps = d.eps; a.flags = flags; a.err = err;
+    a.B = io->B; a.eps = d.eps; a.flags = flags; a.err = err;
     a.stamp_layer = -1;
 #ifdef OMNI_DEBUG_HOOKS
     a.stamps = g_bba_stamps; a.stamp_layer = g_bba_stamp_layer;

@@ -5,7 +5,7 @@
 // stage looks for its operands, so the HBM stream keeps running through the hand-off instead of stopping for a kernel boundary (1.65 us)
 // plus a cold first fetch.
 //   bb_flow_kernel, bb_flow_small_kernel   one rank, the whole chip: activations cross by content (chain_flow.cuh)
-//   bb_chain_kernel                        a tensor-parallel rank (AR), the half grid (HALF), the debug library's arms: behind flags (chain_gemm.cuh)
+//   bb_chain_kernel                        a tensor-parallel rank (AR), the half grid (HALF): behind flags (chain_gemm.cuh)
 // K-step ownership, combine order and rounding points are the launch path's: results are bit-identical.
 // A decode step, behind flags and by content, one card: 64 rows of the 1.7B shape 3050 -> 2886 us, 5 rows of the 0.6B one 2091 -> 1859.
 // Of a 64-row launch (32 us, 100 MB) gate_up is half: its 50 MB come out of HBM at 5.5 TB/s, and a wave's loads return in order, so half of a wave's
@@ -24,11 +24,10 @@
 #include "common.cuh"
 #include "kernels.h"
 
-#define BB_LDS_BYTES ((CH_WAVES * 12 * 64 * 16) + CH_WAVES * 64 * 4)      // combine slots (gate_up: 12 tiles, ONE pass since round 4) + rstd area
+#define BB_LDS_BYTES ((CH_WAVES * 12 * 64 * 16) + CH_WAVES * 64 * 4)      // bb_chain_kernel: combine slots (gate_up: 12 tiles) + rstd area
 
 struct BbArgs {
     const uint16_t *wo, *ln2, *wgu, *wdown, *ln1_next, *wqkv_next;      // *_next == NULL: last layer, no qkv stage
-    int pf;                             // cross-stage weight prefetch (0: every stage fetches its own slice at its entry)
     const uint16_t* attn;               // fragment-major [64][2048]: the attention launch's output
     uint16_t* resid; float* part;       // fragment-major residual stream [64][2048] + sum(r^2) slabs [128][64]
     uint16_t* act;                      // fragment-major [64][6144]
@@ -37,7 +36,7 @@ struct BbArgs {
     // the LAST layer's launch (no next qkv) may end in the talker's own head instead (round 6): final norm folded into the lm_head GEMM, its
     // normalised rows = h[t + 1] (row-major, rows below *num_live), logits fp32 [B][V] holding bf16-rounded values, the codec mask applied
     const uint16_t *lm_head, *final_norm; float* logits; uint16_t* last_hidden; const uint8_t* mask; const int32_t* num_live; float mask_fill; int V;
-    int B, nap; float eps;
+    int B; float eps;
     uint32_t* flags; int32_t* err;
     unsigned long long* stamps;
     // tensor-parallel rank (round 6): o_proj and down_proj are row-parallel partials; their all-reduce rides in the two residual epilogues
@@ -50,112 +49,53 @@ struct BbArgs {
 };
 static_assert(BB_WAVES == CH_WAVES, "bb_areas.h");
 
-// (Round 3 also tried a ninth wave that warms the XCD's L2 with the next stage's slice -- one dword per 64 bytes, nothing
-// depending on it: +0.10 ms per step, removed; and the loader / consumer split of bb_engine.hip.  What is kept is below:
-// the NEXT stage's weight loads issued by the compute waves themselves, behind their last activation load.)
-// GU_G / DN_G / QK_G: activation-ring depth (k-steps per wave in flight behind the flags) of gate_up (its weights ride in the same
-// ring) / down_proj / the next qkv; PF: the cross-stage weight prefetch arm
-// GU1P: gate_up's 12 tiles combine in one pass (chain_gemm ONEPASS; round 4: epilogue 2.4 -> 1.0 us); GUW0: gate_up's whole weight
-// slice (96 registers) goes out at stage entry, ahead of the flags, instead of riding in the activation ring (A/B arm)
-// DEFER: the RMSNorm's rstd applied in the epilogue (chain_gemm PRO 3) -- round 4's A/B arm of VERDICT r3 item 1b; the product form since
-// round 6 (gemm_skinny_kernel takes it for the same GEMMs); false = round 5's exact-rstd stages, debug library only
-// WNT: bit 0 = non-temporal weight loads in gate_up (every byte read by exactly ONE workgroup), bit 1 = in o_proj / down_proj / qkv (each slice
-// read by the two workgroups of a column tile's row halves) -- round 5 A/B arm (MI355X_MICROARCH "nt-weights")
+// Rings: gate_up's activations and weights two k-steps deep, down_proj's and qkv's activations four.  gate_up's 12 tiles combine in one pass, the RMSNorm's
+// rstd is applied in the epilogues (chain_gemm PRO 3).
 // HEAD: the instantiation the LAST layer launches when the step's head rides along (its own code object entry: the other 27 launches keep the
 // leaner kernel -- with the head stage compiled into every launch the segment cost 0.9 us more per layer, register allocation of the shared stages)
 // AR: the instantiation of a tensor-parallel rank (the all-reduces inside the o_proj / down_proj stages); HALF: 128 workgroups play the 256 of the
 // stage grid, two VIRTUAL workgroups each, stage by stage (a virtual workgroup's stage needs only stages that every physical workgroup has
 // already run or will run before it waits again: no cycle) -- two such launches of two processes fit the chip side by side, which is how the
 // cross-process exchange is tested on one GPU (tests/test_gpu_tp.py) and how a co-located second engine keeps its backbone chain
-template <int KO, int KH, int KI, int GU_G, int DN_G, int QK_G, bool PF, bool GU1P = true, bool GUW0 = false, bool DEFER = true, int WNT = 0, bool HEAD = false,
-          bool AR = false, bool HALF = false>
+template <int KO, int KH, int KI, bool HEAD, bool AR, bool HALF>
 __global__ __launch_bounds__(CH_THREADS) void bb_chain_kernel(const BbArgs a) {
     extern __shared__ __attribute__((aligned(16))) float lds[];
-    static_assert(!PF || (!AR && !HALF), "the cross-stage prefetch arm is a single-rank, full-grid experiment");
+    static_assert((AR || HALF) && !(HEAD && HALF), "bb_chain: one rank on the whole chip runs bb_flow_kernel; the half grid has no head stage");
     uint32_t e0 = 0;
     if constexpr (AR) e0 = __builtin_amdgcn_readfirstlane(__hip_atomic_load(a.ar_epoch, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
     ChainGate g;
     chain_gate_init(g, a.flags, a.err);
     g.dom = 8;                          // gate_up's 64-row tiles tie every row group together
-    g.nap = a.nap;
     const int wg = blockIdx.x;
     const int H = a.H, I = a.I, NQ = a.NQ;
     // workgroup -> tile: o_proj / down_proj 16 columns x 32 rows, gate_up 24 activation columns x 64 rows, qkv 32 columns x 32 rows; a
     // workgroup past a stage's grid (column tiles x row tiles < 256 at widths below the 1.7B shape's) publishes the stage and runs ahead
     const int nc_h = H >> 4, nc_gu = I / 24, nc_q = NQ >> 5;
-    // stage codes (error word): 0x1001 .. 0x1004.  Weight registers of the stage AFTER the current one are filled by the current
-    // stage (chain_gemm WSRC 3): gate_up's 96 registers during o_proj, down_proj's 96 during gate_up (the allocator reuses
-    // gate_up's as its k-steps retire), the next qkv's 64 during down_proj.
-    if constexpr (PF) {
-        static_assert(!PF || (KO == 8 && KH == 8 && KI == 24), "the cross-stage prefetch arm (debug library) is built for the 1.7B shape");
-        const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-        const uint32_t lane16 = lane * 16;
-        u32x4 Wg[8][3], Wd[24][1], Wk[8][2];
-        auto pf_g_ = [&]() {
-            const coh_rsrc_t rs = coh_rsrc(a.wgu);
-#pragma unroll
-            for (int d = 0; d < 8; ++d)
-#pragma unroll
-                for (int j = 0; j < 3; ++j)
-                    Wg[d][j] = __builtin_amdgcn_raw_buffer_load_b128(rs, lane16, (uint32_t)(((wg * 3 + j) * 64 + wave + d * CH_WAVES) * 1024), 0);
-        };
-        auto pf_d_ = [&]() {
-            const coh_rsrc_t rs = coh_rsrc(a.wdown);
-#pragma unroll
-            for (int d = 0; d < 24; ++d) Wd[d][0] = __builtin_amdgcn_raw_buffer_load_b128(rs, lane16, (uint32_t)(((wg & 127) * 192 + wave + d * CH_WAVES) * 1024), 0);
-        };
-        auto pf_k_ = [&]() {
-            if (a.wqkv_next == nullptr) return;
-            const coh_rsrc_t rs = coh_rsrc(a.wqkv_next);
-#pragma unroll
-            for (int d = 0; d < 8; ++d)
-#pragma unroll
-                for (int j = 0; j < 2; ++j)
-                    Wk[d][j] = __builtin_amdgcn_raw_buffer_load_b128(rs, lane16, (uint32_t)((((wg & 127) * 2 + j) * 64 + wave + d * CH_WAVES) * 1024), 0);
-        };
-        ChainPrefetch<24, decltype(pf_g_)> pf_g{pf_g_};
-        ChainPrefetch<24, decltype(pf_d_)> pf_d{pf_d_};
-        ChainPrefetch<16, decltype(pf_k_)> pf_k{pf_k_};
-        chain_gemm<2, 1, 8, 0, OMNI_EPI_RESID, 0, 0>(a.wo, nullptr, a.attn, nullptr, 0, a.resid, 0, a.part, a.B, H, a.eps, wg & 127, wg >> 7, lds, g,
-                                                     false, 0x1001, a.stamps, nullptr, pf_g);
-        chain_gemm<4, 3, 8, 3, OMNI_EPI_SILU_MUL_GU8, 2, 3>(a.wgu, a.ln2, a.resid, a.part, H / 16, a.act, 0, nullptr, a.B, I, a.eps, wg, 0, lds, g,
-                                                            true, 0x1002, a.stamps, Wg, pf_d);
-        chain_gemm<2, 1, 24, 0, OMNI_EPI_RESID, 4, 3>(a.wdown, nullptr, a.act, nullptr, 0, a.resid, 0, a.part, a.B, H, a.eps, wg & 127, wg >> 7, lds,
-                                                      g, true, 0x1003, a.stamps, Wd, pf_k);
-        if (a.wqkv_next)
-            chain_gemm<2, 2, 8, 3, OMNI_EPI_BF16, 4, 3>(a.wqkv_next, a.ln1_next, a.resid, a.part, H / 16, a.qkv, NQ, nullptr, a.B, NQ, a.eps,
-                                                        wg & 127, wg >> 7, lds, g, true, 0x1004, a.stamps, Wk);
-        return;
-    } else {
-    constexpr int NT1 = (WNT & 1) ? OMNI_AUX_NT : 0, NT2 = (WNT & 2) ? OMNI_AUX_NT : 0;
+    // stage codes (error word): 0x1001 .. 0x1005
     // the four stages of (virtual) workgroup WG_ behind gate G_
 #define BB_O(WG_, G_)                                                                                                                                   \
-    chain_gemm<2, 1, KO, 0, OMNI_EPI_RESID, 0, 0, ChainNoPrefetch, false, 64, NT2, AR>(a.wo, nullptr, a.attn, nullptr, 0, a.resid, 0, a.part, a.B, H, a.eps,    \
-                                                                                       (WG_) % nc_h, (WG_) / nc_h, lds, G_, false, 0x1001, a.stamps, nullptr,  \
-                                                                                       ChainNoPrefetch(), nullptr, nullptr, 0.f, nullptr, &a.ar_o, e0 + 1u)
+    chain_gemm<2, 1, KO, 0, OMNI_EPI_RESID, 0, 0, ChainNoPrefetch, false, AR>(a.wo, nullptr, a.attn, nullptr, 0, a.resid, 0, a.part, a.B, H, a.eps,         \
+                                                                              (WG_) % nc_h, (WG_) / nc_h, lds, G_, false, 0x1001, a.stamps,                \
+                                                                              ChainNoPrefetch(), nullptr, nullptr, 0.f, nullptr, &a.ar_o, e0 + 1u)
 #define BB_GU(WG_, G_)                                                                                                                                  \
     do {                                                                                                                                                \
         if ((WG_) < nc_gu)                                                                                                                              \
-            chain_gemm<4, 3, KH, DEFER ? 3 : 2, OMNI_EPI_SILU_MUL_GU8, GU_G, GUW0 ? 0 : 1, ChainNoPrefetch, GU1P, 64, NT1>(                              \
-                a.wgu, a.ln2, a.resid, a.part, H / 16, a.act, 0, nullptr, a.B, I, a.eps, WG_, 0, lds, G_, true, 0x1002, a.stamps);                        \
+            chain_gemm<4, 3, KH, 3, OMNI_EPI_SILU_MUL_GU8, 2, 1, ChainNoPrefetch, true>(a.wgu, a.ln2, a.resid, a.part, H / 16, a.act, 0, nullptr, a.B, I,   \
+                                                                                        a.eps, WG_, 0, lds, G_, true, 0x1002, a.stamps);                   \
         else                                                                                                                                            \
             chain_gate_skip(G_);                                                                                                                        \
     } while (0)
 #define BB_DN(WG_, G_)                                                                                                                                  \
-    chain_gemm<2, 1, KI, 0, OMNI_EPI_RESID, DN_G, 0, ChainNoPrefetch, false, 64, NT2, AR>(a.wdown, nullptr, a.act, nullptr, 0, a.resid, 0, a.part, a.B, H,       \
-                                                                                          a.eps, (WG_) % nc_h, (WG_) / nc_h, lds, G_, true, 0x1003, a.stamps,   \
-                                                                                          nullptr, ChainNoPrefetch(), nullptr, nullptr, 0.f, nullptr, &a.ar_dn,  \
-                                                                                          e0 + 2u)
+    chain_gemm<2, 1, KI, 0, OMNI_EPI_RESID, 4, 0, ChainNoPrefetch, false, AR>(a.wdown, nullptr, a.act, nullptr, 0, a.resid, 0, a.part, a.B, H, a.eps,        \
+                                                                              (WG_) % nc_h, (WG_) / nc_h, lds, G_, true, 0x1003, a.stamps,                 \
+                                                                              ChainNoPrefetch(), nullptr, nullptr, 0.f, nullptr, &a.ar_dn, e0 + 2u)
 #define BB_QK(WG_, G_)                                                                                                                                  \
-    chain_gemm<2, 2, KH, DEFER ? 3 : 2, OMNI_EPI_BF16, QK_G, 0, ChainNoPrefetch, false, 64, NT2>(a.wqkv_next, a.ln1_next, a.resid, a.part, H / 16, a.qkv, NQ,    \
-                                                                                                 nullptr, a.B, NQ, a.eps, (WG_) % nc_q, (WG_) / nc_q, lds, G_,   \
-                                                                                                 true, 0x1004, a.stamps)
+    chain_gemm<2, 2, KH, 3, OMNI_EPI_BF16, 4>(a.wqkv_next, a.ln1_next, a.resid, a.part, H / 16, a.qkv, NQ, nullptr, a.B, NQ, a.eps, (WG_) % nc_q,            \
+                                              (WG_) / nc_q, lds, G_, true, 0x1004, a.stamps)
     if constexpr (HALF) {
-        static_assert(!HALF || !HEAD, "the half grid has no head stage (a tensor-parallel rank's lm_head stays its own launch)");
         ChainGate g2;
         chain_gate_init(g2, a.flags, a.err, wg + OMNI_CHAIN_WGS / 2);
         g2.dom = 8;
-        g2.nap = a.nap;
         const int wg2 = wg + OMNI_CHAIN_WGS / 2;
         BB_O(wg, g); BB_O(wg2, g2);
         BB_GU(wg, g); BB_GU(wg2, g2);
@@ -171,10 +111,9 @@ __global__ __launch_bounds__(CH_THREADS) void bb_chain_kernel(const BbArgs a) {
         // the step's head as the last stage of its last backbone launch (one launch and one cold start less: 9.8 us + a boundary -> a stage):
         // gemm_skinny_kernel<2, 2, PRO 2, F32_BF16RND>'s tile and arithmetic (exact norm: its normalised rows are h[t + 1])
         const int nc_v = a.V >> 5;
-        chain_gemm<2, 2, KH, 2, OMNI_EPI_F32_BF16RND, QK_G, 0, ChainNoPrefetch, false, 64, NT2>(a.lm_head, a.final_norm, a.resid, a.part, H / 16, a.logits, a.V,
-                                                                                                nullptr, a.B, a.V, a.eps, wg % nc_v, wg / nc_v, lds, g, true, 0x1005,
-                                                                                                a.stamps, nullptr, ChainNoPrefetch(), a.last_hidden, a.mask,
-                                                                                                a.mask_fill, a.num_live);
+        chain_gemm<2, 2, KH, 2, OMNI_EPI_F32_BF16RND, 4>(a.lm_head, a.final_norm, a.resid, a.part, H / 16, a.logits, a.V, nullptr, a.B, a.V, a.eps, wg % nc_v,
+                                                         wg / nc_v, lds, g, true, 0x1005, a.stamps, ChainNoPrefetch(), a.last_hidden, a.mask, a.mask_fill,
+                                                         a.num_live);
     }
     }
 #undef BB_O
@@ -191,7 +130,6 @@ __global__ __launch_bounds__(CH_THREADS) void bb_chain_kernel(const BbArgs a) {
                 __hip_atomic_store(a.ar_epoch, e0 + 2u, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_AGENT);
             }
         }
-    }
     }
 }
 
@@ -357,14 +295,13 @@ __global__ __launch_bounds__(CH_THREADS) void bb_flow_small_kernel(const BbArgs 
 
 size_t k_bb_flow_bytes(const omni_talker_desc& d) { return 2 * (size_t)BbFlowMap(d.hidden, d.inter).copy; }
 
-OMNI_KNOB g_bb_chain = 1, g_bb_nap = 1, g_bb_prefetch = 0, g_bb_deep = 0, g_bb_min_rows = 33, g_bb_b32 = 1, g_bb_ar = 1;      // cross-stage prefetch: measured +0.4 ms per step, off
+OMNI_KNOB g_bb_chain = 1, g_bb_min_rows = 33, g_bb_b32 = 1, g_bb_ar = 1;
 #ifdef OMNI_DEBUG_HOOKS
 static unsigned long long* g_bb_stamps = nullptr;
-extern "C" void omni_debug_bb_chain(int on) { g_bb_chain = on != 0; g_bb_prefetch = on == 2; }      // 2: with the cross-stage weight prefetch
+extern "C" void omni_debug_bb_chain(int on) { g_bb_chain = on; }
 extern "C" void omni_debug_bb_stamps(void* buf) { g_bb_stamps = (unsigned long long*)buf; }
-extern "C" void omni_debug_bb_deep(int mode) { g_bb_deep = mode; }
 extern "C" void omni_debug_bb_ar(int on) { g_bb_ar = on; }                  // 0: tensor-parallel ranks keep the launch-per-op backbone (round 5)
-extern "C" void omni_debug_bb_min_rows(int rows) { g_bb_min_rows = rows; g_bb_b32 = rows <= 49; }                          // smallest batch the backbone chain takes                                  // deeper activation / weight rings
+extern "C" void omni_debug_bb_min_rows(int rows) { g_bb_min_rows = rows; g_bb_b32 = rows <= 49; }      // smallest batch of the 64-row split
 #endif
 
 // the instantiated shape triples (KO, KH, KI) = (q_heads * 128, hidden, intermediate) / 256: the released 1.7B shape and one no released
@@ -434,24 +371,19 @@ static int bb_launch_small(const BbArgs& a, hipStream_t stream) {
 }
 
 // the all-reduce / half-grid instantiations of one triple (64-row stage set)
-template <int KO, int KH, int KI, bool AR>
-static int bb_launch_ar(const BbArgs& a, bool half, hipStream_t stream) {
-    static bool attr = false;
-    if (!attr) {
-        (void)hipFuncSetAttribute((const void*)bb_chain_kernel<KO, KH, KI, 2, 4, 4, false, true, false, true, 0, false, AR, false>, hipFuncAttributeMaxDynamicSharedMemorySize, BB_LDS_BYTES);
-        (void)hipFuncSetAttribute((const void*)bb_chain_kernel<KO, KH, KI, 2, 4, 4, false, true, false, true, 0, false, AR, true>, hipFuncAttributeMaxDynamicSharedMemorySize, BB_LDS_BYTES);
-        if (AR) (void)hipFuncSetAttribute((const void*)bb_chain_kernel<KO, KH, KI, 2, 4, 4, false, true, false, true, 0, true, AR, false>, hipFuncAttributeMaxDynamicSharedMemorySize, BB_LDS_BYTES);
-        attr = true;
-    }
-    if (AR && !half && a.lm_head != nullptr) {      // a tensor-parallel rank's last layer: the (replicated) lm_head as the launch's last stage
-        hipLaunchKernelGGL((bb_chain_kernel<KO, KH, KI, 2, 4, 4, false, true, false, true, 0, true, AR, false>), dim3(OMNI_CHAIN_WGS), dim3(CH_THREADS), BB_LDS_BYTES, stream, a);
-        OMNI_CHECK_LAUNCH("bb_chain(all-reduce, head)");
-        return OMNI_OK;
-    }
-    if (half) hipLaunchKernelGGL((bb_chain_kernel<KO, KH, KI, 2, 4, 4, false, true, false, true, 0, false, AR, true>), dim3(OMNI_CHAIN_WGS / 2), dim3(CH_THREADS), BB_LDS_BYTES, stream, a);
-    else hipLaunchKernelGGL((bb_chain_kernel<KO, KH, KI, 2, 4, 4, false, true, false, true, 0, false, AR, false>), dim3(OMNI_CHAIN_WGS), dim3(CH_THREADS), BB_LDS_BYTES, stream, a);
+template <int KO, int KH, int KI, bool HEAD, bool AR, bool HALF>
+static int bb_launch_flags(const BbArgs& a, hipStream_t stream) {
+    static const hipError_t attr = hipFuncSetAttribute((const void*)bb_chain_kernel<KO, KH, KI, HEAD, AR, HALF>, hipFuncAttributeMaxDynamicSharedMemorySize, BB_LDS_BYTES);
+    (void)attr;
+    hipLaunchKernelGGL((bb_chain_kernel<KO, KH, KI, HEAD, AR, HALF>), dim3(HALF ? OMNI_CHAIN_WGS / 2 : OMNI_CHAIN_WGS), dim3(CH_THREADS), BB_LDS_BYTES, stream, a);
     OMNI_CHECK_LAUNCH("bb_chain(all-reduce / half grid)");
     return OMNI_OK;
+}
+template <int KO, int KH, int KI>
+static int bb_launch_ar(const BbArgs& a, bool half, hipStream_t stream) {
+    if (half) return bb_launch_flags<KO, KH, KI, false, true, true>(a, stream);
+    // a rank's last layer: the (replicated) lm_head as the launch's last stage
+    return a.lm_head != nullptr ? bb_launch_flags<KO, KH, KI, true, true, false>(a, stream) : bb_launch_flags<KO, KH, KI, false, true, false>(a, stream);
 }
 
 static void bb_fill_ar(ChainAr& c, const omni_ar_peers& p) {
@@ -465,8 +397,7 @@ static void bb_fill_ar(ChainAr& c, const omni_ar_peers& p) {
 }
 
 bool k_bb_chain_head_supported(const omni_talker_desc& d) {      // the lm_head stage's tile grid: 32 columns x 2 row tiles inside 256 workgroups
-    return !k_bb_chain_small(d) && d.vocab % 32 == 0 && (d.vocab / 32) * 2 <= OMNI_CHAIN_WGS && d.lm_head != nullptr &&
-           !g_bb_prefetch && !g_bb_deep;      // (the debug library's A/B arms keep the head as its own launch)
+    return !k_bb_chain_small(d) && d.vocab % 32 == 0 && (d.vocab / 32) * 2 <= OMNI_CHAIN_WGS && d.lm_head != nullptr;
 }
 
 int k_bb_chain(const omni_talker_desc& d, const omni_layer_weights& w, const omni_layer_weights* next, const void* attn, void* resid, float* part,
@@ -478,7 +409,7 @@ int k_bb_chain(const omni_talker_desc& d, const omni_layer_weights& w, const omn
     a.wqkv_next = next ? (const uint16_t*)next->wqkv : nullptr;
     a.attn = (const uint16_t*)attn; a.resid = (uint16_t*)resid; a.part = part; a.act = (uint16_t*)act; a.qkv = (uint16_t*)qkv;
     a.H = d.hidden; a.I = d.inter; a.NQ = (d.q_heads + 2 * d.kv_heads) * 128;
-    a.B = B; a.nap = g_bb_nap; a.eps = eps; a.flags = flags; a.err = err;
+    a.B = B; a.eps = eps; a.flags = flags; a.err = err;
     if (head != nullptr && next == nullptr && !small) {
         a.lm_head = (const uint16_t*)d.lm_head; a.final_norm = (const uint16_t*)d.final_norm; a.logits = head->logits; a.V = d.vocab;
         a.last_hidden = (uint16_t*)head->last_hidden; a.mask = (const uint8_t*)d.allowed_mask; a.mask_fill = head->mask_fill; a.num_live = head->num_live;
@@ -506,51 +437,15 @@ int k_bb_chain(const omni_talker_desc& d, const omni_layer_weights& w, const omn
             bb_fill_ar(a.ar_o, *ar->attn);
             bb_fill_ar(a.ar_dn, *ar->mlp);
             a.ar_epoch = ar->attn->epoch;
-#define X(KO_, KH_, KI_) if (ko == KO_ && kh == KH_ && ki == KI_) return bb_launch_ar<KO_, KH_, KI_, true>(a, half, (hipStream_t)stream);
+#define X(KO_, KH_, KI_) if (ko == KO_ && kh == KH_ && ki == KI_) return bb_launch_ar<KO_, KH_, KI_>(a, half, (hipStream_t)stream);
             BB_AR_SHAPES(X)
 #undef X
         } else if (ko == 8 && kh == 8 && ki == 24) {
-            return bb_launch_ar<8, 8, 24, false>(a, true, (hipStream_t)stream);
+            return bb_launch_flags<8, 8, 24, false, false, true>(a, (hipStream_t)stream);
         }
         omni_set_error("bb_chain: no all-reduce / half-grid stage set for (q width, hidden, intermediate) = (%d, %d, %d)", d.q_heads * 128, d.hidden, d.inter);
         return OMNI_EINVAL;
     }
-#ifdef OMNI_DEBUG_HOOKS      // the A/B arms of rounds 3-5 (1.7B triple only)
-    a.pf = g_bb_prefetch;
-    if (ko == 8 && kh == 8 && ki == 24 && B > 32 && (a.pf || g_bb_deep) && a.lm_head == nullptr) {
-        static bool attr = false;
-#define BB_ARM(...) bb_chain_kernel<8, 8, 24, __VA_ARGS__>
-        if (!attr) {
-            (void)hipFuncSetAttribute((const void*)BB_ARM(2, 4, 4, true), hipFuncAttributeMaxDynamicSharedMemorySize, BB_LDS_BYTES);
-            (void)hipFuncSetAttribute((const void*)BB_ARM(4, 8, 8, false), hipFuncAttributeMaxDynamicSharedMemorySize, BB_LDS_BYTES);
-            (void)hipFuncSetAttribute((const void*)BB_ARM(3, 6, 8, false), hipFuncAttributeMaxDynamicSharedMemorySize, BB_LDS_BYTES);
-            (void)hipFuncSetAttribute((const void*)BB_ARM(2, 8, 8, false), hipFuncAttributeMaxDynamicSharedMemorySize, BB_LDS_BYTES);
-            (void)hipFuncSetAttribute((const void*)BB_ARM(2, 4, 4, false, false), hipFuncAttributeMaxDynamicSharedMemorySize, BB_LDS_BYTES);
-            (void)hipFuncSetAttribute((const void*)BB_ARM(2, 4, 4, false, true, true), hipFuncAttributeMaxDynamicSharedMemorySize, BB_LDS_BYTES);
-            (void)hipFuncSetAttribute((const void*)BB_ARM(2, 4, 4, false, true, false, false), hipFuncAttributeMaxDynamicSharedMemorySize, BB_LDS_BYTES);
-            (void)hipFuncSetAttribute((const void*)BB_ARM(2, 4, 4, false, true, false, true, 1), hipFuncAttributeMaxDynamicSharedMemorySize, BB_LDS_BYTES);
-            (void)hipFuncSetAttribute((const void*)BB_ARM(2, 4, 4, false, true, false, true, 2), hipFuncAttributeMaxDynamicSharedMemorySize, BB_LDS_BYTES);
-            (void)hipFuncSetAttribute((const void*)BB_ARM(2, 4, 4, false, true, false, true, 3), hipFuncAttributeMaxDynamicSharedMemorySize, BB_LDS_BYTES);
-            attr = true;
-        }
-#define BB_LAUNCH(...) hipLaunchKernelGGL((BB_ARM(__VA_ARGS__)), dim3(OMNI_CHAIN_WGS), dim3(CH_THREADS), BB_LDS_BYTES, (hipStream_t)stream, a)
-        if (a.pf) BB_LAUNCH(2, 4, 4, true);
-        else if (g_bb_deep == 1) BB_LAUNCH(4, 8, 8, false);
-        else if (g_bb_deep == 2) BB_LAUNCH(3, 6, 8, false);
-        else if (g_bb_deep == 3) BB_LAUNCH(2, 8, 8, false);
-        else if (g_bb_deep == 4) BB_LAUNCH(2, 4, 4, false, false);             // round 3's two-pass gate_up combine
-        else if (g_bb_deep == 5) BB_LAUNCH(2, 4, 4, false, true, true);        // gate_up weights ahead of the flags
-        else if (g_bb_deep == 6) BB_LAUNCH(2, 4, 4, false, true, false, false); // round 5's exact rstd (timing arm: no longer the launch path's bits)
-        else if (g_bb_deep == 7) BB_LAUNCH(2, 4, 4, false, true, false, true, 1);   // nt weight loads: gate_up only
-        else if (g_bb_deep == 8) BB_LAUNCH(2, 4, 4, false, true, false, true, 2);   // nt: o_proj / down_proj / qkv
-        else if (g_bb_deep == 9) BB_LAUNCH(2, 4, 4, false, true, false, true, 3);   // nt: every weight load of the launch
-        else BB_LAUNCH(2, 4, 4, false);
-#undef BB_LAUNCH
-#undef BB_ARM
-        OMNI_CHECK_LAUNCH("bb_chain(arm)");
-        return OMNI_OK;
-    }
-#endif
 #define X(KO_, KH_, KI_) if (ko == KO_ && kh == KH_ && ki == KI_) return bb_launch_shape<KO_, KH_, KI_>(a, B, (hipStream_t)stream);
     BB_SHAPES(X)
 #undef X

@@ -35,7 +35,7 @@ struct EngArgs {
     uint16_t* resid; float* part;
     uint16_t* act;
     uint16_t* qkv;
-    int B, nap; float eps;
+    int B; float eps;
     uint32_t* flags; int32_t* err;
     unsigned long long* stamps;
 };
@@ -140,7 +140,6 @@ __global__ __launch_bounds__(ENG_THREADS) void bb_engine_kernel(const EngArgs a)
     ChainGate g;
     chain_gate_init(g, a.flags, a.err);
     g.dom = 8;
-    g.nap = a.nap;
     g.es = es; g.fifo = fifo;
     const int wg = blockIdx.x;
     constexpr int H = 2048, I = 6144, NQ = 4096;
@@ -162,7 +161,7 @@ __global__ __launch_bounds__(ENG_THREADS) void bb_engine_kernel(const EngArgs a)
     if (threadIdx.x == 0 && __hip_atomic_load(&es->dead, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP) != 0) atomicCAS(a.err, 0, 0x2fff);
 }
 
-OMNI_KNOB g_bb_engine = 0, g_eng_nap = 1;      // off: correct (bit-identical) but 2.03 ms of backbone per step against the plain chain's 1.56
+OMNI_KNOB g_bb_engine = 0;      // off: correct (bit-identical) but 2.03 ms of backbone per step against the plain chain's 1.56
 #ifdef OMNI_DEBUG_HOOKS
 static unsigned long long* g_eng_stamps = nullptr;
 extern "C" void omni_debug_bb_engine(int on) { g_bb_engine = on; }
@@ -183,7 +182,7 @@ int k_bb_engine(const omni_layer_weights& w, const omni_layer_weights* next, con
     a.ln1_next = next ? (const uint16_t*)next->ln1 : nullptr;
     a.wqkv_next = next ? (const uint16_t*)next->wqkv : nullptr;
     a.attn = (const uint16_t*)attn; a.resid = (uint16_t*)resid; a.part = part; a.act = (uint16_t*)act; a.qkv = (uint16_t*)qkv;
-    a.B = B; a.nap = g_eng_nap; a.eps = eps; a.flags = flags; a.err = err;
+    a.B = B; a.eps = eps; a.flags = flags; a.err = err;
 #ifdef OMNI_DEBUG_HOOKS
     a.stamps = g_eng_stamps;
 #endif

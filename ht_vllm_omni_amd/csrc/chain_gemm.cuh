@@ -26,8 +26,8 @@
 #define CH_STAMP_BY(buf, sidx, k, thread) do { (void)(buf); (void)(sidx); } while (0)
 #endif
 
-// PRO 3 (round 4: an A/B arm; round 6: the product form of every norm-fused stage whose normalised rows are nobody's output -- qkv, gate_up --
-// in the chains and, with the same arithmetic, in gemm_skinny_kernel): the RMSNorm's rstd OFF the critical path.  PRO 2 needs rstd before the first MFMA
+// PRO 3 (every norm-fused stage whose normalised rows are nobody's output -- qkv, gate_up -- in the chains and, with the same arithmetic, in
+// gemm_skinny_kernel): the RMSNorm's rstd OFF the critical path.  PRO 2 needs rstd before the first MFMA
 // (x = w * bf16(r * rstd)): slab loads -> LDS reduction -> barrier sit between the flags and the arithmetic.  PRO 3 feeds the MFMAs
 // bf16(w * r) -- no rstd -- and scales the fp32 sums by rstd[row] in the epilogue: the slab reduction shares the combine barrier.
 // One rounding point moves (bf16(w * bf16(r * rstd)) -> rstd * sum(W * bf16(w * r))): NOT the reference's bits; gated on the accuracy
@@ -39,11 +39,8 @@
 // WSRC: where the weight fragments come from -- 0: fetched whole into registers ahead of the flags; 1: they ride in the x ring
 // (wide slices under a tight register budget); 2: the workgroup's LDS FIFO that loader waves fill by LDS-DMA (bb_engine.hip):
 // round d = the k-steps 8 d .. 8 d + 7 of every n-tile = 8 NT pieces in the order [tile][k-step], wave w reads piece (j, w).
-//        3: registers the PREVIOUS stage filled (Wpre): a stage calls `prefetch()` -- PF::LOADS loads of the next stage's slice
-//        per wave -- behind its epilogue stores and then drains only down to vmcnt(PF::LOADS): the stores are out, the weight
-//        loads stay in flight through the barrier, the flag and the next hand-off.  (Issued earlier -- behind the last
-//        activation load -- they sit in front of the stores in the wave's in-order queue and the flag waits for the whole
-//        slice: measured +0.2 ms per step.)
+// prefetch: PF::LOADS loads per wave that belong to a later stage (bb_all.hip: the attention's first K / V pieces) go out behind the epilogue stores, and the
+// stage drains only down to vmcnt(PF::LOADS): the stores are out, the loads stay in flight through the barrier, the flag and the next hand-off.
 struct ChainNoPrefetch { static constexpr int LOADS = 0; __device__ __forceinline__ void operator()() const {} };
 // ---- round 6: the tensor-parallel all-reduce INSIDE a residual stage (bb_chain.hip on a tensor-parallel rank; allreduce.hip is the same
 // exchange as a launch of its own).  The stage's workgroup owns one 16-column x (16 MT)-row tile of the row-parallel GEMM's output on EVERY
@@ -73,15 +70,11 @@ struct ChainPrefetch {           // N = loads per wave that F issues
 };
 // ONEPASS: more than 6 tiles still combine in ONE pass (the caller's LDS holds CH_WAVES * NT * MT KB of slots): one barrier
 // instead of three and twice the epilogue threads at work; same order of additions.
-// PS: rows per sum(r^2) slab (64; 128 for the code predictor's two-position pass, whose stream holds 128 rows)
-// WAUX: cache policy of the WEIGHT loads (0 default, OMNI_AUX_NT = non-temporal: MI355X_MICROARCH "nt-weights" -- for slices that exactly
-// one workgroup reads once per launch; round 5 A/B, profiles/r05_ab_table.txt)
-template <int MT, int NT, int NTW, int PRO, int EPI, int XG = 0, int WSRC = 0, class PF = ChainNoPrefetch, bool ONEPASS = false, int PS = 64, int WAUX = 0,
-          bool AR = false>
+template <int MT, int NT, int NTW, int PRO, int EPI, int XG = 0, int WSRC = 0, class PF = ChainNoPrefetch, bool ONEPASS = false, bool AR = false>
 __device__ __forceinline__ void chain_gemm(const uint16_t* __restrict__ W, const uint16_t* __restrict__ norm_w, const uint16_t* x,
                                            const float* part_in, int np_in, void* out, int ldo, float* part_out, int M, int N, float eps,
                                            int bx, int by, float* lds, ChainGate& g, bool wait, int code,
-                                           unsigned long long* stamps, const u32x4 (*Wpre)[NT] = nullptr, PF prefetch = PF(),
+                                           unsigned long long* stamps, PF prefetch = PF(),
                                            uint16_t* normed_out = nullptr /* PRO 2: the normalised rows, row-major [M][K] (plain stores:
                                            for the NEXT launch), written by the workgroup columns bx < 8 as gemm_skinny_kernel spreads them */,
                                            const uint8_t* mask = nullptr /* EPI_F32_BF16RND: logit n is `mask_fill` where mask[n] == 0 (the codec mask) */,
@@ -121,7 +114,7 @@ __device__ __forceinline__ void chain_gemm(const uint16_t* __restrict__ W, const
     // ---- before the flags: everything that does not depend on the previous stage.  (The polling wave's first poll returns
     // behind its own weight loads -- a wave's loads return in order -- but letting wave 0 fetch its share of the slice behind
     // the flags instead measured WORSE: the predictor 1.80 -> 2.11 ms; its weights then arrive later than the activations.)
-    constexpr int WS = (WFIFO || WSRC == 3) ? 1 : (WRING ? G : NTW);      // weight slots held at a time
+    constexpr int WS = WFIFO ? 1 : (WRING ? G : NTW);      // weight slots held at a time
     u32x4 Wq[WS][NT], NWq[G];
 #pragma unroll
     for (int d = 0; d < NTW; ++d) {
@@ -129,7 +122,7 @@ __device__ __forceinline__ void chain_gemm(const uint16_t* __restrict__ W, const
         if (WSRC == 0) {
 #pragma unroll
             for (int j = 0; j < NT; ++j)
-                Wq[d][j] = __builtin_amdgcn_raw_buffer_load_b128(wrs, lane16, (uint32_t)((wtile(j) * nsteps + ks) * 1024), WAUX);
+                Wq[d][j] = __builtin_amdgcn_raw_buffer_load_b128(wrs, lane16, (uint32_t)((wtile(j) * nsteps + ks) * 1024), 0);
         }
         if (NW_EARLY) NWq[d % G] = __builtin_amdgcn_raw_buffer_load_b128(nrs, q * 16, ks * 64, 0);
     }
@@ -155,7 +148,7 @@ __device__ __forceinline__ void chain_gemm(const uint16_t* __restrict__ W, const
 #pragma unroll
         for (int e = 0; e < SO::PE; ++e) {
             const int p = SO::index(wave, sub, e);
-            pv[e] = coh_ldf(prs, (uint32_t)(min(p, np_in - 1) * PS + m_base + row) * 4);
+            pv[e] = coh_ldf(prs, (uint32_t)(min(p, np_in - 1) * 64 + m_base + row) * 4);
             if (p >= np_in) pv[e] = 0.f;
         }
     }
@@ -164,7 +157,7 @@ __device__ __forceinline__ void chain_gemm(const uint16_t* __restrict__ W, const
         if (WRING) {
 #pragma unroll
             for (int j = 0; j < NT; ++j)
-                Wq[d % G][j] = __builtin_amdgcn_raw_buffer_load_b128(wrs, lane16, (uint32_t)(((bx * NT + j) * nsteps + wave + d * CH_WAVES) * 1024), WAUX);
+                Wq[d % G][j] = __builtin_amdgcn_raw_buffer_load_b128(wrs, lane16, (uint32_t)(((bx * NT + j) * nsteps + wave + d * CH_WAVES) * 1024), 0);
         }
         if (NORM && !NW_EARLY) NWq[d % G] = __builtin_amdgcn_raw_buffer_load_b128(nrs, q * 16, (wave + d * CH_WAVES) * 64, 0);
 #pragma unroll
@@ -209,9 +202,6 @@ __device__ __forceinline__ void chain_gemm(const uint16_t* __restrict__ W, const
 #pragma unroll
             for (int j = 0; j < NT; ++j)
                 Wn[j] = *reinterpret_cast<const u32x4*>(g.fifo + (size_t)((first + j * 8 + wave) % ENG_FIFO_PIECES) * 1024 + lane16);
-        } else if (WSRC == 3) {
-#pragma unroll
-            for (int j = 0; j < NT; ++j) Wn[j] = Wpre[d][j];
         } else {
 #pragma unroll
             for (int j = 0; j < NT; ++j) Wn[j] = Wq[WRING ? d % G : d][j];
@@ -319,7 +309,7 @@ __device__ __forceinline__ void chain_gemm(const uint16_t* __restrict__ W, const
         }
         float ss = sq4_sum(rv[0], rv[1], rv[2], rv[3]);
         ss = xor32_sum(xor16_sum(ss));                                         // (whole waves: rows past Mloc add into lanes nobody stores)
-        if (has && l < 16) coh_st4(coh_rsrc(part_out), (uint32_t)(bx * PS + m) * 4, __float_as_uint(ss));
+        if (has && l < 16) coh_st4(coh_rsrc(part_out), (uint32_t)(bx * 64 + m) * 4, __float_as_uint(ss));
     } else
     for (int it = threadIdx.x; it < ITEMS; it += CH_THREADS) {
         const int l = it % LN;
@@ -366,7 +356,7 @@ __device__ __forceinline__ void chain_gemm(const uint16_t* __restrict__ W, const
             coh_st8(ors, (uint32_t)frag_off(m, n, N) * 2, (u32x2){pack_bf2(rv[0], rv[1]), pack_bf2(rv[2], rv[3])});
             float ss = sq4_sum(rv[0], rv[1], rv[2], rv[3]);
             ss = xor32_sum(xor16_sum(ss));
-            if (l < 16) coh_st4(coh_rsrc(part_out), (uint32_t)(bx * PS + m) * 4, __float_as_uint(ss));
+            if (l < 16) coh_st4(coh_rsrc(part_out), (uint32_t)(bx * 64 + m) * 4, __float_as_uint(ss));
         } else if (EPI == OMNI_EPI_F32_BF16RND) {
             // logits: fp32 cells holding bf16-rounded values (the reference's bf16 head output), row-major
             const int n = (bx * NT + j) * 16 + 4 * (l >> 4);

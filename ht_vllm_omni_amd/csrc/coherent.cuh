@@ -94,9 +94,7 @@ struct ChainGate {
     int32_t* err;
     bool dead;             // a spin ran out (here or in an earlier launch): stop waiting
     int dom;               // log2 of the flag domain: 6 = the row group's 64 workgroups, 7 = a pair of groups, 8 = all 256
-    int nap;               // s_sleep units (64 clocks) between two polls: 0, 1, 2, 4, 8
     int ahead;             // stages this workgroup has passed without rows since it last waited (chain_gate_skip)
-    int skip_units;        // sleep per skipped stage before the first poll, in units of 32 x 64 clocks (3 = ~2.9 us; A/B knob)
     unsigned long long* stamps;   // debug library only: timeline stamps of the attention stage (pa_body.cuh, CHAIN), or NULL
     // engine mode (NULL / unused in the plain chains): barriers among the 8 compute waves only, weights from the LDS FIFO
     EngSync* es;
@@ -159,8 +157,6 @@ __device__ __forceinline__ void chain_gate_init(ChainGate& g, uint32_t* flags, i
     g.epoch = __builtin_amdgcn_readfirstlane(coh_ld4(g.frs, wg * 4));
     g.dead = __builtin_amdgcn_readfirstlane(__hip_atomic_load(err, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) != 0;
     g.dom = 8;
-    g.nap = 1;
-    g.skip_units = 3;
     g.stamps = nullptr;
     g.ahead = 0;
     g.es = nullptr; g.bgen = 0; g.fifo = nullptr; g.piece_base = 0; g.ready = 0;
@@ -178,29 +174,11 @@ __device__ __forceinline__ void chain_gate_init(ChainGate& g, uint32_t* flags, i
 // stages early: it sleeps ~2.5 us per skipped stage (a stage takes 3-5.5 us) before its first poll.
 __device__ __forceinline__ void chain_gate_wait(ChainGate& g, int code) {
     if (threadIdx.x < 64 && !g.dead) {
-        for (int i = 0; i < g.ahead * g.skip_units; ++i) __builtin_amdgcn_s_sleep(32);
+        for (int i = 0; i < g.ahead * 3; ++i) __builtin_amdgcn_s_sleep(32);
         // (1 << dom) / 4 lanes x 4 flags each (the other lanes read copies)
         const uint32_t off = chain_flag_copy() + ((g.wg >> g.dom) << (g.dom + 2)) + (threadIdx.x & ((1u << (g.dom - 2)) - 1)) * 16;
         unsigned spins = 0;
         unsigned long long t0 = 0;
-        if (g.nap >= 16) {
-            // two polls in flight, half a round trip apart: the flags are sampled twice as often as one load's latency allows
-            u32x4 fa = coh_ld16(g.frs, off);
-            for (;;) {
-                asm volatile("" ::: "memory");
-                __builtin_amdgcn_s_sleep(4);
-                const u32x4 fb = coh_ld16(g.frs, off);
-                const bool behind = (int)(fa[0] - g.epoch) < 0 || (int)(fa[1] - g.epoch) < 0 || (int)(fa[2] - g.epoch) < 0 ||
-                                    (int)(fa[3] - g.epoch) < 0;
-                if (__builtin_amdgcn_ballot_w64(behind) == 0) break;
-                fa = fb;
-                if (chain_wait_expired(++spins, t0)) {
-                    if (threadIdx.x == 0) atomicCAS(g.err, 0, code);
-                    g.dead = true;
-                    break;
-                }
-            }
-        } else
         for (;;) {
             asm volatile("" ::: "memory");                // the buffer load is a plain read to the compiler: keep it inside the loop
             const u32x4 f = coh_ld16(g.frs, off);
@@ -209,10 +187,7 @@ __device__ __forceinline__ void chain_gate_wait(ChainGate& g, int code) {
             if (__builtin_amdgcn_ballot_w64(behind) == 0) break;
             // back-to-back polls from 256 waves slow every other memory access of the chip down (measured: the whole
             // predictor 1.90 -> 2.55 ms without any pause)
-            if (g.nap == 1) __builtin_amdgcn_s_sleep(1);
-            else if (g.nap == 2) __builtin_amdgcn_s_sleep(2);
-            else if (g.nap == 4) __builtin_amdgcn_s_sleep(4);
-            else if (g.nap >= 8) __builtin_amdgcn_s_sleep(8);
+            __builtin_amdgcn_s_sleep(1);
             if (chain_wait_expired(++spins, t0)) {
                 if (threadIdx.x == 0) atomicCAS(g.err, 0, code);
                 g.dead = true;

@@ -25,7 +25,7 @@ struct MoeChainArgs {
     uint16_t* act;                     // fragment-major [64][768]
     uint16_t* shared;                  // row-major [B][1024]: the shared expert's output (combined by the expert launch)
     int32_t* topk_idx; uint16_t* topk_w;
-    int B, top_k, norm_topk, nap; float eps;
+    int B, top_k, norm_topk; float eps;
     uint32_t* flags; int32_t* err;
 };
 
@@ -91,7 +91,6 @@ __global__ __launch_bounds__(CH_THREADS) void moe_chain_kernel(const MoeChainArg
     ChainGate g;
     chain_gate_init(g, a.flags, a.err);
     g.dom = 8;                          // the stages deal rows to workgroups differently (64 / 48 / 8 column groups): one domain
-    g.nap = a.nap;
     const int wg = blockIdx.x;
     constexpr int H = 1024, KO = 2048, E = 128, IS = 768;
     static_assert(KO == 8 * 256 && H == 4 * 256 && IS == 3 * 256, "moe_chain: k-steps per wave");
@@ -103,7 +102,7 @@ __global__ __launch_bounds__(CH_THREADS) void moe_chain_kernel(const MoeChainArg
                                                   0x2002, nullptr);
     else if (wg < 224)       // router: 8 column groups x 4 row groups; column group x also writes k-steps x, x + 8, ... of the normalised rows
         chain_gemm<1, 1, 4, 2, OMNI_EPI_BF16>(a.router, a.ln2, a.resid, a.part, H / 16, a.logits, E, nullptr, a.B, E, a.eps, (wg - 192) & 7, (wg - 192) >> 3,
-                                              lds, g, true, 0x2002, nullptr, nullptr, ChainNoPrefetch(), a.normed_rm);
+                                              lds, g, true, 0x2002, nullptr, ChainNoPrefetch(), a.normed_rm);
     else
         chain_gate_skip(g);
     chain_gemm<1, 1, 3, 0, OMNI_EPI_BF16>(a.sdown, nullptr, a.act, nullptr, 0, a.shared, H, nullptr, a.B, H, a.eps, wg & 63, wg >> 6, lds, g, true, 0x2003,
@@ -123,7 +122,7 @@ struct MoeTailArgs {
     const uint16_t *y, *x, *w_sg, *shared; const int32_t* topk_idx;
     uint16_t* resid; float* part;
     const uint16_t *ln1_next, *wqkv_next; uint16_t* qkv;
-    int B, top_k, e_lo, e_hi, nap; float eps;
+    int B, top_k, e_lo, e_hi; float eps;
     uint32_t* flags; int32_t* err;
 };
 
@@ -197,7 +196,6 @@ __global__ __launch_bounds__(CH_THREADS) void moe_tail_kernel(const MoeTailArgs 
     ChainGate g;
     chain_gate_init(g, a.flags, a.err);
     g.dom = 8;
-    g.nap = a.nap;
     const int wg = blockIdx.x;
     constexpr int H = 1024, NQ = 2560;
     if (wg < a.B) {                      // stage 0x2101: the combine of row wg
@@ -213,7 +211,7 @@ __global__ __launch_bounds__(CH_THREADS) void moe_tail_kernel(const MoeTailArgs 
         chain_gate_skip(g);
 }
 
-OMNI_KNOB g_moe_chain = 1, g_moe_chain_nap = 1, g_moe_tail = 1;
+OMNI_KNOB g_moe_chain = 1, g_moe_tail = 1;
 #ifdef OMNI_DEBUG_HOOKS
 extern "C" void omni_debug_moe_chain(int on) { g_moe_chain = on != 0; g_moe_tail = on != 2; }      // 2: the first chain only (the tail as launches)
 #endif
@@ -226,7 +224,7 @@ int k_moe_tail(const omni_talker_desc& d, const omni_layer_weights& w, const omn
     a.topk_idx = topk_idx; a.resid = (uint16_t*)resid; a.part = part;
     a.ln1_next = (const uint16_t*)next.ln1; a.wqkv_next = (const uint16_t*)next.wqkv; a.qkv = (uint16_t*)qkv;
     a.B = B; a.top_k = d.moe_top_k; a.e_lo = d.moe_e0; a.e_hi = d.moe_e0 + (d.moe_experts_local > 0 ? d.moe_experts_local : d.moe_experts);
-    a.nap = g_moe_chain_nap; a.eps = d.eps; a.flags = flags; a.err = err;
+    a.eps = d.eps; a.flags = flags; a.err = err;
     hipLaunchKernelGGL(moe_tail_kernel, dim3(OMNI_CHAIN_WGS), dim3(CH_THREADS), 0, (hipStream_t)stream, a);
     OMNI_CHECK_LAUNCH("moe_tail");
     return OMNI_OK;
@@ -251,7 +249,7 @@ int k_moe_chain(const omni_talker_desc& d, const omni_layer_weights& w, const vo
     a.sgu = (const uint16_t*)w.moe_shared_gate_up; a.sdown = (const uint16_t*)w.moe_shared_down;
     a.attn = (const uint16_t*)attn; a.resid = (uint16_t*)resid; a.part = part; a.normed_rm = (uint16_t*)normed_rm; a.logits = (uint16_t*)logits;
     a.act = (uint16_t*)act; a.shared = (uint16_t*)shared; a.topk_idx = topk_idx; a.topk_w = (uint16_t*)topk_w;
-    a.B = B; a.top_k = d.moe_top_k; a.norm_topk = d.moe_norm_topk; a.nap = g_moe_chain_nap; a.eps = d.eps;
+    a.B = B; a.top_k = d.moe_top_k; a.norm_topk = d.moe_norm_topk; a.eps = d.eps;
     a.flags = flags; a.err = err;
     hipLaunchKernelGGL(moe_chain_kernel, dim3(OMNI_CHAIN_WGS), dim3(CH_THREADS), 0, (hipStream_t)stream, a);
     OMNI_CHECK_LAUNCH("moe_chain");

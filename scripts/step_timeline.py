@@ -14,7 +14,7 @@ ap.add_argument("--batch", type=int, default=64)
 ap.add_argument("--ctx", type=int, default=352)
 ap.add_argument("--kv", default="fp8")
 ap.add_argument("--model", default="tts-1.7b")
-ap.add_argument("--knobs", default="", help="debug knobs applied before capture, e.g. chain_pair=0,bb_deep=6")
+ap.add_argument("--knobs", default="", help="debug knobs applied before capture, e.g. chain_pair=0,chain_tail=0")
 ap.add_argument("--stages", action="store_true", help="per-stage medians of passes 2, 3, 8, 15")
 a = ap.parse_args()
 args = types.SimpleNamespace(allreduce="rccl", model=a.model, kv=a.kv, batch=a.batch, num_blocks=8192, device_weights=True, parallel="tp", sub_batches=1,

@@ -149,26 +149,24 @@ def _decode_engine(d, w, B, kv="fp8"):
 UNRELEASED = dict(hidden=1536, inter=4608, q_heads=12, kv_heads=6)
 
 
-@pytest.mark.parametrize("mode,B,kv,shape", [("engine", 64, "fp8", None), ("plain-chain", 64, "fp8", None), ("deep-rings", 64, "fp8", None),
-                                             ("engine", 49, "bf16", None), ("plain-chain", 49, "bf16", None), ("deep-rings", 49, "bf16", None),
+@pytest.mark.parametrize("mode,B,kv,shape", [("engine", 64, "fp8", None), ("plain-chain", 64, "fp8", None),
+                                             ("engine", 49, "bf16", None), ("plain-chain", 49, "bf16", None),
                                              ("plain-chain", 64, "fp8", UNRELEASED), ("plain-chain", 41, "int8", UNRELEASED)])
 def test_backbone_segment_chain_against_the_launch_path(B, kv, mode, shape):
     """o_proj -> gate_up -> down_proj -> next qkv as one persistent launch per layer against the launch-per-op backbone of the
-    same library at the 1.7B shape.  The plain chain (csrc/bb_chain.hip) and the loader / consumer engine (bb_engine.hip) keep
-    the launch path's tiles and summation order: logits, hidden state, sampled ids, codes and every KV byte of three decode
-    steps are identical.  (Rounds 3's two-group and split-role arms -- bb_pp.hip, bb_xw.hip: both lost -- left the tree in round 6, when
-    the deferred rstd became the product arithmetic; NOTEBOOK "Round 3" keeps their measurements.)  No flag wait times out in any mode."""
+    same library at the 1.7B shape.  The chain (csrc/bb_chain.hip bb_flow_kernel) and the debug library's loader / consumer engine (bb_engine.hip) keep the
+    launch path's tiles and summation order: logits, hidden state, sampled ids, codes and every KV byte of three decode steps are identical.  No wait
+    times out in any mode."""
     d = get_dims("tts-1.7b").with_(layers=3, max_model_len=256, **(shape or {}))
     w = make_weights(d, seed=8, std=0.02)
     res = {}
     with L.debug_library() as lib:
-        for fn in (lib.omni_debug_bb_chain, lib.omni_debug_bb_engine, lib.omni_debug_bb_deep):
+        for fn in (lib.omni_debug_bb_chain, lib.omni_debug_bb_engine):
             fn.argtypes = [C.c_int]; fn.restype = None
         try:
             for on in (0, 1):
                 lib.omni_debug_bb_chain(on)
                 lib.omni_debug_bb_engine(int(mode == "engine"))
-                lib.omni_debug_bb_deep(int(mode == "deep-rings"))
                 eng = _decode_engine(d, w, B, kv)
                 outs = []
                 for _ in range(3):
@@ -181,7 +179,6 @@ def test_backbone_segment_chain_against_the_launch_path(B, kv, mode, shape):
         finally:
             lib.omni_debug_bb_chain(1)
             lib.omni_debug_bb_engine(0)
-            lib.omni_debug_bb_deep(0)
     for s, (a, b) in enumerate(zip(res[1][0], res[0][0])):
         for name, x, y in zip(("logits", "hidden", "ids", "codes"), a, b):
             assert torch.equal(x, y), f"step {s}: {name} differ between the backbone chain and the launch path"
@@ -356,7 +353,7 @@ def test_words_of_all_ones_pass_the_backbones_hand_offs(model, B):
 def test_whole_backbone_launch_against_the_launch_path(B, kv, base):
     """The whole decoder stack -- qkv(0), then attention -> o_proj -> gate_up -> down_proj -> next qkv per layer -- as ONE persistent
     launch (csrc/bb_all.hip: the paged attention is a stage of the grid, two (row, kv head) pairs per workgroup) against the
-    launch-per-op backbone and against round 3's per-layer chain of the same library: pa_body.cuh / chain_gemm.cuh are the launch
+    launch-per-op backbone and against the per-layer chain of the same library: pa_body.cuh / chain_gemm.cuh are the launch
     path's arithmetic, so logits, hidden state, sampled ids, codes, slot mapping and every KV byte of three decode steps are
     identical; no flag wait times out.  Reference: the vLLM Qwen3 decoder stack behind qwen3_tts_talker.py:341,414-422."""
     d = get_dims("tts-1.7b").with_(layers=3, max_model_len=256)
@@ -392,7 +389,7 @@ def test_whole_backbone_launch_against_the_launch_path(B, kv, base):
 
 @pytest.mark.parametrize("B,kv", [(64, "int8"), (37, "fp8"), (8, "bf16"), (1, "int8")])
 def test_moe_layer_chain_against_the_launch_path(B, kv):
-    """Round 5 (BASELINE configs #4 / #5): the Omni talker's sparse-MoE layer as TWO persistent launches around its
+    """The Omni talker's sparse-MoE layer as TWO persistent launches around its
     expert GEMMs (csrc/moe_chain.hip) -- o_proj -> { router GEMM + normalised rows | shared-expert gate_up } -> { shared-expert down_proj,
     top-k routing }, and { combine into the residual stream -> the next layer's qkv } -- against the seven launches they replace (mode 2:
     the first chain alone): the launch path's tiles, k-step ownership, combine orders and the routing / combine kernels' arithmetic, so three

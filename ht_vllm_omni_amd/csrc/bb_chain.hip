@@ -8,10 +8,12 @@
 //   bb_chain_kernel                        a tensor-parallel rank (AR), the half grid (HALF): behind flags (chain_gemm.cuh)
 // K-step ownership, combine order and rounding points are the launch path's: results are bit-identical.
 // A decode step, behind flags and by content, one card: 64 rows of the 1.7B shape 3050 -> 2886 us, 5 rows of the 0.6B one 2091 -> 1859.
-// Of a 64-row launch (32 us, 100 MB) gate_up is half: its 50 MB come out of HBM at 5.5 TB/s, and a wave's loads return in order, so half of a wave's
-// slice goes out in front of the first look at the operands and half behind the first of them (down_proj: half of its 24 k-steps, x twelve deep): 2866 ->
-// 2837 us a step.  Slices with a single reader are loaded past the caches, which leaves the last-level cache to the predictor's weights (157 MB): 64 rows
-// 2837 -> 2805, 24 rows 2409 -> 2371, 7 rows 2112 -> 2065, 0.6B, 5 rows 1772 -> 1744; those that the two row halves share are not (64 rows 2817 -> 2839).
+// Of a 64-row launch (32 us, 100 MB) gate_up takes 13 us, in which its 50 MB come out of HBM; a wave's loads return in order, so half of a wave's
+// slice goes out in front of the first look at the operands and half behind the first of them (down_proj: half of its 24 k-steps, x twelve deep): 64 rows
+// 2807 -> 2771 us a step, 24 rows 2354 -> 2342.  Slices with a single reader are loaded past the caches, which leaves the last-level cache to the predictor's
+// weights (157 MB): 64 rows 2786 -> 2771, 24 rows 2352 -> 2342, 7 rows 2079 -> 2031, 0.6B, 5 rows 1750 -> 1717; those that the two row halves share are not
+// (64 rows 2817 -> 2839).  The splits for few rows alone: 24 rows 2488 -> 2342, 7 rows 2310 -> 2031, 0.6B, 5 rows 2030 -> 1717 (with the predictor's;
+// profiles/talker_step_sweeps.txt, talker_step_timeline.txt).
 // Tried: gate_up's slice asked for by o_proj's waves (their combine waits for the queue: the same), half of qkv's behind the look (64 rows + 10 us).
 // Shapes are parameters, not literals (the checkpoint decides them, configuration_qwen3_tts.py:192-216): the stage set is a template
 // on the k-steps per wave of its three reduction widths -- KO = q_heads * 128 / 256 (o_proj), KH = hidden / 256 (gate_up, qkv), KI =
@@ -33,13 +35,13 @@ struct BbArgs {
     uint16_t* act;                      // fragment-major [64][6144]
     uint16_t* qkv;                      // row-major [B][NQ]
     int H, I, NQ;                       // output widths: hidden, intermediate, (q_heads + 2 kv_heads) * 128
-    // the LAST layer's launch (no next qkv) may end in the talker's own head instead (round 6): final norm folded into the lm_head GEMM, its
+    // the LAST layer's launch (no next qkv) may end in the talker's own head instead: final norm folded into the lm_head GEMM, its
     // normalised rows = h[t + 1] (row-major, rows below *num_live), logits fp32 [B][V] holding bf16-rounded values, the codec mask applied
     const uint16_t *lm_head, *final_norm; float* logits; uint16_t* last_hidden; const uint8_t* mask; const int32_t* num_live; float mask_fill; int V;
     int B; float eps;
     uint32_t* flags; int32_t* err;
     unsigned long long* stamps;
-    // tensor-parallel rank (round 6): o_proj and down_proj are row-parallel partials; their all-reduce rides in the two residual epilogues
+    // tensor-parallel rank: o_proj and down_proj are row-parallel partials; their all-reduce rides in the two residual epilogues
     // (chain_gemm AR).  ar_epoch = allreduce.hip's epoch / ticket words: this launch makes calls epoch + 1 (o_proj) and epoch + 2 (down_proj)
     ChainAr ar_o, ar_dn;
     uint32_t* ar_epoch;
@@ -300,7 +302,7 @@ OMNI_KNOB g_bb_chain = 1, g_bb_min_rows = 33, g_bb_b32 = 1, g_bb_ar = 1;
 static unsigned long long* g_bb_stamps = nullptr;
 extern "C" void omni_debug_bb_chain(int on) { g_bb_chain = on; }
 extern "C" void omni_debug_bb_stamps(void* buf) { g_bb_stamps = (unsigned long long*)buf; }
-extern "C" void omni_debug_bb_ar(int on) { g_bb_ar = on; }                  // 0: tensor-parallel ranks keep the launch-per-op backbone (round 5)
+extern "C" void omni_debug_bb_ar(int on) { g_bb_ar = on; }                  // 0: tensor-parallel ranks keep the launch-per-op backbone
 extern "C" void omni_debug_bb_min_rows(int rows) { g_bb_min_rows = rows; g_bb_b32 = rows <= 49; }      // smallest batch of the 64-row split
 #endif
 

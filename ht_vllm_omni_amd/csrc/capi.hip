@@ -632,7 +632,7 @@ static int run_code_predictor(omni_talker* t, const int32_t* layer0_ids, const v
             }
             if (!in_pair) {
                 if (d.cp_chain && !t->chain_half && k_cp_chain_supported(d, g)) {
-                    // the layer stack of this pass as one persistent launch: 25 stages behind flag hand-offs
+                    // the layer stack of this pass as one persistent launch: 25 stages, hand-offs by content
                     TRY(k_cp_chain(d, t->cp_layer.data(), t->cp_k.data(), t->cp_v.data(), B, g, g + 1, np, t->cp_resid, t->cp_part, cflags,
                                    cerr, t->cp_flow, nullptr, st));
                     t->ran |= 1;

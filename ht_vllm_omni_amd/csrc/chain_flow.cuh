@@ -45,9 +45,10 @@ __device__ __forceinline__ int flow_failed(const int32_t* err) {
     return __builtin_amdgcn_readfirstlane(__hip_atomic_load(err, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) != 0;
 }
 // another look at the operands is due: false = carry on with what is there.  (Looks at lines nobody has written since are served by the XCD's
-// own L2.  The predictor's launch, pauses of 0 / 64 / 128 / 256 / 384 clocks: 64 rows 2807 / 2810 / 2781 / 2770 / 2785 us a step, 40 rows of the 0.6B talker
-// 2208 / 2204 / 2214 (128 / 256 / 384), 24 rows 1992 / 2002 / 2006, 5 rows 1719 / 1717 / 1719 / 1722 and, on another card, 1697 / 1700 / 1705 (128 / 256 / 384): twice as long above 32 rows, where every
-// workgroup waits in every stage.  The backbone's layers: no difference.)
+// own L2.  The predictor's launch, pauses of 0 / 64 / 128 / 256 / 384 clocks: 64 rows 2807 / 2810 / 2781 / 2770 / 2785 us a step, 5 rows 1719 / 1717 / 1719 / 1722 and,
+// on another card, 1697 / 1700 / 1705 (128 / 256 / 384): twice as long above 32 rows, where every workgroup waits in every stage.  That is little, and in every one of
+// twelve pairs of runs: 64 rows 2779 -> 2776, 44 rows 2596 -> 2591, 40 rows of the 0.6B talker 2201 -> 2198, 64 rows 2298 -> 2289, runs of one side within 3 us
+// (profiles/talker_step_sweeps.txt).  The backbone's layers: no difference.)
 __device__ __forceinline__ bool flow_again(FlowWait& f, int code, unsigned& spins, unsigned long long& t0) {
     if (f.dead) return false;
     if (f.calm) __builtin_amdgcn_s_sleep(4);
@@ -90,7 +91,7 @@ __device__ __forceinline__ void flow_ask(const uint16_t* W, int bx, u32x4 (&Wq)[
 // One skinny-GEMM stage: chain_gemm's k-steps per wave, accumulation, combine order and rounding points (the launch path's bits), its x and
 // slabs awaited by content.  x: fragment-major, 32-column k-steps; `x` / `part_in` / `out` / `part_out` lie in this use's copy (or, the launch's
 // first input, in the plain buffers its predecessor filled: never EMPTY).  clr / clr_part: the same places in the copy to clear, NULL: none.
-// Output layouts (whatever a workgroup writes lies together: no line has two writers):
+// Output layouts (a workgroup's tiles lie together, so that no line of them has two writers; the slabs' 64-byte groups of 16 rows share lines):
 //   RESID, GU8    fragment-major
 //   BF16          16 x 16 bf16 tiles, 512 B: tile t of row group r at (r * (N / 16) + t) * 512, rows of 32 B
 //   F32_BF16RND   16 x 16 fp32 tiles, 1 KB:  tile t of row group r at (r * (N / 16) + t) * 1024, rows of 64 B

@@ -42,7 +42,7 @@
 // prefetch: PF::LOADS loads per wave that belong to a later stage (bb_all.hip: the attention's first K / V pieces) go out behind the epilogue stores, and the
 // stage drains only down to vmcnt(PF::LOADS): the stores are out, the loads stay in flight through the barrier, the flag and the next hand-off.
 struct ChainNoPrefetch { static constexpr int LOADS = 0; __device__ __forceinline__ void operator()() const {} };
-// ---- round 6: the tensor-parallel all-reduce INSIDE a residual stage (bb_chain.hip on a tensor-parallel rank; allreduce.hip is the same
+// ---- the tensor-parallel all-reduce INSIDE a residual stage (bb_chain.hip on a tensor-parallel rank; allreduce.hip is the same
 // exchange as a launch of its own).  The stage's workgroup owns one 16-column x (16 MT)-row tile of the row-parallel GEMM's output on EVERY
 // rank, so the exchange is per tile and needs no stage of its own:
 //   partial   the tile's K-combined sums, rounded to bf16, into this rank's peer-mapped buffer data[rank] (system-scope write-through stores)
@@ -87,7 +87,7 @@ __device__ __forceinline__ void chain_gemm(const uint16_t* __restrict__ W, const
     constexpr int K = NTW * CH_WAVES * 32;
     constexpr int nsteps = K / 32;
     constexpr bool GU8 = EPI == OMNI_EPI_SILU_MUL_GU8;
-    // OMNI_EPI_SILU_MUL (round 5: the MoE layer's shared expert): W = [gate rows | up rows], n-tiles [0, NT/2) are gate tiles, [NT/2, NT)
+    // OMNI_EPI_SILU_MUL (the MoE layer's shared expert): W = [gate rows | up rows], n-tiles [0, NT/2) are gate tiles, [NT/2, NT)
     // the matching up tiles N rows further down (gemm_skinny_kernel's pairing); out = N activation columns
     constexpr bool SILU2 = EPI == OMNI_EPI_SILU_MUL;
     constexpr bool WRING = WSRC == 1, WFIFO = WSRC == 2;

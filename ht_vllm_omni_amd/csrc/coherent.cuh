@@ -5,8 +5,8 @@
 //             storing wave runs `s_waitcnt vmcnt(0)`; a workgroup barrier; then ONE lane publishes the workgroup's flag (sc1 store)
 //   consumer  one wave polls the flags with sc1 loads; the other waves pass a workgroup barrier behind it; every load of the
 //             handed-off bytes is an sc1 buffer load to registers (bypasses the L1; 4-, 8- or 16-byte accesses only)
-// No release / acquire fence anywhere: a fence writes back or invalidates whole caches (38-43 us per grid barrier measured in
-// round 2), an sc1 access costs what a plain one costs at 16 bytes.
+// No release / acquire fence anywhere: a fence writes back or invalidates whole caches (38-43 us per grid
+// barrier), an sc1 access costs what a plain one costs at 16 bytes.
 //
 // Buffer addressing: the resource descriptor is built from a wave-uniform base (SGPRs), lanes supply 32-bit byte offsets
 // (`buffer_load_dwordx4 v, v_off, s[rsrc], 0 offen sc1`); hipcc counts these loads in vmcnt like any other.
@@ -64,8 +64,7 @@ __device__ __forceinline__ uint32_t chain_flag_copy() { return (uint32_t)(blockI
 // workgroup that never sees its peers (a grid that is not co-resident, a lost launch) sets *err and the launch runs to its
 // end without waiting -- a wrong step that the host sees in the error word, never a hung GPU.
 #define OMNI_CHAIN_WGS 256
-#define OMNI_CHAIN_SPIN_BOUND (1u << 21)   // (round-3 arms of the debug library)
-// the product chains wait by WALL CLOCK (ADVICE r3): 2 s of the constant 100 MHz counter, read once per 1024 polls -- a poll is
+// the product chains wait by WALL CLOCK: 2 s of the constant 100 MHz counter, read once per 1024 polls -- a poll is
 // a memory round trip of 0.5-2 us, so the first reading comes after about a millisecond of waiting and costs a healthy stage nothing
 #define OMNI_CHAIN_WAIT_TICKS 200000000ull
 __device__ __forceinline__ bool chain_wait_expired(unsigned spins, unsigned long long& t0) {

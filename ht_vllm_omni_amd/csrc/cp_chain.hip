@@ -3,13 +3,14 @@
 //
 // Launch-per-op, a predictor pass is 25 dependent launches (5 layers x { qkv, attention, o_proj, gate_up, down_proj }) of
 // ~5.5 us each although a workgroup's share of a GEMM is 16-48 KB of weights and a few MFMAs: a dependent launch pays the
-// kernel boundary (1.65 us), a cold weight fetch, a cold activation fetch and a store drain, one after the other (DESIGN 6).
+// kernel boundary (1.65 us), a cold weight fetch, a cold activation fetch and a store drain, one after the other.
 // Here the stages run inside one grid of 256 co-resident workgroups (one per CU):
 //   * a stage's WEIGHT slice does not depend on its predecessor: every wave loads its whole slice before it looks for its operands;
 //   * cp_chain_kernel (passes 2 .. 15, their heads and samplers) hands activations over by content: an operand is there when none of its words
 //     is EMPTY (chain_flow.cuh).  No drain, no flag, no barrier between a stage's last store and its successor's first MFMA.  What bounds it is
-//     that chain of dependent trips: 27 stages a pass of about 2.6 us (5 rows: 69 us a pass; 64 rows: 89), of which 0.6 to 1.6 us are a stage's own
-//     arithmetic, LDS combine and epilogue and the rest the operands' way.  Behind flags (coherent.cuh) a pass took 104 / 110 us;
+//     that chain of dependent trips: 27 stages a pass of about 2.6 us at 5 rows (69 us a pass) and 3.3 at 64 (89), of which 0.6 to 1.6 us are a stage's own
+//     arithmetic, LDS combine and epilogue and the rest the operands' way (profiles/talker_step_timeline.txt).  Behind flags (coherent.cuh) a pass took
+//     104 / 110 us;
 //   * cp_pair_kernel (positions 0 and 1, group 1) likewise, over both positions' rows; a decode step of 64 / of 5 rows, us, behind flags 2886 / 1859, by
 //     content 2860 / 1784 (the stages of up to 16 rows over all 256 workgroups: 64 of them owned every column of qkv);
 //   * what a stage may read without waiting (besides weights): bytes that were final two or more stages earlier -- the K / V history of the
@@ -52,7 +53,7 @@ struct ChainArgs {
     const uint16_t* ptab;                 // folded projection tables [Q - 1][codebook][Hc]: pass g < Q - 1 gathers row `code` of table g - 1
     uint32_t* flags;
     int32_t* err;
-    // tail of the all-pass launch (round 6): input assembly of the backbone by the last sampler stage's row owners, then layer 0's qkv
+    // tail of the all-pass launch: input assembly of the backbone by the last sampler stage's row owners, then layer 0's qkv
     struct Tail {
         const int32_t* input_ids; const uint16_t* embed; int vocab; const uint16_t* cp_embed; const uint16_t* text_step;
         uint16_t* x_out; uint16_t* resid; float* part; int64_t* audio_codes; int H;
@@ -722,7 +723,8 @@ __global__ __launch_bounds__(CH_THREADS) void cp_chain_kernel(const ChainArgs a)
         for (int l = 0; l < a.layers; ++l) {
             const ChainLayer& L = a.layer[l];
             // the workgroup index, opaque per layer: hipcc otherwise hoists every tile / k-step offset of every stage (they depend on
-            // blockIdx only) out of both loops and parks them in VGPR lanes for the whole launch (v_writelane / v_readlane)
+            // blockIdx only) out of both loops and parks them in VGPR lanes for the whole launch (v_writelane / v_readlane; some 240 other
+            // SGPRs, mostly arguments and descriptors, still lie there, in 4 VGPRs)
             int wg = blockIdx.x;
             asm volatile("" : "+s"(wg));
             const int cn = cl == FLOW_COPIES - 1 ? 0 : cl + 1;
@@ -887,7 +889,7 @@ int k_cp_pair(const omni_talker_desc& d, const omni_layer_weights* layers, uint1
 #define CP_TAIL_WIDTHS(X) X(8) X(6)
 OMNI_KNOB g_chain_tail = 1;
 #ifdef OMNI_DEBUG_HOOKS
-extern "C" void omni_debug_chain_tail(int on) { g_chain_tail = on; }      // 0: mtp_finalize and the first qkv as launches of their own (round 5)
+extern "C" void omni_debug_chain_tail(int on) { g_chain_tail = on; }      // 0: mtp_finalize and the first qkv as launches of their own
 #endif
 bool k_cp_chain_tail_supported(const omni_talker_desc& d, int B) {
     bool listed = false;

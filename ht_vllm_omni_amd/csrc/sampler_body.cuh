@@ -333,7 +333,7 @@ __device__ __forceinline__ int smp_pick(float (&xr)[NPT], int V, int greedy, int
     return pick;
 }
 
-// ---- Round 6: the pick of one row by ONE wave, no workgroup barrier (the code-predictor chain's sampler stage: 8.4 us of its 11.4 were the
+// ---- the pick of one row by ONE wave, no workgroup barrier (the code-predictor chain's sampler stage: 8.4 us of its 11.4 were the
 // 4-wave pick above -- 6 barriers, a 64-step readlane rank loop, two LDS compaction passes; profiles/r06_step_timeline.txt).  Same function
 // of the row as smp_pick without top-p (top-k with ties kept -> Gumbel-max with the counter RNG, smallest index on equal scores; greedy =
 // first argmax), so both paths pick the same id bit for bit (tests/test_gpu_chain.py: chain == launch path).

@@ -19,22 +19,22 @@ void omni_debug_bb_chain(int on);                          /* backbone: o_proj -
 void omni_debug_bb_all(int on);                            /* backbone: the whole decoder stack, attention included, as ONE persistent launch (bb_all.hip) */
 void omni_debug_bb_all_stamps(void* buf, int layer);       /* uint64 [8][8][256] timeline stamps of one layer's stages of that launch (NULL: off) */
 void omni_debug_chain_pair(int on);                        /* code predictor: positions 0 / 1 + group 1's head and sampler as one persistent launch (cp_pair_kernel) */
-void omni_debug_chain_tail(int on);                         /* 1 (default): the step's input assembly + layer 0's qkv as the tail of the predictor's all-pass launch; 0: launches of their own (round 5) */
-void omni_debug_bb_min_rows(int rows);                     /* backbone chain: smallest batch the 64-row stage set takes (33 since round 5; 49: round 4's policy, 33-48 rows launch per op) */
+void omni_debug_chain_tail(int on);                         /* 1 (default): the step's input assembly + layer 0's qkv as the tail of the predictor's all-pass launch; 0: launches of their own */
+void omni_debug_bb_min_rows(int rows);                     /* backbone chain: smallest batch the 64-row stage set takes (33; 49: 33-48 rows launch per op) */
 void omni_debug_moe_chain(int on);                         /* sparse-MoE layer: o_proj -> router | shared gate_up -> shared down + routing as one persistent launch (moe_chain.hip) */
 void omni_debug_pa_tail(int on);                           /* decode attention: the last, partial 128-token round as contiguous 32-token chunks per wave (0: interleaved groups) */
 void omni_debug_pa_merge(int inkernel);                    /* KV splits of a decode attention launch: 1 merged by their last arriver inside it (every workspace then opens with zeros), 0 by a merge launch, -1 (default) the first for a talker's own workspace, the second for a caller's */
-void omni_debug_bb_ar(int on);                             /* 0: tensor-parallel ranks keep the launch-per-op backbone with all-reduce launches (round 5) */
-void omni_debug_sample_wave(int on);                       /* row sampler: 1 = one wave per row (smp_pick_wave, round 6) where eligible, 0 = always the 4-wave sample_kernel */
+void omni_debug_bb_ar(int on);                             /* 0: tensor-parallel ranks keep the launch-per-op backbone with all-reduce launches */
+void omni_debug_sample_wave(int on);                       /* row sampler: 1 = one wave per row (smp_pick_wave) where eligible, 0 = always the 4-wave sample_kernel */
 void omni_debug_bb_engine(int on);                         /* backbone segment as the loader / consumer engine (bb_engine.hip) instead of the plain chain */
 void omni_debug_eng_stamps(void* buf);                     /* stage stamps of the engine's compute wave 0 */
 void omni_debug_bb_stamps(void* buf);                      /* as omni_debug_chain_stamps for the backbone segment launches */
-void omni_debug_gemm_defer(int on);                         /* launch path: 1 = rstd of the qkv / gate_up GEMMs applied in the epilogue (round 6 default, the chains' arithmetic), 0 = round 5's exact form */
+void omni_debug_gemm_defer(int on);                         /* launch path: 1 = rstd of the qkv / gate_up GEMMs applied in the epilogue (default, the chains' arithmetic), 0 = the exact form */
 void omni_debug_gemm_stage(int stage);                      /* leave every GEMM kernel after stage 1..4 (timing attribution only) */
 void omni_debug_small_splitq(int on);                       /* small attention: one wave per (row, q head)            */
 void omni_debug_small_tiny(int on);                         /* code-predictor attention: the (token, quarter) / readlane kernel */
 void omni_debug_prefill_mfma(int on);                       /* prefill attention on MFMA (off: per-token VALU path)   */
-void omni_debug_bb_head(int on);                            /* 1 (default): the talker's lm_head rides as the last stage of the last backbone launch; 0: its own launch (round 5) */
+void omni_debug_bb_head(int on);                            /* 1 (default): the talker's lm_head rides as the last stage of the last backbone launch; 0: its own launch */
 void omni_debug_extra_trivial(int n);                       /* append n no-op launches per layer phase                */
 int omni_debug_launch(int mode, int blocks, int threads, void* p0, void* p1, int arg, int reps, void* stream);
 int omni_debug_mix(int pattern, float* small, const void* big, size_t big_bytes, int reps, void* stream);

@@ -1,4 +1,4 @@
-"""Round 6: the code predictor's passes INSIDE the real decode step (W3: 28-layer backbone in front, sampling on, one hipGraph) against the
+"""The code predictor's passes INSIDE the real decode step (W3: 28-layer backbone in front, sampling on, one hipGraph) against the
 same passes with the predictor phase replayed alone (its 161 MB of weights warm in the Infinity Cache): wave 0 of every workgroup stamps
 the 100 MHz counter at 8 points of every stage of every pass (debug library, one stamp block per pass).  Prints per pass its span on the
 chip in both settings, and the per-stage medians of passes 2, 3, 8, 15 and of the pair kernel.
@@ -69,7 +69,7 @@ def run(g, reps=8):
     return out
 
 def spans(t):
-    """per pass: first stage entry (any workgroup) -> last flag of the sampler; pair kernel = block 0"""
+    """per pass: first stage entry (any workgroup) -> last store of the sampler; pair kernel = block 0"""
     res = {}
     for p in [0] + list(range(2, 16)):
         x = t[p]
@@ -100,7 +100,7 @@ for p in [0] + list(range(2, 16)):
     print(f"{'pair' if p == 0 else p:>4}   {vs:10.2f}                                {vc:10.2f}          {vs - vc:+6.2f}")
 print(f" sum   {tot_s:10.2f}                                {tot_c:10.2f}          {tot_s - tot_c:+6.2f}")
 if a.stages:
-    seg = ["W issue", "flag wait", "slabs->rstd", "x+MFMA", "barrier", "epilogue", "drain+flag"]
+    seg = ["W issue", "first look", "operands", "MFMA", "barrier", "epilogue", "-"]      # chain_flow.cuh: the look that found something, all operands there
     for label, tt in (("in-step", ts[-1]), ("alone", tc[-1])):
         for p in (0, 2, 3, 8, 15):
             t = tt[p]

@@ -119,6 +119,7 @@ __global__ __launch_bounds__(256) void attn_small_fused_kernel(const PAArgs a, i
             }
         }
         const bool ok = t0 + tg < cur;
+        if (!ok) vr.a = vr.b = (u32x4){0u, 0u, 0u, 0u};          // an earlier step's row, possibly NaN, which a weight of 0 does not mask
         float kf[16], vf[16];
         to_f32<KV>(kr, kf);
         to_f32<KV>(vr, vf);

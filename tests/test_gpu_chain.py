@@ -87,9 +87,9 @@ def test_all_pass_chain_at_the_edges_of_its_row_splits(B, top_p):
         assert torch.equal(x, y)
 
 
-@pytest.mark.parametrize("chain", [0, 2], ids=["launches", "chain"])
+@pytest.mark.parametrize("chain,fused_norm", [(0, None), (2, None), (0, False)], ids=["launches", "chain", "separate-norms"])
 @pytest.mark.parametrize("B", [5, 24, 40, 64])
-def test_a_row_of_nans_leaves_nothing_behind(B, chain):
+def test_a_row_of_nans_leaves_nothing_behind(B, chain, fused_norm):
     """One row's input is NaN for one call.  What the private K / V cache keeps of it lies past the position of every later pass that has not written
     there again yet: the row's next call, with finite inputs, gives what it gave before."""
     d = get_dims("tts-1.7b").with_(layers=1, max_model_len=256)
@@ -101,7 +101,7 @@ def test_a_row_of_nans_leaves_nothing_behind(B, chain):
         lib.omni_debug_cp_chain.argtypes = [C.c_int]; lib.omni_debug_cp_chain.restype = None
         try:
             lib.omni_debug_cp_chain(chain)
-            eng = _engine(d, w, kv_dtype="bf16", num_blocks=8, max_batch=64)
+            eng = _engine(d, w, kv_dtype="bf16", num_blocks=8, max_batch=64, fused_norm=fused_norm)
             outs = [eng.code_predictor(code0.to(torch.int32), e0, x, greedy=True, return_logits=True) for x in (lh, bad, lh)]
             assert eng.chain_error() == 0
             assert eng.chains_ran() == (1 if chain else 0)

@@ -493,6 +493,16 @@ __device__ __forceinline__ void pa_decode_body(const PAArgs& a, float* lds, cons
         }                                                                                            \
     }
 
+    // ---- batch 0 went out without a limit: its rows past the history are what an earlier request left there, possibly NaN, which a weight of 0 does not
+    // mask (the other batches re-read the history's last row).  Contexts of less than a round only: one branch for the others
+    if ((spec || pre != nullptr) && n_hist < ROUND) {
+#pragma unroll
+        for (int u = 0; u < U; ++u)
+            if (t_begin + wave * 8 + u * (PA_WAVES * 8) + tg >= t_end) {
+                v0[u].a = v0[u].b = (u32x4){0u, 0u, 0u, 0u};
+                vs0[u] = 0.f;
+            }
+    }
     // ---- main loop, loads one batch ahead
     for (int b = 0; b < nb;) {
         if (b + 1 < nb) { PA_LOAD(k1, v1, ks1, vs1, b_t0(b + 1), b_str(b + 1)) }

@@ -509,6 +509,50 @@ def test_attn_decode_fused(ops, kv, hq, hkv, split):
         torch.testing.assert_close(sc.cpu(), pk.scales, rtol=1e-2, atol=0)
 
 
+@pytest.mark.parametrize("kv", ["bf16", "fp16", "fp8", "int8"])
+@pytest.mark.parametrize("hq,hkv", [(16, 8), (4, 1)])
+@pytest.mark.parametrize("max_len", [64, 512])
+def test_rows_past_the_context_may_hold_nans(ops, kv, hq, hkv, max_len):
+    """Blocks keep what an earlier request left in them: NaN in every row that is no row's history, in the table's unused blocks too, changes no bit."""
+    from ht_vllm_omni_amd import _lib as L
+    D, bs, nb = 128, 16, 96
+    g = torch.Generator().manual_seed(hq + len(kv) + max_len)
+    seq_lens = [n for n in (1, 2, 15, 16, 17, 33, 64, 100, 129, 400) if n <= max_len]
+    B = len(seq_lens)
+    perm, bt, ptr = torch.randperm(nb - 1, generator=g) + 1, torch.zeros(B, 32, dtype=torch.int32), 0
+    for r, n in enumerate(seq_lens):                    # disjoint blocks (this op WRITES the new token), one more than the context needs
+        need = (n + bs - 1) // bs + 1
+        bt[r, :need] = perm[ptr:ptr + need]
+        ptr += need
+    stale = torch.ones(nb * bs, dtype=torch.bool)
+    for r, n in enumerate(seq_lens):
+        t = torch.arange(n - 1)
+        stale[bt[r].long()[t // bs] * bs + t % bs] = False
+    shape, dt = (2, nb, bs, hkv, D), {"bf16": BF16, "fp16": torch.float16, "fp8": torch.float8_e4m3fn, "int8": torch.int8}[kv]
+    clean = (torch.randn(shape, generator=g) * (20 if kv == "int8" else 1)).to(dt)
+    sc = torch.rand(2, nb, bs, hkv, generator=g) * 0.02
+    q = _rand(g, B, hq * D).cuda()
+    qkv = _rand(g, B, (hq + 2 * hkv) * D, scale=2.0).cuda()
+    w = torch.ones(D, dtype=BF16).cuda()
+    cos_sin, sl = ops.rope_table(512, D, 1e6).cuda(), torch.tensor(seq_lens, dtype=torch.int32).cuda()
+    res = {}
+    for what in ("clean", "stale"):
+        c, s2 = clean.clone(), sc.clone()
+        if what == "stale" and kv == "int8":
+            s2.view(2, nb * bs, hkv)[:, stale] = float("nan")
+        elif what == "stale":
+            c.view(2, nb * bs, hkv, D).view(torch.uint8 if kv == "fp8" else torch.int16)[:, stale] = {"bf16": 0x7fc0, "fp16": 0x7e00, "fp8": 0x7f}[kv]
+        c, s2 = (c.view(torch.uint8) if kv == "fp8" else c).cuda(), s2.cuda()
+        kw = dict(q_heads=hq, kv_heads=hkv, head_dim=D, block_size=bs, kv_dtype=L.KV_CODES[kv], k_scales=s2[0] if kv == "int8" else None,
+                  v_scales=s2[1] if kv == "int8" else None, max_seq_len=max_len)
+        fused, _ = ops.attn_decode_fused(qkv, w, w, sl - 1, cos_sin, c[0], c[1], bt.cuda(), sl, eps=1e-6, split=False, **kw)
+        # behind the fused call: the new tokens' rows are written now
+        plain = ops.paged_attn_decode(q, c[0], c[1], bt.cuda(), sl, split=False, **kw)
+        res[what] = (fused.cpu(), plain.cpu())
+    for x, y in zip(res["stale"], res["clean"]):
+        assert y.isfinite().all() and torch.equal(x, y)
+
+
 @pytest.mark.parametrize("hq,hkv", [(4, 2), (16, 8), (2, 2), (16, 2)])
 def test_attn_decode_fused_short_context(ops, hq, hkv):
     """Code-predictor geometry: block = one request's 17 positions, contexts 1..17 (one-wave kernel)."""

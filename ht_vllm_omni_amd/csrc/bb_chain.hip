@@ -302,6 +302,7 @@ OMNI_KNOB g_bb_chain = 1, g_bb_min_rows = 33, g_bb_b32 = 1, g_bb_ar = 1;
 static unsigned long long* g_bb_stamps = nullptr;
 extern "C" void omni_debug_bb_chain(int on) { g_bb_chain = on; }
 extern "C" void omni_debug_bb_stamps(void* buf) { g_bb_stamps = (unsigned long long*)buf; }
+extern "C" void omni_debug_bb_deep(int) {}                                  // the arms that it chose timed a launch that is gone
 extern "C" void omni_debug_bb_ar(int on) { g_bb_ar = on; }                  // 0: tensor-parallel ranks keep the launch-per-op backbone
 extern "C" void omni_debug_bb_min_rows(int rows) { g_bb_min_rows = rows; g_bb_b32 = rows <= 49; }      // smallest batch of the 64-row split
 #endif

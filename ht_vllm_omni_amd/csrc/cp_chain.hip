@@ -811,8 +811,8 @@ __global__ __launch_bounds__(CH_THREADS) void cp_chain_kernel(const ChainArgs a)
 // ---- host
 OMNI_KNOB g_cp_chain = 1, g_chain_split48 = 0, g_chain_span = 2, g_chain_pair = 1;
 #ifdef OMNI_DEBUG_HOOKS
-// above 48 rows too the 48-row split of the stages (16-row gate_up tiles)
-extern "C" void omni_debug_chain_split48(int on) { g_chain_split48 = on; }
+// wide 0: above 48 rows too the 48-row split of the stages (16-row gate_up tiles); the other two were the flag domain and the poll pause
+extern "C" void omni_debug_chain_mode(int, int wide, int) { g_chain_split48 = wide == 0; }
 extern "C" void omni_debug_chain_pair(int on) { g_chain_pair = on; }            // positions 0 / 1 + group 1 as a persistent launch (0: the launch path's pair pass)
 static unsigned long long* g_chain_stamps = nullptr;
 // 0: launch per op; 1: one persistent launch per pass (layer stack only); 2: one persistent launch for all passes incl. heads + samplers

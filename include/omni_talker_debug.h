@@ -13,7 +13,8 @@ void omni_debug_tile(int nt, int mt);                       /* force the GEMM ti
 void omni_debug_int8_max_g(int g);                         /* int8-KV decode attention: q heads per workgroup (2 | 4) */
 void omni_debug_cp_pair01(int on);                         /* code predictor: positions 0 and 1 as one two-block pass */
 void omni_debug_cp_chain(int on);                          /* code predictor: the layer stack of a pass as one persistent launch */
-void omni_debug_chain_split48(int on);                      /* predictor chain: above 48 rows too the 48-row split of its stages */
+void omni_debug_chain_mode(int, int wide, int);            /* predictor chain: wide 0 = above 48 rows too the 48-row split of its stages (the other arguments have nothing left to set) */
+void omni_debug_bb_deep(int mode);                         /* nothing left to choose (ring depths and cache policy of a launch that is gone): no effect */
 void omni_debug_chain_stamps(void* buf);                   /* device uint64 [16 passes][40][8][256]: per-stage timeline stamps of every chain launch, one block per predictor pass, block 0 = the pair kernel (NULL: off) */
 void omni_debug_bb_chain(int on);                          /* backbone: o_proj -> gate_up -> down_proj -> next qkv as one persistent launch per layer */
 void omni_debug_bb_all(int on);                            /* backbone: the whole decoder stack, attention included, as ONE persistent launch (bb_all.hip) */

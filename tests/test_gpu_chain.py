@@ -39,11 +39,11 @@ def test_chain_is_bit_identical_to_the_launch_chain(model, B, span, split48):
     res = {}
     with L.debug_library() as lib:
         lib.omni_debug_cp_chain.argtypes = [C.c_int]; lib.omni_debug_cp_chain.restype = None
-        lib.omni_debug_chain_split48.argtypes = [C.c_int]; lib.omni_debug_chain_split48.restype = None
+        lib.omni_debug_chain_mode.argtypes = [C.c_int, C.c_int, C.c_int]; lib.omni_debug_chain_mode.restype = None
         try:
             for on in (0, 1):
                 lib.omni_debug_cp_chain(span if on else 0)
-                lib.omni_debug_chain_split48(split48)
+                lib.omni_debug_chain_mode(0, int(not split48), 0)
                 eng = _engine(d, w, kv_dtype="bf16", num_blocks=8, max_batch=64)
                 for rep in range(3):                                 # flags and hand-off buffers carry over from call to call
                     codes, lg = eng.code_predictor(code0.to(torch.int32).cuda(), e0.cuda(), lh.cuda(), greedy=True, return_logits=True)
@@ -54,7 +54,7 @@ def test_chain_is_bit_identical_to_the_launch_chain(model, B, span, split48):
                 res[on] = (codes.cpu(), lg.cpu(), sampled.cpu())
         finally:
             lib.omni_debug_cp_chain(2)
-            lib.omni_debug_chain_split48(0)
+            lib.omni_debug_chain_mode(0, 1, 0)
     bad = (res[1][0] != res[0][0]).any(dim=1).nonzero().flatten().tolist()
     assert torch.equal(res[1][0], res[0][0]), f"greedy codes differ between the persistent chain and the launch chain in rows {bad}: first differing group per row {[int((res[1][0][b] != res[0][0][b]).nonzero()[0]) for b in bad]}"
     assert torch.equal(res[1][1], res[0][1]), "logits differ between the persistent chain and the launch chain"
